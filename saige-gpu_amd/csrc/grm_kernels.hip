@@ -325,10 +325,6 @@ __device__ __forceinline__ void store_tile256(float* S, int64_t ldS, int64_t bi,
     }
 }
 
-// wait for this wave's LDS traffic, then the workgroup barrier; outstanding
-// global loads (the next chunk's bytes and tables) stay in flight
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Double-buffered: while the MFMAs run on chunk k from one LDS buffer, the
 // same waves decode chunk k+1 into the other, so the matrix pipe and the
 // VALU decode overlap (one workgroup per CU); one LDS-only barrier per chunk.
@@ -565,7 +561,7 @@ __global__ __launch_bounds__(512) void k_syrk_pk256_split(const uint8_t* __restr
 // Re-tile the packed genotypes for k_syrk_pk: block (p, c) byte (b, m) =
 // byte 32p + b of QC'd marker 64c + m, with padding codes 0b01.
 __global__ __launch_bounds__(256) void k_pack_tiles(const uint8_t* __restrict__ packed, int64_t Mqc, int64_t Nnm,
-                                                    int64_t bpm_nm, int64_t nchunk, uint8_t* __restrict__ tp) {
+                                                    int64_t ldp, int64_t nchunk, uint8_t* __restrict__ tp) {
     const int64_t p = blockIdx.x, c = blockIdx.y;
     uint8_t* blk = tp + (p * nchunk + c) * 2048;
     for (int i = threadIdx.x; i < 2048; i += 256) {
@@ -574,8 +570,8 @@ __global__ __launch_bounds__(256) void k_pack_tiles(const uint8_t* __restrict__ 
         const int64_t byte_idx = p * 32 + b;
         const int64_t s0 = byte_idx * 4;
         unsigned v = 0x55u;
-        if (j < Mqc && byte_idx < bpm_nm) {
-            v = packed[j * bpm_nm + byte_idx];
+        if (j < Mqc && s0 < Nnm) {
+            v = packed[j * ldp + byte_idx];
 #pragma unroll
             for (int q = 0; q < 4; q++)
                 if (s0 + q >= Nnm) v = (v & ~(3u << (2 * q))) | (1u << (2 * q));
@@ -707,10 +703,10 @@ int syrk_kchunk_f32() { return BK32; }
 int syrk_kchunk_bf16() { return BK16; }
 
 hipError_t launch_pack_tiles(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t Mqc, int64_t Nnm,
-                             int64_t Npad, int64_t bpm_nm, uint8_t* tp, uint64_t* lut64) {
+                             int64_t Npad, int64_t ldp, uint8_t* tp, uint64_t* lut64) {
     const int64_t nchunk = (Mqc + 63) / 64;
     hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)(Npad / BT), (unsigned)nchunk), dim3(256), 0, s, packed, Mqc,
-                       Nnm, bpm_nm, nchunk, tp);
+                       Nnm, ldp, nchunk, tp);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_lut64, dim3((unsigned)((nchunk * 64 + 255) / 256)), dim3(256), 0, s, lut, (int64_t)0, Mqc,

@@ -33,10 +33,6 @@ __device__ __forceinline__ float wave_sum_f(float v) {
     return v;
 }
 
-// wait for this wave's LDS traffic, then the workgroup barrier; outstanding
-// global loads stay in flight
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Sigma p for one element (getCrossprod, FG.cpp:2412): the reference forms
 // 1/w, then b % (1/w), then tau0 * that, plus tau1 * (K b); tau1 == 0
 // returns the first term alone (FG.cpp:2401-2404).

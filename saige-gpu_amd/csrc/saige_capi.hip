@@ -154,7 +154,7 @@ void free_geno(saige_ctx* c) {
     c->loco_start = c->loco_end = -1;
     c->loco_chrom = -1;
     c->loco_m = 0;
-    c->N = c->M = c->Nnm = c->Npad = c->Mqc = c->Mvr = c->bpm_nm = 0;
+    c->N = c->M = c->Nnm = c->Npad = c->Mqc = c->Mvr = c->ldp = 0;
 }
 
 int64_t count_lines(const char* path, int* err) {
@@ -616,7 +616,7 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
     c->M = M;
     c->Nnm = n_sub;
     c->Npad = round_up(n_sub, NPAD_ALIGN);
-    c->bpm_nm = (n_sub + 3) / 4;
+    c->ldp = round_up((n_sub + 3) / 4, PACKED_ALIGN);
     c->diag_one = diag_one;
     const int64_t bpm = (N + 3) / 4;
 
@@ -689,8 +689,8 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
         c->Mqc = (int64_t)c->qc_index.size();
         c->Mvr = (int64_t)c->vr_index.size();
         const int64_t nl = std::max<int64_t>(c->Mqc, c->Mvr);
-        if (dalloc(&d_list, nl) || dalloc(&c->d_packed, c->Mqc * c->bpm_nm) ||
-            dalloc(&c->d_packed_vr, c->Mvr * c->bpm_nm) || dalloc(&c->d_lut, c->Mqc) ||
+        if (dalloc(&d_list, nl) || dalloc(&c->d_packed, (c->Mqc + PACKED_PAD_ROWS) * c->ldp) ||
+            dalloc(&c->d_packed_vr, c->Mvr * c->ldp) || dalloc(&c->d_lut, c->Mqc + PACKED_PAD_ROWS) ||
             dalloc(&c->d_lut_vr, c->Mvr) || dalloc(&c->d_diag, c->Npad) || dalloc(&c->d_vec, 4 * c->Npad)) {
             set_error("device allocation failed (packed genotypes)");
             rc = SAIGE_E_NOMEM;
@@ -701,19 +701,19 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
             e = hipMemcpyAsync(d_list, c->qc_index.data(), 4 * c->Mqc, hipMemcpyHostToDevice, st);
         if (e == hipSuccess)
             e = launch_repack(st, d_bed, bpm, d_list, c->Mqc, c->d_stats, identity ? nullptr : d_sub, n_sub,
-                              c->bpm_nm, c->d_packed);
+                              c->ldp, c->d_packed);
         if (e == hipSuccess) e = launch_lut(st, d_list, c->Mqc, c->d_stats, c->d_lut);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e == hipSuccess && c->Mvr > 0) {
             e = hipMemcpyAsync(d_list, c->vr_index.data(), 4 * c->Mvr, hipMemcpyHostToDevice, st);
             if (e == hipSuccess)
                 e = launch_repack(st, d_bed, bpm, d_list, c->Mvr, c->d_stats, identity ? nullptr : d_sub,
-                                  n_sub, c->bpm_nm, c->d_packed_vr);
+                                  n_sub, c->ldp, c->d_packed_vr);
             if (e == hipSuccess) e = launch_lut(st, d_list, c->Mvr, c->d_stats, c->d_lut_vr);
         }
         // diag(Z Z^T) in FP32 marker order (Get_Diagof_StdGeno, FG.cpp:665-704)
         if (e == hipSuccess && c->Mqc > 0)
-            e = launch_diag_std(st, c->d_packed, c->d_lut, c->Mqc, n_sub, c->bpm_nm, c->d_diag);
+            e = launch_diag_std(st, c->d_packed, c->d_lut, c->Mqc, n_sub, c->ldp, c->d_diag);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess) {
             set_error("repack failed: %s", hipGetErrorString(e));
@@ -1004,7 +1004,7 @@ static int get_geno_impl(saige_ctx* c, const uint8_t* packed, int64_t n, int64_t
         return SAIGE_E_ARG;
     }
     int32_t* d = reinterpret_cast<int32_t*>(c->d_vec);
-    SAIGE_HIP_TRY(launch_get_geno(c->stream, packed + idx * c->bpm_nm, c->Nnm, d));
+    SAIGE_HIP_TRY(launch_get_geno(c->stream, packed + idx * c->ldp, c->Nnm, d));
     SAIGE_HIP_TRY(hipMemcpyAsync(out, d, 4 * c->Nnm, hipMemcpyDeviceToHost, c->stream));
     SAIGE_HIP_TRY(hipStreamSynchronize(c->stream));
     return SAIGE_OK;
@@ -1029,7 +1029,7 @@ int saige_get_one_snp_std_geno(saige_ctx* c, int64_t idx, float* out) {
         set_error("marker index %lld out of range", (long long)idx);
         return SAIGE_E_ARG;
     }
-    SAIGE_HIP_TRY(launch_std_geno(c->stream, c->d_packed + idx * c->bpm_nm, c->d_lut + idx, c->Nnm, c->d_vec));
+    SAIGE_HIP_TRY(launch_std_geno(c->stream, c->d_packed + idx * c->ldp, c->d_lut + idx, c->Nnm, c->d_vec));
     SAIGE_HIP_TRY(hipMemcpyAsync(out, c->d_vec, 4 * c->Nnm, hipMemcpyDeviceToHost, c->stream));
     SAIGE_HIP_TRY(hipStreamSynchronize(c->stream));
     return SAIGE_OK;
@@ -1112,7 +1112,7 @@ int saige_build_grm(saige_ctx* c, int precision) {
         }
         hipError_t e = hipMemcpyAsync(d_tiles, order.data(), sizeof(int2) * order.size(), hipMemcpyHostToDevice, st);
         if (e == hipSuccess) e = hipEventRecord(c->ev0, st);
-        if (e == hipSuccess) e = launch_pack_tiles(st, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->bpm_nm, d_tp, d_l64);
+        if (e == hipSuccess) e = launch_pack_tiles(st, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, d_tp, d_l64);
         if (e == hipSuccess && split) e = launch_lut64_range(st, c->d_lut, c->Mqc, 0, c->Mqc, 1, d_llo);
         if (e == hipSuccess)
             e = syrk_pk_passes(st, d_tp, d_l64, d_llo, c->Mqc, Np, d_tiles, c->d_grm, 0, 0, -1, tile);
@@ -1165,13 +1165,13 @@ int saige_build_grm(saige_ctx* c, int precision) {
         const int64_t np = std::min(pw, c->Mqc - j0);
         const int64_t ldz = round_up(np, 64);
         if (bf16) {
-            e = launch_std_panel_bf16(st, c->d_packed, c->d_lut, j0, np, c->Nnm, Np, c->bpm_nm, ldz,
+            e = launch_std_panel_bf16(st, c->d_packed, c->d_lut, j0, np, c->Nnm, Np, c->ldp, ldz,
                                       static_cast<__hip_bfloat16*>(d_panel));
             if (e == hipSuccess)
                 e = launch_syrk_bf16(st, static_cast<__hip_bfloat16*>(d_panel), Np, ldz, ldz, d_tiles, c->d_grm,
                                      !first);
         } else {
-            e = launch_std_panel_f32(st, c->d_packed, c->d_lut, j0, np, c->Nnm, Np, c->bpm_nm, ldz,
+            e = launch_std_panel_f32(st, c->d_packed, c->d_lut, j0, np, c->Nnm, Np, c->ldp, ldz,
                                      static_cast<float*>(d_panel));
             if (e == hipSuccess)
                 e = launch_syrk_f32(st, static_cast<float*>(d_panel), Np, ldz, ldz, d_tiles, c->d_grm, !first);
@@ -1477,7 +1477,7 @@ hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, int ac
         e = dalloc(&d_tp, (Np / syrk_tile()) * nchunk * 2048);
         if (e == hipSuccess) e = dalloc(&d_l64, nchunk * 64);
         if (e == hipSuccess && split) e = dalloc(&d_llo, nchunk * 64);
-        if (e == hipSuccess) e = launch_pack_tiles(st, c->d_packed, c->d_lut, c->Mqc, N, Np, c->bpm_nm, d_tp, d_l64);
+        if (e == hipSuccess) e = launch_pack_tiles(st, c->d_packed, c->d_lut, c->Mqc, N, Np, c->ldp, d_tp, d_l64);
         if (e == hipSuccess) e = launch_lut64_range(st, c->d_lut, c->Mqc, start, end + 1, 0, d_l64);
         if (e == hipSuccess && split) e = launch_lut64_range(st, c->d_lut, c->Mqc, start, end + 1, 1, d_llo);
         if (e == hipSuccess)
@@ -1497,13 +1497,13 @@ hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, int ac
             const int64_t np = std::min(pw, end + 1 - j0);
             const int64_t ldz = round_up(np, 64);
             if (bf16) {
-                e = launch_std_panel_bf16(st, c->d_packed, c->d_lut, j0, np, N, Np, c->bpm_nm, ldz,
+                e = launch_std_panel_bf16(st, c->d_packed, c->d_lut, j0, np, N, Np, c->ldp, ldz,
                                           static_cast<__hip_bfloat16*>(d_panel));
                 if (e == hipSuccess)
                     e = launch_syrk_bf16(st, static_cast<__hip_bfloat16*>(d_panel), Np, ldz, ldz, d_tiles, S,
                                          accumulate);
             } else {
-                e = launch_std_panel_f32(st, c->d_packed, c->d_lut, j0, np, N, Np, c->bpm_nm, ldz,
+                e = launch_std_panel_f32(st, c->d_packed, c->d_lut, j0, np, N, Np, c->ldp, ldz,
                                          static_cast<float*>(d_panel));
                 if (e == hipSuccess)
                     e = launch_syrk_f32(st, static_cast<float*>(d_panel), Np, ldz, ldz, d_tiles, S, accumulate);
@@ -1599,7 +1599,7 @@ int saige_set_start_end_index(saige_ctx* c, int64_t start, int64_t end, int chro
     // marker order (set_Diagof_StdGeno_LOCO, FG.cpp:4947-4955)
     if (e == hipSuccess) e = launch_fill_zero(st, d_rdiag, 4 * Np);
     if (e == hipSuccess)
-        e = launch_diag_std(st, c->d_packed + start * c->bpm_nm, c->d_lut + start, cnt, N, c->bpm_nm, d_rdiag);
+        e = launch_diag_std(st, c->d_packed + start * c->ldp, c->d_lut + start, cnt, N, c->ldp, d_rdiag);
     if (e == hipSuccess) e = launch_sub(st, c->d_diag, d_rdiag, Np, c->d_diag_loco);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     dfree(d_rdiag);

@@ -45,6 +45,13 @@ struct DecodeParams {
 constexpr int EW = 64;
 // Row padding of all N-length device arrays and of the GRM.
 constexpr int64_t NPAD_ALIGN = 256;
+// Row stride alignment (bytes) of the packed genotypes: a marker's 128-byte
+// segments (512 samples) are whole cache lines, whatever the sample count.
+constexpr int64_t PACKED_ALIGN = 128;
+// Rows allocated behind the GRM markers' packed genotypes and their lookup
+// table (contents unused), so that a kernel may load whole tiles of up to 128
+// markers from any first marker.
+constexpr int64_t PACKED_PAD_ROWS = 128;
 
 // Block-GEMM shape: rt = 32-row tiles per wave (1 or 2), pd = 32-column
 // chunks of S requested ahead (1 or 3), nsplit = column slices of S (1, 2, 4
@@ -180,15 +187,16 @@ struct saige_ctx {
     std::vector<int32_t> vr_rand;
     int diag_one = 0;
     // sizes
-    int64_t N = 0, M = 0, Nnm = 0, Npad = 0, Mqc = 0, Mvr = 0, bpm_nm = 0;
+    int64_t N = 0, M = 0, Nnm = 0, Npad = 0, Mqc = 0, Mvr = 0;
+    int64_t ldp = 0;                             // packed genotypes' row stride in bytes
     bool loaded = false;
     // decode outputs
     saige::MarkerStat* d_stats = nullptr;        // [M]
     std::vector<saige::MarkerStat> h_stats;      // [M]
     std::vector<int32_t> qc_index, vr_index;     // original marker index of QC'd / VR markers
-    uint8_t* d_packed = nullptr;                 // [Mqc][bpm_nm] internal code
-    uint8_t* d_packed_vr = nullptr;              // [Mvr][bpm_nm]
-    float4* d_lut = nullptr;                     // [Mqc] (L0, L1, L2, 0)
+    uint8_t* d_packed = nullptr;                 // [Mqc + PACKED_PAD_ROWS][ldp] internal code
+    uint8_t* d_packed_vr = nullptr;              // [Mvr][ldp]
+    float4* d_lut = nullptr;                     // [Mqc + PACKED_PAD_ROWS] (L0, L1, L2, 0)
     float4* d_lut_vr = nullptr;
     float* d_diag = nullptr;                     // [Npad] sum z^2
     // GRM S = Z Z^T, [Npad][Npad] FP32
@@ -256,6 +264,10 @@ inline int64_t round_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 __device__ __forceinline__ float div_rn(float a, float b) { return (float)((double)a / (double)b); }
 __device__ __forceinline__ float sqrt_rn(float a) { return (float)__builtin_sqrt((double)a); }
 
+// wait for this wave's LDS traffic, then the workgroup barrier; outstanding
+// global loads stay in flight (__syncthreads would drain them)
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // ---- genotype kernels (geno_kernels.hip)
 // imask: NULL when every .fam sample is phenotyped, else 16 copies (stride
 // ld, a multiple of 16) of the rows' 2-bit code mask, copy r shifted by r
@@ -264,11 +276,12 @@ hipError_t launch_decode_stats(hipStream_t s, const uint8_t* bed, const uint8_t*
                                const uint8_t* randset, DecodeParams p, MarkerStat* stats);
 hipError_t launch_repack(hipStream_t s, const uint8_t* bed, int64_t bpm, const int32_t* markers,
                          int64_t nmark, const MarkerStat* stats, const int32_t* subidx,
-                         int64_t Nnm, int64_t bpm_nm, uint8_t* out);
+                         int64_t Nnm, int64_t ldp, uint8_t* out);
 hipError_t launch_lut(hipStream_t s, const int32_t* markers, int64_t nmark,
                       const MarkerStat* stats, float4* lut);
+// packed and lut: readable for up to PACKED_PAD_ROWS - 1 rows past Mqc
 hipError_t launch_diag_std(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t Mqc,
-                           int64_t Nnm, int64_t bpm_nm, float* diag);
+                           int64_t Nnm, int64_t ldp, float* diag);
 hipError_t launch_get_geno(hipStream_t s, const uint8_t* packed_row, int64_t Nnm, int32_t* out);
 hipError_t launch_std_geno(hipStream_t s, const uint8_t* packed_row, const float4* lut_row,
                            int64_t Nnm, float* out);
@@ -277,10 +290,10 @@ hipError_t launch_synth_bed(hipStream_t s, uint8_t* bed, int64_t N, int64_t M, f
 // Z panel [Npad][ldz] for markers [j0, j0+np) (np <= ldz; columns beyond np
 // and rows beyond Nnm are zero).  Element type float or bf16.
 hipError_t launch_std_panel_f32(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t j0,
-                                int64_t np, int64_t Nnm, int64_t Npad, int64_t bpm_nm, int64_t ldz,
+                                int64_t np, int64_t Nnm, int64_t Npad, int64_t ldp, int64_t ldz,
                                 float* Zp);
 hipError_t launch_std_panel_bf16(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t j0,
-                                 int64_t np, int64_t Nnm, int64_t Npad, int64_t bpm_nm, int64_t ldz,
+                                 int64_t np, int64_t Nnm, int64_t Npad, int64_t ldp, int64_t ldz,
                                  __hip_bfloat16* Zp);
 
 // ---- GRM kernels (grm_kernels.hip)
@@ -295,7 +308,7 @@ std::vector<int2> syrk_tile_order(int64_t nt, int64_t g);
 // 2-bit-input SYRK: tp = tiled packed genotypes ((Npad/128) x nchunk x 2 KB,
 // nchunk = ceil(Mqc/64)), lut64 = nchunk*64 entries; both from launch_pack_tiles
 hipError_t launch_pack_tiles(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t Mqc, int64_t Nnm,
-                             int64_t Npad, int64_t bpm_nm, uint8_t* tp, uint64_t* lut64);
+                             int64_t Npad, int64_t ldp, uint8_t* tp, uint64_t* lut64);
 // markers [j0, j1) only (j1 < 0: all); lut64 must be zero outside the range.
 // accumulate: 0 overwrite, 1 add, -1 subtract.
 // tile: 128 or 256 (tiles from syrk_tile_order(Npad / tile, ...)).
