@@ -134,10 +134,14 @@ void free_parked(saige_ctx* c) {
     c->parked.clear();
 }
 
-void free_geno(saige_ctx* c) {
+// Everything that belongs to the cohort, except the ingest's kept blocks.
+void clear_geno(saige_ctx* c) {
     free_parked(c);
-    dfree(c->d_stats); dfree(c->d_packed); dfree(c->d_packed_vr); dfree(c->d_lut); dfree(c->d_lut_vr);
-    dfree(c->d_diag); dfree(c->d_grm); dfree(c->d_vec); dfree(c->d_grm_loco); dfree(c->d_diag_loco);
+    c->d_stats = nullptr;
+    c->d_packed = c->d_packed_vr = nullptr;
+    c->d_lut = c->d_lut_vr = nullptr;
+    c->d_diag = c->d_vec = nullptr;
+    dfree(c->d_grm); dfree(c->d_grm_loco); dfree(c->d_diag_loco);
     dfree(c->d_mv_in); dfree(c->d_mv_blk); dfree(c->d_mv_out); dfree(c->d_mv_ypart);
     dfree(c->d_dots_partial); dfree(c->d_dots_out);
     tri_plan_free(c->tri);
@@ -155,6 +159,13 @@ void free_geno(saige_ctx* c) {
     c->loco_chrom = -1;
     c->loco_m = 0;
     c->N = c->M = c->Nnm = c->Npad = c->Mqc = c->Mvr = c->ldp = 0;
+}
+
+void free_geno(saige_ctx* c) {
+    clear_geno(c);
+    for (KeptBlock* b : {&c->kb_stats, &c->kb_packed, &c->kb_packed_vr, &c->kb_lut, &c->kb_lut_vr, &c->kb_vec,
+                         &c->kb_lists})
+        b->release();
 }
 
 int64_t count_lines(const char* path, int* err) {
@@ -610,7 +621,7 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
         }
         if (subidx[i] != i + 1) identity = false;
     }
-    free_geno(c);
+    clear_geno(c);
     hipStream_t st = c->stream;
     c->N = N;
     c->M = M;
@@ -643,17 +654,21 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
         for (int64_t r = 0; r < 16; r++) std::memcpy(imask.data() + r * ldm + r, mb.data(), bpm);
     }
 
-    uint8_t *d_ind = nullptr, *d_rset = nullptr;
-    int32_t *d_sub = nullptr, *d_list = nullptr;
-    auto cleanup = [&]() { dfree(d_ind); dfree(d_rset); dfree(d_sub); dfree(d_list); };
+    // setgeno's lists in one block: the mask copies, the VR pool's flags, the
+    // sample list and the marker list, each at a multiple of 256 bytes
+    const int64_t o_rset = round_up(all_in ? 0 : 16 * ldm, 256), o_sub = o_rset + round_up(M, 256),
+                  o_list = o_sub + round_up(4 * n_sub, 256);
     int rc = SAIGE_OK;
     do {
-        if (dalloc(&d_ind, all_in ? 16 : 16 * ldm) || dalloc(&d_rset, M) || dalloc(&d_sub, n_sub) ||
-            dalloc(&c->d_stats, M)) {
+        if (c->kb_lists.reserve(o_list + 4 * M) || c->kb_stats.reserve((int64_t)sizeof(MarkerStat) * M)) {
             set_error("device allocation failed (setgeno)");
             rc = SAIGE_E_NOMEM;
             break;
         }
+        uint8_t* const base = static_cast<uint8_t*>(c->kb_lists.p);
+        uint8_t *d_ind = base, *d_rset = base + o_rset;
+        int32_t *d_sub = reinterpret_cast<int32_t*>(base + o_sub), *d_list = reinterpret_cast<int32_t*>(base + o_list);
+        c->d_stats = static_cast<MarkerStat*>(c->kb_stats.p);
         if ((!all_in && hipMemcpyAsync(d_ind, imask.data(), 16 * ldm, hipMemcpyHostToDevice, st)) ||
             hipMemcpyAsync(d_rset, rset.data(), M, hipMemcpyHostToDevice, st) ||
             hipMemcpyAsync(d_sub, subidx, 4 * n_sub, hipMemcpyHostToDevice, st)) {
@@ -688,14 +703,20 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
         }
         c->Mqc = (int64_t)c->qc_index.size();
         c->Mvr = (int64_t)c->vr_index.size();
-        const int64_t nl = std::max<int64_t>(c->Mqc, c->Mvr);
-        if (dalloc(&d_list, nl) || dalloc(&c->d_packed, (c->Mqc + PACKED_PAD_ROWS) * c->ldp) ||
-            dalloc(&c->d_packed_vr, c->Mvr * c->ldp) || dalloc(&c->d_lut, c->Mqc + PACKED_PAD_ROWS) ||
-            dalloc(&c->d_lut_vr, c->Mvr) || dalloc(&c->d_diag, c->Npad) || dalloc(&c->d_vec, 4 * c->Npad)) {
+        if (c->kb_packed.reserve((c->Mqc + PACKED_PAD_ROWS) * c->ldp) || c->kb_packed_vr.reserve(c->Mvr * c->ldp) ||
+            c->kb_lut.reserve((int64_t)sizeof(float4) * (c->Mqc + PACKED_PAD_ROWS)) ||
+            c->kb_lut_vr.reserve((int64_t)sizeof(float4) * c->Mvr) ||
+            c->kb_vec.reserve((int64_t)sizeof(float) * 5 * c->Npad)) {
             set_error("device allocation failed (packed genotypes)");
             rc = SAIGE_E_NOMEM;
             break;
         }
+        c->d_packed = static_cast<uint8_t*>(c->kb_packed.p);
+        c->d_packed_vr = static_cast<uint8_t*>(c->kb_packed_vr.p);
+        c->d_lut = static_cast<float4*>(c->kb_lut.p);
+        c->d_lut_vr = static_cast<float4*>(c->kb_lut_vr.p);
+        c->d_diag = static_cast<float*>(c->kb_vec.p);
+        c->d_vec = c->d_diag + c->Npad;
         e = launch_fill_zero(st, c->d_diag, 4 * c->Npad);
         if (e == hipSuccess && c->Mqc > 0)
             e = hipMemcpyAsync(d_list, c->qc_index.data(), 4 * c->Mqc, hipMemcpyHostToDevice, st);
@@ -721,7 +742,6 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
             break;
         }
     } while (0);
-    cleanup();
     if (rc != SAIGE_OK) {
         free_geno(c);
         return rc;

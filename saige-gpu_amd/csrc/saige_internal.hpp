@@ -173,6 +173,28 @@ struct Engine {
     int64_t gemm_launches[4] = {0, 0, 0, 0};
 };
 
+// A device block that outlives the cohort it was made for (a context reads
+// one after another): reserve() keeps the block when it is large enough and
+// not more than twice (plus 64 MB) too large, else replaces it.
+struct KeptBlock {
+    void* p = nullptr;
+    int64_t cap = 0;
+    hipError_t reserve(int64_t bytes) {
+        if (bytes < 16) bytes = 16;
+        if (p && cap >= bytes && cap <= 2 * bytes + ((int64_t)64 << 20)) return hipSuccess;
+        release();
+        const hipError_t e = hipMalloc(&p, (size_t)bytes);
+        if (e == hipSuccess) cap = bytes;
+        else p = nullptr;
+        return e;
+    }
+    void release() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        cap = 0;
+    }
+};
+
 }  // namespace saige
 
 struct saige_ctx {
@@ -190,6 +212,9 @@ struct saige_ctx {
     int64_t N = 0, M = 0, Nnm = 0, Npad = 0, Mqc = 0, Mvr = 0;
     int64_t ldp = 0;                             // packed genotypes' row stride in bytes
     bool loaded = false;
+    // the device blocks of an ingest, kept for the context's next cohort: the
+    // pointers below and setgeno's own lists point into them
+    saige::KeptBlock kb_stats, kb_packed, kb_packed_vr, kb_lut, kb_lut_vr, kb_vec, kb_lists;
     // decode outputs
     saige::MarkerStat* d_stats = nullptr;        // [M]
     std::vector<saige::MarkerStat> h_stats;      // [M]
