@@ -21,3 +21,35 @@ def test_diag_tile_edges(session, N, M):
     og = O.setgeno(body, N, M)
     assert session.getMsub_MAFge_minMAFtoConstructGRM() == og["Mqc"]
     assert np.array_equal(session.Get_Diagof_StdGeno().view(np.uint32), O.diag_std(og).view(np.uint32))
+
+
+def _same_genotypes(session, body, N, M, sub):
+    session.setminMAFforGRM(0.0)
+    session.setmaxMissingRateforGRM(1.0)
+    session.setminMAC_VarianceRatio(20, -1, False)
+    session.setgeno_bytes(body, N, M, sub)
+    og = O.setgeno(body, N, M, subidx=sub)
+    assert session.getMsub_MAFge_minMAFtoConstructGRM() == og["Mqc"] == M
+    n = len(sub)
+    for j in range(M):
+        assert np.array_equal(session.Get_OneSNP_Geno(j), O.get_geno(og["packed"][j], n)), j
+
+
+@pytest.mark.parametrize("N", [1, 4, 15, 16, 17, 63, 64, 65, 255, 257, 1030, 16390])
+def test_repack_in_order(session, N):
+    """One wave per marker, 16 output bytes (64 samples) per lane and step,
+    four steps (16,384 samples) at a time; rows of every alignment."""
+    print(f"case: repack in order N={N}", flush=True)
+    body, _, _ = random_bed(N, 9, 0.3, seed=N)
+    _same_genotypes(session, body, N, 9, np.arange(1, N + 1, dtype=np.int32))
+
+
+@pytest.mark.parametrize("N,n,M", [(5, 1, 1), (17, 16, 3), (64, 15, 4), (130, 129, 5), (1003, 1003, 6), (8201, 8190, 7),
+                                   (163840, 40, 3), (163841, 41, 3)])
+def test_repack_listed(session, N, n, M):
+    """Samples in an order of their own, four markers per workgroup; the last
+    case's rows are too long for LDS."""
+    print(f"case: repack listed N={N} n={n} M={M}", flush=True)
+    body, _, _ = random_bed(N, M, 0.3, seed=N + n)
+    sub = (np.random.default_rng(n).permutation(N)[:n] + 1).astype(np.int32)
+    _same_genotypes(session, body, N, M, sub)
