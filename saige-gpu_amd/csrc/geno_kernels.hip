@@ -172,18 +172,6 @@ __device__ __forceinline__ uint32_t impute_word(uint32_t w, uint32_t f0, uint32_
 __device__ __forceinline__ uint32_t fill_lo(int fill) { return fill == 0 ? 0xFFFFFFFFu : 0u; }
 __device__ __forceinline__ uint32_t fill_hi(int fill) { return fill <= 1 ? 0xFFFFFFFFu : 0u; }
 
-// rows a..d of four bytes -> their byte columns: t[k] = byte k of a, b, c, d
-__device__ __forceinline__ void transpose4x4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t (&t)[4]) {
-    const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u);   // a0 b0 a1 b1
-    const uint32_t ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u);   // a2 b2 a3 b3
-    const uint32_t cd0 = __builtin_amdgcn_perm(d, c, 0x05010400u);
-    const uint32_t cd1 = __builtin_amdgcn_perm(d, c, 0x07030602u);
-    t[0] = __builtin_amdgcn_perm(cd0, ab0, 0x05040100u);
-    t[1] = __builtin_amdgcn_perm(cd0, ab0, 0x07060302u);
-    t[2] = __builtin_amdgcn_perm(cd1, ab1, 0x05040100u);
-    t[3] = __builtin_amdgcn_perm(cd1, ab1, 0x07060302u);
-}
-
 // four bytes at any address (one unaligned dword load)
 __device__ __forceinline__ uint32_t load4(const uint8_t* p) {
     uint32_t v;
@@ -505,8 +493,6 @@ __global__ void k_std_geno(const uint8_t* __restrict__ row, const float4* __rest
 template <typename T>
 __device__ __forceinline__ T to_elem(float v);
 template <>
-__device__ __forceinline__ float to_elem<float>(float v) { return v; }
-template <>
 __device__ __forceinline__ __hip_bfloat16 to_elem<__hip_bfloat16>(float v) { return __float2bfloat16(v); }
 
 template <typename T>
@@ -675,15 +661,6 @@ hipError_t launch_synth_bed(hipStream_t s, uint8_t* bed, int64_t N, int64_t M, f
     const int64_t n = M * bpm;
     hipLaunchKernelGGL(k_synth_bed, dim3(grid_for((n + 255) / 256, 1 << 16)), dim3(256), 0, s, bed, N, M, bpm,
                        maf_lo, maf_hi, miss, npairs, seed);
-    return hipGetLastError();
-}
-
-hipError_t launch_std_panel_f32(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t j0,
-                                int64_t np, int64_t Nnm, int64_t Npad, int64_t ldp, int64_t ldz,
-                                float* Zp) {
-    dim3 grid((unsigned)(Npad / 128), (unsigned)((ldz + 63) / 64));
-    hipLaunchKernelGGL(k_std_panel<float>, grid, dim3(256), 0, s, packed, lut, j0, np, Nnm, ldp, ldz,
-                       Zp);
     return hipGetLastError();
 }
 

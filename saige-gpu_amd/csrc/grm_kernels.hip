@@ -618,6 +618,17 @@ __global__ __launch_bounds__(256) void k_mirror_diag(float* __restrict__ S, int6
         S[(base + c) * ld + base + r] = S[(base + r) * ld + base + c];
 }
 
+// out[nr][nc] = S[r0 + i][c0 + j] / m, rounded once (div_rn): the read-back of a
+// block of K.  One row per blockIdx.y step, four columns per thread.
+__global__ __launch_bounds__(256) void k_grm_block(const float* __restrict__ S, int64_t ld, int64_t nr, int64_t nc,
+                                                   float m, float* __restrict__ out) {
+    const int64_t j0 = 4 * (blockIdx.x * (int64_t)256 + threadIdx.x);
+    for (int64_t i = blockIdx.y; i < nr; i += gridDim.y)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (j0 + e < nc) out[i * nc + j0 + e] = div_rn(S[i * ld + j0 + e], m);
+}
+
 // ------------------------------------------------------------------ FP32
 constexpr int BK32 = 32;            // markers per K chunk
 constexpr int P32 = BK32 + 4;       // LDS row pitch (floats)
@@ -758,6 +769,13 @@ hipError_t launch_syrk_pk_split(hipStream_t s, const uint8_t* tp, const uint64_t
 hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile) {
     if (tile <= 0 || Npad % tile != 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_mirror_diag, dim3((unsigned)(Npad / tile), (unsigned)tile), dim3(256), 0, s, S, Npad, tile);
+    return hipGetLastError();
+}
+
+hipError_t launch_grm_block(hipStream_t s, const float* S, int64_t ld, int64_t nr, int64_t nc, float m, float* out) {
+    if (nr <= 0 || nc <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_grm_block, dim3((unsigned)((nc + 1023) / 1024), (unsigned)std::min<int64_t>(nr, 32768)),
+                       dim3(256), 0, s, S, ld, nr, nc, m, out);
     return hipGetLastError();
 }
 

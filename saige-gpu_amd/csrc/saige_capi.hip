@@ -164,7 +164,7 @@ void clear_geno(saige_ctx* c) {
 void free_geno(saige_ctx* c) {
     clear_geno(c);
     for (KeptBlock* b : {&c->kb_stats, &c->kb_packed, &c->kb_packed_vr, &c->kb_lut, &c->kb_lut_vr, &c->kb_vec,
-                         &c->kb_lists})
+                         &c->kb_lists, &c->kb_block})
         b->release();
 }
 
@@ -1226,10 +1226,21 @@ int saige_get_grm_block(saige_ctx* c, int64_t r0, int64_t c0, int64_t nr, int64_
         set_error("GRM block out of range");
         return SAIGE_E_ARG;
     }
-    SAIGE_HIP_TRY(hipMemcpy2D(out, sizeof(float) * nc, c->d_grm + r0 * c->Npad + c0, sizeof(float) * c->Npad,
-                              sizeof(float) * nc, nr, hipMemcpyDeviceToHost));
-    const float m = (float)c->Mqc;
-    for (int64_t i = 0; i < nr * nc; i++) out[i] = out[i] / m;
+    if (nr == 0 || nc == 0) return SAIGE_OK;
+    // rows divided on the device into a contiguous block (at most 64 MB, or one
+    // row) and copied from there: a pitched copy goes to the host row by row
+    const int64_t rows = std::min(nr, std::max<int64_t>(1, ((int64_t)16 << 20) / nc));
+    if (c->kb_block.reserve((int64_t)sizeof(float) * rows * nc)) {
+        set_error("device allocation failed (GRM block)");
+        return SAIGE_E_NOMEM;
+    }
+    float* d = static_cast<float*>(c->kb_block.p);
+    for (int64_t i = 0; i < nr; i += rows) {
+        const int64_t n = std::min(rows, nr - i);
+        SAIGE_HIP_TRY(launch_grm_block(c->stream, c->d_grm + (r0 + i) * c->Npad + c0, c->Npad, n, nc, (float)c->Mqc, d));
+        SAIGE_HIP_TRY(hipMemcpyAsync(out + i * nc, d, sizeof(float) * n * nc, hipMemcpyDeviceToHost, c->stream));
+        SAIGE_HIP_TRY(hipStreamSynchronize(c->stream));
+    }
     return SAIGE_OK;
 }
 

@@ -215,6 +215,7 @@ struct saige_ctx {
     // the device blocks of an ingest, kept for the context's next cohort: the
     // pointers below and setgeno's own lists point into them
     saige::KeptBlock kb_stats, kb_packed, kb_packed_vr, kb_lut, kb_lut_vr, kb_vec, kb_lists;
+    saige::KeptBlock kb_block;                   // saige_get_grm_block's rows on their way to the host
     // decode outputs
     saige::MarkerStat* d_stats = nullptr;        // [M]
     std::vector<saige::MarkerStat> h_stats;      // [M]
@@ -350,6 +351,8 @@ hipError_t launch_syrk_pk_split(hipStream_t s, const uint8_t* tp, const uint64_t
 // piece 0: the values rounded to BF16 (hi); 1: the remainders rounded to BF16 (lo)
 hipError_t launch_lut64_range(hipStream_t s, const float4* lut, int64_t Mqc, int64_t j0, int64_t j1, int piece,
                               uint64_t* lut64);
+// out[nr][nc] (contiguous) = S[i][j] / m for S at its block's first element
+hipError_t launch_grm_block(hipStream_t s, const float* S, int64_t ld, int64_t nr, int64_t nc, float m, float* out);
 hipError_t launch_sub(hipStream_t s, const float* a, const float* b, int64_t n, float* out);
 int syrk_tile();
 int syrk_kchunk_f32();
