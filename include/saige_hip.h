@@ -40,7 +40,11 @@ extern "C" {
 #define SAIGE_PENDING 1       /* saige_poll: the request has not finished */
 
 /* GRM arithmetic for saige_build_grm */
-#define SAIGE_GRM_FP32 0        /* FP32 Z panels, FP32 MFMA (v_mfma_f32_32x32x2_f32) */
+#define SAIGE_GRM_FP32 0        /* 2-bit genotypes; z_i z_j = (g_i - c) beta z_j + a term of
+                                   j alone: g - c whole, beta z in three BF16 pieces (24
+                                   bits), three products on the BF16 MFMA with FP32
+                                   accumulation, the terms of j alone in FP64; an FP32
+                                   sum over the markers' exact products               */
 #define SAIGE_GRM_BF16 1        /* 2-bit genotypes standardised to BF16 inside the SYRK,
                                    BF16 MFMA with FP32 accumulation                    */
 #define SAIGE_GRM_BF16_PANEL 2  /* same arithmetic from materialised BF16 Z panels     */

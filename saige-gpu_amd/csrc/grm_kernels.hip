@@ -2,8 +2,8 @@
 //
 // Zp is the standardised panel, [Npad][ldz] row-major (sample rows, marker
 // columns), so both MFMA operands are K-contiguous rows of the same matrix.
-// Each workgroup computes one 128x128 tile of the lower triangle (tile row
-// >= tile column) and writes it and its mirror into the full row-major S.
+// Each workgroup computes one tile of the lower triangle (tile row >= tile
+// column) and writes it and its mirror into the full row-major S.
 // Tile order: the host lists the triangle's tiles grouped into 8x8-tile
 // super-blocks, and the launch index is remapped so that each XCD (launch
 // order round-robins over the 8 XCDs) walks a contiguous run of that list.
@@ -14,6 +14,8 @@
 // Operand staging: global -> registers (prefetch of the next K chunk while
 // the current one is multiplied) -> LDS -> MFMA fragments.
 #include <algorithm>
+#include <cmath>
+#include <cstdlib>
 
 #include "saige_internal.hpp"
 
@@ -36,34 +38,53 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t bid, int64_t nblk) {
     return (x < rem) ? x * (q + 1) + loc : rem * (q + 1) + (x - rem) * q + loc;
 }
 
-// Accumulator layout of a 32x32 MFMA block: lane l, register r holds
-// row 8*(r/4) + 4*(l/32) + (r%4), column l%32.
-__device__ __forceinline__ void store_tile(float* S, int64_t ldS, int64_t bi, int64_t bj, int wr,
-                                           int wc, int lane, const f32x16 (&acc)[2][2],
-                                           int accumulate) {
-    const bool mirror = bi != bj;
+// x rounded to nearest (ties to even) at 16 significant bits: the FP32
+// value with the low 8 of its 23 fraction bits cleared.  Such a value is
+// exactly the sum of its two BF16 pieces by truncation (the upper half of
+// its bits, then the upper half of the remainder's), which the block GEMM
+// over the lower triangle relies on.  Finite x only.
+__device__ __forceinline__ float round16(float x) {
+    const uint32_t b = __float_as_uint(x);
+    return __uint_as_float((b + 0x7Fu + ((b >> 8) & 1u)) & 0xFFFFFF00u);
+}
+
+// Store a wave's block of 32*MI rows from row0 and 32*NI columns from col0,
+// mirrored for off-diagonal tiles; accumulate: +1 add to S, -1 subtract from
+// S, 0 store.  center: the column's value taken off each sum first (nullptr:
+// none).  R16: the stored values (after the add or subtract) rounded by
+// round16.  Accumulator layout of a 32x32 MFMA block: lane l, register r
+// holds row 8*(r/4) + 4*(l/32) + (r%4), column l%32.
+template <int MI, int NI, bool R16>
+__device__ __forceinline__ void store_block(float* S, int64_t ldS, int64_t row0, int64_t col0, bool mirror, int lane,
+                                            const f32x16 (&acc)[MI][NI], int accumulate,
+                                            const float* center = nullptr) {
 #pragma unroll
-    for (int mi = 0; mi < 2; mi++) {
+    for (int mi = 0; mi < MI; mi++) {
 #pragma unroll
-        for (int ni = 0; ni < 2; ni++) {
-            const int64_t col = bj * BT + wc * 64 + ni * 32 + (lane & 31);
+        for (int ni = 0; ni < NI; ni++) {
+            const int64_t col = col0 + ni * 32 + (lane & 31);
+            const float cc = center ? center[col] : 0.0f;
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const int64_t row0 = bi * BT + wr * 64 + mi * 32 + 8 * g + 4 * (lane >> 5);
+                const int64_t row = row0 + mi * 32 + 8 * g + 4 * (lane >> 5);
                 float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = acc[mi][ni][4 * g + e];
+                for (int e = 0; e < 4; e++) v[e] = center ? acc[mi][ni][4 * g + e] - cc : acc[mi][ni][4 * g + e];
                 if (accumulate > 0) {        // S += tile
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = S[(row0 + e) * ldS + col] + v[e];
+                    for (int e = 0; e < 4; e++) v[e] = S[(row + e) * ldS + col] + v[e];
                 } else if (accumulate < 0) { // S -= tile (LOCO: remove one chromosome's markers)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = S[(row0 + e) * ldS + col] - v[e];
+                    for (int e = 0; e < 4; e++) v[e] = S[(row + e) * ldS + col] - v[e];
+                }
+                if (R16) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = round16(v[e]);
                 }
 #pragma unroll
-                for (int e = 0; e < 4; e++) S[(row0 + e) * ldS + col] = v[e];
+                for (int e = 0; e < 4; e++) S[(row + e) * ldS + col] = v[e];
                 if (mirror) {
-                    float4* dst = reinterpret_cast<float4*>(S + col * ldS + row0);
+                    float4* dst = reinterpret_cast<float4*>(S + col * ldS + row);
                     *dst = make_float4(v[0], v[1], v[2], v[3]);
                 }
             }
@@ -139,7 +160,7 @@ __global__ __launch_bounds__(256) void k_syrk_bf16(const __hip_bfloat16* __restr
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fb[ni], acc[mi][ni], 0, 0, 0);
         }
     }
-    store_tile(S, ldS, bi, bj, wr, wc, lane, acc, accumulate);
+    store_block<2, 2, false>(S, ldS, bi * BT + wr * 64, bj * BT + wc * 64, bi != bj, lane, acc, accumulate);
 }
 
 // ------------------------------------------------------- BF16, 2-bit in
@@ -154,24 +175,10 @@ __global__ __launch_bounds__(256) void k_syrk_bf16(const __hip_bfloat16* __restr
 // lut64[j]: four BF16 values of marker j indexed by the internal code:
 // 00 -> L[2], 01 -> 0, 10 -> L[1], 11 -> L[0].
 //
-// Thread t decodes byte b = t/8 of markers 8*(t%8)..+7: four sample rows of
-// eight consecutive markers, i.e. four 16-byte LDS rows of the operand.
-__device__ __forceinline__ u32x4 decode_row(const uint64_t (&lut)[8], const uint8_t (&byte)[8], int j) {
-    u32x4 r;
-#pragma unroll
-    for (int h = 0; h < 4; h++) {
-        const unsigned c0 = (byte[2 * h] >> (2 * j)) & 3u;
-        const unsigned c1 = (byte[2 * h + 1] >> (2 * j)) & 3u;
-        const unsigned v0 = (unsigned)(lut[2 * h] >> (16 * c0)) & 0xFFFFu;
-        const unsigned v1 = (unsigned)(lut[2 * h + 1] >> (16 * c1)) & 0xFFFFu;
-        r[h] = v0 | (v1 << 16);
-    }
-    return r;
-}
-
-// The same row as decode_row, by byte permutes: lo[e] / hi[e] hold the low /
-// high bytes of marker e's four BF16 table entries (entry c in byte c), so
-// the 8-byte pair table {lo[2k+1], lo[2k]} is indexed by c_even and
+// Eight consecutive markers' values of one sample (samples 4b + j of byte b;
+// bytes: the eight markers' bytes), i.e. one 16-byte LDS row of an operand, by
+// byte permutes: lo[e] / hi[e] hold the low / high bytes of marker e's four
+// BF16 table entries (entry c in byte c), so the 8-byte pair table {lo[2k+1], lo[2k]} is indexed by c_even and
 // 4 + c_odd.  (byte >> 2j) & 3 of all eight markers at once gives the
 // selectors; four permutes pick the low and high bytes of two marker pairs
 // and two more interleave them into packed BF16 pairs.
@@ -192,138 +199,12 @@ __device__ __forceinline__ u32x4 decode_row_perm(const uint32_t (&lo)[8], const 
     return r;
 }
 
-__global__ __launch_bounds__(256) void k_syrk_pk(const uint8_t* __restrict__ tp, int64_t nchunk, int64_t c0,
-                                                 int64_t c1, const uint64_t* __restrict__ lut64,
-                                                 const int2* __restrict__ tiles, int64_t nblk,
-                                                 float* __restrict__ S, int64_t ldS, int accumulate) {
-    __shared__ __attribute__((aligned(16))) __hip_bfloat16 sA[BT * P16];
-    __shared__ __attribute__((aligned(16))) __hip_bfloat16 sB[BT * P16];
-    const int2 t = tiles[xcd_remap(blockIdx.x, nblk)];
-    const int64_t bi = t.x, bj = t.y;
-    const bool diag = bi == bj;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wr = wv >> 1, wc = wv & 1;
-    const int o = tid & 7, b = tid >> 3;          // marker octet, byte within the panel
-    const uint64_t* gA = reinterpret_cast<const uint64_t*>(tp + (bi * nchunk * 32 + b) * 64 + 8 * o);
-    const uint64_t* gB = reinterpret_cast<const uint64_t*>(tp + (bj * nchunk * 32 + b) * 64 + 8 * o);
-    // one chunk = 2048 bytes = 256 uint64; this launch covers chunks [c0, c1)
-    uint64_t ra = gA[c0 * 256], rb = gB[c0 * 256];
-    const uint64_t* gl = lut64 + 8 * o;
-    uint64_t la[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) la[e] = gl[c0 * 64 + e];
-
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-        for (int ni = 0; ni < 2; ni++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[mi][ni][r] = 0.0f;
-
-    for (int64_t kc = c0; kc < c1; kc++) {
-        uint8_t ba[8], bb[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            ba[e] = (uint8_t)(ra >> (8 * e));
-            bb[e] = (uint8_t)(rb >> (8 * e));
-        }
-        uint64_t lc[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) lc[e] = la[e];
-        // prefetch the next chunk's bytes and LUT entries (re-read the last one at the end)
-        const int64_t kn = (kc + 1 < c1) ? kc + 1 : kc;
-        ra = gA[kn * 256];
-        rb = gB[kn * 256];
-#pragma unroll
-        for (int e = 0; e < 8; e++) la[e] = gl[kn * 64 + e];
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            *reinterpret_cast<u32x4*>(sA + (4 * b + j) * P16 + 8 * o) = decode_row(lc, ba, j);
-            if (!diag) *reinterpret_cast<u32x4*>(sB + (4 * b + j) * P16 + 8 * o) = decode_row(lc, bb, j);
-        }
-        __syncthreads();
-        const __hip_bfloat16* pB = diag ? sA : sB;
-#pragma unroll
-        for (int ks = 0; ks < BK16 / 16; ks++) {
-            const int kk = ks * 16 + (lane >> 5) * 8;
-            bf16x8 fa[2], fb[2];
-#pragma unroll
-            for (int mi = 0; mi < 2; mi++)
-                fa[mi] = *reinterpret_cast<const bf16x8*>(sA + (wr * 64 + mi * 32 + (lane & 31)) * P16 + kk);
-#pragma unroll
-            for (int ni = 0; ni < 2; ni++)
-                fb[ni] = *reinterpret_cast<const bf16x8*>(pB + (wc * 64 + ni * 32 + (lane & 31)) * P16 + kk);
-#pragma unroll
-            for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-                for (int ni = 0; ni < 2; ni++)
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fb[ni], acc[mi][ni], 0, 0, 0);
-        }
-    }
-    store_tile(S, ldS, bi, bj, wr, wc, lane, acc, accumulate);
-}
-
-// 256x256 tiles for the 2-bit input: 512 threads (8 waves as 4 x 2), each
-// wave a 64 x 128 block of the tile (2 x 4 MFMA 32x32 blocks, 128
-// accumulator registers).  Per 64-marker chunk a thread decodes the same 64
-// values as in k_syrk_pk, but each decoded value feeds twice the MFMA work,
-// which halves the VALU decode per MFMA (the bound of the 128 tile).  The
-// per-element accumulation order (chunk by chunk, 16 markers per MFMA) is
-// that of k_syrk_pk, so both give bitwise equal S.
+// The single-pass BF16 GRM on 256x256 tiles: 512 threads (8 waves as 4 x 2),
+// each wave a 64 x 128 block of the tile (2 x 4 MFMA 32x32 blocks, 128
+// accumulator registers).  The per-element accumulation order (chunk by
+// chunk, 16 markers per MFMA) is that of every tile size, so all give
+// bitwise equal S.
 constexpr int BT2 = 256;
-
-// x rounded to nearest (ties to even) at 16 significant bits: the FP32
-// value with the low 8 of its 23 fraction bits cleared.  Such a value is
-// exactly the sum of its two BF16 pieces by truncation (the upper half of
-// its bits, then the upper half of the remainder's), which the block GEMM
-// over the lower triangle relies on.  Finite x only.
-__device__ __forceinline__ float round16(float x) {
-    const uint32_t b = __float_as_uint(x);
-    return __uint_as_float((b + 0x7Fu + ((b >> 8) & 1u)) & 0xFFFFFF00u);
-}
-
-// Store a 256x256 tile from waves of (32*MI) x 128 (wave (wr, wc) owns rows
-// wr*32*MI + [0, 32*MI) and columns wc*128 + [0, 128)), mirrored for
-// off-diagonal tiles; accumulate: +1 add to S, -1 subtract from S, 0 store.
-// R16: the stored values (after the add or subtract) rounded by round16.
-template <int MI, bool R16>
-__device__ __forceinline__ void store_tile256(float* S, int64_t ldS, int64_t bi, int64_t bj, int wr, int wc,
-                                              int lane, const f32x16 (&acc)[MI][4], int accumulate) {
-    const bool mirror = bi != bj;
-#pragma unroll
-    for (int mi = 0; mi < MI; mi++) {
-#pragma unroll
-        for (int ni = 0; ni < 4; ni++) {
-            const int64_t col = bj * BT2 + wc * 128 + ni * 32 + (lane & 31);
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int64_t row0 = bi * BT2 + wr * 32 * MI + mi * 32 + 8 * g + 4 * (lane >> 5);
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = acc[mi][ni][4 * g + e];
-                if (accumulate > 0) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = S[(row0 + e) * ldS + col] + v[e];
-                } else if (accumulate < 0) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = S[(row0 + e) * ldS + col] - v[e];
-                }
-                if (R16) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = round16(v[e]);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; e++) S[(row0 + e) * ldS + col] = v[e];
-                if (mirror) {
-                    float4* dst = reinterpret_cast<float4*>(S + col * ldS + row0);
-                    *dst = make_float4(v[0], v[1], v[2], v[3]);
-                }
-            }
-        }
-    }
-}
 
 // Double-buffered: while the MFMAs run on chunk k from one LDS buffer, the
 // same waves decode chunk k+1 into the other, so the matrix pipe and the
@@ -333,6 +214,16 @@ __device__ __forceinline__ void store_tile256(float* S, int64_t ldS, int64_t bi,
 // never alias and can interleave them; the loop body is one basic block (the
 // last step decodes a clamped copy of the last chunk that nothing reads, and
 // diagonal tiles, both panels the same, decode their B copy too).
+// eight tables' low and high bytes of their BF16 entries
+__device__ __forceinline__ void split_bytes(const uint64_t (&t)[8], uint32_t (&lo)[8], uint32_t (&hi)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const uint32_t l = (uint32_t)t[e], h = (uint32_t)(t[e] >> 32);
+        lo[e] = __builtin_amdgcn_perm(h, l, 0x06040200u);
+        hi[e] = __builtin_amdgcn_perm(h, l, 0x07050301u);
+    }
+}
+
 __global__ __launch_bounds__(512) void k_syrk_pk256(const uint8_t* __restrict__ tp, int64_t nchunk, int64_t c0,
                                                     int64_t c1, const uint64_t* __restrict__ lut64,
                                                     const int2* __restrict__ tiles, int64_t nblk,
@@ -367,15 +258,6 @@ __global__ __launch_bounds__(512) void k_syrk_pk256(const uint8_t* __restrict__ 
         rb = gB[kc * 256];
 #pragma unroll
         for (int e = 0; e < 8; e++) la[e] = gl[kc * 64 + e];
-    };
-    // a table's low and high bytes of its BF16 entries
-    auto split_bytes = [&](const uint64_t (&t)[8], uint32_t (&lo)[8], uint32_t (&hi)[8]) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const uint32_t l = (uint32_t)t[e], h = (uint32_t)(t[e] >> 32);
-            lo[e] = __builtin_amdgcn_perm(h, l, 0x06040200u);
-            hi[e] = __builtin_amdgcn_perm(h, l, 0x07050301u);
-        }
     };
     // decode the chunk held in ra/rb/la into (dA, dB), fetching chunk kn
     auto decode_next = [&](__hip_bfloat16* dA, __hip_bfloat16* dB, int64_t kn) {
@@ -429,120 +311,161 @@ __global__ __launch_bounds__(512) void k_syrk_pk256(const uint8_t* __restrict__ 
         step(sA1, sB1, sA0, sB0, kc + 1);
     }
     if (kc < c1) multiply(sA0, sB0);
-    store_tile256<2, false>(S, ldS, bi, bj, wr, wc, lane, acc, accumulate);
+    store_block<2, 4, false>(S, ldS, bi * BT2 + wr * 64, bj * BT2 + wc * 128, bi != bj, lane, acc, accumulate);
 }
 
-// The split GRM in one pass: per 32-marker chunk each thread decodes its
-// panel's bytes through both tables, hi and lo, and every wave adds
-// hi.hi, hi.lo and lo.hi of its 64 x 128 block in that order (three MFMAs
-// per operand pair into one accumulator).  Against three separate passes
-// this reads the genotypes and the tables once, keeps a single set of
-// accumulators and stores S once.  LDS: two buffers of the four decoded
-// operands (A hi, A lo, B hi, B lo; 256 samples x 32 markers each, pitch 40
-// for conflict-free 16-byte reads) = 160 KiB.  Threads 0-255 decode the row
-// panel, 256-511 the column panel: thread (o, b) holds marker octet o of the
-// chunk and byte row b (four samples).  S is stored rounded to 16 significant
-// bits (round16, after the add or subtract of an accumulating pass), which
-// moves each value by at most 2^-16 of itself; the block GEMM then needs two
-// BF16 pieces of S instead of three.
-constexpr int BKS = 32;            // markers per chunk
-constexpr int PS = BKS + 8;        // LDS row pitch (bf16 elements)
-
-__global__ __launch_bounds__(512) void k_syrk_pk256_split(const uint8_t* __restrict__ tp, int64_t nchunk,
-                                                          int64_t k0, int64_t k1,
-                                                          const uint64_t* __restrict__ lhi,
-                                                          const uint64_t* __restrict__ llo,
-                                                          const int2* __restrict__ tiles, int64_t nblk,
-                                                          float* __restrict__ S, int64_t ldS, int accumulate) {
-    __shared__ __attribute__((aligned(16))) __hip_bfloat16 s0[4 * BT2 * PS];   // [A hi | A lo | B hi | B lo]
-    __shared__ __attribute__((aligned(16))) __hip_bfloat16 s1[4 * BT2 * PS];
+// k_syrk_pk<T, F>: the GRM from 2-bit genotypes on T x T tiles, by operand
+// form F:
+// * SYRK_HI: one BF16 piece of z, hi.hi (the single-pass GRM; T < 256, the
+//   256 tile is k_syrk_pk256);
+// * SYRK_SPLIT: z in two BF16 pieces, hi.hi + hi.lo + lo.hi (the split GRM),
+//   stored rounded to 16 significant bits (round16, after the add or subtract
+//   of an accumulating pass), which moves each value by at most 2^-16 of
+//   itself; the block GEMM then needs two BF16 pieces of S instead of three;
+// * SYRK_FP32: z_i z_j = (g_i - c) beta z_j + (alpha + beta c) z_j with the
+//   marker's z = alpha + beta g and c the whole number nearest its mean.  g - c
+//   is a whole number, exact in one BF16 piece, so the row operand needs one
+//   piece and only the column operand beta z needs three (24 bits and more):
+//   three products instead of the six of two three-piece operands, on the
+//   BF16 pipe instead of the FP32 one (1/16 of its rate).  The second term
+//   depends on the column alone: its sum over the markers is formed in FP64
+//   beforehand and taken off at the store (center).
+// Per chunk of BK markers each thread decodes two operand rows' worth of its
+// byte row through two tables (one for SYRK_HI), then every wave adds the
+// products of its block in a fixed order.  LDS: two buffers of the operands
+// (four for the multi-piece forms), so the next chunk's decode runs beside
+// this chunk's MFMAs.  SYRK_SPLIT: threads of the lower half decode the row
+// panel (hi, lo), of the upper half the column panel; SYRK_FP32: the lower
+// half the row operand and the column's lo, the upper half its hi and mid.
+//
+// T: the 256 tile (8 waves of 64 x 128) does the most MFMA work per decoded
+// value and is bound by the matrix pipe and its power (split GRM at N = 40,000:
+// 1380 TFLOP/s of BF16 products); a small GRM has too few of its tiles for 256
+// CUs, each walking all markers, and takes 128 (4 waves of 64 x 64) or 64 (4
+// waves of 32 x 32) tiles, see syrk_pk_tile.  The per-element order is the
+// same for every T: bitwise equal S.
+template <int T, int F>
+__global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t* __restrict__ tp, int64_t nchunk,
+                                                                  int64_t k0, int64_t k1, SyrkTables tb,
+                                                                  const int2* __restrict__ tiles, int64_t nblk,
+                                                                  float* __restrict__ S, int64_t ldS,
+                                                                  int accumulate) {
+    constexpr int BK = T == 64 ? 64 : 32;            // markers per chunk
+    constexpr int P = BK + 8;                        // LDS row pitch (bf16 elements), conflict-free 16-byte reads
+    constexpr int NOP = F == SYRK_HI ? 2 : 4;        // operands in LDS
+    constexpr int HALF = T == 256 ? 256 : 128;       // threads per panel
+    constexpr int OCT = BK / 8;                      // marker octets per chunk
+    constexpr int WC = 2;                            // waves across the tile's columns
+    constexpr int MI = T == 64 ? 1 : 2, NI = T == 256 ? 4 : MI;
+    constexpr int NPROD = F == SYRK_HI ? 1 : 3;
+    __shared__ __attribute__((aligned(16))) __hip_bfloat16 s0[NOP * T * P];
+    __shared__ __attribute__((aligned(16))) __hip_bfloat16 s1[NOP * T * P];
     const int2 t = tiles[xcd_remap(blockIdx.x, nblk)];
     const int64_t bi = t.x, bj = t.y;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wr = wv >> 1, wc = wv & 1;
-    const int r = tid >> 8, o = tid & 3, b = (tid & 255) >> 2;   // panel (0 rows, 1 columns), octet, byte row
-    const int64_t pn = 2 * (r ? bj : bi) + (b >> 5);
-    // uint64 units: 64-marker chunk c is 256 words on from chunk c-1, its
-    // second 32 markers 4 words into a byte row
-    const uint64_t* g = reinterpret_cast<const uint64_t*>(tp + (pn * nchunk * 32 + (b & 31)) * 64 + 8 * o);
-    const uint64_t* gh = lhi + 8 * o;
-    const uint64_t* gl = llo + 8 * o;
-    const int dst = (2 * r) * BT2 * PS + (4 * b) * PS + 8 * o;   // this thread's hi rows; lo rows BT2*PS on
+    const int wr = wv / WC, wc = wv % WC;
+    // half (0, 1), octet and byte row of this thread
+    const int h = tid / HALF, o = tid % OCT, b = (tid % HALF) / OCT;
+    // its byte row of tile row / column index x: uint64 units, a 64-marker
+    // chunk is 256 words on from the one before, its second 32 markers 4 words
+    // into a byte row
+    auto byte_row = [&](int64_t x) {
+        const int64_t s4 = x * (T / 4) + b;          // byte row of the matrix: 32 per 128-sample panel
+        return reinterpret_cast<const uint64_t*>(tp + ((s4 >> 5) * nchunk * 32 + (s4 & 31)) * 64 + 8 * o);
+    };
+    const bool lower = h == 0;
+    const uint64_t* g0 = byte_row(lower ? bi : bj);
+    const uint64_t* g1 = byte_row(F == SYRK_FP32 || !lower ? bj : bi);
+    const uint64_t* t0 = (F == SYRK_FP32 && !lower ? tb.t[1] : tb.t[0]) + 8 * o;
+    const uint64_t* t1 = (F == SYRK_FP32 ? (lower ? tb.t[3] : tb.t[2]) : tb.t[1]) + 8 * o;
+    constexpr int OPS = T * P;                       // one operand
+    const int dst = (F == SYRK_HI ? h : 2 * h) * OPS + (4 * b) * P + 8 * o;
 
-    f32x16 acc[2][4];
+    f32x16 acc[MI][NI];
 #pragma unroll
-    for (int mi = 0; mi < 2; mi++)
+    for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-        for (int ni = 0; ni < 4; ni++)
+        for (int ni = 0; ni < NI; ni++)
 #pragma unroll
             for (int q = 0; q < 16; q++) acc[mi][ni][q] = 0.0f;
 
-    uint64_t raw, th[8], tl[8];
+    uint64_t raw0, raw1, l0[8], l1[8];
     auto fetch = [&](int64_t kc) {
-        raw = g[(kc >> 1) * 256 + (kc & 1) * 4];
+        const int64_t off = BK == 64 ? kc * 256 : (kc >> 1) * 256 + (kc & 1) * 4;
+        raw0 = g0[off];
+        if (F == SYRK_FP32) raw1 = g1[off];
 #pragma unroll
-        for (int e = 0; e < 8; e++) th[e] = gh[kc * 32 + e];
+        for (int e = 0; e < 8; e++) l0[e] = t0[kc * BK + e];
+        if (F != SYRK_HI) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) tl[e] = gl[kc * 32 + e];
-    };
-    auto split_bytes = [&](const uint64_t (&tb)[8], uint32_t (&lo)[8], uint32_t (&hi)[8]) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const uint32_t l = (uint32_t)tb[e], h = (uint32_t)(tb[e] >> 32);
-            lo[e] = __builtin_amdgcn_perm(h, l, 0x06040200u);
-            hi[e] = __builtin_amdgcn_perm(h, l, 0x07050301u);
+            for (int e = 0; e < 8; e++) l1[e] = t1[kc * BK + e];
         }
     };
-    // decode the chunk held in raw/th/tl into buffer d, fetching chunk kn
+    // decode the chunk held in the registers into buffer d, fetching chunk kn
     auto decode_next = [&](__hip_bfloat16* d, int64_t kn) {
-        const uint64_t c = raw;
-        uint32_t hlo[8], hhi[8], llo8[8], lhi8[8];
-        split_bytes(th, hlo, hhi);
-        split_bytes(tl, llo8, lhi8);
+        const uint64_t c0 = raw0, c1 = F == SYRK_FP32 ? raw1 : raw0;
+        uint32_t lo0[8], hi0[8], lo1[8], hi1[8];
+        split_bytes(l0, lo0, hi0);
+        if (F != SYRK_HI) split_bytes(l1, lo1, hi1);
         fetch(kn);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            *reinterpret_cast<u32x4*>(d + dst + j * PS) = decode_row_perm(hlo, hhi, c, j);
-            *reinterpret_cast<u32x4*>(d + dst + BT2 * PS + j * PS) = decode_row_perm(llo8, lhi8, c, j);
+            *reinterpret_cast<u32x4*>(d + dst + j * P) = decode_row_perm(lo0, hi0, c0, j);
+            if (F != SYRK_HI) *reinterpret_cast<u32x4*>(d + dst + OPS + j * P) = decode_row_perm(lo1, hi1, c1, j);
         }
     };
     auto multiply = [&](const __hip_bfloat16* d) {
-        const __hip_bfloat16* Ah = d;
-        const __hip_bfloat16* Al = d + BT2 * PS;
-        const __hip_bfloat16* Bh = d + 2 * BT2 * PS;
-        const __hip_bfloat16* Bl = d + 3 * BT2 * PS;
 #pragma unroll
-        for (int ks = 0; ks < BKS / 16; ks++) {
+        for (int ks = 0; ks < BK / 16; ks++) {
             const int kk = ks * 16 + (lane >> 5) * 8;
-            bf16x8 fah[2], fal[2];
+            // operand q of row block r
+            auto frag = [&](int q, int r) {
+                return *reinterpret_cast<const bf16x8*>(d + q * OPS + (r + (lane & 31)) * P + kk);
+            };
+            bf16x8 fa[MI], fl[MI];
 #pragma unroll
-            for (int mi = 0; mi < 2; mi++) {
-                const int row = (wr * 64 + mi * 32 + (lane & 31)) * PS + kk;
-                fah[mi] = *reinterpret_cast<const bf16x8*>(Ah + row);
-                fal[mi] = *reinterpret_cast<const bf16x8*>(Al + row);
+            for (int mi = 0; mi < MI; mi++) {
+                fa[mi] = frag(0, wr * 32 * MI + mi * 32);
+                if (F == SYRK_SPLIT) fl[mi] = frag(1, wr * 32 * MI + mi * 32);
             }
 #pragma unroll
-            for (int ni = 0; ni < 4; ni++) {
-                const int col = (wc * 128 + ni * 32 + (lane & 31)) * PS + kk;
-                const bf16x8 fbh = *reinterpret_cast<const bf16x8*>(Bh + col);
-                const bf16x8 fbl = *reinterpret_cast<const bf16x8*>(Bl + col);
+            for (int ni = 0; ni < NI; ni++) {
+                const int c = wc * 32 * NI + ni * 32;
+                if (F == SYRK_HI) {
+                    const bf16x8 fb = frag(1, c);
 #pragma unroll
-                for (int mi = 0; mi < 2; mi++) {
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fah[mi], fbh, acc[mi][ni], 0, 0, 0);
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fah[mi], fbl, acc[mi][ni], 0, 0, 0);
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fal[mi], fbh, acc[mi][ni], 0, 0, 0);
+                    for (int mi = 0; mi < MI; mi++)
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fb, acc[mi][ni], 0, 0, 0);
+                } else if (F == SYRK_SPLIT) {
+                    const bf16x8 fbh = frag(2, c), fbl = frag(3, c);
+#pragma unroll
+                    for (int mi = 0; mi < MI; mi++) {
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fbh, acc[mi][ni], 0, 0, 0);
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fbl, acc[mi][ni], 0, 0, 0);
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fl[mi], fbh, acc[mi][ni], 0, 0, 0);
+                    }
+                } else {
+                    const bf16x8 fbl = frag(1, c), fbh = frag(2, c), fbm = frag(3, c);
+#pragma unroll
+                    for (int mi = 0; mi < MI; mi++) {
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fbl, acc[mi][ni], 0, 0, 0);
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fbm, acc[mi][ni], 0, 0, 0);
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fbh, acc[mi][ni], 0, 0, 0);
+                    }
                 }
             }
         }
     };
-    // multiply chunk kc from cur while decoding chunk kc+1 into nxt
+    // multiply chunk kc from cur while decoding chunk kc+1 into nxt: one MFMA,
+    // then its share of the decode's VALU instructions
     auto step = [&](const __hip_bfloat16* cur, __hip_bfloat16* nxt, int64_t kc) {
+        constexpr int NM = MI * NI * (BK / 16) * NPROD;
         decode_next(nxt, kc + 2 < k1 ? kc + 2 : k1 - 1);
         multiply(cur);
 #pragma unroll
-        for (int i = 0; i < 48; i++) {
+        for (int i = 0; i < NM; i++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, (F == SYRK_HI ? 72 : 144) / NM, 0);
         }
         lds_barrier();
     };
@@ -555,54 +478,167 @@ __global__ __launch_bounds__(512) void k_syrk_pk256_split(const uint8_t* __restr
         step(s1, s0, kc + 1);
     }
     if (kc < k1) multiply(s0);
-    store_tile256<2, true>(S, ldS, bi, bj, wr, wc, lane, acc, accumulate);
+    store_block<MI, NI, F == SYRK_SPLIT>(S, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane, acc,
+                                         accumulate, F == SYRK_FP32 ? tb.center : nullptr);
 }
 
-// Re-tile the packed genotypes for k_syrk_pk: block (p, c) byte (b, m) =
-// byte 32p + b of QC'd marker 64c + m, with padding codes 0b01.
+// Re-tile the packed genotypes for the SYRK: block (p, c) byte (b, m) = byte
+// 32p + b of GRM marker 64(c0 + c) + m, with padding codes 0b01 (samples >= Nnm,
+// markers >= Mqc).  A workgroup takes four panels (a cache line of each row)
+// of one chunk: dwords of four markers' rows are transposed in registers,
+// collected in LDS and stored 16 bytes per thread.  Bound by its two streams:
+// 215 us for 1.2 GB at N = 40,000, M = 60,000, 5.6 TB/s (1431 us with a byte per
+// thread and 32 bytes of a row at a time, which fetched the genotypes several
+// times over).
 __global__ __launch_bounds__(256) void k_pack_tiles(const uint8_t* __restrict__ packed, int64_t Mqc, int64_t Nnm,
-                                                    int64_t ldp, int64_t nchunk, uint8_t* __restrict__ tp) {
-    const int64_t p = blockIdx.x, c = blockIdx.y;
-    uint8_t* blk = tp + (p * nchunk + c) * 2048;
-    for (int i = threadIdx.x; i < 2048; i += 256) {
-        const int b = i >> 6, m = i & 63;
-        const int64_t j = c * 64 + m;
-        const int64_t byte_idx = p * 32 + b;
-        const int64_t s0 = byte_idx * 4;
-        unsigned v = 0x55u;
-        if (j < Mqc && s0 < Nnm) {
-            v = packed[j * ldp + byte_idx];
+                                                    int64_t ldp, int64_t npanel, int64_t c0, int64_t nchunk,
+                                                    uint8_t* __restrict__ tp) {
+    __shared__ uint32_t tile[128 * 17];              // [byte row of four panels][16 marker quads + 1]
+    const int64_t p0 = 4 * (int64_t)blockIdx.x, c = blockIdx.y;
+    const int tid = threadIdx.x, c4 = tid & 31, mq = tid >> 5;
+    const int64_t left = Nnm - (p0 * 128 + 16 * c4); // samples from this dword on
+    const uint32_t keep = left >= 16 ? 0xFFFFFFFFu : (left <= 0 ? 0u : (1u << (2 * left)) - 1u);
+    const uint8_t* src = packed + p0 * 32 + 4 * c4;  // p0 * 32 + 128 <= ldp
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                if (s0 + q >= Nnm) v = (v & ~(3u << (2 * q))) | (1u << (2 * q));
+    for (int q = 0; q < 2; q++) {
+        const int quad = mq + 8 * q;
+        uint32_t w[4], t[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int64_t j = (c0 + c) * 64 + 4 * quad + e;
+            // rows past the markers are the buffer's padding
+            const uint32_t k = j < Mqc ? keep : 0u;
+            w[e] = (*reinterpret_cast<const uint32_t*>(src + j * ldp) & k) | (0x55555555u & ~k);
         }
-        blk[i] = (uint8_t)v;
+        transpose4x4(w[0], w[1], w[2], w[3], t);
+#pragma unroll
+        for (int e = 0; e < 4; e++) tile[(4 * c4 + e) * 17 + quad] = t[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int i = tid + 256 * q;                 // 16 bytes: four marker quads of byte row i / 4
+        const int64_t p = p0 + (i >> 7);
+        const uint32_t* v = tile + (i >> 2) * 17 + 4 * (i & 3);
+        if (p < npanel)
+            *reinterpret_cast<uint4*>(tp + (p * nchunk + c) * 2048 + 16 * (i & 127)) =
+                make_uint4(v[0], v[1], v[2], v[3]);
     }
 }
 
-// lut64[j] for j < nchunk*64 (zero for padding markers).  piece 0: each
-// value rounded to BF16 (hi); piece 1: the remainder x - hi, exact in FP32,
-// rounded to BF16 (lo), so that x - hi - lo is within 2^-16 |x| (BF16 keeps
-// 8 significant bits: each rounding is within 2^-8 relative).
-__device__ __forceinline__ uint64_t bf16_piece(float x, int piece) {
-    const __hip_bfloat16 hi = __float2bfloat16(x);
-    if (piece == 0) return __bfloat16_as_ushort(hi);
-    return __bfloat16_as_ushort(__float2bfloat16(__fsub_rn(x, __bfloat162float(hi))));
+// The SYRK's tables: entry j of a table is GRM marker base + j, four BF16
+// values indexed by the internal code (00 -> two copies, 01 -> 0, 10 -> one,
+// 11 -> none); zero outside markers [j0, j1).
+// SYRK_HI / SYRK_SPLIT: t[0] z rounded to BF16 (hi), t[1] the remainder z - hi,
+// exact in FP32, rounded to BF16 (lo), so that z - hi - lo is within 2^-16 |z|.
+// SYRK_FP32: t[0] g - c, t[1..3] beta z in three BF16 pieces (each the rounded
+// remainder of the ones before), and corr[j] = -(alpha + beta c) z in FP64 per
+// genotype, from z(0), z(1), z(2) as alpha = z(0), beta = (z(2) - z(0)) / 2.
+__device__ __forceinline__ uint64_t bf16_code(double x) { return __bfloat16_as_ushort(__float2bfloat16((float)x)); }
+__device__ __forceinline__ uint64_t four_codes(uint64_t v0, uint64_t v1, uint64_t v2) {
+    return v2 | (v1 << 32) | (v0 << 48);
 }
 
-__global__ void k_lut64(const float4* __restrict__ lut, int64_t j0, int64_t j1, int64_t n, int piece,
-                        uint64_t* __restrict__ out) {
-    const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    uint64_t v = 0;
+__global__ void k_syrk_tables(const float4* __restrict__ lut, int64_t base, int64_t n, int64_t j0, int64_t j1,
+                              int form, SyrkTables tb) {
+    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const int64_t j = base + k;
+    uint64_t out[4] = {0, 0, 0, 0};
+    double cor[3] = {0.0, 0.0, 0.0};
     if (j >= j0 && j < j1) {
         const float4 L = lut[j];
-        const uint64_t l0 = bf16_piece(L.x, piece);
-        const uint64_t l1 = bf16_piece(L.y, piece);
-        const uint64_t l2 = bf16_piece(L.z, piece);
-        v = l2 | (0ull << 16) | (l1 << 32) | (l0 << 48);   // codes 00, 01, 10, 11
+        const float z[3] = {L.x, L.y, L.z};
+        if (form != SYRK_FP32) {
+            uint64_t hi[3], lo[3];
+#pragma unroll
+            for (int g = 0; g < 3; g++) {
+                const __hip_bfloat16 h = __float2bfloat16(z[g]);
+                hi[g] = __bfloat16_as_ushort(h);
+                lo[g] = __bfloat16_as_ushort(__float2bfloat16(__fsub_rn(z[g], __bfloat162float(h))));
+            }
+            out[0] = four_codes(hi[0], hi[1], hi[2]);
+            out[1] = four_codes(lo[0], lo[1], lo[2]);
+        } else {
+            const double alpha = z[0], beta = 0.5 * ((double)z[2] - (double)z[0]);
+            // the mean genotype is -alpha / beta
+            const double c = beta > 0.0 ? fmin(fmax(rint(-alpha / beta), 0.0), 2.0) : 0.0;
+            out[0] = four_codes(bf16_code(0.0 - c), bf16_code(1.0 - c), bf16_code(2.0 - c));
+            uint64_t pc[3][3];
+#pragma unroll
+            for (int g = 0; g < 3; g++) {
+                double x = beta * (double)z[g];
+                cor[g] = -(alpha + beta * c) * (double)z[g];
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    const __hip_bfloat16 h = __float2bfloat16((float)x);
+                    pc[q][g] = __bfloat16_as_ushort(h);
+                    x -= (double)__bfloat162float(h);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 3; q++) out[1 + q] = four_codes(pc[q][0], pc[q][1], pc[q][2]);
+        }
     }
-    out[j] = v;
+    for (int q = 0; q < 4; q++)
+        if (tb.t[q]) tb.t[q][k] = out[q];
+    if (tb.corr)
+        for (int g = 0; g < 3; g++) tb.corr[3 * k + g] = cor[g];
+}
+
+// SYRK_FP32's column terms: per sample the FP64 sum of corr over the markers'
+// genotypes.  k_center_part: 16 samples (a dword of codes) per lane, one wave
+// per 1024 samples and slice of the markers, four rows' loads in flight;
+// k_center_sum adds the slices in order.
+__global__ __launch_bounds__(64) void k_center_part(const uint8_t* __restrict__ packed, int64_t ldp,
+                                                    const double* __restrict__ corr, int64_t base, int64_t n,
+                                                    int64_t per, int64_t Npad, double* __restrict__ part) {
+    const int64_t d = blockIdx.x * (int64_t)64 + threadIdx.x;    // dword of the row
+    if (16 * d >= Npad) return;                                  // ldp >= Npad / 4
+    const int64_t a = blockIdx.y * per, b = min(a + per, n);
+    const uint8_t* src = packed + base * ldp + 4 * d;
+    double s[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) s[i] = 0.0;
+    for (int64_t j = a; j < b; j += 4) {
+        uint32_t w[4];
+        double c[4][3];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int64_t jj = min(j + u, b - 1);
+            const double on = j + u < b ? 1.0 : 0.0;
+            w[u] = *reinterpret_cast<const uint32_t*>(src + jj * ldp);
+#pragma unroll
+            for (int g = 0; g < 3; g++) c[u][g] = on * corr[3 * jj + g];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const uint32_t v = w[u] >> (2 * i);
+                s[i] += (v & 2u) ? ((v & 1u) ? c[u][0] : c[u][1]) : c[u][2];
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) part[blockIdx.y * Npad + 16 * d + i] = s[i];
+}
+
+__global__ __launch_bounds__(256) void k_center_sum(const double* __restrict__ part, int64_t nslice, int64_t Npad,
+                                                    int64_t Nnm, float* __restrict__ center) {
+    // 32 samples per workgroup, eight threads each: thread q adds slices q, q + 8, ...
+    __shared__ double sm[8][32];
+    const int l = threadIdx.x & 31, q = threadIdx.x >> 5;
+    const int64_t i = blockIdx.x * (int64_t)32 + l;              // Npad is a multiple of 32
+    double s = 0.0;
+#pragma unroll 8
+    for (int64_t k = q; k < nslice; k += 8) s += part[k * Npad + i];
+    sm[q][l] = s;
+    __syncthreads();
+    if (q == 0) {
+#pragma unroll
+        for (int k = 1; k < 8; k++) s += sm[k][l];
+        center[i] = i < Nnm ? (float)s : 0.0f;
+    }
 }
 
 // Copy each diagonal tile's lower half onto its upper half: S[c][r] =
@@ -629,141 +665,100 @@ __global__ __launch_bounds__(256) void k_grm_block(const float* __restrict__ S, 
             if (j0 + e < nc) out[i * nc + j0 + e] = div_rn(S[i * ld + j0 + e], m);
 }
 
-// ------------------------------------------------------------------ FP32
-constexpr int BK32 = 32;            // markers per K chunk
-constexpr int P32 = BK32 + 4;       // LDS row pitch (floats)
-// LDS element (row, k) lives at row*P32 + (k&1)*16 + (k>>1), so lane l's
-// k = 2s + l/32 sequence over s is contiguous (four b128 reads per chunk).
-
-__global__ __launch_bounds__(256) void k_syrk_f32(const float* __restrict__ Zp, int64_t ldz, int64_t kdim,
-                                                  const int2* __restrict__ tiles, int64_t nblk,
-                                                  float* __restrict__ S, int64_t ldS, int accumulate) {
-    __shared__ __attribute__((aligned(16))) float sA[BT * P32];
-    __shared__ __attribute__((aligned(16))) float sB[BT * P32];
-    const int2 t = tiles[xcd_remap(blockIdx.x, nblk)];
-    const int64_t bi = t.x, bj = t.y;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wr = wv >> 1, wc = wv & 1;
-
-    // 16-byte chunk c = tid + 256 q: row c/8, k (c%8)*4
-    const int lrow = tid >> 3, lk = (tid & 7) * 4;
-    const float* gA = Zp + (bi * BT + lrow) * ldz + lk;
-    const float* gB = Zp + (bj * BT + lrow) * ldz + lk;
-    float4 ra[4], rb[4];
-    const int64_t nk = kdim / BK32;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        ra[q] = *reinterpret_cast<const float4*>(gA + (int64_t)(32 * q) * ldz);
-        rb[q] = *reinterpret_cast<const float4*>(gB + (int64_t)(32 * q) * ldz);
-    }
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-        for (int ni = 0; ni < 2; ni++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[mi][ni][r] = 0.0f;
-
-    const int hk = lk >> 1;  // k/2 of the chunk's first element
-    for (int64_t kc = 0; kc < nk; kc++) {
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            float* a = sA + (lrow + 32 * q) * P32;
-            float* b = sB + (lrow + 32 * q) * P32;
-            *reinterpret_cast<float2*>(a + hk) = make_float2(ra[q].x, ra[q].z);
-            *reinterpret_cast<float2*>(a + 16 + hk) = make_float2(ra[q].y, ra[q].w);
-            *reinterpret_cast<float2*>(b + hk) = make_float2(rb[q].x, rb[q].z);
-            *reinterpret_cast<float2*>(b + 16 + hk) = make_float2(rb[q].y, rb[q].w);
-        }
-        __syncthreads();
-        {
-            const int64_t off = ((kc + 1 < nk) ? kc + 1 : kc) * BK32;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                ra[q] = *reinterpret_cast<const float4*>(gA + (int64_t)(32 * q) * ldz + off);
-                rb[q] = *reinterpret_cast<const float4*>(gB + (int64_t)(32 * q) * ldz + off);
-            }
-        }
-        const int h = (lane >> 5) * 16;
-#pragma unroll
-        for (int sq = 0; sq < 4; sq++) {
-            float4 fa[2], fb[2];
-#pragma unroll
-            for (int mi = 0; mi < 2; mi++)
-                fa[mi] = *reinterpret_cast<const float4*>(sA + (wr * 64 + mi * 32 + (lane & 31)) * P32 + h + 4 * sq);
-#pragma unroll
-            for (int ni = 0; ni < 2; ni++)
-                fb[ni] = *reinterpret_cast<const float4*>(sB + (wc * 64 + ni * 32 + (lane & 31)) * P32 + h + 4 * sq);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-#pragma unroll
-                for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-                    for (int ni = 0; ni < 2; ni++)
-                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[mi][e], fb[ni][e], acc[mi][ni], 0, 0, 0);
-            }
-        }
-    }
-    store_tile(S, ldS, bi, bj, wr, wc, lane, acc, accumulate);
-}
-
 }  // namespace
 
-int syrk_kchunk_f32() { return BK32; }
 int syrk_kchunk_bf16() { return BK16; }
 
-hipError_t launch_pack_tiles(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t Mqc, int64_t Nnm,
-                             int64_t Npad, int64_t ldp, uint8_t* tp, uint64_t* lut64) {
-    const int64_t nchunk = (Mqc + 63) / 64;
-    hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)(Npad / BT), (unsigned)nchunk), dim3(256), 0, s, packed, Mqc,
-                       Nnm, ldp, nchunk, tp);
+// slices of the markers in k_center_part: enough waves to fill the chip,
+// at least 32 markers each
+static int64_t center_slices(int64_t n, int64_t Npad) {
+    const int64_t blocks = (Npad + 1023) / 1024;
+    return std::max<int64_t>(1, std::min<int64_t>({(n + 31) / 32, (2048 + blocks - 1) / blocks, (int64_t)512}));
+}
+
+hipError_t SyrkOperands::build(hipStream_t s, int form_, const uint8_t* packed, const float4* lut, int64_t Mqc,
+                               int64_t Nnm, int64_t Npad_, int64_t ldp, int64_t j0, int64_t j1) {
+    release();
+    if (j0 < 0 || j1 > Mqc || j0 >= j1 || Npad_ % 256 != 0 || 4 * ldp < Npad_) return hipErrorInvalidValue;
+    form = form_;
+    Npad = Npad_;
+    const int64_t c0 = j0 / 64;
+    nchunk = (j1 + 63) / 64 - c0;
+    const int64_t npanel = Npad / BT, n = nchunk * 64;
+    const int ntab = form == SYRK_HI ? 1 : (form == SYRK_SPLIT ? 2 : 4);
+    const int64_t nsl = form == SYRK_FP32 ? center_slices(n, Npad) : 0;
+    // one block: tiled genotypes, tables, then (SYRK_FP32) corr, center, slices
+    const int64_t b_tp = npanel * nchunk * 2048, b_tab = 8 * n;
+    const int64_t b_cor = nsl ? round_up(24 * n, 256) : 0, b_cen = nsl ? round_up(4 * Npad, 256) : 0;
+    hipError_t e = hipMalloc(&block, (size_t)(b_tp + ntab * b_tab + b_cor + b_cen + 8 * nsl * Npad));
+    if (e != hipSuccess) {
+        block = nullptr;
+        return e;
+    }
+    uint8_t* p = static_cast<uint8_t*>(block);
+    tp = p;
+    p += b_tp;
+    for (int q = 0; q < ntab; q++, p += b_tab) tb.t[q] = reinterpret_cast<uint64_t*>(p);
+    double* part = nullptr;
+    if (nsl) {
+        tb.corr = reinterpret_cast<double*>(p);
+        tb.center = reinterpret_cast<float*>(p + b_cor);
+        part = reinterpret_cast<double*>(p + b_cor + b_cen);
+    }
+    hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)((npanel + 3) / 4), (unsigned)nchunk), dim3(256), 0, s, packed,
+                       Mqc, Nnm, ldp, npanel, c0, nchunk, tp);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_syrk_tables, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, lut, c0 * 64, n, j0, j1,
+                       form, tb);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (nsl) {
+        const int64_t per = round_up((n + nsl - 1) / nsl, 4);
+        hipLaunchKernelGGL(k_center_part, dim3((unsigned)((Npad + 1023) / 1024), (unsigned)nsl), dim3(64), 0, s, packed,
+                           ldp, tb.corr, c0 * 64, n, per, Npad, part);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL(k_center_sum, dim3((unsigned)(Npad / 32)), dim3(256), 0, s, part, nsl, Npad, Nnm,
+                           tb.center);
+    }
+    return hipGetLastError();
+}
+
+void SyrkOperands::release() {
+    if (block) (void)hipFree(block);
+    *this = SyrkOperands{};
+}
+
+template <int T, int F>
+static void launch_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, int accumulate) {
+    constexpr int BK = T == 64 ? 64 : 32;
+    const int64_t nt = op.Npad / T, nblk = nt * (nt + 1) / 2;
+    hipLaunchKernelGGL((k_syrk_pk<T, F>), dim3((unsigned)nblk), dim3(T == 256 ? 512 : 256), 0, s, op.tp, op.nchunk,
+                       (int64_t)0, op.nchunk * (64 / BK), op.tb, tiles, nblk, S, op.Npad, accumulate);
+}
+
+hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, int accumulate,
+                          int tile) {
+    if ((tile != 64 && tile != BT && tile != BT2) || op.Npad % tile != 0 || !op.block) return hipErrorInvalidValue;
+    if (op.form == SYRK_HI && tile == BT2) {
+        const int64_t nt = op.Npad / BT2, nblk = nt * (nt + 1) / 2;
+        hipLaunchKernelGGL(k_syrk_pk256, dim3((unsigned)nblk), dim3(512), 0, s, op.tp, op.nchunk, (int64_t)0, op.nchunk,
+                           op.tb.t[0], tiles, nblk, S, op.Npad, accumulate);
+    } else if (op.form == SYRK_HI) {
+        if (tile == BT) launch_pk<128, SYRK_HI>(s, op, tiles, S, accumulate);
+        else launch_pk<64, SYRK_HI>(s, op, tiles, S, accumulate);
+    } else if (op.form == SYRK_SPLIT) {
+        if (tile == BT2) launch_pk<256, SYRK_SPLIT>(s, op, tiles, S, accumulate);
+        else if (tile == BT) launch_pk<128, SYRK_SPLIT>(s, op, tiles, S, accumulate);
+        else launch_pk<64, SYRK_SPLIT>(s, op, tiles, S, accumulate);
+    } else {
+        if (tile == BT2) launch_pk<256, SYRK_FP32>(s, op, tiles, S, accumulate);
+        else if (tile == BT) launch_pk<128, SYRK_FP32>(s, op, tiles, S, accumulate);
+        else launch_pk<64, SYRK_FP32>(s, op, tiles, S, accumulate);
+    }
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_lut64, dim3((unsigned)((nchunk * 64 + 255) / 256)), dim3(256), 0, s, lut, (int64_t)0, Mqc,
-                       nchunk * 64, 0, lut64);
-    return hipGetLastError();
-}
-
-hipError_t launch_lut64_range(hipStream_t s, const float4* lut, int64_t Mqc, int64_t j0, int64_t j1, int piece,
-                              uint64_t* lut64) {
-    const int64_t nchunk = (Mqc + 63) / 64;
-    hipLaunchKernelGGL(k_lut64, dim3((unsigned)((nchunk * 64 + 255) / 256)), dim3(256), 0, s, lut, j0, j1,
-                       nchunk * 64, piece, lut64);
-    return hipGetLastError();
-}
-
-hipError_t launch_syrk_pk(hipStream_t s, const uint8_t* tp, const uint64_t* lut64, int64_t Mqc, int64_t Npad,
-                          const int2* tiles, float* S, int accumulate, int64_t j0, int64_t j1, int tile) {
-    if ((tile != BT && tile != BT2) || Npad % tile != 0) return hipErrorInvalidValue;
-    const int64_t nt = Npad / tile;
-    const int64_t nblk = nt * (nt + 1) / 2;
-    const int64_t nchunk = (Mqc + 63) / 64;
-    if (j1 < 0) j1 = Mqc;
-    const int64_t c0 = j0 / 64, c1 = (j1 + 63) / 64;
-    if (c0 >= c1) return hipSuccess;
-    if (tile == BT2)
-        hipLaunchKernelGGL(k_syrk_pk256, dim3((unsigned)nblk), dim3(512), 0, s, tp, nchunk, c0, c1, lut64, tiles,
-                           nblk, S, Npad, accumulate);
-    else
-        hipLaunchKernelGGL(k_syrk_pk, dim3((unsigned)nblk), dim3(256), 0, s, tp, nchunk, c0, c1, lut64, tiles,
-                           nblk, S, Npad, accumulate);
-    return hipGetLastError();
-}
-
-hipError_t launch_syrk_pk_split(hipStream_t s, const uint8_t* tp, const uint64_t* lhi, const uint64_t* llo,
-                                int64_t Mqc, int64_t Npad, const int2* tiles, float* S, int accumulate, int64_t j0,
-                                int64_t j1) {
-    if (Npad % BT2 != 0 || !lhi || !llo) return hipErrorInvalidValue;
-    const int64_t nt = Npad / BT2;
-    const int64_t nblk = nt * (nt + 1) / 2;
-    const int64_t nchunk = (Mqc + 63) / 64;
-    if (j1 < 0) j1 = Mqc;
-    const int64_t k0 = j0 / BKS, k1 = (j1 + BKS - 1) / BKS;
-    if (k0 >= k1) return hipSuccess;
-    hipLaunchKernelGGL(k_syrk_pk256_split, dim3((unsigned)nblk), dim3(512), 0, s, tp, nchunk, k0, k1, lhi, llo,
-                       tiles, nblk, S, Npad, accumulate);
-    return hipGetLastError();
+    // the multi-piece forms reach a diagonal tile's two mirror entries by
+    // different sums: keep S exactly symmetric
+    if (e == hipSuccess && op.form != SYRK_HI) e = launch_mirror_diag(s, S, op.Npad, tile);
+    return e;
 }
 
 hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile) {
@@ -779,12 +774,26 @@ hipError_t launch_grm_block(hipStream_t s, const float* S, int64_t ld, int64_t n
     return hipGetLastError();
 }
 
-// Tile edge of the 2-bit-input SYRK: 256 unless SAIGE_SYRK_TILE=128 (the
-// tests compare the two, which are bitwise equal).
-int syrk_pk_tile() {
-    if (const char* env = std::getenv("SAIGE_SYRK_TILE"))
-        if (std::atoi(env) == BT) return BT;
-    return BT2;
+// Tile edge of the 2-bit-input SYRK at Npad rows (every size gives the same
+// bits): the one of least time by a model of rounds on 256 CUs, in us for the
+// split form over 8192 markers.  A 256 tile fills a CU and takes 525 us
+// whatever their number up to 256; two 128 tiles share a CU (390 us; 290 us
+// alone); 64 tiles run at 0.36 us each, at least 130 us.  Measured us at
+// N = 1000, 2000, 3000, 4000, 8000, 20,000: 64 tiles 144, 292, 454, 726, 2477,
+// 13,996; 128 tiles 293, 301, 394, 644, 1708, 9335; 256 tiles 534, 538, 548,
+// 556, 1745, 8053; the other forms cross at the same places.
+// SAIGE_SYRK_TILE=64, 128 or 256 sets it (the tests compare them).
+int syrk_pk_tile(int64_t Npad) {
+    if (const char* env = std::getenv("SAIGE_SYRK_TILE")) {
+        const int t = std::atoi(env);
+        if (t == 64 || t == BT || t == BT2) return t;
+    }
+    auto tiles = [&](int64_t T) { return (double)(Npad / T) * (double)(Npad / T + 1) / 2.0; };
+    const double t256 = 525.0 * std::ceil(tiles(256) / 256.0);
+    const double t128 = tiles(128) <= 256.0 ? 290.0 : 390.0 * std::ceil(tiles(128) / 512.0);
+    const double t64 = std::max(130.0, 60.0 + 0.36 * tiles(64));
+    if (t256 <= t128 && t256 <= t64) return BT2;
+    return t128 <= t64 ? BT : 64;
 }
 
 int syrk_tile() { return BT; }
@@ -808,15 +817,6 @@ hipError_t launch_syrk_bf16(hipStream_t s, const __hip_bfloat16* Zp, int64_t Npa
     const int64_t nt = Npad / BT;
     const int64_t nblk = nt * (nt + 1) / 2;
     hipLaunchKernelGGL(k_syrk_bf16, dim3((unsigned)nblk), dim3(256), 0, s, Zp, ldz, kdim, tiles, nblk, S, Npad,
-                       accumulate);
-    return hipGetLastError();
-}
-
-hipError_t launch_syrk_f32(hipStream_t s, const float* Zp, int64_t Npad, int64_t ldz, int64_t kdim,
-                           const int2* tiles, float* S, int accumulate) {
-    const int64_t nt = Npad / BT;
-    const int64_t nblk = nt * (nt + 1) / 2;
-    hipLaunchKernelGGL(k_syrk_f32, dim3((unsigned)nblk), dim3(256), 0, s, Zp, ldz, kdim, tiles, nblk, S, Npad,
                        accumulate);
     return hipGetLastError();
 }

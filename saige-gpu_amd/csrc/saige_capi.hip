@@ -1075,19 +1075,36 @@ int saige_get_diag_of_kin(saige_ctx* c, float* out) {
     return SAIGE_OK;
 }
 
-// The 2-bit-input SYRK over markers [j0, j1) into S: one pass with the BF16
-// table (hi), or, for the split GRM (llo given), hi x hi + hi x lo + lo x hi
-// in one pass over both tables.  accumulate: 0 store, +1 add, -1 subtract.
-static hipError_t syrk_pk_passes(hipStream_t st, const uint8_t* tp, const uint64_t* lhi, const uint64_t* llo,
-                                 int64_t Mqc, int64_t Np, const int2* tiles, float* S, int accumulate, int64_t j0,
-                                 int64_t j1, int tile) {
-    if (!llo) return launch_syrk_pk(st, tp, lhi, Mqc, Np, tiles, S, accumulate, j0, j1, tile);
-    hipError_t e = launch_syrk_pk_split(st, tp, lhi, llo, Mqc, Np, tiles, S, accumulate, j0, j1);
-    // the cross terms reach a diagonal tile's mirror entries in opposite
-    // orders: keep S exactly symmetric
-    if (e == hipSuccess) e = launch_mirror_diag(st, S, Np, tile);
+namespace {
+// S (= / += / -=) the GRM part of markers [j0, j1) from the 2-bit genotypes, in
+// the operand form of `precision` (accumulate: 0, 1, -1).  Waits for the
+// stream; t (may be null): device seconds between its start and end.
+hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1, float* S, int accumulate, double* t) {
+    hipStream_t st = c->stream;
+    const int64_t Np = c->Npad;
+    const int form = precision == SAIGE_GRM_FP32 ? SYRK_FP32 : (precision == SAIGE_GRM_BF16_SPLIT ? SYRK_SPLIT : SYRK_HI);
+    const int tile = syrk_pk_tile(Np);
+    // super-blocks of 1024 rows in the dispatch order
+    const std::vector<int2> order = syrk_tile_order(Np / tile, 1024 / tile);
+    SyrkOperands op;
+    int2* d_tiles = nullptr;
+    hipError_t e = dalloc(&d_tiles, (int64_t)order.size());
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(d_tiles, order.data(), sizeof(int2) * order.size(), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess && t) e = hipEventRecord(c->ev0, st);
+    if (e == hipSuccess) e = op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j0, j1);
+    if (e == hipSuccess) e = launch_syrk_pk(st, op, d_tiles, S, accumulate, tile);
+    if (e == hipSuccess && t) e = hipEventRecord(c->ev1, st);
+    const hipError_t w = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = w;
+    op.release();
+    dfree(d_tiles);
+    float ms = 0.f;
+    if (e == hipSuccess && t) e = hipEventElapsedTime(&ms, c->ev0, c->ev1);
+    if (e == hipSuccess && t) *t = ms * 1e-3;
     return e;
 }
+}  // namespace
 
 int saige_build_grm(saige_ctx* c, int precision) {
     CHECK_CTX(c);
@@ -1114,50 +1131,23 @@ int saige_build_grm(saige_ctx* c, int precision) {
     c->grm_ready = false;
     c->loco_ready = false;   // S_loco derives from S
     c->loco_inplace = false;
-    if (precision == SAIGE_GRM_BF16 || precision == SAIGE_GRM_BF16_SPLIT) {
+    if (precision != SAIGE_GRM_BF16_PANEL) {
         // 2-bit operands straight into the MFMA SYRK: no Z panel
-        const bool split = precision == SAIGE_GRM_BF16_SPLIT;
-        const int64_t nchunk = (c->Mqc + 63) / 64;
-        uint8_t* d_tp = nullptr;
-        uint64_t *d_l64 = nullptr, *d_llo = nullptr;
-        int2* d_tiles = nullptr;
-        const int tile = split ? 256 : syrk_pk_tile();   // the split kernel: 256 tiles only
-        const std::vector<int2> order = syrk_tile_order(Np / tile, tile == 256 ? 4 : 8);
-        auto release = [&]() { dfree(d_tp); dfree(d_l64); dfree(d_llo); dfree(d_tiles); };
-        if (dalloc(&d_tp, (Np / syrk_tile()) * nchunk * 2048) || dalloc(&d_l64, nchunk * 64) ||
-            (split && dalloc(&d_llo, nchunk * 64)) || dalloc(&d_tiles, (int64_t)order.size())) {
-            release();
-            set_error("cannot allocate the tiled genotypes for the SYRK");
-            return SAIGE_E_NOMEM;
-        }
-        hipError_t e = hipMemcpyAsync(d_tiles, order.data(), sizeof(int2) * order.size(), hipMemcpyHostToDevice, st);
-        if (e == hipSuccess) e = hipEventRecord(c->ev0, st);
-        if (e == hipSuccess) e = launch_pack_tiles(st, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, d_tp, d_l64);
-        if (e == hipSuccess && split) e = launch_lut64_range(st, c->d_lut, c->Mqc, 0, c->Mqc, 1, d_llo);
-        if (e == hipSuccess)
-            e = syrk_pk_passes(st, d_tp, d_l64, d_llo, c->Mqc, Np, d_tiles, c->d_grm, 0, 0, -1, tile);
-        if (e == hipSuccess) e = hipEventRecord(c->ev1, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        release();
+        const hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, 0, &c->grm_seconds);
         if (e != hipSuccess) {
             set_error("GRM build failed: %s", hipGetErrorString(e));
-            return SAIGE_E_DEVICE;
+            return e == hipErrorOutOfMemory ? SAIGE_E_NOMEM : SAIGE_E_DEVICE;
         }
-        float ms = 0.f;
-        SAIGE_HIP_TRY(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-        c->grm_seconds = ms * 1e-3;
         c->grm_ready = true;
         c->grm_precision = precision;
         return SAIGE_OK;
     }
-    const bool bf16 = precision == SAIGE_GRM_BF16_PANEL;
-    const int64_t esz = bf16 ? 2 : 4;
-    const int64_t kc = bf16 ? syrk_kchunk_bf16() : syrk_kchunk_f32();
+    const int64_t kc = syrk_kchunk_bf16();
     size_t free_b = 0, total_b = 0;
     SAIGE_HIP_TRY(hipMemGetInfo(&free_b, &total_b));
     // panel budget: at most 32 GB and half of what is free
     int64_t budget = std::min<int64_t>((int64_t)32 << 30, (int64_t)(free_b / 2));
-    int64_t pw = budget / (Np * esz);
+    int64_t pw = budget / (Np * 2);
     pw = std::max<int64_t>(kc, pw / 64 * 64);
     const int64_t full = round_up(c->Mqc, 64);
     pw = std::min(pw, full);
@@ -1168,7 +1158,7 @@ int saige_build_grm(saige_ctx* c, int precision) {
         pw = std::min(pw, cap);
     }
     void* d_panel = nullptr;
-    SAIGE_HIP_TRY(hipMalloc(&d_panel, (size_t)(Np * pw * esz)));
+    SAIGE_HIP_TRY(hipMalloc(&d_panel, (size_t)(Np * pw * 2)));
     const std::vector<int2> order = syrk_tile_order(Np / syrk_tile(), 8);
     int2* d_tiles = nullptr;
     if (dalloc(&d_tiles, (int64_t)order.size()) ||
@@ -1184,18 +1174,10 @@ int saige_build_grm(saige_ctx* c, int precision) {
     for (int64_t j0 = 0; j0 < c->Mqc && e == hipSuccess; j0 += pw) {
         const int64_t np = std::min(pw, c->Mqc - j0);
         const int64_t ldz = round_up(np, 64);
-        if (bf16) {
-            e = launch_std_panel_bf16(st, c->d_packed, c->d_lut, j0, np, c->Nnm, Np, c->ldp, ldz,
-                                      static_cast<__hip_bfloat16*>(d_panel));
-            if (e == hipSuccess)
-                e = launch_syrk_bf16(st, static_cast<__hip_bfloat16*>(d_panel), Np, ldz, ldz, d_tiles, c->d_grm,
-                                     !first);
-        } else {
-            e = launch_std_panel_f32(st, c->d_packed, c->d_lut, j0, np, c->Nnm, Np, c->ldp, ldz,
-                                     static_cast<float*>(d_panel));
-            if (e == hipSuccess)
-                e = launch_syrk_f32(st, static_cast<float*>(d_panel), Np, ldz, ldz, d_tiles, c->d_grm, !first);
-        }
+        e = launch_std_panel_bf16(st, c->d_packed, c->d_lut, j0, np, c->Nnm, Np, c->ldp, ldz,
+                                  static_cast<__hip_bfloat16*>(d_panel));
+        if (e == hipSuccess)
+            e = launch_syrk_bf16(st, static_cast<__hip_bfloat16*>(d_panel), Np, ldz, ldz, d_tiles, c->d_grm, !first);
         first = 0;
     }
     if (e == hipSuccess) e = hipEventRecord(c->ev1, st);
@@ -1482,66 +1464,38 @@ int saige_pcg_block(saige_ctx* c, const float* w, const float* tau, const float*
 namespace {
 // S (+/-)= Z_r Z_r^T over GRM markers [start, end], with the kernel and
 // operand precision the resident S was built with (accumulate: 1 add, -1
-// subtract).  Asynchronous on the context's stream.
+// subtract).
 hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, int accumulate) {
+    if (c->grm_precision != SAIGE_GRM_BF16_PANEL)
+        return syrk_from_packed(c, c->grm_precision, start, end + 1, S, accumulate, nullptr);
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
     const int64_t cnt = end - start + 1;
-    const bool split = c->grm_precision == SAIGE_GRM_BF16_SPLIT;
-    const bool pk = c->grm_precision == SAIGE_GRM_BF16 || split;
-    const int tile = split ? 256 : (pk ? syrk_pk_tile() : syrk_tile());
-    const std::vector<int2> order = syrk_tile_order(Np / tile, tile == 256 ? 4 : 8);
+    const std::vector<int2> order = syrk_tile_order(Np / syrk_tile(), 8);
     int2* d_tiles = nullptr;
-    uint8_t* d_tp = nullptr;
-    uint64_t *d_l64 = nullptr, *d_llo = nullptr;
     void* d_panel = nullptr;
-    auto release = [&]() {
-        (void)hipStreamSynchronize(st);
-        dfree(d_tiles); dfree(d_tp); dfree(d_l64); dfree(d_llo);
-        if (d_panel) (void)hipFree(d_panel);
-    };
     hipError_t e = dalloc(&d_tiles, (int64_t)order.size());
     if (e == hipSuccess)
         e = hipMemcpyAsync(d_tiles, order.data(), sizeof(int2) * order.size(), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess && pk) {
-        const int64_t nchunk = (c->Mqc + 63) / 64;
-        e = dalloc(&d_tp, (Np / syrk_tile()) * nchunk * 2048);
-        if (e == hipSuccess) e = dalloc(&d_l64, nchunk * 64);
-        if (e == hipSuccess && split) e = dalloc(&d_llo, nchunk * 64);
-        if (e == hipSuccess) e = launch_pack_tiles(st, c->d_packed, c->d_lut, c->Mqc, N, Np, c->ldp, d_tp, d_l64);
-        if (e == hipSuccess) e = launch_lut64_range(st, c->d_lut, c->Mqc, start, end + 1, 0, d_l64);
-        if (e == hipSuccess && split) e = launch_lut64_range(st, c->d_lut, c->Mqc, start, end + 1, 1, d_llo);
+    const int64_t kc = syrk_kchunk_bf16();
+    size_t free_b = 0, total_b = 0;
+    if (e == hipSuccess) e = hipMemGetInfo(&free_b, &total_b);
+    int64_t pw = std::min<int64_t>((int64_t)32 << 30, (int64_t)(free_b / 2)) / (Np * 2);
+    pw = std::min(std::max<int64_t>(kc, pw / 64 * 64), round_up(cnt, 64));
+    if (const char* env = std::getenv("SAIGE_GRM_PANEL_MARKERS"))
+        pw = std::min(pw, std::max<int64_t>(64, std::atoll(env) / 64 * 64));
+    if (e == hipSuccess) e = hipMalloc(&d_panel, (size_t)(Np * pw * 2));
+    for (int64_t j0 = start; j0 <= end && e == hipSuccess; j0 += pw) {
+        const int64_t np = std::min(pw, end + 1 - j0);
+        const int64_t ldz = round_up(np, 64);
+        e = launch_std_panel_bf16(st, c->d_packed, c->d_lut, j0, np, N, Np, c->ldp, ldz,
+                                  static_cast<__hip_bfloat16*>(d_panel));
         if (e == hipSuccess)
-            e = syrk_pk_passes(st, d_tp, d_l64, d_llo, c->Mqc, Np, d_tiles, S, accumulate, start, end + 1, tile);
-    } else if (e == hipSuccess) {
-        const bool bf16 = c->grm_precision == SAIGE_GRM_BF16_PANEL;
-        const int64_t esz = bf16 ? 2 : 4;
-        const int64_t kc = bf16 ? syrk_kchunk_bf16() : syrk_kchunk_f32();
-        size_t free_b = 0, total_b = 0;
-        e = hipMemGetInfo(&free_b, &total_b);
-        int64_t pw = std::min<int64_t>((int64_t)32 << 30, (int64_t)(free_b / 2)) / (Np * esz);
-        pw = std::min(std::max<int64_t>(kc, pw / 64 * 64), round_up(cnt, 64));
-        if (const char* env = std::getenv("SAIGE_GRM_PANEL_MARKERS"))
-            pw = std::min(pw, std::max<int64_t>(64, std::atoll(env) / 64 * 64));
-        if (e == hipSuccess) e = hipMalloc(&d_panel, (size_t)(Np * pw * esz));
-        for (int64_t j0 = start; j0 <= end && e == hipSuccess; j0 += pw) {
-            const int64_t np = std::min(pw, end + 1 - j0);
-            const int64_t ldz = round_up(np, 64);
-            if (bf16) {
-                e = launch_std_panel_bf16(st, c->d_packed, c->d_lut, j0, np, N, Np, c->ldp, ldz,
-                                          static_cast<__hip_bfloat16*>(d_panel));
-                if (e == hipSuccess)
-                    e = launch_syrk_bf16(st, static_cast<__hip_bfloat16*>(d_panel), Np, ldz, ldz, d_tiles, S,
-                                         accumulate);
-            } else {
-                e = launch_std_panel_f32(st, c->d_packed, c->d_lut, j0, np, N, Np, c->ldp, ldz,
-                                         static_cast<float*>(d_panel));
-                if (e == hipSuccess)
-                    e = launch_syrk_f32(st, static_cast<float*>(d_panel), Np, ldz, ldz, d_tiles, S, accumulate);
-            }
-        }
+            e = launch_syrk_bf16(st, static_cast<__hip_bfloat16*>(d_panel), Np, ldz, ldz, d_tiles, S, accumulate);
     }
-    release();
+    (void)hipStreamSynchronize(st);
+    dfree(d_tiles);
+    if (d_panel) (void)hipFree(d_panel);
     return e;
 }
 }  // namespace

@@ -195,6 +195,30 @@ struct KeptBlock {
     }
 };
 
+// lookup tables of the 2-bit-input SYRK, one entry per marker of its chunks
+// (k_syrk_tables), and the FP32 form's column terms
+struct SyrkTables {
+    uint64_t* t[4] = {nullptr, nullptr, nullptr, nullptr};
+    double* corr = nullptr;        // [markers][3]
+    float* center = nullptr;       // [Npad]
+};
+
+// The operands of a 2-bit-input SYRK over markers [j0, j1): the genotypes
+// re-tiled ((Npad / 128) panels x nchunk chunks of 64 markers x 2 KB) and the
+// tables, in one device block.  build() only enqueues (packed and lut must stay
+// until the stream has run it); release() frees, with the stream idle.
+enum SyrkForm { SYRK_HI = 0, SYRK_SPLIT = 1, SYRK_FP32 = 2 };
+struct SyrkOperands {
+    void* block = nullptr;
+    int form = SYRK_HI;
+    int64_t Npad = 0, nchunk = 0;
+    uint8_t* tp = nullptr;
+    SyrkTables tb;
+    hipError_t build(hipStream_t s, int form, const uint8_t* packed, const float4* lut, int64_t Mqc, int64_t Nnm,
+                     int64_t Npad, int64_t ldp, int64_t j0, int64_t j1);
+    void release();
+};
+
 }  // namespace saige
 
 struct saige_ctx {
@@ -290,6 +314,18 @@ inline int64_t round_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 __device__ __forceinline__ float div_rn(float a, float b) { return (float)((double)a / (double)b); }
 __device__ __forceinline__ float sqrt_rn(float a) { return (float)__builtin_sqrt((double)a); }
 
+// rows a..d of four bytes -> their byte columns: t[k] = byte k of a, b, c, d
+__device__ __forceinline__ void transpose4x4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t (&t)[4]) {
+    const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u);   // a0 b0 a1 b1
+    const uint32_t ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u);   // a2 b2 a3 b3
+    const uint32_t cd0 = __builtin_amdgcn_perm(d, c, 0x05010400u);
+    const uint32_t cd1 = __builtin_amdgcn_perm(d, c, 0x07030602u);
+    t[0] = __builtin_amdgcn_perm(cd0, ab0, 0x05040100u);
+    t[1] = __builtin_amdgcn_perm(cd0, ab0, 0x07060302u);
+    t[2] = __builtin_amdgcn_perm(cd1, ab1, 0x05040100u);
+    t[3] = __builtin_amdgcn_perm(cd1, ab1, 0x07060302u);
+}
+
 // wait for this wave's LDS traffic, then the workgroup barrier; outstanding
 // global loads stay in flight (__syncthreads would drain them)
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -313,11 +349,8 @@ hipError_t launch_std_geno(hipStream_t s, const uint8_t* packed_row, const float
                            int64_t Nnm, float* out);
 hipError_t launch_synth_bed(hipStream_t s, uint8_t* bed, int64_t N, int64_t M, float maf_lo,
                             float maf_hi, float miss, int64_t npairs, uint64_t seed);
-// Z panel [Npad][ldz] for markers [j0, j0+np) (np <= ldz; columns beyond np
-// and rows beyond Nnm are zero).  Element type float or bf16.
-hipError_t launch_std_panel_f32(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t j0,
-                                int64_t np, int64_t Nnm, int64_t Npad, int64_t ldp, int64_t ldz,
-                                float* Zp);
+// Z panel [Npad][ldz] in BF16 for markers [j0, j0+np) (np <= ldz; columns
+// beyond np and rows beyond Nnm are zero).
 hipError_t launch_std_panel_bf16(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t j0,
                                  int64_t np, int64_t Nnm, int64_t Npad, int64_t ldp, int64_t ldz,
                                  __hip_bfloat16* Zp);
@@ -326,36 +359,21 @@ hipError_t launch_std_panel_bf16(hipStream_t s, const uint8_t* packed, const flo
 // S (Npad x Npad, ld = Npad) (+)= Zp Zp^T over the lower-triangle tiles,
 // mirrored into the upper triangle.  kdim is a multiple of the kernel's k-chunk.
 // tiles: the lower-triangle tile list from syrk_tile_order(Npad / syrk_tile())
-hipError_t launch_syrk_f32(hipStream_t s, const float* Zp, int64_t Npad, int64_t ldz, int64_t kdim,
-                           const int2* tiles, float* S, int accumulate);
 hipError_t launch_syrk_bf16(hipStream_t s, const __hip_bfloat16* Zp, int64_t Npad, int64_t ldz,
                             int64_t kdim, const int2* tiles, float* S, int accumulate);
 std::vector<int2> syrk_tile_order(int64_t nt, int64_t g);
-// 2-bit-input SYRK: tp = tiled packed genotypes ((Npad/128) x nchunk x 2 KB,
-// nchunk = ceil(Mqc/64)), lut64 = nchunk*64 entries; both from launch_pack_tiles
-hipError_t launch_pack_tiles(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t Mqc, int64_t Nnm,
-                             int64_t Npad, int64_t ldp, uint8_t* tp, uint64_t* lut64);
-// markers [j0, j1) only (j1 < 0: all); lut64 must be zero outside the range.
-// accumulate: 0 overwrite, 1 add, -1 subtract.
-// tile: 128 or 256 (tiles from syrk_tile_order(Npad / tile, ...)).
-hipError_t launch_syrk_pk(hipStream_t s, const uint8_t* tp, const uint64_t* lut64, int64_t Mqc, int64_t Npad,
-                          const int2* tiles, float* S, int accumulate, int64_t j0, int64_t j1, int tile);
-int syrk_pk_tile();
+// the 2-bit-input SYRK of op on T x T tiles (64, 128 or 256; tiles from
+// syrk_tile_order(Npad / tile, ...)); accumulate: 0 overwrite, 1 add, -1
+// subtract.  S comes out exactly symmetric.
+hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, int accumulate,
+                          int tile);
+int syrk_pk_tile(int64_t Npad);
 // copy each diagonal tile's lower half onto its upper half (tile edge `tile`)
 hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile);
-// the split GRM in one pass over markers [j0, j1): hi.hi + hi.lo + lo.hi per
-// 32-marker chunk from the two tables (256 tiles; accumulate as launch_syrk_pk)
-hipError_t launch_syrk_pk_split(hipStream_t s, const uint8_t* tp, const uint64_t* lhi, const uint64_t* llo,
-                                int64_t Mqc, int64_t Npad, const int2* tiles, float* S, int accumulate, int64_t j0,
-                                int64_t j1);
-// piece 0: the values rounded to BF16 (hi); 1: the remainders rounded to BF16 (lo)
-hipError_t launch_lut64_range(hipStream_t s, const float4* lut, int64_t Mqc, int64_t j0, int64_t j1, int piece,
-                              uint64_t* lut64);
 // out[nr][nc] (contiguous) = S[i][j] / m for S at its block's first element
 hipError_t launch_grm_block(hipStream_t s, const float* S, int64_t ld, int64_t nr, int64_t nc, float m, float* out);
 hipError_t launch_sub(hipStream_t s, const float* a, const float* b, int64_t n, float* out);
 int syrk_tile();
-int syrk_kchunk_f32();
 int syrk_kchunk_bf16();
 
 // ---- PCG kernels (pcg_kernels.hip)
