@@ -406,7 +406,7 @@ int saige_engine_stats(const saige_ctx* ctx, int kind, double* gemm_seconds, int
 int saige_synth_bed_device(saige_ctx* ctx, void* bed_body_dev, int64_t N, int64_t M,
                            float maf_lo, float maf_hi, float miss_rate, float pair_frac,
                            uint64_t seed);
-/* Device allocation helper for the above (freed by saige_free_device). */
+/* Device allocation helper for the above, zeroed (freed by saige_free_device). */
 int saige_alloc_device(saige_ctx* ctx, int64_t bytes, void** out);
 int saige_free_device(saige_ctx* ctx, void* p);
 /* Page-locked host memory (freed by saige_free_host): host columns staged in

@@ -2177,6 +2177,16 @@ int saige_alloc_device(saige_ctx* c, int64_t bytes, void** out) {
         return SAIGE_E_ARG;
     }
     SAIGE_HIP_TRY(hipMalloc(out, (size_t)bytes));
+    // zeroed, so that what a caller reads before writing it does not depend on
+    // what the block held before
+    hipError_t e = hipMemsetAsync(*out, 0, (size_t)bytes, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) {
+        (void)hipFree(*out);
+        *out = nullptr;
+        set_error("clearing a device block failed: %s", hipGetErrorString(e));
+        return SAIGE_E_DEVICE;
+    }
     return SAIGE_OK;
 }
 
