@@ -33,23 +33,14 @@ __device__ __forceinline__ float wave_sum_f(float v) {
     return v;
 }
 
-// Sigma p for one element (getCrossprod, FG.cpp:2412): the reference forms
-// 1/w, then b % (1/w), then tau0 * that, plus tau1 * (K b); tau1 == 0
-// returns the first term alone (FG.cpp:2401-2404).
-__device__ __forceinline__ float sigma_elem(float p, float y, float winv, float tau0, float tau1,
-                                            float mqc) {
-    float t = __fmul_rn(tau0, __fmul_rn(p, winv));
-    if (tau1 == 0.0f) return t;
-    return __fadd_rn(t, __fmul_rn(tau1, div_rn(y, mqc)));
-}
-
 // --------------------------------------------------------------- GEMV
 constexpr int GEMV_ROWS = 4;  // rows (waves) per workgroup
 
 __global__ __launch_bounds__(256) void k_gemv(const float* __restrict__ S, int64_t ld, int64_t Nnm,
                                               const float* __restrict__ in, float* __restrict__ out,
-                                              SigmaArgs a, double* __restrict__ partial) {
+                                              VecArgs a, double* __restrict__ partial) {
     __shared__ double s_dot[GEMV_ROWS];
+    if (a.over && *a.over <= a.iter) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int64_t row = (int64_t)blockIdx.x * GEMV_ROWS + wv;
     const float4* Srow = reinterpret_cast<const float4*>(S + row * ld);
@@ -76,11 +67,8 @@ __global__ __launch_bounds__(256) void k_gemv(const float* __restrict__ S, int64
         if (a.mode == 0) {
             o = div_rn(y, a.mqc);
         } else {
-            const int s = a.sys[0];
-            const bool on = a.live[0] && row < Nnm && a.mask[(int64_t)s * ld + row];
             const float p = in[row];
-            o = on ? sigma_elem(p, y, a.winv[(int64_t)s * ld + row], a.tau[2 * s], a.tau[2 * s + 1], a.mqc)
-                   : 0.0f;
+            o = row < Nnm ? sigma_elem(p, y, a.winv[row], a.tau0, a.tau1, a.mqc) : 0.0f;
             d = (double)p * (double)o;
         }
         out[row] = o;
@@ -89,7 +77,7 @@ __global__ __launch_bounds__(256) void k_gemv(const float* __restrict__ S, int64
     if (a.mode == 1) {
         __syncthreads();
         if (threadIdx.x == 0)
-            partial[(int64_t)blockIdx.x * 2] = (s_dot[0] + s_dot[1]) + (s_dot[2] + s_dot[3]);
+            partial[blockIdx.x] = (s_dot[0] + s_dot[1]) + (s_dot[2] + s_dot[3]);
     }
 }
 
@@ -116,8 +104,10 @@ __host__ __device__ __forceinline__ int64_t triv_y2_first(int64_t c, int64_t NR)
 
 __global__ __launch_bounds__(512) void k_gemv_tri(const float* __restrict__ S, int64_t ld,
                                                   const float* __restrict__ x, const int4* __restrict__ items,
-                                                  float* __restrict__ y1p, float* __restrict__ y2p) {
+                                                  float* __restrict__ y1p, float* __restrict__ y2p,
+                                                  const int32_t* __restrict__ over, int iter) {
     __shared__ float4 sz[2][8][64];    // use-2 strip sums, two chunks
+    if (over && *over <= iter) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int4 item = items[blockIdx.x];
     const int64_t R = item.x, ca = item.y, cb = item.z, slot = item.w;
@@ -176,8 +166,9 @@ __global__ __launch_bounds__(512) void k_gemv_tri(const float* __restrict__ S, i
 __global__ __launch_bounds__(256) void k_gemv_tri_epi(const float* __restrict__ y1p, const float* __restrict__ y2p,
                                                       const int2* __restrict__ rtab, int64_t ld, int64_t Nnm,
                                                       const float* __restrict__ in, float* __restrict__ out,
-                                                      SigmaArgs a, double* __restrict__ partial) {
+                                                      VecArgs a, double* __restrict__ partial) {
     __shared__ double sm[256];
+    if (a.over && *a.over <= a.iter) return;
     const int tid = threadIdx.x;
     const int64_t R = blockIdx.x, row = R * TV_ROWS + tid, NR = ld / TV_ROWS;
     const int2 rt = rtab[R];
@@ -192,10 +183,8 @@ __global__ __launch_bounds__(256) void k_gemv_tri_epi(const float* __restrict__ 
     if (a.mode == 0) {
         o = div_rn(y, a.mqc);
     } else {
-        const int s = a.sys[0];
-        const bool on = a.live[0] && row < Nnm && a.mask[(int64_t)s * ld + row];
         const float p = in[row];
-        o = on ? sigma_elem(p, y, a.winv[(int64_t)s * ld + row], a.tau[2 * s], a.tau[2 * s + 1], a.mqc) : 0.0f;
+        o = row < Nnm ? sigma_elem(p, y, a.winv[row], a.tau0, a.tau1, a.mqc) : 0.0f;
         d = (double)p * (double)o;
     }
     out[row] = o;
@@ -205,7 +194,7 @@ __global__ __launch_bounds__(256) void k_gemv_tri_epi(const float* __restrict__ 
             __syncthreads();
             if (tid < st) sm[tid] += sm[tid + st];
         }
-        if (tid == 0) partial[R * 2] = sm[0];
+        if (tid == 0) partial[R] = sm[0];
     }
 }
 
@@ -1195,53 +1184,16 @@ __global__ __launch_bounds__(256) void k_sigma_setup(const float* __restrict__ w
     if (!on) {
         winv[i] = 0.f;
         minv[i] = 0.f;
-        mask_out[i] = 0;
+        if (mask_out) mask_out[i] = 0;
         if (dout) dout[i] = 0.f;
         return;
     }
     const float wi = w[i];
-    // getDiagOfSigma (FG.cpp:2335-2358): (tau1 * diag) / Mqc + tau0 / w, >= 1e-4
-    float d = diag_one ? __fadd_rn(tau1, div_rn(tau0, wi))
-                       : __fadd_rn(div_rn(__fmul_rn(tau1, diag[i]), mqc), div_rn(tau0, wi));
-    if (d < 1e-4f) d = 1e-4f;
+    const float d = sigma_diag(wi, diag, i, tau0, tau1, mqc, diag_one);
     if (dout) dout[i] = d;
     winv[i] = div_rn(1.0f, wi);
     minv[i] = div_rn(1.0f, d);   // minvVec = 1/getDiagOfSigma (FG.cpp:2637)
-    mask_out[i] = 1;
-}
-
-// Start column `slot`: x = 0, r = b, z = minv r, p = z (FG.cpp:2615-2690).
-__global__ __launch_bounds__(256) void k_col_init(const float* __restrict__ b, int slot, int kpad,
-                                                  int64_t Nnm, const float* __restrict__ minv,
-                                                  const uint8_t* __restrict__ mask, float* X, float* R,
-                                                  float* Z, float* P, double* __restrict__ partial) {
-    __shared__ double sm[2][256];
-    const int tid = threadIdx.x;
-    const int64_t i = (int64_t)blockIdx.x * VROWS + tid;
-    double rz = 0.0, rr = 0.0;
-    const bool on = i < Nnm && mask[i];
-    const float r = on ? b[i] : 0.0f;
-    const float z = __fmul_rn(minv[i], r);
-    const int64_t o = i * kpad + slot;
-    X[o] = 0.0f;
-    R[o] = r;
-    Z[o] = z;
-    P[o] = z;
-    rz = (double)z * (double)r;
-    rr = (double)r * (double)r;
-    sm[0][tid] = rz;
-    sm[1][tid] = rr;
-    for (int s = 128; s >= 1; s >>= 1) {
-        __syncthreads();
-        if (tid < s) {
-            sm[0][tid] += sm[0][tid + s];
-            sm[1][tid] += sm[1][tid + s];
-        }
-    }
-    if (tid == 0) {
-        partial[(int64_t)blockIdx.x * 2] = sm[0][0];
-        partial[(int64_t)blockIdx.x * 2 + 1] = sm[1][0];
-    }
+    if (mask_out) mask_out[i] = 1;
 }
 
 // Sum partial[p][col][comp] over p in a fixed order: one workgroup per
@@ -1260,23 +1212,6 @@ __device__ __forceinline__ double sum_parts(const double* partial, int64_t npart
     double r = sm[0];
     __syncthreads();
     return r;
-}
-
-__global__ __launch_bounds__(256) void k_col_init_finish(int slot, const double* __restrict__ partial,
-                                                         int64_t nparts, double* rz, double* sumr2,
-                                                         const int32_t* maxiter, const double* tol,
-                                                         int32_t* iter, uint8_t* done, uint8_t* live) {
-    __shared__ double sm[256];
-    const double a = sum_parts(partial, nparts, 1, 0, 0, sm);
-    const double b = sum_parts(partial, nparts, 1, 0, 1, sm);
-    if (threadIdx.x == 0) {
-        rz[slot] = a;
-        sumr2[slot] = b;
-        iter[slot] = 0;
-        live[slot] = 1;
-        // while (sumr2 > tolPCG && iter < maxiterPCG) (FG.cpp:2696)
-        done[slot] = (b > tol[slot] && 0 < maxiter[slot]) ? 0 : 1;
-    }
 }
 
 // alpha = r^T z / p^T A p (FG.cpp:2710)
@@ -1446,12 +1381,6 @@ __global__ void k_cols_gather(const float* __restrict__ src, const int32_t* __re
     if (i < Nnm) dst[(int64_t)j * Nnm + i] = src[i * kpad + slots[j]];
 }
 
-__global__ void k_gather_col(const float* __restrict__ src, int slot, int kpad, int64_t Nnm,
-                             float* __restrict__ dst) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < Nnm) dst[i] = src[i * kpad + slot];
-}
-
 // slot results to chosen columns of a column-major buffer: dst[:, cols[j]]
 __global__ void k_cols_gather_to(const float* __restrict__ src, const int32_t* __restrict__ slots,
                                  const int32_t* __restrict__ cols, int kpad, int64_t Nnm, int64_t ld,
@@ -1592,11 +1521,11 @@ int64_t gemm_max_parts(int64_t Npad) { return Npad / EROWS; }
 int64_t vec_max_parts(int64_t Npad, int) { return Npad / VROWS; }
 
 hipError_t launch_grm_gemv(hipStream_t s, const float* S, int64_t Npad, int64_t Nnm, const float* in,
-                           float* out, SigmaArgs a, double* partial, int64_t* nparts, const GemvPlan* tri) {
+                           float* out, VecArgs a, double* partial, int64_t* nparts, const GemvPlan* tri) {
     if (tri) {
         if (tri->Npad != Npad || !tri->items || Npad % TV_ROWS != 0) return hipErrorInvalidValue;
         hipLaunchKernelGGL(k_gemv_tri, dim3((unsigned)tri->nitems), dim3(512), 0, s, S, Npad, in, tri->items,
-                           tri->y1p, tri->y2p);
+                           tri->y1p, tri->y2p, a.over, a.iter);
         const int64_t nb = Npad / TV_ROWS;
         hipLaunchKernelGGL(k_gemv_tri_epi, dim3((unsigned)nb), dim3(256), 0, s, tri->y1p, tri->y2p, tri->rtab, Npad,
                            Nnm, in, out, a, partial);
@@ -1869,25 +1798,6 @@ hipError_t launch_sigma_setup(hipStream_t s, const float* w, const uint8_t* mask
     return hipGetLastError();
 }
 
-hipError_t launch_col_init(hipStream_t s, const float* b, int slot, int kpad, int64_t Nnm, int64_t Npad,
-                           const float* minv_sys, const uint8_t* mask_sys, float* X, float* R, float* Z,
-                           float* P, double* partial, int64_t* nparts) {
-    const int64_t nb = Npad / VROWS;
-    hipLaunchKernelGGL(k_col_init, dim3((unsigned)nb), dim3(256), 0, s, b, slot, kpad, Nnm, minv_sys,
-                       mask_sys, X, R, Z, P, partial);
-    if (nparts) *nparts = nb;
-    return hipGetLastError();
-}
-
-hipError_t launch_col_init_finish(hipStream_t s, int slot, int kpad, const double* partial,
-                                  int64_t nparts, double* rz, double* sumr2, const int32_t* maxiter,
-                                  const double* tol, int32_t* iter, uint8_t* done, uint8_t* live) {
-    (void)kpad;
-    hipLaunchKernelGGL(k_col_init_finish, dim3(1), dim3(256), 0, s, slot, partial, nparts, rz, sumr2,
-                       maxiter, tol, iter, done, live);
-    return hipGetLastError();
-}
-
 hipError_t launch_alpha(hipStream_t s, int kpad, const double* partial, int64_t nparts, const double* rz,
                         const uint8_t* done, const uint8_t* live, const uint8_t* kind, float* alpha) {
     hipLaunchKernelGGL(k_alpha, dim3((unsigned)kpad), dim3(256), 0, s, kpad, partial, nparts, rz, done,
@@ -1944,12 +1854,6 @@ hipError_t launch_cols_init_finish(hipStream_t s, int k, const int32_t* slots, i
 hipError_t launch_cols_gather(hipStream_t s, const float* src, int k, const int32_t* slots, int kpad, int64_t Nnm,
                               float* dst) {
     hipLaunchKernelGGL(k_cols_gather, dim3(nblk(Nnm, 256), (unsigned)k), dim3(256), 0, s, src, slots, kpad, Nnm, dst);
-    return hipGetLastError();
-}
-
-hipError_t launch_gather_col(hipStream_t s, const float* src, int slot, int kpad, int64_t Nnm,
-                             float* dst) {
-    hipLaunchKernelGGL(k_gather_col, dim3(nblk(Nnm, 256)), dim3(256), 0, s, src, slot, kpad, Nnm, dst);
     return hipGetLastError();
 }
 

@@ -147,7 +147,7 @@ void clear_geno(saige_ctx* c) {
     tri_plan_free(c->tri);
     gemv_plan_free(c->triv);
     free_engine(c->eng);
-    free_engine(c->eng1);
+    c->s1.release();
     c->h_stats.clear();
     c->qc_index.clear();
     c->vr_index.clear();
@@ -290,22 +290,10 @@ int engine_set_system(saige_ctx* c, Engine& e, int s, const float* w_host, const
     return SAIGE_OK;
 }
 
-// uploads the per-slot state after the host changed it (live slots and
-// their systems)
-int engine_sync_host_arrays(saige_ctx* c, Engine& e) {
-    SAIGE_HIP_TRY(push_slot_state(c, e));
-    SAIGE_HIP_TRY(hipStreamSynchronize(c->stream));
-    return SAIGE_OK;
-}
-
 // Start k solves at once: column j of B_host (N x k, column-major) in slot
 // slots[j] with system systems[j].  One upload, two launches, one sync.
 int engine_add_batch(saige_ctx* c, Engine& e, int k, const int32_t* slots, const int32_t* systems,
                      const float* B_host, int maxiter, float tol, int product = 0, bool b_on_device = false) {
-    if (product && e.kpad != EW) {
-        set_error("GRM-product slots need the block engine");
-        return SAIGE_E_STATE;
-    }
     if (k < 1 || k > e.kpad || !slots || !systems || !B_host) {
         set_error("invalid batch of %d columns (engine width %d)", k, e.kpad);
         return SAIGE_E_ARG;
@@ -376,16 +364,23 @@ int ensure_tri(saige_ctx* c) {
     return SAIGE_OK;
 }
 
-// items of the lower-triangle GEMV: at most TRIV_CHUNKS chunks of 256
-// columns left of a row set's diagonal block
-constexpr int TRIV_CHUNKS = 24;
+// items of the lower-triangle GEMV: at most this many 256-column chunks left of
+// a row set's diagonal block, two to twelve, as leave about 200 items of more
+// than the diagonal blocks' work.  Fewer chunks spread a small triangle over
+// the CUs (us per solve of N = 8000 at 24, 8, 4, 2 chunks: 838, 520, 443, 495;
+// N = 20,000: 1669, 1454, 1544, 1661), and from 40,000 samples on 8 to 24 are
+// within 2%.
+int triv_chunks(int64_t Npad) {
+    const int64_t nr = Npad / 256, chunks = nr * (nr - 1) / 2;
+    return (int)std::max<int64_t>(2, std::min<int64_t>(12, (chunks + 199) / 200));
+}
 
 // the lower-triangle GEMV's plan when that mode is on (else nullptr); rc != 0
 // on an allocation failure
 const GemvPlan* gemv_plan(saige_ctx* c, int* rc) {
     *rc = SAIGE_OK;
     if (c->gemv_mode != SAIGE_GEMV_TRI) return nullptr;
-    const hipError_t e = gemv_plan_build(c->triv, c->Npad, TRIV_CHUNKS);
+    const hipError_t e = gemv_plan_build(c->triv, c->Npad, triv_chunks(c->Npad));
     if (e != hipSuccess) {
         saige::set_error("lower-triangle GEMV scratch for Npad=%lld: %s", (long long)c->Npad, hipGetErrorString(e));
         *rc = e == hipErrorOutOfMemory ? SAIGE_E_NOMEM : SAIGE_E_DEVICE;
@@ -396,11 +391,7 @@ const GemvPlan* gemv_plan(saige_ctx* c, int* rc) {
 int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t* iters_out) {
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
-    if (e.kpad != 1)
-        if (int rc = ensure_tri(c)) return rc;
-    int prc = 0;
-    const GemvPlan* tv = e.kpad == 1 ? gemv_plan(c, &prc) : nullptr;
-    if (prc) return prc;
+    if (int rc = ensure_tri(c)) return rc;
     SigmaArgs a;
     a.winv = e.winv;
     a.mask = e.mask;
@@ -446,14 +437,11 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
         if (!any) break;
         int64_t np = 0;
         SAIGE_HIP_TRY(hipEventRecord(c->ev0, st));
-        if (e.kpad == 1)
-            SAIGE_HIP_TRY(launch_grm_gemv(st, g.S, Np, N, e.P, e.AP, a, e.partial, &np, tv));
-        else
-            SAIGE_HIP_TRY(launch_grm_gemm(st, g.S, Np, N, e.P, e.AP, a, e.partial, &np, e.ypart,
-                                          quarter       ? c->gemm_cfg_quarter
-                                          : halves == 3 ? c->gemm_cfg
-                                                        : c->gemm_cfg_half,
-                                          halves, &c->tri, g.s16, narrow ? &nc : nullptr));
+        SAIGE_HIP_TRY(launch_grm_gemm(st, g.S, Np, N, e.P, e.AP, a, e.partial, &np, e.ypart,
+                                      quarter       ? c->gemm_cfg_quarter
+                                      : halves == 3 ? c->gemm_cfg
+                                                    : c->gemm_cfg_half,
+                                      halves, &c->tri, g.s16, narrow ? &nc : nullptr));
         SAIGE_HIP_TRY(hipEventRecord(c->ev1, st));
         SAIGE_HIP_TRY(launch_alpha(st, e.kpad, e.partial, np, e.rz, e.done, e.live, e.kind, e.alpha));
         int64_t np2 = 0;
@@ -466,10 +454,9 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
         SAIGE_HIP_TRY(hipStreamSynchronize(st));
         float ms = 0.f;
         SAIGE_HIP_TRY(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-        const int kind = e.kpad == 1 ? SAIGE_LAUNCH_GEMV
-                         : quarter      ? SAIGE_LAUNCH_GEMM_QUARTER
-                         : halves == 3  ? SAIGE_LAUNCH_GEMM_FULL
-                                        : SAIGE_LAUNCH_GEMM_HALF;
+        const int kind = quarter       ? SAIGE_LAUNCH_GEMM_QUARTER
+                         : halves == 3 ? SAIGE_LAUNCH_GEMM_FULL
+                                       : SAIGE_LAUNCH_GEMM_HALF;
         e.gemm_seconds[kind] += ms * 1e-3;
         e.gemm_launches[kind]++;
     }
@@ -1226,6 +1213,20 @@ int saige_get_grm_block(saige_ctx* c, int64_t r0, int64_t c0, int64_t nr, int64_
     return SAIGE_OK;
 }
 
+namespace {
+int reserve_solve1(saige_ctx* c) {
+    const hipError_t e = c->s1.reserve(c->Npad);
+    if (e == hipSuccess) return SAIGE_OK;
+    set_error("device allocation failed (single-column vectors): %s", hipGetErrorString(e));
+    return e == hipErrorOutOfMemory ? SAIGE_E_NOMEM : SAIGE_E_DEVICE;
+}
+
+// zeroes rows [Nnm, Npad) of a vector (padded rows read as zero in products)
+hipError_t zero_tail(saige_ctx* c, float* v) {
+    return launch_fill_zero(c->stream, v + c->Nnm, 4 * (c->Npad - c->Nnm));
+}
+}  // namespace
+
 static int grm_matvec(saige_ctx* c, int loco, const float* B, int64_t k, float* Y) {
     if (k <= 0 || !B || !Y) {
         set_error("invalid matvec arguments");
@@ -1234,22 +1235,24 @@ static int grm_matvec(saige_ctx* c, int loco, const float* B, int64_t k, float* 
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
     const GrmView g = grm_view(c, loco);
-    SigmaArgs a{};
-    a.mqc = (float)g.m;
-    a.mode = 0;
     if (k == 1) {
-        int rc = engine_reserve(c, c->eng1, 1, 1);
-        if (rc) return rc;
-        Engine& e = c->eng1;
-        SAIGE_HIP_TRY(hipMemcpyAsync(e.stage, B, 4 * N, hipMemcpyHostToDevice, st));
+        if (int rc = reserve_solve1(c)) return rc;
+        Solve1& v = c->s1;
         int prc = 0;
         const GemvPlan* tv = gemv_plan(c, &prc);
         if (prc) return prc;
-        SAIGE_HIP_TRY(launch_grm_gemv(st, g.S, Np, N, e.stage, e.AP, a, nullptr, nullptr, tv));
-        SAIGE_HIP_TRY(hipMemcpyAsync(Y, e.AP, 4 * N, hipMemcpyDeviceToHost, st));
+        VecArgs va;
+        va.mqc = (float)g.m;
+        SAIGE_HIP_TRY(hipMemcpyAsync(v.p, B, 4 * N, hipMemcpyHostToDevice, st));
+        SAIGE_HIP_TRY(zero_tail(c, v.p));
+        SAIGE_HIP_TRY(launch_grm_gemv(st, g.S, Np, N, v.p, v.ap, va, nullptr, nullptr, tv));
+        SAIGE_HIP_TRY(hipMemcpyAsync(Y, v.ap, 4 * N, hipMemcpyDeviceToHost, st));
         SAIGE_HIP_TRY(hipStreamSynchronize(st));
         return SAIGE_OK;
     }
+    SigmaArgs a{};
+    a.mqc = (float)g.m;
+    a.mode = 0;
     if (int rc = ensure_tri(c)) return rc;
     // own scratch (not the engine's), so live engine slots are untouched
     if (!c->d_mv_in) {
@@ -1330,39 +1333,29 @@ static int get_crossprod(saige_ctx* c, int loco, const float* b, const float* w,
         set_error("invalid arguments");
         return SAIGE_E_ARG;
     }
-    int rc = engine_reserve(c, c->eng1, 1, 1);
-    if (rc) return rc;
-    Engine& e = c->eng1;
-    e.loco = loco;
-    rc = engine_set_system(c, e, 0, w, tau, nullptr);
-    if (rc) return rc;
+    if (int rc = reserve_solve1(c)) return rc;
+    Solve1& v = c->s1;
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
-    e.h_slot_sys[0] = 0;
-    e.h_live[0] = 1;
-    rc = engine_sync_host_arrays(c, e);
-    if (rc) return rc;
-    SAIGE_HIP_TRY(hipMemcpyAsync(e.stage, b, 4 * N, hipMemcpyHostToDevice, st));
-    SigmaArgs a;
-    a.winv = e.winv;
-    a.mask = e.mask;
-    a.tau = e.tau;
-    a.sys = e.slot_sys;
-    a.live = e.live;
     const GrmView g = grm_view(c, loco);
-    a.inv_m = 0.f;
-    a.mqc = (float)g.m;
-    a.mode = 1;
-    a.kind = nullptr;
-    a.xout = nullptr;
     int prc = 0;
     const GemvPlan* tv = gemv_plan(c, &prc);
     if (prc) return prc;
-    SAIGE_HIP_TRY(launch_grm_gemv(st, g.S, Np, N, e.stage, e.AP, a, e.partial, nullptr, tv));
-    SAIGE_HIP_TRY(hipMemcpyAsync(out, e.AP, 4 * N, hipMemcpyDeviceToHost, st));
+    SAIGE_HIP_TRY(hipMemcpyAsync(v.w, w, 4 * N, hipMemcpyHostToDevice, st));
+    SAIGE_HIP_TRY(hipMemcpyAsync(v.p, b, 4 * N, hipMemcpyHostToDevice, st));
+    SAIGE_HIP_TRY(zero_tail(c, v.p));
+    SAIGE_HIP_TRY(launch_sigma_setup(st, v.w, nullptr, g.diag, N, Np, tau[0], tau[1], (float)g.m, g.diag_one, v.winv,
+                                     v.minv, nullptr, nullptr));
+    VecArgs a;
+    a.winv = v.winv;
+    a.tau0 = tau[0];
+    a.tau1 = tau[1];
+    a.mqc = (float)g.m;
+    a.mode = 1;
+    SAIGE_HIP_TRY(launch_grm_gemv(st, g.S, Np, N, v.p, v.ap, a, v.pap, nullptr, tv));
+    SAIGE_HIP_TRY(hipMemcpyAsync(out, v.ap, 4 * N, hipMemcpyDeviceToHost, st));
     SAIGE_HIP_TRY(hipStreamSynchronize(st));
-    e.h_live[0] = 0;
-    return engine_sync_host_arrays(c, e);
+    return SAIGE_OK;
 }
 
 int saige_get_crossprod(saige_ctx* c, const float* b, const float* w, const float* tau, float* out) {
@@ -1378,18 +1371,17 @@ static int pcg1(saige_ctx* c, int loco, const float* w, const float* tau, const 
         set_error("invalid arguments");
         return SAIGE_E_ARG;
     }
-    int rc = engine_reserve(c, c->eng1, 1, 1);
-    if (rc) return rc;
-    Engine& e = c->eng1;
-    e.loco = loco;
-    if ((rc = engine_set_system(c, e, 0, w, tau, nullptr))) return rc;
-    if ((rc = engine_add(c, e, 0, 0, b, maxiter, tol))) return rc;
-    uint8_t done = 0;
-    int32_t it = 0;
-    while (!done) {
-        if ((rc = engine_step(c, e, 64, &done, &it))) return rc;
-    }
-    if ((rc = engine_take(c, e, 0, x))) return rc;
+    if (int rc = reserve_solve1(c)) return rc;
+    Solve1& v = c->s1;
+    hipStream_t st = c->stream;
+    const int64_t N = c->Nnm;
+    const GrmView g = grm_view(c, loco);
+    int prc = 0;
+    const GemvPlan* tv = gemv_plan(c, &prc);
+    if (prc) return prc;
+    int it = 0;
+    SAIGE_HIP_TRY(solve1(st, v, w, b, x, g.S, g.diag, N, tau[0], tau[1], (float)g.m, g.diag_one, maxiter, (double)tol,
+                         tv, &it));
     if (iters) *iters = it;
     if (it >= maxiter && maxiter > 0) {
         set_error("pcg did not converge. You may increase maxiter number.");
@@ -2137,8 +2129,9 @@ int saige_engine_stats(const saige_ctx* c, int kind, double* secs, int64_t* laun
         set_error("unknown launch kind %d", kind);
         return SAIGE_E_ARG;
     }
-    if (secs) *secs = c->eng.gemm_seconds[kind] + c->eng1.gemm_seconds[kind];
-    if (launches) *launches = c->eng.gemm_launches[kind] + c->eng1.gemm_launches[kind];
+    const bool gemv = kind == SAIGE_LAUNCH_GEMV;
+    if (secs) *secs = gemv ? c->s1.seconds : c->eng.gemm_seconds[kind];
+    if (launches) *launches = gemv ? c->s1.launches : c->eng.gemm_launches[kind];
     return SAIGE_OK;
 }
 

@@ -121,11 +121,41 @@ struct GemmConfig {
     int mode = GEMM_FP32;
 };
 
+// The width-1 solver's device state and what it publishes to the host
+// (page-locked, coherent): the iteration last decided, the iteration count and
+// whether the solve is over.
+struct P1State {
+    double rz[2];                  // z'r of the even / odd iteration
+    int32_t over;                  // the iteration whose decision ended the solve; INT32_MAX while it runs
+};
+struct P1Host {
+    volatile int32_t decided, it, done;
+};
+
+// The buffers of single-column products and solves for one Npad (one device
+// block), kept by the context.
+struct Solve1 {
+    static constexpr int EVENTS = 16;
+    void* block = nullptr;
+    int64_t Npad = 0;
+    float *w = nullptr, *b = nullptr, *winv = nullptr, *minv = nullptr, *x = nullptr, *r = nullptr, *z = nullptr,
+          *p = nullptr, *p2 = nullptr, *ap = nullptr;       // [Npad]
+    double *pap = nullptr, *partial = nullptr;
+    P1State* st = nullptr;
+    P1Host* host = nullptr;
+    float* hvec = nullptr;         // page-locked [3][Npad]: a small solve's w and b, read in place, and its x
+    hipEvent_t ev[EVENTS] = {};
+    double seconds = 0.0;          // device time and count of the GRM products
+    int64_t launches = 0;
+    hipError_t reserve(int64_t Npad);
+    void release();
+};
+
 struct Engine {
     int width = 0;        // live slot capacity (<= EW)
     int nsys = 0;
     int loco = 0;         // 1: products with the LOCO GRM S_loco, divisor M_loco
-    int kpad = 0;         // 1 (GEMV) or EW (MFMA GEMM)
+    int kpad = 0;         // EW once reserved
     // [Npad][kpad] row-major column blocks
     float* X = nullptr; float* R = nullptr; float* Z = nullptr; float* P = nullptr; float* AP = nullptr;
     // per system [nsys][Npad]
@@ -167,8 +197,8 @@ struct Engine {
     int32_t* h_iter = nullptr;
     int32_t* h_slot_sys = nullptr;
     uint8_t* h_live = nullptr;
-    // device time of the GRM product launches by kind: [0] GEMV (width 1),
-    // [1] GEMM over one 32-column half, [2] GEMM over both halves
+    // device time of the GRM product launches by kind: [1] GEMM over one
+    // 32-column half, [2] GEMM over both halves, [3] over 16 columns
     double gemm_seconds[4] = {0.0, 0.0, 0.0, 0.0};   // by SAIGE_LAUNCH_* kind
     int64_t gemm_launches[4] = {0, 0, 0, 0};
 };
@@ -288,7 +318,7 @@ struct saige_ctx {
     float* d_mv_out = nullptr;                   // [Npad][EW]
     float* d_mv_ypart = nullptr;                 // split-K scratch
     saige::Engine eng;
-    saige::Engine eng1;                          // kpad = 1 engine for saige_pcg1
+    saige::Solve1 s1;                            // single-column products and solves
 };
 
 namespace saige {
@@ -376,7 +406,34 @@ hipError_t launch_sub(hipStream_t s, const float* a, const float* b, int64_t n, 
 int syrk_tile();
 int syrk_kchunk_bf16();
 
+// Sigma p for one element (getCrossprod, FG.cpp:2412): the reference forms
+// 1/w, then b % (1/w), then tau0 * that, plus tau1 * (K b); tau1 == 0
+// returns the first term alone (FG.cpp:2401-2404).
+__device__ __forceinline__ float sigma_elem(float p, float y, float winv, float tau0, float tau1,
+                                            float mqc) {
+    float t = __fmul_rn(tau0, __fmul_rn(p, winv));
+    if (tau1 == 0.0f) return t;
+    return __fadd_rn(t, __fmul_rn(tau1, div_rn(y, mqc)));
+}
+
+// getDiagOfSigma (FG.cpp:2335-2358): (tau1 * diag) / Mqc + tau0 / w, >= 1e-4
+__device__ __forceinline__ float sigma_diag(float w, const float* diag, int64_t i, float tau0, float tau1, float mqc,
+                                            int diag_one) {
+    const float d = diag_one ? __fadd_rn(tau1, div_rn(tau0, w))
+                             : __fadd_rn(div_rn(__fmul_rn(tau1, diag[i]), mqc), div_rn(tau0, w));
+    return d < 1e-4f ? 1e-4f : d;
+}
+
 // ---- PCG kernels (pcg_kernels.hip)
+// arguments of a single-column product's epilogue
+struct VecArgs {
+    const float* winv = nullptr;     // [Npad], mode 1
+    float tau0 = 0.0f, tau1 = 0.0f;
+    float mqc = 1.0f;                // Mqc as float (divisor, FG.cpp:1706)
+    int mode = 0;                    // 0: out = S p / Mqc ; 1: out = Sigma p, zero past Nnm
+    const int32_t* over = nullptr;   // the launch returns at once when *over <= iter; may be null
+    int iter = 0;
+};
 struct SigmaArgs {
     const float* winv;     // [nsys][Npad]
     const uint8_t* mask;   // [nsys][Npad]
@@ -389,13 +446,18 @@ struct SigmaArgs {
     const uint8_t* kind;   // [kpad] 1 = product slot (out = K p, also written to xout); may be null
     float* xout;           // result block of product slots
 };
-// out[N][kpad] = epilogue(S * in), plus per-column partial p^T out dots when
-// mode == 1 (partial: [nparts][kpad][2], slot 0).  Returns nparts used.
+// out = epilogue(S * in), plus partial p^T out dots when mode == 1 (partial:
+// one double per part).  Returns the number of parts.
 // tri: read only the lower triangle (k_gemv_tri + k_gemv_tri_epi) with this
 // plan for Npad; nullptr: k_gemv over all of S.
 hipError_t launch_grm_gemv(hipStream_t s, const float* S, int64_t Npad, int64_t Nnm, const float* in,
-                           float* out, SigmaArgs a, double* partial, int64_t* nparts,
+                           float* out, VecArgs a, double* partial, int64_t* nparts,
                            const GemvPlan* tri = nullptr);
+// Sigma x = b by PCG for host vectors w, b and x; the iteration count in
+// *iters.  Waits for the stream.
+hipError_t solve1(hipStream_t s, Solve1& v, const float* w_host, const float* b_host, float* x_host, const float* S,
+                  const float* diag, int64_t Nnm, float tau0, float tau1, float m, int diag_one, int maxiter,
+                  double tol, const GemvPlan* tri, int* iters);
 bool gemm_config_valid(GemmConfig g);
 // ypart: gemm_ypart_floats(Npad) floats of scratch for the split-K slices.
 // halves: bit h set = columns [32h, 32h+32) are computed; the epilogue's
@@ -419,14 +481,6 @@ int64_t vec_max_parts(int64_t Npad, int kpad);
 hipError_t launch_sigma_setup(hipStream_t s, const float* w, const uint8_t* mask_in, const float* diag,
                               int64_t Nnm, int64_t Npad, float tau0, float tau1, float mqc,
                               int diag_one, float* winv, float* minv, uint8_t* mask_out, float* dout);
-// column init: X=0, R=b (staged), Z=minv*R, P=Z; partial rz/rr dots
-hipError_t launch_col_init(hipStream_t s, const float* b, int slot, int kpad, int64_t Nnm,
-                           int64_t Npad, const float* minv_sys, const uint8_t* mask_sys,
-                           float* X, float* R, float* Z, float* P, double* partial,
-                           int64_t* nparts);
-hipError_t launch_col_init_finish(hipStream_t s, int slot, int kpad, const double* partial,
-                                  int64_t nparts, double* rz, double* sumr2, const int32_t* maxiter,
-                                  const double* tol, int32_t* iter, uint8_t* done, uint8_t* live);
 hipError_t launch_alpha(hipStream_t s, int kpad, const double* partial, int64_t nparts,
                         const double* rz, const uint8_t* done, const uint8_t* live, const uint8_t* kind,
                         float* alpha);
@@ -448,8 +502,6 @@ hipError_t launch_cols_init_finish(hipStream_t s, int k, const int32_t* slots, i
                                    const double* tol, int32_t* iter, uint8_t* done, int product);
 hipError_t launch_cols_gather(hipStream_t s, const float* src, int k, const int32_t* slots, int kpad, int64_t Nnm,
                               float* dst);
-hipError_t launch_gather_col(hipStream_t s, const float* src, int slot, int kpad, int64_t Nnm,
-                             float* dst);
 hipError_t launch_scatter_cols(hipStream_t s, const float* src, int64_t k, int64_t Nnm,
                                int64_t Npad, int kpad, float* dst);
 hipError_t launch_gather_cols(hipStream_t s, const float* src, int64_t k, int64_t Nnm, int kpad,

@@ -12,7 +12,7 @@
 //   two launches, where the whole of S comes from the caches;
 // * else: k_p1_dir (decide, p), the GEMV and its epilogue (Sigma p, p'Ap),
 //   k_p1_update.
-// 1000 samples: SMALLUS us per solve of three iterations; six launches and a host
+// 1000 samples: 76 us per solve of three iterations; six launches and a host
 // round trip per iteration took 277 us.
 #include "saige_internal.hpp"
 
