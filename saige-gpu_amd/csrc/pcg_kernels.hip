@@ -1103,72 +1103,109 @@ __global__ __launch_bounds__(256) void k_tri_reduce(const float* __restrict__ y1
     }
 }
 
-constexpr int EROWS = 256;   // rows per workgroup of the epilogue
+// The vector kernels of the block engine move four columns per thread (16
+// bytes) and 64 rows per workgroup, four passes of 16 rows, all loads of a
+// thread in flight together: at 256 rows and one column per thread a workgroup
+// ran 64 dependent passes (epilogue 83 us at N = 50,000, 132 us at 10,000, now
+// 19 and 13 us; update 38 and 32 us, now 19 and 6 us).  Groups of four columns
+// with no column at work are skipped.
+constexpr int EROWS = 64;
+constexpr int EPASS = EROWS / 16;
+
+// per-column FP64 sums over a workgroup's rows: thread (row group t / 16,
+// columns 4 (t % 16) + e) brings v[e]; column n's sum goes to dst[2 n]
+__device__ __forceinline__ void block_col_sums(const double (&v)[4], double* sm, double* dst) {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int e = 0; e < 4; e++) sm[e * 256 + tid] = v[e];
+    for (int st = 128; st >= 16; st >>= 1) {
+        __syncthreads();
+        if (tid < st) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) sm[e * 256 + tid] += sm[e * 256 + tid + st];
+        }
+    }
+    __syncthreads();
+    if (tid < EW) dst[2 * tid] = sm[(tid & 3) * 256 + (tid >> 2)];
+    __syncthreads();
+}
 
 __global__ __launch_bounds__(256) void k_gemm_epi(const float* __restrict__ ypart, int nsplit, int64_t Npad,
                                                   int64_t Nnm, const float* __restrict__ in,
                                                   float* __restrict__ out, SigmaArgs a,
                                                   double* __restrict__ partial) {
-    __shared__ double sm[256];
-    const int tid = threadIdx.x;
-    const int n = tid & 63;
-    int s = 0;
-    float tau0 = 0.f, tau1 = 0.f;
-    bool col_on = false, product = false;
-    if (a.mode == 1) {
-        s = a.sys[n];
-        tau0 = a.tau[2 * s];
-        tau1 = a.tau[2 * s + 1];
-        col_on = a.live[n] != 0;
-        product = a.kind != nullptr && a.kind[n] != 0;
-    }
-    double dsum = 0.0;
-    const int64_t rb = (int64_t)blockIdx.x * EROWS;
-    for (int rl = tid >> 6; rl < EROWS; rl += 4) {
-        const int64_t row = rb + rl;
-        const int64_t o = row * EW + n;
-        float y = ypart[o];
+    __shared__ double sm[4 * 256];
+    const int tid = threadIdx.x, n0 = 4 * (tid & 15);
+    int s[4] = {0, 0, 0, 0};
+    float tau0[4], tau1[4];
+    bool on_col[4], product[4], work = a.mode == 0, prod_any = false;
 #pragma unroll
-        for (int sp = 1; sp < nsplit; sp++) y += ypart[(int64_t)sp * Npad * EW + o];
-        float r;
-        if (a.mode == 0) {
-            r = div_rn(y, a.mqc);
-        } else if (product) {
-            // a product slot: K p on the system's samples, stored as the result
-            const bool on = col_on && row < Nnm && a.mask[(int64_t)s * Npad + row];
-            r = on ? div_rn(y, a.mqc) : 0.0f;
-            a.xout[o] = r;
-        } else {
-            const bool on = col_on && row < Nnm && a.mask[(int64_t)s * Npad + row];
-            const float p = in[o];
-            r = on ? sigma_elem(p, y, a.winv[(int64_t)s * Npad + row], tau0, tau1, a.mqc) : 0.0f;
-            dsum += (double)p * (double)r;
+    for (int e = 0; e < 4; e++) {
+        tau0[e] = tau1[e] = 0.0f;
+        on_col[e] = product[e] = false;
+        if (a.mode == 1) {
+            s[e] = a.sys[n0 + e];
+            tau0[e] = a.tau[2 * s[e]];
+            tau1[e] = a.tau[2 * s[e] + 1];
+            on_col[e] = a.live[n0 + e] != 0;
+            product[e] = a.kind != nullptr && a.kind[n0 + e] != 0;
+            work |= on_col[e];
+            prod_any |= on_col[e] && product[e];
         }
-        out[o] = r;
     }
-    if (a.mode == 1) {
-        sm[tid] = dsum;
-        for (int st = 128; st >= EW; st >>= 1) {
-            __syncthreads();
-            if (tid < st) sm[tid] += sm[tid + st];
+    double dsum[4] = {0.0, 0.0, 0.0, 0.0};
+    const int64_t rb = (int64_t)blockIdx.x * EROWS + (tid >> 4);
+    if (work) {
+        float4 y[EPASS], p[EPASS];
+#pragma unroll
+        for (int k = 0; k < EPASS; k++) {
+            const int64_t o = (rb + 16 * k) * EW + n0;
+            y[k] = *reinterpret_cast<const float4*>(ypart + o);
+            p[k] = a.mode == 1 ? *reinterpret_cast<const float4*>(in + o) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
-        __syncthreads();
-        if (tid < EW) partial[((int64_t)blockIdx.x * EW + tid) * 2] = sm[tid];
+        for (int sp = 1; sp < nsplit; sp++)
+#pragma unroll
+            for (int k = 0; k < EPASS; k++) {
+                const float4 v = *reinterpret_cast<const float4*>(ypart + ((int64_t)sp * Npad + rb + 16 * k) * EW + n0);
+                y[k].x += v.x;
+                y[k].y += v.y;
+                y[k].z += v.z;
+                y[k].w += v.w;
+            }
+#pragma unroll
+        for (int k = 0; k < EPASS; k++) {
+            const int64_t row = rb + 16 * k, o = row * EW + n0;
+            const float yv[4] = {y[k].x, y[k].y, y[k].z, y[k].w}, pv[4] = {p[k].x, p[k].y, p[k].z, p[k].w};
+            float r[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (a.mode == 0) {
+                    r[e] = div_rn(yv[e], a.mqc);
+                    continue;
+                }
+                const int64_t i = (int64_t)s[e] * Npad + row;
+                const bool on = on_col[e] && row < Nnm && a.mask[i];
+                if (product[e]) {
+                    // a product slot: K p on the system's samples
+                    r[e] = on ? div_rn(yv[e], a.mqc) : 0.0f;
+                } else {
+                    r[e] = on ? sigma_elem(pv[e], yv[e], a.winv[i], tau0[e], tau1[e], a.mqc) : 0.0f;
+                    dsum[e] += (double)pv[e] * (double)r[e];
+                }
+            }
+            *reinterpret_cast<float4*>(out + o) = make_float4(r[0], r[1], r[2], r[3]);
+            if (prod_any) {                       // product slots' results
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (on_col[e] && product[e]) a.xout[o + e] = r[e];
+            }
+        }
     }
+    if (a.mode == 1) block_col_sums(dsum, sm, partial + (int64_t)blockIdx.x * EW * 2);
 }
 
 // ------------------------------------------------------ vector kernels
-constexpr int VROWS = 256;   // rows per workgroup in the elementwise kernels
-
-// In-workgroup reduction of per-thread values to per-column sums
-// (threads tid and tid + s share a column when kpad divides s).
-__device__ __forceinline__ void col_reduce(double* sm, int tid, int kpad) {
-    for (int s = 128; s >= kpad; s >>= 1) {
-        __syncthreads();
-        if (tid < s) sm[tid] += sm[tid + s];
-    }
-    __syncthreads();
-}
+constexpr int VROWS = EROWS; // rows per workgroup in the elementwise kernels
 
 __global__ __launch_bounds__(256) void k_sigma_setup(const float* __restrict__ w,
                                                      const uint8_t* __restrict__ mask_in,
@@ -1228,7 +1265,7 @@ __global__ __launch_bounds__(256) void k_alpha(int kpad, const double* __restric
 }
 
 // x += a p; r1 = r - a Ap; z1 = minv r1 (FG.cpp:2734-2767), partial z1.r1, r1.r1
-__global__ __launch_bounds__(256) void k_update(int kpad, int64_t Npad, const float* __restrict__ alpha,
+__global__ __launch_bounds__(256) void k_update(int64_t Npad, const float* __restrict__ alpha,
                                                 const uint8_t* __restrict__ done,
                                                 const uint8_t* __restrict__ live,
                                                 const uint8_t* __restrict__ kind,
@@ -1237,43 +1274,62 @@ __global__ __launch_bounds__(256) void k_update(int kpad, int64_t Npad, const fl
                                                 float* Z, const float* __restrict__ P,
                                                 const float* __restrict__ AP,
                                                 double* __restrict__ partial) {
-    __shared__ double sm[2][256];
-    const int tid = threadIdx.x;
-    const int c = tid % kpad;
-    const int rstep = 256 / kpad;
-    const bool act = live[c] && !done[c] && !kind[c];
-    const float a = alpha[c];
-    const float* mv = minv + (int64_t)sys[c] * Npad;
-    double rz = 0.0, rr = 0.0;
-    const int64_t rbase = (int64_t)blockIdx.x * VROWS;
-    if (act) {
-        for (int rl = tid / kpad; rl < VROWS; rl += rstep) {
-            const int64_t i = rbase + rl;
-            const int64_t o = i * kpad + c;
-            const float x = __fadd_rn(X[o], __fmul_rn(a, P[o]));
-            const float r1 = __fsub_rn(R[o], __fmul_rn(a, AP[o]));
-            const float z1 = __fmul_rn(mv[i], r1);
-            X[o] = x;
-            R[o] = r1;
-            Z[o] = z1;
-            rz += (double)z1 * (double)r1;
-            rr += (double)r1 * (double)r1;
+    __shared__ double sm[4 * 256];
+    const int tid = threadIdx.x, n0 = 4 * (tid & 15);
+    bool act[4], any = false, all = true;
+    float al[4];
+    const float* mv[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        act[e] = live[n0 + e] && !done[n0 + e] && !kind[n0 + e];
+        any |= act[e];
+        all &= act[e];
+        al[e] = alpha[n0 + e];
+        mv[e] = minv + (int64_t)sys[n0 + e] * Npad;
+    }
+    double rz[4] = {0.0, 0.0, 0.0, 0.0}, rr[4] = {0.0, 0.0, 0.0, 0.0};
+    const int64_t rb = (int64_t)blockIdx.x * VROWS + (tid >> 4);
+    if (any) {
+        float4 x[EPASS], r[EPASS], p[EPASS], ap[EPASS], z[EPASS];
+        float m[EPASS][4];
+#pragma unroll
+        for (int k = 0; k < EPASS; k++) {
+            const int64_t i = rb + 16 * k, o = i * EW + n0;
+            x[k] = *reinterpret_cast<const float4*>(X + o);
+            r[k] = *reinterpret_cast<const float4*>(R + o);
+            p[k] = *reinterpret_cast<const float4*>(P + o);
+            ap[k] = *reinterpret_cast<const float4*>(AP + o);
+            z[k] = all ? make_float4(0.f, 0.f, 0.f, 0.f) : *reinterpret_cast<const float4*>(Z + o);
+#pragma unroll
+            for (int e = 0; e < 4; e++) m[k][e] = mv[e][i];
+        }
+#pragma unroll
+        for (int k = 0; k < EPASS; k++) {
+            const int64_t o = (rb + 16 * k) * EW + n0;
+            float xv[4] = {x[k].x, x[k].y, x[k].z, x[k].w}, rv[4] = {r[k].x, r[k].y, r[k].z, r[k].w};
+            float zv[4] = {z[k].x, z[k].y, z[k].z, z[k].w};
+            const float pv[4] = {p[k].x, p[k].y, p[k].z, p[k].w}, av[4] = {ap[k].x, ap[k].y, ap[k].z, ap[k].w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float x1 = __fadd_rn(xv[e], __fmul_rn(al[e], pv[e]));
+                const float r1 = __fsub_rn(rv[e], __fmul_rn(al[e], av[e]));
+                const float z1 = __fmul_rn(m[k][e], r1);
+                if (act[e]) {                     // a column that is not at work keeps its values
+                    xv[e] = x1;
+                    rv[e] = r1;
+                    zv[e] = z1;
+                    rz[e] += (double)z1 * (double)r1;
+                    rr[e] += (double)r1 * (double)r1;
+                }
+            }
+            *reinterpret_cast<float4*>(X + o) = make_float4(xv[0], xv[1], xv[2], xv[3]);
+            *reinterpret_cast<float4*>(R + o) = make_float4(rv[0], rv[1], rv[2], rv[3]);
+            *reinterpret_cast<float4*>(Z + o) = make_float4(zv[0], zv[1], zv[2], zv[3]);
         }
     }
-    sm[0][tid] = rz;
-    sm[1][tid] = rr;
-    for (int s = 128; s >= kpad; s >>= 1) {
-        __syncthreads();
-        if (tid < s) {
-            sm[0][tid] += sm[0][tid + s];
-            sm[1][tid] += sm[1][tid + s];
-        }
-    }
-    __syncthreads();
-    if (tid < kpad) {
-        partial[((int64_t)blockIdx.x * kpad + tid) * 2] = sm[0][tid];
-        partial[((int64_t)blockIdx.x * kpad + tid) * 2 + 1] = sm[1][tid];
-    }
+    double* dst = partial + (int64_t)blockIdx.x * EW * 2;
+    block_col_sums(rz, sm, dst);
+    block_col_sums(rr, sm, dst + 1);
 }
 
 // beta = z1^T r1 / z^T r; sumr2 = r1^T r1; stop test (FG.cpp:2770-2792)
@@ -1306,54 +1362,80 @@ __global__ __launch_bounds__(256) void k_beta(int kpad, const double* __restrict
     }
 }
 
-// p = z1 + beta p (FG.cpp:2772)
-__global__ __launch_bounds__(256) void k_pupdate(int kpad, int64_t Npad, const float* __restrict__ beta,
+// p = z1 + beta p (FG.cpp:2772); four columns per thread
+__global__ __launch_bounds__(256) void k_pupdate(int64_t Npad, const float* __restrict__ beta,
                                                  const uint8_t* __restrict__ done,
                                                  const uint8_t* __restrict__ live,
                                                  const uint8_t* __restrict__ kind,
                                                  const float* __restrict__ Z, float* P) {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= Npad * kpad) return;
-    const int c = (int)(t % kpad);
-    if (!live[c] || done[c] || kind[c]) return;
-    P[t] = __fadd_rn(Z[t], __fmul_rn(beta[c], P[t]));
+    if (t >= Npad * (EW / 4)) return;
+    const int n0 = 4 * (int)(t % (EW / 4));
+    bool act[4], any = false;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        act[e] = live[n0 + e] && !done[n0 + e] && !kind[n0 + e];
+        any |= act[e];
+    }
+    if (!any) return;
+    const float4 z = *reinterpret_cast<const float4*>(Z + 4 * t), p = *reinterpret_cast<const float4*>(P + 4 * t);
+    const float zv[4] = {z.x, z.y, z.z, z.w};
+    float pv[4] = {p.x, p.y, p.z, p.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (act[e]) pv[e] = __fadd_rn(zv[e], __fmul_rn(beta[n0 + e], pv[e]));
+    *reinterpret_cast<float4*>(P + 4 * t) = make_float4(pv[0], pv[1], pv[2], pv[3]);
 }
 
 // Start the listed columns together: column j of the staged block B
 // ([k][Nnm]) goes to slot slots[j] with system sys[j] (FG.cpp:2615-2690).
 // product != 0 starts GRM-product slots instead: P = b on the system's
-// samples, and the slot is done after the next GEMM pass.
-__global__ __launch_bounds__(256) void k_cols_init(const float* __restrict__ B, const int32_t* __restrict__ slots,
-                                                   const int32_t* __restrict__ sys, int kpad, int64_t Nnm,
+// samples, and the slot is done after the next GEMM pass.  A workgroup takes
+// 64 rows of all k columns and turns them in LDS: read along the rows of B,
+// written along the columns of the engine's row-major blocks.
+__global__ __launch_bounds__(256) void k_cols_init(const float* __restrict__ B, int k,
+                                                   const int32_t* __restrict__ slots,
+                                                   const int32_t* __restrict__ sys, int64_t Nnm,
                                                    int64_t Npad, const float* __restrict__ minv,
                                                    const uint8_t* __restrict__ mask, float* X, float* R, float* Z,
                                                    float* P, double* __restrict__ partial, int product) {
-    __shared__ double sm[2][256];
-    const int tid = threadIdx.x;
-    const int j = blockIdx.y;
-    const int slot = slots[j];
-    const int64_t so = (int64_t)sys[j] * Npad;
-    const int64_t i = (int64_t)blockIdx.x * VROWS + tid;
-    const bool on = i < Nnm && mask[so + i];
-    const float r = on ? B[(int64_t)j * Nnm + i] : 0.0f;
-    const float z = __fmul_rn(minv[so + i], r);
-    const int64_t o = i * kpad + slot;
-    X[o] = 0.0f;
-    R[o] = r;
-    Z[o] = z;
-    P[o] = product ? r : z;
-    sm[0][tid] = (double)z * (double)r;
-    sm[1][tid] = (double)r * (double)r;
-    for (int s = 128; s >= 1; s >>= 1) {
-        __syncthreads();
-        if (tid < s) {
-            sm[0][tid] += sm[0][tid + s];
-            sm[1][tid] += sm[1][tid + s];
+    __shared__ float tile[VROWS][EW + 1];
+    __shared__ double2 sm[256];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t r0 = (int64_t)blockIdx.x * VROWS;
+    for (int j = tid >> 6; j < k; j += 4) tile[lane][j] = r0 + lane < Nnm ? B[(int64_t)j * Nnm + r0 + lane] : 0.0f;
+    __syncthreads();
+    int kp = 1;                                   // columns rounded up to a power of two
+    while (kp < k) kp *= 2;
+    const int j = tid % kp, rstep = 256 / kp;
+    double2 v = make_double2(0.0, 0.0);
+    if (j < k) {
+        const int slot = slots[j];
+        const int64_t so = (int64_t)sys[j] * Npad;
+        for (int rl = tid / kp; rl < VROWS; rl += rstep) {
+            const int64_t i = r0 + rl, o = i * EW + slot;
+            const float r = i < Nnm && mask[so + i] ? tile[rl][j] : 0.0f;
+            const float z = __fmul_rn(minv[so + i], r);
+            X[o] = 0.0f;
+            R[o] = r;
+            Z[o] = z;
+            P[o] = product ? r : z;
+            v.x += (double)z * (double)r;
+            v.y += (double)r * (double)r;
         }
     }
-    if (tid == 0) {
-        partial[((int64_t)blockIdx.x * kpad + slot) * 2] = sm[0][0];
-        partial[((int64_t)blockIdx.x * kpad + slot) * 2 + 1] = sm[1][0];
+    sm[tid] = v;
+    for (int s = 128; s >= kp; s >>= 1) {
+        __syncthreads();
+        if (tid < s) {
+            sm[tid].x += sm[tid + s].x;
+            sm[tid].y += sm[tid + s].y;
+        }
+    }
+    if (tid < k) {
+        double* dst = partial + ((int64_t)blockIdx.x * EW + slots[tid]) * 2;
+        dst[0] = sm[tid].x;
+        dst[1] = sm[tid].y;
     }
 }
 
@@ -1374,20 +1456,25 @@ __global__ __launch_bounds__(256) void k_cols_init_finish(const int32_t* __restr
     }
 }
 
-__global__ void k_cols_gather(const float* __restrict__ src, const int32_t* __restrict__ slots, int kpad,
-                              int64_t Nnm, float* __restrict__ dst) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    if (i < Nnm) dst[(int64_t)j * Nnm + i] = src[i * kpad + slots[j]];
-}
-
-// slot results to chosen columns of a column-major buffer: dst[:, cols[j]]
-__global__ void k_cols_gather_to(const float* __restrict__ src, const int32_t* __restrict__ slots,
-                                 const int32_t* __restrict__ cols, int kpad, int64_t Nnm, int64_t ld,
-                                 float* __restrict__ dst) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    if (i < Nnm) dst[(int64_t)cols[j] * ld + i] = src[i * kpad + slots[j]];
+// Slot results to columns of a column-major buffer, dst[:, cols[j]] (cols
+// nullptr: j): 64 rows of all k columns per workgroup, turned in LDS.
+__global__ __launch_bounds__(256) void k_cols_gather(const float* __restrict__ src, int k,
+                                                     const int32_t* __restrict__ slots,
+                                                     const int32_t* __restrict__ cols, int64_t Nnm, int64_t ld,
+                                                     float* __restrict__ dst) {
+    __shared__ float tile[64][EW + 1];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t r0 = (int64_t)blockIdx.x * 64;
+    int kp = 1;
+    while (kp < k) kp *= 2;
+    const int j = tid % kp;
+    if (j < k) {
+        const int slot = slots[j];
+        for (int rl = tid / kp; rl < 64 && r0 + rl < Nnm; rl += 256 / kp) tile[rl][j] = src[(r0 + rl) * EW + slot];
+    }
+    __syncthreads();
+    if (r0 + lane < Nnm)
+        for (int c = tid >> 6; c < k; c += 4) dst[(int64_t)(cols ? cols[c] : c) * ld + r0 + lane] = tile[lane][c];
 }
 
 // column-major [k][Nnm] (host layout) <-> [Npad][kpad] row-major blocks
@@ -1502,14 +1589,16 @@ __global__ __launch_bounds__(256) void k_col_dots(const float* __restrict__ X, i
     }
 }
 
-__global__ void k_col_dots_finish(const double* __restrict__ partial, int64_t nb, int k, int nd,
-                                  double* __restrict__ out) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= k * nd) return;
-    const int j = t / nd, d = t - j * nd;
+// one wave per dot: lane l adds blocks l, l + 64, ..., then a fixed tree
+__global__ __launch_bounds__(64) void k_col_dots_finish(const double* __restrict__ partial, int64_t nb, int k, int nd,
+                                                        double* __restrict__ out) {
+    const int64_t t = blockIdx.x, n = (int64_t)k * nd;
     double s = 0.0;
-    for (int64_t b = 0; b < nb; b++) s += partial[(b * k + j) * nd + d];
-    out[t] = s;
+#pragma unroll 4
+    for (int64_t b = threadIdx.x; b < nb; b += 64) s += partial[b * n + t];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (threadIdx.x == 0) out[t] = s;
 }
 
 inline unsigned nblk(int64_t n, int64_t b) { return (unsigned)((n + b - 1) / b); }
@@ -1810,8 +1899,9 @@ hipError_t launch_update(hipStream_t s, int kpad, int64_t Nnm, int64_t Npad, con
                          const int32_t* sys, float* X, float* R, float* Z, const float* P, const float* AP,
                          double* partial, int64_t* nparts) {
     (void)Nnm;
+    if (kpad != EW) return hipErrorInvalidValue;
     const int64_t nb = Npad / VROWS;
-    hipLaunchKernelGGL(k_update, dim3((unsigned)nb), dim3(256), 0, s, kpad, Npad, alpha, done, live, kind, minv,
+    hipLaunchKernelGGL(k_update, dim3((unsigned)nb), dim3(256), 0, s, Npad, alpha, done, live, kind, minv,
                        sys, X, R, Z, P, AP, partial);
     if (nparts) *nparts = nb;
     return hipGetLastError();
@@ -1828,7 +1918,8 @@ hipError_t launch_beta(hipStream_t s, int kpad, const double* partial, int64_t n
 hipError_t launch_pupdate(hipStream_t s, int kpad, int64_t Nnm, int64_t Npad, const float* beta,
                           const uint8_t* done, const uint8_t* live, const uint8_t* kind, const float* Z, float* P) {
     (void)Nnm;
-    hipLaunchKernelGGL(k_pupdate, dim3(nblk(Npad * kpad, 256)), dim3(256), 0, s, kpad, Npad, beta, done,
+    if (kpad != EW) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_pupdate, dim3(nblk(Npad * (EW / 4), 256)), dim3(256), 0, s, Npad, beta, done,
                        live, kind, Z, P);
     return hipGetLastError();
 }
@@ -1836,9 +1927,10 @@ hipError_t launch_pupdate(hipStream_t s, int kpad, int64_t Nnm, int64_t Npad, co
 hipError_t launch_cols_init(hipStream_t s, const float* B, int k, const int32_t* slots, const int32_t* sys,
                             int kpad, int64_t Nnm, int64_t Npad, const float* minv, const uint8_t* mask, float* X,
                             float* R, float* Z, float* P, double* partial, int64_t* nparts, int product) {
+    if (kpad != EW || k < 1 || k > EW) return hipErrorInvalidValue;
     const int64_t nb = Npad / VROWS;
-    hipLaunchKernelGGL(k_cols_init, dim3((unsigned)nb, (unsigned)k), dim3(256), 0, s, B, slots, sys, kpad, Nnm, Npad,
-                       minv, mask, X, R, Z, P, partial, product);
+    hipLaunchKernelGGL(k_cols_init, dim3((unsigned)nb), dim3(256), 0, s, B, k, slots, sys, Nnm, Npad, minv, mask, X, R,
+                       Z, P, partial, product);
     if (nparts) *nparts = nb;
     return hipGetLastError();
 }
@@ -1851,9 +1943,10 @@ hipError_t launch_cols_init_finish(hipStream_t s, int k, const int32_t* slots, i
     return hipGetLastError();
 }
 
-hipError_t launch_cols_gather(hipStream_t s, const float* src, int k, const int32_t* slots, int kpad, int64_t Nnm,
-                              float* dst) {
-    hipLaunchKernelGGL(k_cols_gather, dim3(nblk(Nnm, 256), (unsigned)k), dim3(256), 0, s, src, slots, kpad, Nnm, dst);
+hipError_t launch_cols_gather(hipStream_t s, const float* src, int k, const int32_t* slots, const int32_t* cols,
+                              int kpad, int64_t Nnm, int64_t ld, float* dst) {
+    if (kpad != EW || k < 1 || k > EW) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_cols_gather, dim3(nblk(Nnm, 64)), dim3(256), 0, s, src, k, slots, cols, Nnm, ld, dst);
     return hipGetLastError();
 }
 
@@ -1894,13 +1987,6 @@ hipError_t launch_rademacher(hipStream_t s, float* dst, int64_t ld, int64_t N, u
 int col_dots_max() { return DOT_MAX; }
 int64_t col_dots_partial_doubles(int64_t Npad, int k) { return (Npad / DOT_ROWS + 1) * (int64_t)k * DOT_MAX; }
 
-hipError_t launch_cols_gather_to(hipStream_t s, const float* src, int k, const int32_t* slots, const int32_t* cols,
-                                 int kpad, int64_t Nnm, int64_t ld, float* dst) {
-    hipLaunchKernelGGL(k_cols_gather_to, dim3(nblk(Nnm, 256), (unsigned)k), dim3(256), 0, s, src, slots, cols, kpad,
-                       Nnm, ld, dst);
-    return hipGetLastError();
-}
-
 hipError_t launch_col_dots(hipStream_t s, const float* X, int64_t ldx, int kpad, const int32_t* slots, int k,
                            const float* P1, const float* P2, int64_t ldp, const int32_t* pcols, const float* Q,
                            int m, int64_t ldq, int64_t Nnm, double* partial, double* out) {
@@ -1911,7 +1997,7 @@ hipError_t launch_col_dots(hipStream_t s, const float* X, int64_t ldx, int kpad,
                        ldp, pcols, Q, m, ldq, Nnm, partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_col_dots_finish, dim3(nblk((int64_t)k * nd, 64)), dim3(64), 0, s, partial, nb, k, nd, out);
+    hipLaunchKernelGGL(k_col_dots_finish, dim3((unsigned)(k * nd)), dim3(64), 0, s, partial, nb, k, nd, out);
     return hipGetLastError();
 }
 

@@ -490,7 +490,7 @@ int engine_take_batch(saige_ctx* c, Engine& e, int k, const int32_t* slots, floa
     for (int j = 0; j < k; j++) e.h_live[slots[j]] = 0;
     SAIGE_HIP_TRY(push_slot_state(c, e));
     if (X_host) {
-        SAIGE_HIP_TRY(launch_cols_gather(st, e.X, k, e.d_list, e.kpad, c->Nnm, e.stageB));
+        SAIGE_HIP_TRY(launch_cols_gather(st, e.X, k, e.d_list, nullptr, e.kpad, c->Nnm, c->Nnm, e.stageB));
         SAIGE_HIP_TRY(hipMemcpyAsync(X_host, e.stageB, sizeof(float) * c->Nnm * k, hipMemcpyDeviceToHost, st));
     }
     SAIGE_HIP_TRY(hipStreamSynchronize(st));
@@ -576,9 +576,9 @@ int engine_take_batch_ex(saige_ctx* c, Engine& e, int k, const int32_t* slots, f
     SAIGE_HIP_TRY(push_slot_state(c, e));
     if (int rc = column_dots(c, e.X, 0, e.kpad, d_slots, k, P1, P2, ldp, d_slots + 2 * EW, Q, m, ldq, dots_host))
         return rc;
-    if (X_dev) SAIGE_HIP_TRY(launch_cols_gather_to(st, e.X, k, d_slots, d_slots + EW, e.kpad, c->Nnm, ldx, X_dev));
+    if (X_dev) SAIGE_HIP_TRY(launch_cols_gather(st, e.X, k, d_slots, d_slots + EW, e.kpad, c->Nnm, ldx, X_dev));
     if (X_host) {
-        SAIGE_HIP_TRY(launch_cols_gather(st, e.X, k, d_slots, e.kpad, c->Nnm, e.stageB));
+        SAIGE_HIP_TRY(launch_cols_gather(st, e.X, k, d_slots, nullptr, e.kpad, c->Nnm, c->Nnm, e.stageB));
         SAIGE_HIP_TRY(hipMemcpyAsync(X_host, e.stageB, sizeof(float) * c->Nnm * k, hipMemcpyDeviceToHost, st));
     }
     SAIGE_HIP_TRY(hipStreamSynchronize(st));

@@ -500,8 +500,9 @@ hipError_t launch_cols_init(hipStream_t s, const float* B, int k, const int32_t*
 hipError_t launch_cols_init_finish(hipStream_t s, int k, const int32_t* slots, int kpad, const double* partial,
                                    int64_t nparts, double* rz, double* sumr2, const int32_t* maxiter,
                                    const double* tol, int32_t* iter, uint8_t* done, int product);
-hipError_t launch_cols_gather(hipStream_t s, const float* src, int k, const int32_t* slots, int kpad, int64_t Nnm,
-                              float* dst);
+// slot results to columns cols[j] (nullptr: j) of a column-major buffer
+hipError_t launch_cols_gather(hipStream_t s, const float* src, int k, const int32_t* slots, const int32_t* cols,
+                              int kpad, int64_t Nnm, int64_t ld, float* dst);
 hipError_t launch_scatter_cols(hipStream_t s, const float* src, int64_t k, int64_t Nnm,
                                int64_t Npad, int kpad, float* dst);
 hipError_t launch_gather_cols(hipStream_t s, const float* src, int64_t k, int64_t Nnm, int kpad,
@@ -520,7 +521,5 @@ int64_t col_dots_partial_doubles(int64_t Npad, int k);
 hipError_t launch_col_dots(hipStream_t s, const float* X, int64_t ldx, int kpad, const int32_t* slots, int k,
                            const float* P1, const float* P2, int64_t ldp, const int32_t* pcols, const float* Q,
                            int m, int64_t ldq, int64_t Nnm, double* partial, double* out);
-hipError_t launch_cols_gather_to(hipStream_t s, const float* src, int k, const int32_t* slots, const int32_t* cols,
-                                 int kpad, int64_t Nnm, int64_t ld, float* dst);
 
 }  // namespace saige
