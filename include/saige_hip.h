@@ -334,7 +334,9 @@ int saige_autotune_candidates(int* rt, int* pd, int* nsplit);
 /* Set the block-GEMM shape explicitly, for full and one-half launches
  * (engine idle). */
 int saige_set_gemm_config(saige_ctx* ctx, int rt, int pd, int nsplit);
-/* Current shape, and its tuned per-launch time in ms (0 if not tuned). */
+/* Current shape, and its tuned per-launch time in ms (0 if not tuned).  Until
+ * a shape is tuned or set, the library takes the prefetch depth it has
+ * measured better for the launch's width in place of pd (the same bits). */
 int saige_get_gemm_config(const saige_ctx* ctx, int* rt, int* pd, int* nsplit, double* tuned_ms);
 /* Shape of one-half launches (nsplit as the full shape). */
 int saige_get_gemm_config_half(const saige_ctx* ctx, int* rt, int* pd, double* tuned_ms);

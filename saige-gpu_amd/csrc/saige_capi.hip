@@ -347,6 +347,19 @@ int engine_add(saige_ctx* c, Engine& e, int slot, int s, const float* b_host, in
     return engine_add_batch(c, e, 1, &slot, &s, b_host, maxiter, tol);
 }
 
+// The shape of a block product over all 64 columns or fewer (`cfg` is the
+// context's for that width).  Until a shape is tuned or set, the prefetch
+// depth, which does not change the bits, is the one measured better at the
+// default shape's other parameters: three chunks ahead (two in the split
+// modes), except where that spills, over 64 columns in the lower-triangle mode.
+// ms at N = 100,000 at depth 1 and 3: FP32 mode 14.4 and 14.0 (half 9.6 and
+// 9.1; N = 10,000: 0.167 and 0.151), lower triangle 7.6 and 11.7, half 5.6 and
+// 5.3, 16 columns 5.2 and 4.6.
+GemmConfig shape_used(const saige_ctx* c, GemmConfig cfg, bool full) {
+    if (!c->gemm_shape_set) cfg.pd = cfg.mode == GEMM_BF16X3_TRI && full ? 1 : 3;
+    return cfg;
+}
+
 // items per row set left of its diagonal block in the lower-triangle
 // product: at most TRI_CHUNKS chunks of 32 columns (3072 columns) per item
 constexpr int TRI_CHUNKS = 96;
@@ -438,9 +451,11 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
         int64_t np = 0;
         SAIGE_HIP_TRY(hipEventRecord(c->ev0, st));
         SAIGE_HIP_TRY(launch_grm_gemm(st, g.S, Np, N, e.P, e.AP, a, e.partial, &np, e.ypart,
-                                      quarter       ? c->gemm_cfg_quarter
-                                      : halves == 3 ? c->gemm_cfg
-                                                    : c->gemm_cfg_half,
+                                      shape_used(c,
+                                                 quarter       ? c->gemm_cfg_quarter
+                                                 : halves == 3 ? c->gemm_cfg
+                                                               : c->gemm_cfg_half,
+                                                 halves == 3 && !narrow),
                                       halves, &c->tri, g.s16, narrow ? &nc : nullptr));
         SAIGE_HIP_TRY(hipEventRecord(c->ev1, st));
         SAIGE_HIP_TRY(launch_alpha(st, e.kpad, e.partial, np, e.rz, e.done, e.live, e.kind, e.alpha));
@@ -1275,7 +1290,8 @@ static int grm_matvec(saige_ctx* c, int loco, const float* B, int64_t k, float* 
         const NarrowCols q0 = NarrowCols::tile(16, 0);
         if (e == hipSuccess)
             e = launch_grm_gemm(st, g.S, Np, N, d_blk, d_out, a, nullptr, nullptr, c->d_mv_ypart,
-                                q ? c->gemm_cfg_quarter : kb <= 32 ? c->gemm_cfg_half : c->gemm_cfg,
+                                shape_used(c, q ? c->gemm_cfg_quarter : kb <= 32 ? c->gemm_cfg_half : c->gemm_cfg,
+                                           kb > 32),
                                 kb <= 32 ? 1 : 3, &c->tri, g.s16, q ? &q0 : nullptr);
         if (e == hipSuccess) e = launch_gather_cols(st, d_out, kb, N, EW, d_in);
         if (e == hipSuccess) e = hipMemcpyAsync(Y + k0 * N, d_in, 4 * N * kb, hipMemcpyDeviceToHost, st);
@@ -2002,6 +2018,7 @@ int saige_autotune(saige_ctx* c, int reps, double* ms_table) {
         }
     }
     c->gemm_cfg = best;
+    c->gemm_shape_set = true;
     c->gemm_tuned_ms = best_ms;
     c->gemm_cfg_half = best_h;
     c->gemm_tuned_ms_half = best_h_ms;
@@ -2029,6 +2046,7 @@ int saige_set_gemm_config(saige_ctx* c, int rt, int pd, int nsplit) {
     }
     if (int rc = engine_idle(c, "changing the block-GEMM shape")) return rc;
     c->gemm_cfg = g;
+    c->gemm_shape_set = true;
     c->gemm_tuned_ms = 0.0;
     c->gemm_cfg_half = g;
     c->gemm_cfg_quarter = g;

@@ -295,6 +295,7 @@ struct saige_ctx {
     // shape for launches over one 32-column half: same nsplit (the summation
     // order, so a column's bits do not depend on the other half), own rt/pd
     saige::GemmConfig gemm_cfg_half;
+    bool gemm_shape_set = false;                 // by saige_autotune or saige_set_gemm_config
     saige::GemmConfig gemm_cfg_quarter;     // 16-column launches (lower-triangle mode)
     saige::TriPlan tri;                          // lower-triangle product (mode 2), built on first use
     int gemv_mode = SAIGE_GEMV_TRI;              // single-column products: lower triangle or all of S
