@@ -26,11 +26,61 @@ namespace saige {
 namespace {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 
 __device__ __forceinline__ float wave_sum_f(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
+}
+
+// ------------------------------------------------------- 24-bit triangle
+// A value of at most 16 significant bits (the split GRM's storage) has its
+// low 8 FP32 bits zero: three bytes hold it.  The products that stream the
+// lower triangle are bound by its bytes, so they read it in this form where
+// it is there (15 GB instead of 20 at N = 100,000): 32 x 32 blocks (I, J),
+// J < I, of 3 KB each, block (I, J) at I (I - 1) / 2 + J, so that a strip of 32
+// rows is one contiguous stream.  Within a block lane (ln = l % 16, g = l / 16)
+// owns rows 16 r + ln (r = 0, 1), columns 8 g + [0, 8), the layout of the MFMA
+// operands: [r][lane] 16 bytes, the upper halves of its eight words (the first
+// BF16 piece by truncation, as it stands), then [lane] 16 bytes, the third byte
+// of the eight words of r = 0 and of r = 1.
+constexpr int64_t S24_BLOCK = 3072;
+__host__ __device__ __forceinline__ int64_t s24_block(int64_t I, int64_t J) { return I * (I - 1) / 2 + J; }
+
+// elements 2k and 2k + 1 (k < 4) of a lane's row from h[k] and their third bytes
+// in l[k / 2]
+__device__ __forceinline__ uint32_t s24_lo(u32x4 h, const uint32_t (&l)[2], int k) {
+    return __builtin_amdgcn_perm(h[k], l[k >> 1], 0x0504000Cu | (uint32_t)((2 * (k & 1)) << 8));
+}
+__device__ __forceinline__ uint32_t s24_hi(u32x4 h, const uint32_t (&l)[2], int k) {
+    return __builtin_amdgcn_perm(h[k], l[k >> 1], 0x0706000Cu | (uint32_t)((2 * (k & 1) + 1) << 8));
+}
+
+// k_pack24: one wave per block of the FP32 triangle.  Reads 20 GB and writes 15
+// GB at N = 100,000: 6.7 ms, 5.2 TB/s.
+__global__ __launch_bounds__(256) void k_pack24(const float* __restrict__ S, int64_t ld, uint8_t* __restrict__ out) {
+    const int lane = threadIdx.x & 63, ln = lane & 15, g = lane >> 4;
+    const int64_t I = blockIdx.y + 1;
+    const int64_t J = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (J >= I) return;
+    u32x4* dst = reinterpret_cast<u32x4*>(out + s24_block(I, J) * S24_BLOCK);
+    u32x4 lo;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const float* p = S + (32 * I + 16 * r + ln) * ld + 32 * J + 8 * g;
+        const u32x4 a = *reinterpret_cast<const u32x4*>(p), b = *reinterpret_cast<const u32x4*>(p + 4);
+        const u32x4 h = {__builtin_amdgcn_perm(a[1], a[0], 0x07060302u), __builtin_amdgcn_perm(a[3], a[2], 0x07060302u),
+                         __builtin_amdgcn_perm(b[1], b[0], 0x07060302u), __builtin_amdgcn_perm(b[3], b[2], 0x07060302u)};
+        // byte 1 of four words
+        const uint32_t a01 = __builtin_amdgcn_perm(a[1], a[0], 0x0C0C0501u), a23 = __builtin_amdgcn_perm(a[3], a[2], 0x0C0C0501u);
+        const uint32_t b01 = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0501u), b23 = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0501u);
+        lo[2 * r] = a01 | (a23 << 16);
+        lo[2 * r + 1] = b01 | (b23 << 16);
+        dst[64 * r + lane] = h;
+    }
+    dst[128 + lane] = lo;
 }
 
 // --------------------------------------------------------------- GEMV
@@ -157,6 +207,115 @@ __global__ __launch_bounds__(512) void k_gemv_tri(const float* __restrict__ S, i
     for (int r = 0; r < 32; r++) {
         const float t = wave_sum_f(acc[r]);
         if (lane == r) yp[r] = t;
+    }
+}
+
+// x summed over the 16 lanes of its group (lanes 16 g + [0, 16)), to the
+// group's last lane: four shifts by 1, 2, 4 and 8 lanes within the group
+__device__ __forceinline__ float row16_sum(float x) {
+    auto shr = [](float v, auto n) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x110 + decltype(n)::value, 0xF, 0xF, true));
+    };
+    x += shr(x, std::integral_constant<int, 1>());
+    x += shr(x, std::integral_constant<int, 2>());
+    x += shr(x, std::integral_constant<int, 4>());
+    x += shr(x, std::integral_constant<int, 8>());
+    return x;
+}
+
+// k_gemv_tri24: k_gemv_tri on the 24-bit triangle, the same items and partials.
+// A wave's strip is a stream of 3 KB blocks, eight per 256-column chunk.  Lane
+// (ln, g) holds rows ln and 16 + ln and eight columns of a block: use 1 adds into
+// two accumulators per lane, use 2 into eight per block, which are summed over
+// the 16 lanes of a column group (DPP) and left in LDS per strip.  Diagonal
+// items read the FP32 square.  Bound by S's bytes: 2.64 ms at N = 100,000 (5.7
+// TB/s), 3.43 on the FP32 triangle; 0.69 ms at 50,000.
+__global__ __launch_bounds__(512) void k_gemv_tri24(const float* __restrict__ S, const uint8_t* __restrict__ S24,
+                                                    int64_t ld, const float* __restrict__ x,
+                                                    const int4* __restrict__ items, float* __restrict__ y1p,
+                                                    float* __restrict__ y2p, const int32_t* __restrict__ over,
+                                                    int iter) {
+    __shared__ __attribute__((aligned(16))) float sz[2][8][TV_COLS];   // use-2 strip sums, two chunks
+    if (over && *over <= iter) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, ln = lane & 15, g = lane >> 4;
+    const int4 item = items[blockIdx.x];
+    const int64_t R = item.x, ca = item.y, cb = item.z, slot = item.w;
+    const int64_t NR = ld / TV_ROWS;
+    const int64_t r0 = R * TV_ROWS + 32 * wv;   // the wave's first row
+    float* yp = y1p + slot * TV_ROWS + 32 * wv;
+    if (ca >= R) {                              // the diagonal block: use 1 only, FP32
+        const float4 xj = *reinterpret_cast<const float4*>(x + TV_COLS * R + 4 * lane);
+        const float* Sb = S + r0 * ld + TV_COLS * R + 4 * lane;
+#pragma unroll 8
+        for (int r = 0; r < 32; r++) {
+            const float4 v = *reinterpret_cast<const float4*>(Sb + r * ld);
+            const float t = wave_sum_f(v.x * xj.x + v.y * xj.y + v.z * xj.z + v.w * xj.w);
+            if (lane == r) yp[r] = t;
+        }
+        return;
+    }
+    const float xr0 = x[r0 + ln], xr1 = x[r0 + 16 + ln];
+    const u32x4* strip = reinterpret_cast<const u32x4*>(S24 + s24_block(r0 / 32, 0) * S24_BLOCK) + lane;
+    float acc0 = 0.0f, acc1 = 0.0f;
+    for (int64_t c = ca; c < cb; c++) {
+        const u32x4* bp = strip + 8 * c * (S24_BLOCK / 16);
+        u32x4 h0[8], h1[8], lo[8];
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            h0[b] = bp[b * 192];
+            h1[b] = bp[b * 192 + 64];
+            lo[b] = bp[b * 192 + 128];
+        }
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const float* xc = x + TV_COLS * c + 32 * b + 8 * g;
+            const float4 xa = *reinterpret_cast<const float4*>(xc), xb = *reinterpret_cast<const float4*>(xc + 4);
+            const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+            const uint32_t l0[2] = {lo[b][0], lo[b][1]}, l1[2] = {lo[b][2], lo[b][3]};
+            float z[8];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float a0 = __uint_as_float(s24_lo(h0[b], l0, k)), a1 = __uint_as_float(s24_hi(h0[b], l0, k));
+                const float b0 = __uint_as_float(s24_lo(h1[b], l1, k)), b1 = __uint_as_float(s24_hi(h1[b], l1, k));
+                acc0 = __fmaf_rn(a0, xv[2 * k], acc0);
+                acc1 = __fmaf_rn(b0, xv[2 * k], acc1);
+                acc0 = __fmaf_rn(a1, xv[2 * k + 1], acc0);
+                acc1 = __fmaf_rn(b1, xv[2 * k + 1], acc1);
+                z[2 * k] = __fmaf_rn(b0, xr1, a0 * xr0);
+                z[2 * k + 1] = __fmaf_rn(b1, xr1, a1 * xr0);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) z[k] = row16_sum(z[k]);
+            if (ln == 15) {
+                float4* d = reinterpret_cast<float4*>(&sz[c & 1][wv][32 * b + 8 * g]);
+                d[0] = make_float4(z[0], z[1], z[2], z[3]);
+                d[1] = make_float4(z[4], z[5], z[6], z[7]);
+            }
+        }
+        // buffer c & 1 was last read for chunk c-2, before chunk c-1's barrier
+        lds_barrier();
+        if (wv == (int)(c & 7)) {
+            float4 sum = *reinterpret_cast<const float4*>(&sz[c & 1][0][4 * lane]);
+#pragma unroll
+            for (int w = 1; w < 8; w++) {
+                const float4 v = *reinterpret_cast<const float4*>(&sz[c & 1][w][4 * lane]);
+                sum.x += v.x;
+                sum.y += v.y;
+                sum.z += v.z;
+                sum.w += v.w;
+            }
+            const int64_t ps = triv_y2_first(c, NR) + (R - c - 1);
+            *reinterpret_cast<float4*>(y2p + ps * TV_COLS + 4 * lane) = sum;
+        }
+    }
+    // the four column groups' sums of each row
+    acc0 += __shfl_xor(acc0, 16, 64);
+    acc1 += __shfl_xor(acc1, 16, 64);
+    acc0 += __shfl_xor(acc0, 32, 64);
+    acc1 += __shfl_xor(acc1, 32, 64);
+    if (g == 0) {
+        yp[ln] = acc0;
+        yp[16 + ln] = acc1;
     }
 }
 
@@ -381,9 +540,6 @@ __global__ __launch_bounds__(256) void k_gemm_part(const float* __restrict__ S, 
 // would also drain every outstanding global load.  W is the waves-per-SIMD
 // bound each shape is compiled for.  Raw sums go to Ypart exactly as
 // k_gemm_part writes them.
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
-
 __device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
     const uint32_t b0 = __float_as_uint(x0), b1 = __float_as_uint(x1);
     const float r0 = x0 - __uint_as_float(b0 & 0xffff0000u);
@@ -425,6 +581,20 @@ __device__ __forceinline__ void split2_8(float4 a, float4 b, u32x4& h, u32x4& m)
     split2_pair(b.z, b.w, h3, m3);
     h = u32x4{h0, h1, h2, h3};
     m = u32x4{m0, m1, m2, m3};
+}
+
+// the second piece of eight 24-bit values: h their upper halves, l0 and l1 their
+// third bytes (split2_pair's remainders, formed the same way)
+__device__ __forceinline__ u32x4 s24_mid(u32x4 h, uint32_t l0, uint32_t l1) {
+    const uint32_t l[2] = {l0, l1};
+    u32x4 m;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float r0 = __uint_as_float(s24_lo(h, l, k)) - __uint_as_float(h[k] << 16);
+        const float r1 = __uint_as_float(s24_hi(h, l, k)) - __uint_as_float(h[k] & 0xffff0000u);
+        m[k] = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
+    }
+    return m;
 }
 
 __device__ __forceinline__ f32x16 mfma_bf(u32x4 a, u32x4 b, f32x16 c) {
@@ -791,8 +961,15 @@ __device__ __forceinline__ int map_col(const ColMap32& m, int k) {
 
 // cm: the block columns of a 16- or 32-column launch (NQ 1 or 2), which
 // holds its P pieces, partials and LDS tiles at launch columns [0, 16*NQ)
-template <int NWV, int PD, int NQ, int SP>
-__global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__ S, int64_t ld,
+// C24 (SP = 2): chunks left of the diagonal come from the 24-bit triangle, whose
+// upper halves are the first piece as they stand; the diagonal squares are read
+// in FP32.  The same values, so the same bits.  Narrow launches are bound by S's
+// bytes, the full one by the matrix cores' rate beside them: 16, 32 and 64
+// columns at N = 100,000 take 3.48, 4.31 and 6.98 ms, 4.61, 5.20 and 7.60 on the
+// FP32 triangle.
+template <int NWV, int PD, int NQ, int SP, bool C24>
+__global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__ S, const uint8_t* __restrict__ S24,
+                                                       int64_t ld,
                                                        const u32x4* __restrict__ pb, const float* __restrict__ P,
                                                        const int4* __restrict__ items, float* __restrict__ y1p,
                                                        float* __restrict__ y2p, ColMap32 cm) {
@@ -813,6 +990,11 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
     const int64_t rw = R * GM + wv * 32;             // the wave's first row
     const bool valid = rw < ld;                      // ld = Npad, a multiple of 32
     const float* srow = S + ((valid ? rw : ld - 32) + ln) * ld + 8 * g;
+    // the strip's blocks (for rows past ld any blocks in range: their results
+    // are not used)
+    const u32x4* strip = C24 ? reinterpret_cast<const u32x4*>(S24 + s24_block((valid ? rw : ld - 32) / 32, 0) * S24_BLOCK) +
+                                   lane
+                             : nullptr;
     constexpr int c0 = 0;                            // the launch's first column in LDS and partials
     // the block column of launch column k (of 16 * NQ)
     auto gcol = [&](int k) { return NQ < 4 ? map_col(cm, k) : k; };
@@ -843,20 +1025,39 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
     for (int r = 0; r < 2; r++)
 #pragma unroll
         for (int t = 0; t < NQ; t++) acc1[r][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float4 ring[RING][2][2];                         // [slot][row tile][half of the lane's 8 columns]
+    // a raw chunk: FP32, [2 * row tile + half of the lane's 8 columns], or (24
+    // bits) the two row tiles' upper halves and their third bytes
+    u32x4 ring[RING][4];
     u32x4 bring[RING][STG];
-    auto issue = [&](float4 (&rs)[2][2], u32x4 (&br)[STG], int64_t ch) {
-#pragma unroll
-        for (int s = 0; s < STG; s++) br[s] = bsrc[s][4 * ch * EW];
-#pragma unroll
-        for (int r = 0; r < 2; r++)
-#pragma unroll
-            for (int h = 0; h < 2; h++)
-                rs[r][h] = *reinterpret_cast<const float4*>(srow + (int64_t)r * 16 * ld + ch * 32 + 4 * h);
-    };
     // the run over the item; U2: chunks left of the diagonal (use 1 and 2)
     auto run = [&](auto u2tag) {
         constexpr bool U2 = decltype(u2tag)::value;
+        constexpr bool S3 = C24 && U2;               // this item's chunks are in the 24-bit form
+        auto issue = [&](u32x4 (&rs)[4], u32x4 (&br)[STG], int64_t ch) {
+#pragma unroll
+            for (int s = 0; s < STG; s++) br[s] = bsrc[s][4 * ch * EW];
+            if constexpr (S3) {
+#pragma unroll
+                for (int k = 0; k < 3; k++) rs[k] = strip[ch * (S24_BLOCK / 16) + 64 * k];
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    rs[k] = *reinterpret_cast<const u32x4*>(srow + (int64_t)(k >> 1) * 16 * ld + ch * 32 + 4 * (k & 1));
+            }
+        };
+        // a raw chunk's pieces of row tile r
+        auto split = [&](const u32x4 (&rs)[4], int r, u32x4& h, u32x4& m, u32x4& l) {
+            if constexpr (S3) {
+                h = rs[r];
+                m = s24_mid(rs[r], rs[2][2 * r], rs[2][2 * r + 1]);
+            } else {
+                const float4 a = __builtin_bit_cast(float4, rs[2 * r]), b = __builtin_bit_cast(float4, rs[2 * r + 1]);
+                if constexpr (SP == 3)
+                    split3_8(a, b, h, m, l);
+                else
+                    split2_8(a, b, h, m);
+            }
+        };
         // the A operand of use 2: P rows rw + 4g + tt (tt < 4) and
         // rw + 16 + 4g + tt - 4 (tt >= 4), launch column 16t + ln, as three
         // pieces (zero for rows past ld)
@@ -965,12 +1166,7 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
             if (pre) issue(ring[(u + PD) % RING], bring[(u + PD) % RING], c + PD < cb ? c + PD : cb - 1);
             u32x4 ah[2], am[2], al[2];
 #pragma unroll
-            for (int r = 0; r < 2; r++) {
-                if (SP == 3)
-                    split3_8(ring[u][r][0], ring[u][r][1], ah[r], am[r], al[r]);
-                else
-                    split2_8(ring[u][r][0], ring[u][r][1], ah[r], am[r]);
-            }
+            for (int r = 0; r < 2; r++) split(ring[u], r, ah[r], am[r], al[r]);
             chunk_mfma(par, c, ah, am, al);
         };
         if (PIPE) {
@@ -984,14 +1180,9 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
             // compile-time indices.
             constexpr int UNR = RING == 3 ? 6 : 2;
             u32x4 pcs[2][SP][2];                      // [set][piece][row tile]
-            auto split_into = [&](const float4 (&rs)[2][2], u32x4 (&p)[SP][2]) {
+            auto split_into = [&](const u32x4 (&rs)[4], u32x4 (&p)[SP][2]) {
 #pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    if constexpr (SP == 3)
-                        split3_8(rs[r][0], rs[r][1], p[0][r], p[1][r], p[2][r]);
-                    else
-                        split2_8(rs[r][0], rs[r][1], p[0][r], p[1][r]);
-                }
+                for (int r = 0; r < 2; r++) split(rs, r, p[0][r], p[1][r], p[SP - 1][r]);
             };
             // k: the chunk's offset from ca modulo UNR
             auto pstep = [&](int k, int64_t c) {
@@ -1609,12 +1800,25 @@ int64_t gemv_max_parts(int64_t Npad) { return Npad / GEMV_ROWS; }
 int64_t gemm_max_parts(int64_t Npad) { return Npad / EROWS; }
 int64_t vec_max_parts(int64_t Npad, int) { return Npad / VROWS; }
 
-hipError_t launch_grm_gemv(hipStream_t s, const float* S, int64_t Npad, int64_t Nnm, const float* in,
+int64_t s24_bytes(int64_t Npad) { return s24_block(Npad / 32, 0) * S24_BLOCK; }
+
+hipError_t launch_pack24(hipStream_t s, const float* S, int64_t Npad, uint8_t* out) {
+    const int64_t nb = Npad / 32;
+    if (nb < 2) return hipSuccess;
+    hipLaunchKernelGGL(k_pack24, dim3((unsigned)((nb + 2) / 4), (unsigned)(nb - 1)), dim3(256), 0, s, S, Npad, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_grm_gemv(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, const float* in,
                            float* out, VecArgs a, double* partial, int64_t* nparts, const GemvPlan* tri) {
     if (tri) {
         if (tri->Npad != Npad || !tri->items || Npad % TV_ROWS != 0) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_gemv_tri, dim3((unsigned)tri->nitems), dim3(512), 0, s, S, Npad, in, tri->items,
-                           tri->y1p, tri->y2p, a.over, a.iter);
+        if (m.s24)
+            hipLaunchKernelGGL(k_gemv_tri24, dim3((unsigned)tri->nitems), dim3(512), 0, s, m.S, m.s24, Npad, in,
+                               tri->items, tri->y1p, tri->y2p, a.over, a.iter);
+        else
+            hipLaunchKernelGGL(k_gemv_tri, dim3((unsigned)tri->nitems), dim3(512), 0, s, m.S, Npad, in, tri->items,
+                               tri->y1p, tri->y2p, a.over, a.iter);
         const int64_t nb = Npad / TV_ROWS;
         hipLaunchKernelGGL(k_gemv_tri_epi, dim3((unsigned)nb), dim3(256), 0, s, tri->y1p, tri->y2p, tri->rtab, Npad,
                            Nnm, in, out, a, partial);
@@ -1622,7 +1826,7 @@ hipError_t launch_grm_gemv(hipStream_t s, const float* S, int64_t Npad, int64_t 
         return hipGetLastError();
     }
     const int64_t nb = Npad / GEMV_ROWS;
-    hipLaunchKernelGGL(k_gemv, dim3((unsigned)nb), dim3(256), 0, s, S, Npad, Nnm, in, out, a, partial);
+    hipLaunchKernelGGL(k_gemv, dim3((unsigned)nb), dim3(256), 0, s, m.S, Npad, Nnm, in, out, a, partial);
     if (nparts) *nparts = nb;
     return hipGetLastError();
 }
@@ -1764,10 +1968,14 @@ hipError_t tri_plan_build(TriPlan& t, int64_t Npad, int nwv, int ch) {
 
 namespace {
 template <int NWV, int PD, int NQ, int SP>
-void launch_t16(hipStream_t s, dim3 grid, const float* S, int64_t Npad, const u32x4* pb, const float* in,
+void launch_t16(hipStream_t s, dim3 grid, GrmMat m, int64_t Npad, const u32x4* pb, const float* in,
                 const TriPlan& t, ColMap32 cm, float* ypart) {
-    hipLaunchKernelGGL((k_gemm_t16<NWV, PD, NQ, SP>), grid, dim3(64 * NWV), 0, s, S, Npad, pb, in, t.items, t.y1p,
-                       t.y2p, cm);
+    if (SP == 2 && m.s24)
+        hipLaunchKernelGGL((k_gemm_t16<NWV, PD, NQ, 2, true>), grid, dim3(64 * NWV), 0, s, m.S, m.s24, Npad, pb, in,
+                           t.items, t.y1p, t.y2p, cm);
+    else
+        hipLaunchKernelGGL((k_gemm_t16<NWV, PD, NQ, SP, false>), grid, dim3(64 * NWV), 0, s, m.S, m.s24, Npad, pb, in,
+                           t.items, t.y1p, t.y2p, cm);
     hipLaunchKernelGGL((k_tri_reduce<NWV, 4 * NQ>), dim3((unsigned)(Npad * 4 * NQ / 256)), dim3(256), 0, s, t.y1p,
                        t.y2p, t.rtab, Npad, cm, ypart);
 }
@@ -1775,7 +1983,7 @@ void launch_t16(hipStream_t s, dim3 grid, const float* S, int64_t Npad, const u3
 // the lower-triangle product over the launch's 64 columns, or the 16 or 32
 // block columns narrow lists (nullptr and halves 1 or 2: the half's 32)
 template <int NWV, int SP>
-hipError_t launch_tri(hipStream_t s, const float* S, int64_t Npad, const float* in, float* ypart, int pd,
+hipError_t launch_tri(hipStream_t s, GrmMat m, int64_t Npad, const float* in, float* ypart, int pd,
                       int halves, const NarrowCols* narrow, const TriPlan& t) {
     const int64_t G = Npad / 8;
     u32x4* pb = reinterpret_cast<u32x4*>(ypart + (int64_t)GSPLIT_MAX * Npad * EW);
@@ -1788,22 +1996,23 @@ hipError_t launch_tri(hipStream_t s, const float* S, int64_t Npad, const float* 
     if (narrow)
         for (int k = 0; k < narrow->width; k++) cm.w[k / 4] |= (uint32_t)narrow->col[k] << (8 * (k % 4));
     if (narrow && narrow->width == 16) {
-        if (deep) launch_t16<NWV, 2, 1, SP>(s, grid, S, Npad, pb, in, t, cm, ypart);
-        else launch_t16<NWV, 1, 1, SP>(s, grid, S, Npad, pb, in, t, cm, ypart);
+        if (deep) launch_t16<NWV, 2, 1, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
+        else launch_t16<NWV, 1, 1, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
     } else if (narrow) {
-        if (deep) launch_t16<NWV, 2, 2, SP>(s, grid, S, Npad, pb, in, t, cm, ypart);
-        else launch_t16<NWV, 1, 2, SP>(s, grid, S, Npad, pb, in, t, cm, ypart);
+        if (deep) launch_t16<NWV, 2, 2, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
+        else launch_t16<NWV, 1, 2, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
     } else {
-        if (deep) launch_t16<NWV, 2, 4, SP>(s, grid, S, Npad, pb, in, t, cm, ypart);
-        else launch_t16<NWV, 1, 4, SP>(s, grid, S, Npad, pb, in, t, cm, ypart);
+        if (deep) launch_t16<NWV, 2, 4, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
+        else launch_t16<NWV, 1, 4, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
     }
     return hipGetLastError();
 }
 }  // namespace
 
-hipError_t launch_grm_gemm(hipStream_t s, const float* S, int64_t Npad, int64_t Nnm, const float* in,
+hipError_t launch_grm_gemm(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, const float* in,
                            float* out, SigmaArgs a, double* partial, int64_t* nparts, float* ypart, GemmConfig g,
-                           int halves, const TriPlan* tri, bool s16, const NarrowCols* narrow) {
+                           int halves, const TriPlan* tri, const NarrowCols* narrow) {
+    const float* S = m.S;
     // Npad is a multiple of 256 = 128 * RT for both RT; a slice holds at least
     // one superchunk when Npad / GKS >= nsplit
     if (!gemm_config_valid(g) || Npad % 256 != 0 || halves < 1 || halves > 3) return hipErrorInvalidValue;
@@ -1821,12 +2030,12 @@ hipError_t launch_grm_gemm(hipStream_t s, const float* S, int64_t Npad, int64_t 
                 seen |= 1ull << col;
             }
         }
-        if (s16)
-            e = tri->nwv == 8 ? launch_tri<8, 2>(s, S, Npad, in, ypart, g.pd, halves, narrow, *tri)
-                              : launch_tri<12, 2>(s, S, Npad, in, ypart, g.pd, halves, narrow, *tri);
+        if (m.s16)
+            e = tri->nwv == 8 ? launch_tri<8, 2>(s, m, Npad, in, ypart, g.pd, halves, narrow, *tri)
+                              : launch_tri<12, 2>(s, m, Npad, in, ypart, g.pd, halves, narrow, *tri);
         else
-            e = tri->nwv == 8 ? launch_tri<8, 3>(s, S, Npad, in, ypart, g.pd, halves, narrow, *tri)
-                              : launch_tri<12, 3>(s, S, Npad, in, ypart, g.pd, halves, narrow, *tri);
+            e = tri->nwv == 8 ? launch_tri<8, 3>(s, m, Npad, in, ypart, g.pd, halves, narrow, *tri)
+                              : launch_tri<12, 3>(s, m, Npad, in, ypart, g.pd, halves, narrow, *tri);
         if (e != hipSuccess) return e;
         const int64_t nb = Npad / EROWS;
         hipLaunchKernelGGL(k_gemm_epi, dim3((unsigned)nb), dim3(256), 0, s, ypart, 1, Npad, Nnm, in, out, a,

@@ -141,7 +141,9 @@ void clear_geno(saige_ctx* c) {
     c->d_packed = c->d_packed_vr = nullptr;
     c->d_lut = c->d_lut_vr = nullptr;
     c->d_diag = c->d_vec = nullptr;
-    dfree(c->d_grm); dfree(c->d_grm_loco); dfree(c->d_diag_loco);
+    dfree(c->d_grm); dfree(c->d_s24); dfree(c->d_grm_loco);
+    c->s24_ok = false;
+    dfree(c->d_diag_loco);
     dfree(c->d_mv_in); dfree(c->d_mv_blk); dfree(c->d_mv_out); dfree(c->d_mv_ypart);
     dfree(c->d_dots_partial); dfree(c->d_dots_out);
     tri_plan_free(c->tri);
@@ -238,23 +240,50 @@ int engine_reserve(saige_ctx* c, Engine& e, int kpad, int nsys) {
 
 // The GRM a product uses: the full one (S/Mqc, diag) or the LOCO one
 // (S_loco/M_loco, diag_loco; getDiagOfSigma_LOCO ignores the diag-as-one
-// option, FG.cpp:2368-2392).  s16: S's values have at most 16 significant
-// bits (the split GRM and its LOCO ranges are stored so), and the block GEMM
-// may split them into two BF16 pieces; SAIGE_GEMM_S_PIECES=3 keeps three
-// (the same bits, more work).
+// option, FG.cpp:2368-2392).  The split GRM and its LOCO ranges have values of
+// at most 16 significant bits; SAIGE_GEMM_S_PIECES=3 has the block GEMM take
+// them as any others (the same bits, more work).
 struct GrmView {
-    const float* S;
+    GrmMat S;
     const float* diag;
     int64_t m;
     int diag_one;
-    bool s16;
 };
 
 GrmView grm_view(const saige_ctx* c, int loco) {
     const char* pieces = std::getenv("SAIGE_GEMM_S_PIECES");
     const bool s16 = c->grm_precision == SAIGE_GRM_BF16_SPLIT && !(pieces && std::atoi(pieces) == 3);
-    if (loco) return {c->loco_inplace ? c->d_grm : c->d_grm_loco, c->d_diag_loco, c->loco_m, 0, s16};
-    return {c->d_grm, c->d_diag, c->Mqc, c->diag_one, s16};
+    if (loco) return {{c->loco_inplace ? c->d_grm : c->d_grm_loco, s16, nullptr}, c->d_diag_loco, c->loco_m, 0};
+    return {{c->d_grm, s16, c->s24_ok ? c->d_s24 : nullptr}, c->d_diag, c->Mqc, c->diag_one};
+}
+
+// Makes the 24-bit triangle of a split GRM when its bytes leave room for
+// everything else a cohort of this size may take: a second GRM (leave one
+// chromosome out) and the products' scratch, a quarter of a GRM at most, and 8
+// GB.  Without it the products read the FP32 triangle.  Asynchronous on the
+// context's stream.
+hipError_t make_s24(saige_ctx* c) {
+    c->s24_ok = false;
+    if (c->grm_precision != SAIGE_GRM_BF16_SPLIT) {
+        dfree(c->d_s24);
+        return hipSuccess;
+    }
+    const int64_t bytes = s24_bytes(c->Npad), grm = 4 * c->Npad * c->Npad;
+    if (bytes == 0) return hipSuccess;
+    if (!c->d_s24) {
+        size_t free_b = 0, total_b = 0;
+        const hipError_t e = hipMemGetInfo(&free_b, &total_b);
+        if (e != hipSuccess) return e;
+        if ((int64_t)free_b < bytes + grm + grm / 4 + ((int64_t)8 << 30)) return hipSuccess;
+        if (dalloc(&c->d_s24, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            c->d_s24 = nullptr;
+            return hipSuccess;
+        }
+    }
+    const hipError_t e = launch_pack24(c->stream, c->d_grm, c->Npad, c->d_s24);
+    c->s24_ok = e == hipSuccess;
+    return e;
 }
 
 int check_loco(const saige_ctx* c) {
@@ -456,7 +485,7 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
                                                  : halves == 3 ? c->gemm_cfg
                                                                : c->gemm_cfg_half,
                                                  halves == 3 && !narrow),
-                                      halves, &c->tri, g.s16, narrow ? &nc : nullptr));
+                                      halves, &c->tri, narrow ? &nc : nullptr));
         SAIGE_HIP_TRY(hipEventRecord(c->ev1, st));
         SAIGE_HIP_TRY(launch_alpha(st, e.kpad, e.partial, np, e.rz, e.done, e.live, e.kind, e.alpha));
         int64_t np2 = 0;
@@ -1135,15 +1164,19 @@ int saige_build_grm(saige_ctx* c, int precision) {
     c->loco_inplace = false;
     if (precision != SAIGE_GRM_BF16_PANEL) {
         // 2-bit operands straight into the MFMA SYRK: no Z panel
-        const hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, 0, &c->grm_seconds);
+        hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, 0, &c->grm_seconds);
+        c->grm_precision = precision;
+        if (e == hipSuccess) e = make_s24(c);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess) {
             set_error("GRM build failed: %s", hipGetErrorString(e));
             return e == hipErrorOutOfMemory ? SAIGE_E_NOMEM : SAIGE_E_DEVICE;
         }
         c->grm_ready = true;
-        c->grm_precision = precision;
         return SAIGE_OK;
     }
+    c->s24_ok = false;
+    dfree(c->d_s24);
     const int64_t kc = syrk_kchunk_bf16();
     size_t free_b = 0, total_b = 0;
     SAIGE_HIP_TRY(hipMemGetInfo(&free_b, &total_b));
@@ -1292,7 +1325,7 @@ static int grm_matvec(saige_ctx* c, int loco, const float* B, int64_t k, float* 
             e = launch_grm_gemm(st, g.S, Np, N, d_blk, d_out, a, nullptr, nullptr, c->d_mv_ypart,
                                 shape_used(c, q ? c->gemm_cfg_quarter : kb <= 32 ? c->gemm_cfg_half : c->gemm_cfg,
                                            kb > 32),
-                                kb <= 32 ? 1 : 3, &c->tri, g.s16, q ? &q0 : nullptr);
+                                kb <= 32 ? 1 : 3, &c->tri, q ? &q0 : nullptr);
         if (e == hipSuccess) e = launch_gather_cols(st, d_out, kb, N, EW, d_in);
         if (e == hipSuccess) e = hipMemcpyAsync(Y + k0 * N, d_in, 4 * N * kb, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1517,6 +1550,8 @@ static int restore_full_grm(saige_ctx* c) {
                 return SAIGE_E_STATE;
             }
     hipError_t e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, 1);
+    // the sums may differ from the first build's in the last bit
+    if (e == hipSuccess) e = make_s24(c);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
         set_error("restoring the GRM after an in-place LOCO range failed: %s", hipGetErrorString(e));
@@ -1583,6 +1618,7 @@ int saige_set_start_end_index(saige_ctx* c, int64_t start, int64_t end, int chro
         e = hipMemcpyAsync(c->d_grm_loco, c->d_grm, sizeof(float) * Np * Np, hipMemcpyDeviceToDevice, st);
         if (e == hipSuccess) e = range_syrk(c, start, end, c->d_grm_loco, -1);
     } else {
+        c->s24_ok = false;           // made anew when S is whole again
         if (c->loco_inplace) e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, 1);
         c->loco_inplace = false;
         if (e == hipSuccess) e = range_syrk(c, start, end, c->d_grm, -1);
@@ -1907,16 +1943,16 @@ int saige_autotune(saige_ctx* c, int reps, double* ms_table) {
     a.mqc = (float)c->Mqc;
     a.mode = 0;
     // time one shape: one warm-up launch, then reps launches between events
-    const bool s16 = grm_view(c, 0).s16;
+    const GrmMat S = grm_view(c, 0).S;
     const NarrowCols q0 = NarrowCols::tile(16, 0);
     auto time_shape = [&](GemmConfig g, int halves, double* out_ms, bool q = false) -> hipError_t {
         const NarrowCols* quarter = q ? &q0 : nullptr;
-        hipError_t e = launch_grm_gemm(st, c->d_grm, Np, N, c->d_mv_blk, c->d_mv_out, a, nullptr, nullptr,
-                                       c->d_mv_ypart, g, halves, &c->tri, s16, quarter);
+        hipError_t e = launch_grm_gemm(st, S, Np, N, c->d_mv_blk, c->d_mv_out, a, nullptr, nullptr, c->d_mv_ypart,
+                                       g, halves, &c->tri, quarter);
         if (e == hipSuccess) e = hipEventRecord(c->ev0, st);
         for (int r = 0; r < reps && e == hipSuccess; r++)
-            e = launch_grm_gemm(st, c->d_grm, Np, N, c->d_mv_blk, c->d_mv_out, a, nullptr, nullptr, c->d_mv_ypart,
-                                g, halves, &c->tri, s16, quarter);
+            e = launch_grm_gemm(st, S, Np, N, c->d_mv_blk, c->d_mv_out, a, nullptr, nullptr, c->d_mv_ypart, g,
+                                halves, &c->tri, quarter);
         if (e == hipSuccess) e = hipEventRecord(c->ev1, st);
         if (e == hipSuccess) e = hipEventSynchronize(c->ev1);
         float ms = 0.f;

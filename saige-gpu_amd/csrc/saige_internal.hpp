@@ -281,6 +281,10 @@ struct saige_ctx {
     float* d_diag = nullptr;                     // [Npad] sum z^2
     // GRM S = Z Z^T, [Npad][Npad] FP32
     float* d_grm = nullptr;
+    // the split GRM's lower triangle in three bytes a value (launch_pack24), when
+    // there is room for it; s24_ok: it holds d_grm's present values
+    uint8_t* d_s24 = nullptr;
+    bool s24_ok = false;
     // LOCO (setStartEndIndex, FG.cpp:3067): S minus one range of GRM markers
     float* d_grm_loco = nullptr;                 // [Npad][Npad]
     float* d_diag_loco = nullptr;                // [Npad]
@@ -426,6 +430,18 @@ __device__ __forceinline__ float sigma_diag(float w, const float* diag, int64_t 
 }
 
 // ---- PCG kernels (pcg_kernels.hip)
+// the GRM a product reads
+struct GrmMat {
+    const float* S = nullptr;        // [Npad][Npad]
+    // every value of S has at most 16 significant bits (the split GRM's
+    // storage): the lower-triangle block product then splits S into two BF16
+    // pieces instead of three, with the same bits
+    bool s16 = false;
+    const uint8_t* s24 = nullptr;    // such an S's lower triangle in three bytes a value (launch_pack24), or null
+};
+int64_t s24_bytes(int64_t Npad);
+hipError_t launch_pack24(hipStream_t s, const float* S, int64_t Npad, uint8_t* out);
+
 // arguments of a single-column product's epilogue
 struct VecArgs {
     const float* winv = nullptr;     // [Npad], mode 1
@@ -451,12 +467,12 @@ struct SigmaArgs {
 // one double per part).  Returns the number of parts.
 // tri: read only the lower triangle (k_gemv_tri + k_gemv_tri_epi) with this
 // plan for Npad; nullptr: k_gemv over all of S.
-hipError_t launch_grm_gemv(hipStream_t s, const float* S, int64_t Npad, int64_t Nnm, const float* in,
+hipError_t launch_grm_gemv(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, const float* in,
                            float* out, VecArgs a, double* partial, int64_t* nparts,
                            const GemvPlan* tri = nullptr);
 // Sigma x = b by PCG for host vectors w, b and x; the iteration count in
 // *iters.  Waits for the stream.
-hipError_t solve1(hipStream_t s, Solve1& v, const float* w_host, const float* b_host, float* x_host, const float* S,
+hipError_t solve1(hipStream_t s, Solve1& v, const float* w_host, const float* b_host, float* x_host, GrmMat S,
                   const float* diag, int64_t Nnm, float tau0, float tau1, float m, int diag_one, int maxiter,
                   double tol, const GemvPlan* tri, int* iters);
 bool gemm_config_valid(GemmConfig g);
@@ -465,14 +481,11 @@ bool gemm_config_valid(GemmConfig g);
 // values for a half that is not computed are meaningless (the caller only
 // passes halves without live columns).
 // tri: the plan for Npad, required in mode GEMM_BF16X3_TRI (else unused).
-// s16: every value of S has at most 16 significant bits (the split GRM's
-// storage); the lower-triangle mode then splits S into two BF16 pieces
-// instead of three, with the same bits.
 // narrow (lower-triangle mode): only the 16 or 32 block columns it lists
 // are computed (halves is then unused); nullptr: the halves.
-hipError_t launch_grm_gemm(hipStream_t s, const float* S, int64_t Npad, int64_t Nnm, const float* in,
+hipError_t launch_grm_gemm(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, const float* in,
                            float* out, SigmaArgs a, double* partial, int64_t* nparts, float* ypart,
-                           GemmConfig g, int halves = 3, const TriPlan* tri = nullptr, bool s16 = false,
+                           GemmConfig g, int halves = 3, const TriPlan* tri = nullptr,
                            const NarrowCols* narrow = nullptr);
 int64_t gemm_ypart_floats(int64_t Npad);
 int64_t gemv_max_parts(int64_t Npad);

@@ -305,7 +305,7 @@ void Solve1::release() {
     launches = n;
 }
 
-hipError_t solve1(hipStream_t s, Solve1& v, const float* w_host, const float* b_host, float* x_host, const float* S,
+hipError_t solve1(hipStream_t s, Solve1& v, const float* w_host, const float* b_host, float* x_host, GrmMat S,
                   const float* diag, int64_t Nnm, float tau0, float tau1, float m, int diag_one, int maxiter,
                   double tol, const GemvPlan* tri, int* iters) {
     const int64_t Np = v.Npad;
@@ -361,7 +361,7 @@ hipError_t solve1(hipStream_t s, Solve1& v, const float* w_host, const float* b_
             npap = (int)(Np / (4 * rw));
             const size_t lds = sizeof(float) * (size_t)Np;
             auto go = [&](auto kernel) {
-                hipLaunchKernelGGL(kernel, dim3((unsigned)npap), dim3(256), lds, s, j, S, Np, Nnm, v.partial, nb, v.st,
+                hipLaunchKernelGGL(kernel, dim3((unsigned)npap), dim3(256), lds, s, j, S.S, Np, Nnm, v.partial, nb, v.st,
                                    h, maxiter, tol, v.z, pv, nx, a, v.ap, v.pap, v.x, v.hvec + 2 * Np);
             };
             if (rw == 1) go(k_p1_row<1>);
