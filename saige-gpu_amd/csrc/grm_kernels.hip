@@ -49,44 +49,50 @@ __device__ __forceinline__ float round16(float x) {
 }
 
 // Store a wave's block of 32*MI rows from row0 and 32*NI columns from col0,
-// mirrored for off-diagonal tiles; accumulate: +1 add to S, -1 subtract from
-// S, 0 store.  center: the column's value taken off each sum first (nullptr:
-// none).  R16: the stored values (after the add or subtract) rounded by
-// round16.  Accumulator layout of a 32x32 MFMA block: lane l, register r
-// holds row 8*(r/4) + 4*(l/32) + (r%4), column l%32.
+// mirrored for off-diagonal tiles; accumulate: +1 S = S0 + block, -1 S = S0 -
+// block (LOCO: one chromosome's markers left out), 0 store.  S0 may be S.
+// center: the column's value taken off each sum first (nullptr: none).  R16:
+// the stored values (after the add or subtract) rounded by round16.
+// Accumulator layout of a 32x32 MFMA block: lane l, register r holds row
+// 8*(r/4) + 4*(l/32) + (r%4), column l%32.  A block's S0 values are requested
+// before the block ahead of it is stored (no entry that is read is stored by
+// another lane).  With few markers the store is a third of the launch and bound
+// by its bytes (S0's triangle read, S written): 1000 of 20,000 markers left out
+// at N = 20,000 take 1.54 ms; a copy of S first and requests at their use took
+// 2.7.
 template <int MI, int NI, bool R16>
-__device__ __forceinline__ void store_block(float* S, int64_t ldS, int64_t row0, int64_t col0, bool mirror, int lane,
-                                            const f32x16 (&acc)[MI][NI], int accumulate,
+__device__ __forceinline__ void store_block(float* S, const float* S0, int64_t ldS, int64_t row0, int64_t col0,
+                                            bool mirror, int lane, const f32x16 (&acc)[MI][NI], int accumulate,
                                             const float* center = nullptr) {
+    float s0[2][16];
+    auto request = [&](int k) {
+        const float* p = S0 + (row0 + k / NI * 32 + 4 * (lane >> 5)) * ldS + col0 + k % NI * 32 + (lane & 31);
 #pragma unroll
-    for (int mi = 0; mi < MI; mi++) {
+        for (int r = 0; r < 16; r++) s0[k & 1][r] = p[(8 * (r >> 2) + (r & 3)) * ldS];
+    };
+    if (accumulate) request(0);
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++) {
-            const int64_t col = col0 + ni * 32 + (lane & 31);
-            const float cc = center ? center[col] : 0.0f;
+    for (int k = 0; k < MI * NI; k++) {
+        const int mi = k / NI, ni = k % NI;
+        const int64_t col = col0 + ni * 32 + (lane & 31);
+        const float cc = center ? center[col] : 0.0f;
+        if (accumulate && k + 1 < MI * NI) request(k + 1);
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int64_t row = row0 + mi * 32 + 8 * g + 4 * (lane >> 5);
-                float v[4];
+        for (int g = 0; g < 4; g++) {
+            const int64_t row = row0 + mi * 32 + 8 * g + 4 * (lane >> 5);
+            float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = center ? acc[mi][ni][4 * g + e] - cc : acc[mi][ni][4 * g + e];
-                if (accumulate > 0) {        // S += tile
+            for (int e = 0; e < 4; e++) {
+                v[e] = center ? acc[mi][ni][4 * g + e] - cc : acc[mi][ni][4 * g + e];
+                if (accumulate > 0) v[e] = s0[k & 1][4 * g + e] + v[e];
+                else if (accumulate < 0) v[e] = s0[k & 1][4 * g + e] - v[e];
+                if (R16) v[e] = round16(v[e]);
+            }
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = S[(row + e) * ldS + col] + v[e];
-                } else if (accumulate < 0) { // S -= tile (LOCO: remove one chromosome's markers)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = S[(row + e) * ldS + col] - v[e];
-                }
-                if (R16) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = round16(v[e]);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; e++) S[(row + e) * ldS + col] = v[e];
-                if (mirror) {
-                    float4* dst = reinterpret_cast<float4*>(S + col * ldS + row);
-                    *dst = make_float4(v[0], v[1], v[2], v[3]);
-                }
+            for (int e = 0; e < 4; e++) S[(row + e) * ldS + col] = v[e];
+            if (mirror) {
+                float4* dst = reinterpret_cast<float4*>(S + col * ldS + row);
+                *dst = make_float4(v[0], v[1], v[2], v[3]);
             }
         }
     }
@@ -98,7 +104,7 @@ constexpr int P16 = BK16 + 8;       // LDS row pitch (bf16 elements): 144 B, con
 
 __global__ __launch_bounds__(256) void k_syrk_bf16(const __hip_bfloat16* __restrict__ Zp, int64_t ldz,
                                                    int64_t kdim, const int2* __restrict__ tiles, int64_t nblk,
-                                                   float* __restrict__ S, int64_t ldS, int accumulate) {
+                                                   float* S, int64_t ldS, int accumulate) {
     __shared__ __attribute__((aligned(16))) __hip_bfloat16 sA[BT * P16];
     __shared__ __attribute__((aligned(16))) __hip_bfloat16 sB[BT * P16];
     const int2 t = tiles[xcd_remap(blockIdx.x, nblk)];
@@ -160,7 +166,7 @@ __global__ __launch_bounds__(256) void k_syrk_bf16(const __hip_bfloat16* __restr
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[mi], fb[ni], acc[mi][ni], 0, 0, 0);
         }
     }
-    store_block<2, 2, false>(S, ldS, bi * BT + wr * 64, bj * BT + wc * 64, bi != bj, lane, acc, accumulate);
+    store_block<2, 2, false>(S, S, ldS, bi * BT + wr * 64, bj * BT + wc * 64, bi != bj, lane, acc, accumulate);
 }
 
 // ------------------------------------------------------- BF16, 2-bit in
@@ -227,7 +233,7 @@ __device__ __forceinline__ void split_bytes(const uint64_t (&t)[8], uint32_t (&l
 __global__ __launch_bounds__(512) void k_syrk_pk256(const uint8_t* __restrict__ tp, int64_t nchunk, int64_t c0,
                                                     int64_t c1, const uint64_t* __restrict__ lut64,
                                                     const int2* __restrict__ tiles, int64_t nblk,
-                                                    float* __restrict__ S, int64_t ldS, int accumulate) {
+                                                    float* S, const float* S0, int64_t ldS, int accumulate) {
     __shared__ __attribute__((aligned(16))) __hip_bfloat16 sA0[BT2 * P16];
     __shared__ __attribute__((aligned(16))) __hip_bfloat16 sB0[BT2 * P16];
     __shared__ __attribute__((aligned(16))) __hip_bfloat16 sA1[BT2 * P16];
@@ -311,7 +317,7 @@ __global__ __launch_bounds__(512) void k_syrk_pk256(const uint8_t* __restrict__ 
         step(sA1, sB1, sA0, sB0, kc + 1);
     }
     if (kc < c1) multiply(sA0, sB0);
-    store_block<2, 4, false>(S, ldS, bi * BT2 + wr * 64, bj * BT2 + wc * 128, bi != bj, lane, acc, accumulate);
+    store_block<2, 4, false>(S, S0, ldS, bi * BT2 + wr * 64, bj * BT2 + wc * 128, bi != bj, lane, acc, accumulate);
 }
 
 // k_syrk_pk<T, F>: the GRM from 2-bit genotypes on T x T tiles, by operand
@@ -348,7 +354,7 @@ template <int T, int F>
 __global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t* __restrict__ tp, int64_t nchunk,
                                                                   int64_t k0, int64_t k1, SyrkTables tb,
                                                                   const int2* __restrict__ tiles, int64_t nblk,
-                                                                  float* __restrict__ S, int64_t ldS,
+                                                                  float* S, const float* S0, int64_t ldS,
                                                                   int accumulate) {
     constexpr int BK = T == 64 ? 64 : 32;            // markers per chunk
     constexpr int P = BK + 8;                        // LDS row pitch (bf16 elements), conflict-free 16-byte reads
@@ -478,7 +484,7 @@ __global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t*
         step(s1, s0, kc + 1);
     }
     if (kc < k1) multiply(s0);
-    store_block<MI, NI, F == SYRK_SPLIT>(S, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane, acc,
+    store_block<MI, NI, F == SYRK_SPLIT>(S, S0, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane, acc,
                                          accumulate, F == SYRK_FP32 ? tb.center : nullptr);
 }
 
@@ -728,31 +734,32 @@ void SyrkOperands::release() {
 }
 
 template <int T, int F>
-static void launch_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, int accumulate) {
+static void launch_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, const float* S0,
+                      int accumulate) {
     constexpr int BK = T == 64 ? 64 : 32;
     const int64_t nt = op.Npad / T, nblk = nt * (nt + 1) / 2;
     hipLaunchKernelGGL((k_syrk_pk<T, F>), dim3((unsigned)nblk), dim3(T == 256 ? 512 : 256), 0, s, op.tp, op.nchunk,
-                       (int64_t)0, op.nchunk * (64 / BK), op.tb, tiles, nblk, S, op.Npad, accumulate);
+                       (int64_t)0, op.nchunk * (64 / BK), op.tb, tiles, nblk, S, S0, op.Npad, accumulate);
 }
 
-hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, int accumulate,
-                          int tile) {
+hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, const float* S0,
+                          int accumulate, int tile) {
     if ((tile != 64 && tile != BT && tile != BT2) || op.Npad % tile != 0 || !op.block) return hipErrorInvalidValue;
     if (op.form == SYRK_HI && tile == BT2) {
         const int64_t nt = op.Npad / BT2, nblk = nt * (nt + 1) / 2;
         hipLaunchKernelGGL(k_syrk_pk256, dim3((unsigned)nblk), dim3(512), 0, s, op.tp, op.nchunk, (int64_t)0, op.nchunk,
-                           op.tb.t[0], tiles, nblk, S, op.Npad, accumulate);
+                           op.tb.t[0], tiles, nblk, S, S0, op.Npad, accumulate);
     } else if (op.form == SYRK_HI) {
-        if (tile == BT) launch_pk<128, SYRK_HI>(s, op, tiles, S, accumulate);
-        else launch_pk<64, SYRK_HI>(s, op, tiles, S, accumulate);
+        if (tile == BT) launch_pk<128, SYRK_HI>(s, op, tiles, S, S0, accumulate);
+        else launch_pk<64, SYRK_HI>(s, op, tiles, S, S0, accumulate);
     } else if (op.form == SYRK_SPLIT) {
-        if (tile == BT2) launch_pk<256, SYRK_SPLIT>(s, op, tiles, S, accumulate);
-        else if (tile == BT) launch_pk<128, SYRK_SPLIT>(s, op, tiles, S, accumulate);
-        else launch_pk<64, SYRK_SPLIT>(s, op, tiles, S, accumulate);
+        if (tile == BT2) launch_pk<256, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate);
+        else if (tile == BT) launch_pk<128, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate);
+        else launch_pk<64, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate);
     } else {
-        if (tile == BT2) launch_pk<256, SYRK_FP32>(s, op, tiles, S, accumulate);
-        else if (tile == BT) launch_pk<128, SYRK_FP32>(s, op, tiles, S, accumulate);
-        else launch_pk<64, SYRK_FP32>(s, op, tiles, S, accumulate);
+        if (tile == BT2) launch_pk<256, SYRK_FP32>(s, op, tiles, S, S0, accumulate);
+        else if (tile == BT) launch_pk<128, SYRK_FP32>(s, op, tiles, S, S0, accumulate);
+        else launch_pk<64, SYRK_FP32>(s, op, tiles, S, S0, accumulate);
     }
     hipError_t e = hipGetLastError();
     // the multi-piece forms reach a diagonal tile's two mirror entries by

@@ -1107,10 +1107,12 @@ int saige_get_diag_of_kin(saige_ctx* c, float* out) {
 }
 
 namespace {
-// S (= / += / -=) the GRM part of markers [j0, j1) from the 2-bit genotypes, in
-// the operand form of `precision` (accumulate: 0, 1, -1).  Waits for the
-// stream; t (may be null): device seconds between its start and end.
-hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1, float* S, int accumulate, double* t) {
+// S = (nothing, S0 plus, S0 minus) the GRM part of markers [j0, j1) from the
+// 2-bit genotypes, in the operand form of `precision` (accumulate: 0, 1, -1; S0
+// may be S).  Waits for the stream; t (may be null): device seconds between its
+// start and end.
+hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1, float* S, const float* S0,
+                            int accumulate, double* t) {
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad;
     const int form = precision == SAIGE_GRM_FP32 ? SYRK_FP32 : (precision == SAIGE_GRM_BF16_SPLIT ? SYRK_SPLIT : SYRK_HI);
@@ -1124,7 +1126,7 @@ hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1,
         e = hipMemcpyAsync(d_tiles, order.data(), sizeof(int2) * order.size(), hipMemcpyHostToDevice, st);
     if (e == hipSuccess && t) e = hipEventRecord(c->ev0, st);
     if (e == hipSuccess) e = op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j0, j1);
-    if (e == hipSuccess) e = launch_syrk_pk(st, op, d_tiles, S, accumulate, tile);
+    if (e == hipSuccess) e = launch_syrk_pk(st, op, d_tiles, S, S0, accumulate, tile);
     if (e == hipSuccess && t) e = hipEventRecord(c->ev1, st);
     const hipError_t w = hipStreamSynchronize(st);
     if (e == hipSuccess) e = w;
@@ -1164,7 +1166,7 @@ int saige_build_grm(saige_ctx* c, int precision) {
     c->loco_inplace = false;
     if (precision != SAIGE_GRM_BF16_PANEL) {
         // 2-bit operands straight into the MFMA SYRK: no Z panel
-        hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, 0, &c->grm_seconds);
+        hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, nullptr, 0, &c->grm_seconds);
         c->grm_precision = precision;
         if (e == hipSuccess) e = make_s24(c);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1503,14 +1505,18 @@ int saige_pcg_block(saige_ctx* c, const float* w, const float* tau, const float*
 // ---------------------------------------------------------------- LOCO
 
 namespace {
-// S (+/-)= Z_r Z_r^T over GRM markers [start, end], with the kernel and
+// S = S0 (+/-) Z_r Z_r^T over GRM markers [start, end], with the kernel and
 // operand precision the resident S was built with (accumulate: 1 add, -1
-// subtract).
-hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, int accumulate) {
+// subtract; S0 may be S).
+hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, const float* S0, int accumulate) {
     if (c->grm_precision != SAIGE_GRM_BF16_PANEL)
-        return syrk_from_packed(c, c->grm_precision, start, end + 1, S, accumulate, nullptr);
+        return syrk_from_packed(c, c->grm_precision, start, end + 1, S, S0, accumulate, nullptr);
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
+    if (S != S0) {                   // the panels add to S one after another
+        const hipError_t ce = hipMemcpyAsync(S, S0, sizeof(float) * Np * Np, hipMemcpyDeviceToDevice, st);
+        if (ce != hipSuccess) return ce;
+    }
     const int64_t cnt = end - start + 1;
     const std::vector<int2> order = syrk_tile_order(Np / syrk_tile(), 8);
     int2* d_tiles = nullptr;
@@ -1549,7 +1555,7 @@ static int restore_full_grm(saige_ctx* c) {
                 set_error("live LOCO slots use the in-place LOCO GRM; take them before using the full GRM");
                 return SAIGE_E_STATE;
             }
-    hipError_t e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, 1);
+    hipError_t e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, c->d_grm, 1);
     // the sums may differ from the first build's in the last bit
     if (e == hipSuccess) e = make_s24(c);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -1615,13 +1621,12 @@ int saige_set_start_end_index(saige_ctx* c, int64_t start, int64_t end, int chro
             }
         }
         // S_loco = S - Z_r Z_r^T with the kernel and operand precision S was built with
-        e = hipMemcpyAsync(c->d_grm_loco, c->d_grm, sizeof(float) * Np * Np, hipMemcpyDeviceToDevice, st);
-        if (e == hipSuccess) e = range_syrk(c, start, end, c->d_grm_loco, -1);
+        e = range_syrk(c, start, end, c->d_grm_loco, c->d_grm, -1);
     } else {
         c->s24_ok = false;           // made anew when S is whole again
-        if (c->loco_inplace) e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, 1);
+        if (c->loco_inplace) e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, c->d_grm, 1);
         c->loco_inplace = false;
-        if (e == hipSuccess) e = range_syrk(c, start, end, c->d_grm, -1);
+        if (e == hipSuccess) e = range_syrk(c, start, end, c->d_grm, c->d_grm, -1);
         if (e == hipSuccess) c->loco_inplace = true;
     }
     // diag_loco = diag - sum over the range of z^2, the range summed from zero in

@@ -398,10 +398,11 @@ hipError_t launch_syrk_bf16(hipStream_t s, const __hip_bfloat16* Zp, int64_t Npa
                             int64_t kdim, const int2* tiles, float* S, int accumulate);
 std::vector<int2> syrk_tile_order(int64_t nt, int64_t g);
 // the 2-bit-input SYRK of op on T x T tiles (64, 128 or 256; tiles from
-// syrk_tile_order(Npad / tile, ...)); accumulate: 0 overwrite, 1 add, -1
-// subtract.  S comes out exactly symmetric.
-hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, int accumulate,
-                          int tile);
+// syrk_tile_order(Npad / tile, ...)); accumulate: 0 overwrite, 1 S = S0 + the
+// product, -1 S = S0 - the product (S0 may be S).  S comes out exactly
+// symmetric.
+hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, const float* S0,
+                          int accumulate, int tile);
 int syrk_pk_tile(int64_t Npad);
 // copy each diagonal tile's lower half onto its upper half (tile edge `tile`)
 hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile);
