@@ -356,10 +356,11 @@ int saige_get_gemm_config_quarter(const saige_ctx* ctx, int* rt, int* pd, double
  * on the split GRM, whose values need two pieces), on the 16x16x32 MFMA,
  * read from the lower triangle of the GRM only (half the bytes): each 32x32
  * block left of the diagonal gives both S_IJ P_J and S_IJ^T P_I.  A launch
- * covers 64, 32 or 16 columns, as few as hold live slots (at most 16 or 32
- * occupied slots run as one 16- or 32-column launch wherever they sit), with
- * the same per-column arithmetic (SAIGE_LAUNCH_GEMM_QUARTER counts the
- * 16-column ones, SAIGE_LAUNCH_GEMM_HALF the 32-column ones).  rt selects
+ * covers 64, 48, 32 or 16 columns, as few as hold live slots (at most 16, 32
+ * or 48 occupied slots run as one launch of that width wherever they sit),
+ * with the same per-column arithmetic (SAIGE_LAUNCH_GEMM_QUARTER counts the
+ * 16-column ones, SAIGE_LAUNCH_GEMM_HALF the 32-column ones,
+ * SAIGE_LAUNCH_GEMM_FULL the wider ones).  rt selects
  * the workgroup (1: twelve waves, 2: eight), pd 1 or 3 the prefetch depth
  * (one or two chunks ahead); nsplit is unused.  It needs device scratch for
  * its partial products, about 128 N^2 / (32 * waves) bytes (3.3 GB at
@@ -392,7 +393,8 @@ int64_t saige_engine_system_bytes(const saige_ctx* ctx);
 #define SAIGE_LAUNCH_GEMV 0       /* width-1 engine (saige_pcg1): k_gemv          */
 #define SAIGE_LAUNCH_GEMM_HALF 1  /* block GEMM over 32 columns: one half, or (lower
                                      triangle) at most 32 occupied slots anywhere */
-#define SAIGE_LAUNCH_GEMM_FULL 2  /* block GEMM over all 64 columns                */
+#define SAIGE_LAUNCH_GEMM_FULL 2  /* block GEMM over all 64 columns, or (lower
+                                     triangle) 48 of them                        */
 #define SAIGE_LAUNCH_GEMM_QUARTER 3 /* lower-triangle block GEMM over 16 columns
                                      (at most 16 occupied slots, anywhere)       */
 int saige_engine_stats(const saige_ctx* ctx, int kind, double* gemm_seconds, int64_t* gemm_launches);

@@ -836,8 +836,8 @@ __global__ __launch_bounds__(768) void k_gemm_x3w(const float* __restrict__ S, i
 // ------------------------------------------------- lower-triangle product
 // k_gemm_t16<NWV, PD, NQ, SP>: the three-piece product read from the lower
 // triangle of S only (half the bytes), on the 16x16x32 BF16 MFMA, over NQ
-// tiles of 16 right-hand sides: NQ = 4 for all 64 columns, 2 for 32 and 1
-// for 16 block columns that a map names.  S is symmetric, so a 32x32 block S_IJ left
+// tiles of 16 right-hand sides: NQ = 4 for all 64 columns, 3, 2 and 1 for the
+// 48, 32 or 16 block columns that a map names.  S is symmetric, so a 32x32 block S_IJ left
 // of the diagonal serves two products:
 //   use 1: Y_I += S_IJ P_J
 //   use 2: Y_J += S_IJ^T P_I
@@ -874,10 +874,9 @@ __global__ __launch_bounds__(768) void k_gemm_x3w(const float* __restrict__ S, i
 // row-set order: a fixed order, so results are reproducible, and a column's
 // arithmetic is the same whatever NQ, so a launch can be as narrow as its
 // live columns (a 16-column launch does a quarter of a full one's MFMA work)
-// and a column's bits still do not depend on its co-tenants.  A 16- or
-// 32-column launch takes any 16 or 32 block columns (a map of launch column
-// -> block column), so at most 16 or 32 live columns anywhere in the block
-// run in one.  The arithmetic of an output column depends only on its own
+// and a column's bits still do not depend on its co-tenants.  A narrow launch
+// takes any 16, 32 or 48 block columns (a map of launch column -> block column),
+// so that many live columns anywhere in the block run in one.  The arithmetic of an output column depends only on its own
 // column of P, in whatever position of the MFMA operands it sits.
 // Eight waves have registers for a software-pipelined loop: chunk c's pieces
 // are split during chunk c-1, beside that chunk's MFMAs.  Twelve waves split
@@ -951,15 +950,14 @@ __device__ __forceinline__ void t16_transpose(const u32x4 (&a)[2], const u32x4 (
     }
 }
 
-// block column of launch column k (< 32) of a narrow launch: byte k of the
+// block column of launch column k (< 48) of a narrow launch: byte k of the
 // map, picked with selects (no indexing into the kernel argument)
-__device__ __forceinline__ int map_col(const ColMap32& m, int k) {
-    const uint32_t lo = (k & 8) ? ((k & 4) ? m.w[3] : m.w[2]) : ((k & 4) ? m.w[1] : m.w[0]);
-    const uint32_t hi = (k & 8) ? ((k & 4) ? m.w[7] : m.w[6]) : ((k & 4) ? m.w[5] : m.w[4]);
-    return (int)((((k & 16) ? hi : lo) >> (8 * (k & 3))) & 0xFFu);
+__device__ __forceinline__ int map_col(const ColMap& m, int k) {
+    auto word = [&](int o) { return (k & 8) ? ((k & 4) ? m.w[o + 3] : m.w[o + 2]) : ((k & 4) ? m.w[o + 1] : m.w[o]); };
+    return (int)(((k & 32 ? word(8) : k & 16 ? word(4) : word(0)) >> (8 * (k & 3))) & 0xFFu);
 }
 
-// cm: the block columns of a 16- or 32-column launch (NQ 1 or 2), which
+// cm: the block columns of a 16-, 32- or 48-column launch (NQ 1 to 3), which
 // holds its P pieces, partials and LDS tiles at launch columns [0, 16*NQ)
 // C24 (SP = 2): chunks left of the diagonal come from the 24-bit triangle, whose
 // upper halves are the first piece as they stand; the diagonal squares are read
@@ -972,7 +970,7 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
                                                        int64_t ld,
                                                        const u32x4* __restrict__ pb, const float* __restrict__ P,
                                                        const int4* __restrict__ items, float* __restrict__ y1p,
-                                                       float* __restrict__ y2p, ColMap32 cm) {
+                                                       float* __restrict__ y2p, ColMap cm) {
     constexpr int GM = 32 * NWV;
     constexpr bool PIPE = NWV == 8;                  // software-pipelined chunk loop (register room)
     constexpr int RING = PD + 1;                     // raw chunks held
@@ -1075,15 +1073,16 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
             }
         }
         // the sum over the waves of chunk cc's use-2 tiles (32 columns x
-        // 16*NQ rhs, NQ values per lane of waves [0, 8)), stored as its
+        // 16*NQ rhs, V values per lane of waves [0, NR2)), stored as its
         // partial for this row set
         auto reduce = [&](int64_t cc, const float* sr) {
-            if (wv < 8) {
-                const int o = (wv * 64 + lane) * NQ;
+            constexpr int V = NQ >= 3 ? 4 : NQ, NR2 = 8 * NQ / V;
+            if (wv < NR2) {
+                const int o = (wv * 64 + lane) * V;
                 const int j = o / (16 * NQ), ql = o % (16 * NQ);
                 const float* src = sr + tri_sr_index(j, ql);
                 float* dst = y2p + (tri_y2_first<NWV>(cc, NR) + (R - cc / NWV - 1)) * (32 * YS) + j * YS + ql;
-                if constexpr (NQ == 4) {
+                if constexpr (V == 4) {
                     float4 sum = *reinterpret_cast<const float4*>(src);
 #pragma unroll
                     for (int w = 1; w < NWV; w++) {
@@ -1094,7 +1093,7 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
                         sum.w += v.w;
                     }
                     *reinterpret_cast<float4*>(dst) = sum;
-                } else if constexpr (NQ == 2) {
+                } else if constexpr (V == 2) {
                     float2 sum = *reinterpret_cast<const float2*>(src);
 #pragma unroll
                     for (int w = 1; w < NWV; w++) {
@@ -1249,16 +1248,18 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
 
 // k_tri_reduce: Y[row][q] = the row set's use-1 partials (rtab[R] = {first
 // slot, count}) in slot order, then the chunk's use-2 partials in row-set
-// order; float4 per thread, QW threads per row (16: all 64 columns; 8 and 4:
-// the 32 or 16 columns of a narrow launch, stored to the block columns of
-// cm).  The partials hold the launch's 4 * QW columns only (row stride
+// order; float4 per thread, QW threads per row (16: all 64 columns; 12, 8 and
+// 4: the 48, 32 or 16 columns of a narrow launch, stored to the block columns
+// of cm), whole rows per workgroup.  The partials hold the launch's 4 * QW columns only (row stride
 // 4 * QW).
+constexpr int tri_reduce_threads(int QW) { return QW == 12 ? 192 : 256; }
+
 template <int NWV, int QW>
-__global__ __launch_bounds__(256) void k_tri_reduce(const float* __restrict__ y1p, const float* __restrict__ y2p,
-                                                    const int2* __restrict__ rtab, int64_t ld, ColMap32 cm,
+__global__ __launch_bounds__(tri_reduce_threads(QW)) void k_tri_reduce(const float* __restrict__ y1p, const float* __restrict__ y2p,
+                                                    const int2* __restrict__ rtab, int64_t ld, ColMap cm,
                                                     float* __restrict__ y) {
     constexpr int GM = 32 * NWV, YS = 4 * QW;
-    const int64_t row = (int64_t)blockIdx.x * (256 / QW) + threadIdx.x / QW;
+    const int64_t row = (int64_t)blockIdx.x * (tri_reduce_threads(QW) / QW) + threadIdx.x / QW;
     const int q = 4 * (threadIdx.x % QW);               // the launch's column
     const int64_t nch = ld / 32, NR = (nch + NWV - 1) / NWV;
     const int64_t c = row / 32, R = c / NWV;
@@ -1969,18 +1970,19 @@ hipError_t tri_plan_build(TriPlan& t, int64_t Npad, int nwv, int ch) {
 namespace {
 template <int NWV, int PD, int NQ, int SP>
 void launch_t16(hipStream_t s, dim3 grid, GrmMat m, int64_t Npad, const u32x4* pb, const float* in,
-                const TriPlan& t, ColMap32 cm, float* ypart) {
+                const TriPlan& t, ColMap cm, float* ypart) {
     if (SP == 2 && m.s24)
         hipLaunchKernelGGL((k_gemm_t16<NWV, PD, NQ, 2, true>), grid, dim3(64 * NWV), 0, s, m.S, m.s24, Npad, pb, in,
                            t.items, t.y1p, t.y2p, cm);
     else
         hipLaunchKernelGGL((k_gemm_t16<NWV, PD, NQ, SP, false>), grid, dim3(64 * NWV), 0, s, m.S, m.s24, Npad, pb, in,
                            t.items, t.y1p, t.y2p, cm);
-    hipLaunchKernelGGL((k_tri_reduce<NWV, 4 * NQ>), dim3((unsigned)(Npad * 4 * NQ / 256)), dim3(256), 0, s, t.y1p,
-                       t.y2p, t.rtab, Npad, cm, ypart);
+    constexpr int QW = 4 * NQ, NT = tri_reduce_threads(QW);     // Npad is a multiple of NT / QW
+    hipLaunchKernelGGL((k_tri_reduce<NWV, QW>), dim3((unsigned)(Npad / (NT / QW))), dim3(NT), 0, s, t.y1p, t.y2p,
+                       t.rtab, Npad, cm, ypart);
 }
 
-// the lower-triangle product over the launch's 64 columns, or the 16 or 32
+// the lower-triangle product over the launch's 64 columns, or the 16, 32 or 48
 // block columns narrow lists (nullptr and halves 1 or 2: the half's 32)
 template <int NWV, int SP>
 hipError_t launch_tri(hipStream_t s, GrmMat m, int64_t Npad, const float* in, float* ypart, int pd,
@@ -1992,12 +1994,15 @@ hipError_t launch_tri(hipStream_t s, GrmMat m, int64_t Npad, const float* in, fl
     const bool deep = pd == 3;
     const NarrowCols half = NarrowCols::tile(32, halves == 2 ? 32 : 0);
     if (!narrow && halves != 3) narrow = &half;
-    ColMap32 cm{};
+    ColMap cm{};
     if (narrow)
         for (int k = 0; k < narrow->width; k++) cm.w[k / 4] |= (uint32_t)narrow->col[k] << (8 * (k % 4));
     if (narrow && narrow->width == 16) {
         if (deep) launch_t16<NWV, 2, 1, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
         else launch_t16<NWV, 1, 1, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
+    } else if (narrow && narrow->width == 48) {
+        if (deep) launch_t16<NWV, 2, 3, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
+        else launch_t16<NWV, 1, 3, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
     } else if (narrow) {
         if (deep) launch_t16<NWV, 2, 2, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
         else launch_t16<NWV, 1, 2, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
@@ -2021,8 +2026,8 @@ hipError_t launch_grm_gemm(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, c
         if (!tri || tri->Npad != Npad || !tri->items) return hipErrorInvalidValue;
         hipError_t e;
         if (narrow) {
-            // 16 or 32 distinct block columns
-            if (narrow->width != 16 && narrow->width != 32) return hipErrorInvalidValue;
+            // 16, 32 or 48 distinct block columns
+            if (narrow->width != 16 && narrow->width != 32 && narrow->width != 48) return hipErrorInvalidValue;
             uint64_t seen = 0;
             for (int k = 0; k < narrow->width; k++) {
                 const int col = narrow->col[k];

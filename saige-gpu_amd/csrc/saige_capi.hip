@@ -457,13 +457,15 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
             nlive++;
         }
     if (halves == 0) halves = 1;
-    // the lower-triangle product runs at most 16 (32) occupied slots,
-    // wherever they sit, as one 16- (32-) column launch: the occupied slots
-    // in order, then free ones (computed, not used)
+    // the lower-triangle product runs at most 16 (32, 48) occupied slots,
+    // wherever they sit, as one 16- (32-, 48-) column launch: the occupied
+    // slots in order, then free ones (computed, not used).  16, 32, 48 and 64
+    // columns of random operands take 0.89, 1.05, 1.37 and 1.69 ms at N = 50,000,
+    // 3.45, 4.9, 6.5 and 7.6 at 100,000.
     NarrowCols nc;
     bool narrow = false;
-    if (e.kpad == EW && c->gemm_cfg.mode == GEMM_BF16X3_TRI && nlive > 0 && nlive <= 32) {
-        nc.width = nlive <= 16 ? 16 : 32;
+    if (e.kpad == EW && c->gemm_cfg.mode == GEMM_BF16X3_TRI && nlive > 0 && nlive <= 48) {
+        nc.width = (nlive + 15) / 16 * 16;
         int n = 0;
         for (int k = 0; k < e.kpad; k++)
             if (e.h_live[k]) nc.col[n++] = (uint8_t)k;
@@ -472,7 +474,7 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
         narrow = true;
     }
     const bool quarter = narrow && nc.width == 16;
-    if (narrow && !quarter) halves = 1;   // for the shape and the statistics below
+    if (narrow) halves = nc.width == 48 ? 3 : 1;   // for the shape and the statistics below
     for (int it = 0; it < n_iter; it++) {
         bool any = false;
         for (int k = 0; k < e.kpad; k++) any |= (e.h_live[k] && !e.h_done[k]);
@@ -484,7 +486,7 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
                                                  quarter       ? c->gemm_cfg_quarter
                                                  : halves == 3 ? c->gemm_cfg
                                                                : c->gemm_cfg_half,
-                                                 halves == 3 && !narrow),
+                                                 halves == 3),
                                       halves, &c->tri, narrow ? &nc : nullptr));
         SAIGE_HIP_TRY(hipEventRecord(c->ev1, st));
         SAIGE_HIP_TRY(launch_alpha(st, e.kpad, e.partial, np, e.rz, e.done, e.live, e.kind, e.alpha));
@@ -1319,15 +1321,17 @@ static int grm_matvec(saige_ctx* c, int loco, const float* B, int64_t k, float* 
         const int kb = (int)std::min<int64_t>(EW, k - k0);
         e = hipMemcpyAsync(d_in, B + k0 * N, 4 * N * kb, hipMemcpyHostToDevice, st);
         if (e == hipSuccess) e = launch_scatter_cols(st, d_in, kb, N, Np, EW, d_blk);
-        // the lower-triangle product runs as narrow as the block: 16, 32 or
-        // 64 columns
-        const bool q = kb <= 16 && c->gemm_cfg.mode == GEMM_BF16X3_TRI;
-        const NarrowCols q0 = NarrowCols::tile(16, 0);
+        // the lower-triangle product runs as narrow as the block: 16, 32, 48
+        // or 64 columns
+        const bool tri = c->gemm_cfg.mode == GEMM_BF16X3_TRI;
+        const bool q = kb <= 16 && tri;
+        const bool narrow = tri && (q || (kb > 32 && kb <= 48));
+        const NarrowCols nc = NarrowCols::tile(q ? 16 : 48, 0);
         if (e == hipSuccess)
             e = launch_grm_gemm(st, g.S, Np, N, d_blk, d_out, a, nullptr, nullptr, c->d_mv_ypart,
                                 shape_used(c, q ? c->gemm_cfg_quarter : kb <= 32 ? c->gemm_cfg_half : c->gemm_cfg,
                                            kb > 32),
-                                kb <= 32 ? 1 : 3, &c->tri, q ? &q0 : nullptr);
+                                kb <= 32 ? 1 : 3, &c->tri, narrow ? &nc : nullptr);
         if (e == hipSuccess) e = launch_gather_cols(st, d_out, kb, N, EW, d_in);
         if (e == hipSuccess) e = hipMemcpyAsync(Y + k0 * N, d_in, 4 * N * kb, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);

@@ -66,12 +66,12 @@ enum GemmMode { GEMM_FP32 = 0, GEMM_BF16X3 = 1, GEMM_BF16X3_TRI = 2 };
 // one Npad.  Row set R = rows 32*nwv*R + [0, 32*nwv); item = (R, chunk range
 // [ca, cb) of 32 columns, use-1 slot); row set R's use-1 partials are the
 // slots rtab[R].x + [0, rtab[R].y).
-// the block columns of a 16- or 32-column launch of the lower-triangle
+// the block columns of a 16-, 32- or 48-column launch of the lower-triangle
 // GEMM: launch column k < width computes block column col[k]; distinct
 // columns below EW
 struct NarrowCols {
     int width = 16;
-    uint8_t col[32] = {};
+    uint8_t col[48] = {};
     static NarrowCols tile(int width, int first) {   // columns first + [0, width)
         NarrowCols c;
         c.width = width;
@@ -80,8 +80,8 @@ struct NarrowCols {
     }
 };
 // the same map as a kernel argument: byte k of w[k / 4] is col[k]
-struct ColMap32 {
-    uint32_t w[8];
+struct ColMap {
+    uint32_t w[12];
 };
 
 struct TriPlan {
@@ -482,7 +482,7 @@ bool gemm_config_valid(GemmConfig g);
 // values for a half that is not computed are meaningless (the caller only
 // passes halves without live columns).
 // tri: the plan for Npad, required in mode GEMM_BF16X3_TRI (else unused).
-// narrow (lower-triangle mode): only the 16 or 32 block columns it lists
+// narrow (lower-triangle mode): only the 16, 32 or 48 block columns it lists
 // are computed (halves is then unused); nullptr: the halves.
 hipError_t launch_grm_gemm(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, const float* in,
                            float* out, SigmaArgs a, double* partial, int64_t* nparts, float* ypart,
