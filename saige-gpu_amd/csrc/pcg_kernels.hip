@@ -381,8 +381,7 @@ constexpr int GSPLIT_MAX = 8;           // most column slices
 
 template <int RT, int PD>
 __global__ __launch_bounds__(256) void k_gemm_part(const float* __restrict__ S, int64_t ld,
-                                                   const float* __restrict__ in, float* __restrict__ ypart,
-                                                   int halves) {
+                                                   const float* __restrict__ in, float* __restrict__ ypart) {
     constexpr int GM = 128 * RT;        // rows per workgroup
     constexpr int CPS = GKS / 32;       // 32-column chunks per superchunk
     constexpr int RING = PD + 1;        // S register buffers; RING divides CPS, so a
@@ -454,60 +453,109 @@ __global__ __launch_bounds__(256) void k_gemm_part(const float* __restrict__ S, 
                             *reinterpret_cast<const float4*>(srow + (int64_t)t * 32 * ld + kf + 4 * q);
             }
             const float* pb = sP + c * 32 + hl * 16;
-            if (halves == 3) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const float4 b0 = *reinterpret_cast<const float4*>(pb + (lane & 31) * GKP + 4 * q);
-                    const float4 b1 = *reinterpret_cast<const float4*>(pb + (32 + (lane & 31)) * GKP + 4 * q);
+            for (int q = 0; q < 4; q++) {
+                const float4 b0 = *reinterpret_cast<const float4*>(pb + (lane & 31) * GKP + 4 * q);
+                const float4 b1 = *reinterpret_cast<const float4*>(pb + (32 + (lane & 31)) * GKP + 4 * q);
 #pragma unroll
-                    for (int t = 0; t < RT; t++) {
-                        const float4 a = ring[c % RING][t][q];
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b0.x, acc[t][0], 0, 0, 0);
-                        acc[t][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b1.x, acc[t][1], 0, 0, 0);
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b0.y, acc[t][0], 0, 0, 0);
-                        acc[t][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b1.y, acc[t][1], 0, 0, 0);
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b0.z, acc[t][0], 0, 0, 0);
-                        acc[t][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b1.z, acc[t][1], 0, 0, 0);
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b0.w, acc[t][0], 0, 0, 0);
-                        acc[t][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b1.w, acc[t][1], 0, 0, 0);
-                    }
-                }
-            } else {
-                // one 32-column half live: half the MFMA work (the other half's
-                // partial sums are left unwritten and ignored by the epilogue)
-                const int h = halves >> 1;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const float4 b = *reinterpret_cast<const float4*>(pb + (32 * h + (lane & 31)) * GKP + 4 * q);
-#pragma unroll
-                    for (int t = 0; t < RT; t++) {
-                        const float4 a = ring[c % RING][t][q];
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc[t][0], 0, 0, 0);
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc[t][0], 0, 0, 0);
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc[t][0], 0, 0, 0);
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc[t][0], 0, 0, 0);
-                    }
+                for (int t = 0; t < RT; t++) {
+                    const float4 a = ring[c % RING][t][q];
+                    acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b0.x, acc[t][0], 0, 0, 0);
+                    acc[t][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b1.x, acc[t][1], 0, 0, 0);
+                    acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b0.y, acc[t][0], 0, 0, 0);
+                    acc[t][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b1.y, acc[t][1], 0, 0, 0);
+                    acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b0.z, acc[t][0], 0, 0, 0);
+                    acc[t][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b1.z, acc[t][1], 0, 0, 0);
+                    acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b0.w, acc[t][0], 0, 0, 0);
+                    acc[t][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b1.w, acc[t][1], 0, 0, 0);
                 }
             }
         }
     }
     // raw sums: lane holds column ni*32 + lane%32, rows 8*(r/4) + 4*(lane/32) + r%4
-    // (with one live half, acc[t][0] holds that half)
     float* yp = ypart + (int64_t)split * (gridDim.x * (int64_t)GM) * EW;
-    const int nh = halves == 3 ? 2 : 1;
-    const int h0 = halves == 2 ? 1 : 0;
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
         for (int ni = 0; ni < 2; ni++) {
-            if (ni >= nh) break;
-            const int n = (h0 + ni) * 32 + (lane & 31);
+            const int n = ni * 32 + (lane & 31);
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int64_t row = r0 + wv * 32 * RT + t * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 yp[row * EW + n] = acc[t][ni][r];
             }
         }
+}
+
+// k_gemm_half<NW>: the same sums for one 32-column half, NW waves of 32 rows per
+// workgroup, only the half's P staged, three chunks ahead.  The same MFMAs in
+// the same order as k_gemm_part.  Four waves share a staged P and stream S at
+// 4.6 to 4.8 TB/s from 20,000 samples on (N = 14,080, 20,224, 30,208, 60,160:
+// 172, 356, 712, 3030 us; staging both halves took 195, 415, 830, 3460).  Few
+// rows leave them on too few CUs or unevenly on all (N = 10,240: 320 workgroups
+// on 256 CUs), and one-wave workgroups, which spread evenly, pay their own
+// staging: see HALF_ONE_WAVE.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_gemm_half(const float* __restrict__ S, int64_t ld,
+                                                       const float* __restrict__ in, float* __restrict__ ypart,
+                                                       int half) {
+    constexpr int CPS = GKS / 32;       // 32-column chunks per superchunk
+    constexpr int PD = 3, RING = 4;     // chunks requested ahead, S register buffers (as in k_gemm_part)
+    constexpr int NP = GKS / (2 * NW);  // P values staged per thread and superchunk
+    static_assert(CPS % RING == 0, "");
+    __shared__ __attribute__((aligned(16))) float sP[32 * GKP];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, hl = lane >> 5;
+    const int64_t r0 = (int64_t)blockIdx.x * 32 * NW + wv * 32;
+    const int split = blockIdx.y, nsplit = gridDim.y;
+    const int64_t nsc = ld / GKS;
+    const int64_t sc0 = nsc * split / nsplit, sc1 = nsc * (split + 1) / nsplit, kend = sc1 * GKS;
+    const float* srow = S + (r0 + (lane & 31)) * ld + hl * 16;
+    const int pn = tid & 31, pq = tid >> 5;
+    const float* pp = in + (int64_t)pq * NP * EW + 32 * half + pn;
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+    float4 ring[RING][4];
+    float pr[NP];
+    auto request = [&](int u, int64_t k) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) ring[u][q] = *reinterpret_cast<const float4*>(srow + k + 4 * q);
+    };
+#pragma unroll
+    for (int d = 0; d < PD; d++)
+        if (sc0 * GKS + 32 * d < kend) request(d, sc0 * GKS + 32 * d);
+#pragma unroll
+    for (int q = 0; q < NP; q++) pr[q] = pp[(sc0 * GKS + q) * EW];
+    for (int64_t sc = sc0; sc < sc1; sc++) {
+        const int64_t k0 = sc * GKS;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NP / 4; q++)
+            *reinterpret_cast<float4*>(sP + pn * GKP + pq * NP + 4 * q) =
+                make_float4(pr[4 * q], pr[4 * q + 1], pr[4 * q + 2], pr[4 * q + 3]);
+        __syncthreads();
+        if (sc + 1 < sc1) {
+#pragma unroll
+            for (int q = 0; q < NP; q++) pr[q] = pp[(k0 + GKS + q) * EW];
+        }
+#pragma unroll
+        for (int c = 0; c < CPS; c++) {
+            const int64_t kf = k0 + 32 * (c + PD);
+            if (kf < kend) request((c + PD) % RING, kf);
+            const float* pb = sP + (lane & 31) * GKP + c * 32 + hl * 16;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float4 b = *reinterpret_cast<const float4*>(pb + 4 * q), a = ring[c % RING][q];
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+            }
+        }
+    }
+    float* yp = ypart + (int64_t)split * ld * EW + 32 * half + (lane & 31);
+#pragma unroll
+    for (int r = 0; r < 16; r++) yp[(r0 + 8 * (r >> 2) + 4 * hl + (r & 3)) * EW] = acc[r];
 }
 
 // ------------------------------------------- GEMM, three-piece BF16 split
@@ -2014,6 +2062,11 @@ hipError_t launch_tri(hipStream_t s, GrmMat m, int64_t Npad, const float* in, fl
 }
 }  // namespace
 
+// Rows up to which a one-half FP32 product runs one-wave workgroups: us per
+// product with one and with four waves at 1024, 2560, 5120, 10,240, 14,080 and
+// 20,224 rows: 7.5, 17.4, 34.2, 111, 217, 487 and 8.5, 17.6, 34.0, 126, 172, 356.
+constexpr int64_t HALF_ONE_WAVE = 12288;
+
 hipError_t launch_grm_gemm(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, const float* in,
                            float* out, SigmaArgs a, double* partial, int64_t* nparts, float* ypart, GemmConfig g,
                            int halves, const TriPlan* tri, const NarrowCols* narrow) {
@@ -2072,14 +2125,21 @@ hipError_t launch_grm_gemm(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, c
             hipLaunchKernelGGL((k_gemm_x3<2, 3, 1>), grid, dim3(256), 0, s, S, Npad, pb, ypart, halves);
         else
             hipLaunchKernelGGL((k_gemm_x3<2, 1, 2>), grid, dim3(256), 0, s, S, Npad, pb, ypart, halves);
+    } else if (halves != 3) {
+        if (Npad <= HALF_ONE_WAVE)
+            hipLaunchKernelGGL((k_gemm_half<1>), dim3((unsigned)(Npad / 32), nsplit), dim3(64), 0, s, S, Npad, in,
+                               ypart, halves - 1);
+        else
+            hipLaunchKernelGGL((k_gemm_half<4>), dim3((unsigned)(Npad / 128), nsplit), dim3(256), 0, s, S, Npad, in,
+                               ypart, halves - 1);
     } else if (g.rt == 2 && g.pd == 3)
-        hipLaunchKernelGGL((k_gemm_part<2, 3>), grid, dim3(256), 0, s, S, Npad, in, ypart, halves);
+        hipLaunchKernelGGL((k_gemm_part<2, 3>), grid, dim3(256), 0, s, S, Npad, in, ypart);
     else if (g.rt == 2)
-        hipLaunchKernelGGL((k_gemm_part<2, 1>), grid, dim3(256), 0, s, S, Npad, in, ypart, halves);
+        hipLaunchKernelGGL((k_gemm_part<2, 1>), grid, dim3(256), 0, s, S, Npad, in, ypart);
     else if (g.pd == 3)
-        hipLaunchKernelGGL((k_gemm_part<1, 3>), grid, dim3(256), 0, s, S, Npad, in, ypart, halves);
+        hipLaunchKernelGGL((k_gemm_part<1, 3>), grid, dim3(256), 0, s, S, Npad, in, ypart);
     else
-        hipLaunchKernelGGL((k_gemm_part<1, 1>), grid, dim3(256), 0, s, S, Npad, in, ypart, halves);
+        hipLaunchKernelGGL((k_gemm_part<1, 1>), grid, dim3(256), 0, s, S, Npad, in, ypart);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int64_t nb = Npad / EROWS;
