@@ -1578,7 +1578,7 @@ __global__ __launch_bounds__(256) void k_beta(int kpad, const double* __restrict
                                               const int32_t* __restrict__ maxiter,
                                               const double* __restrict__ tol, int32_t* iter,
                                               uint8_t* done, const uint8_t* __restrict__ live,
-                                              const uint8_t* __restrict__ kind, float* beta) {
+                                              const uint8_t* __restrict__ kind, float* beta, SlotHost h) {
     __shared__ double sm[256];
     const int c = blockIdx.x;
     const double rzn = sum_parts(partial, nparts, kpad, c, 0, sm);
@@ -1599,6 +1599,9 @@ __global__ __launch_bounds__(256) void k_beta(int kpad, const double* __restrict
         } else {
             beta[c] = 0.0f;
         }
+        h.iter[c] = iter[c];
+        h.done[c] = done[c];
+        __threadfence_system();          // there before k_pupdate says so
     }
 }
 
@@ -1607,8 +1610,9 @@ __global__ __launch_bounds__(256) void k_pupdate(int64_t Npad, const float* __re
                                                  const uint8_t* __restrict__ done,
                                                  const uint8_t* __restrict__ live,
                                                  const uint8_t* __restrict__ kind,
-                                                 const float* __restrict__ Z, float* P) {
+                                                 const float* __restrict__ Z, float* P, int32_t* seq, int32_t step) {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (t == 0) __hip_atomic_store(seq, step, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     if (t >= Npad * (EW / 4)) return;
     const int n0 = 4 * (int)(t % (EW / 4));
     bool act[4], any = false;
@@ -1683,7 +1687,7 @@ __global__ __launch_bounds__(256) void k_cols_init_finish(const int32_t* __restr
                                                           const double* __restrict__ partial, int64_t nparts,
                                                           double* rz, double* sumr2, const int32_t* maxiter,
                                                           const double* tol, int32_t* iter, uint8_t* done,
-                                                          int product) {
+                                                          int product, SlotHost h) {
     __shared__ double sm[256];
     const int slot = slots[blockIdx.x];
     const double a = sum_parts(partial, nparts, kpad, slot, 0, sm);
@@ -1692,7 +1696,10 @@ __global__ __launch_bounds__(256) void k_cols_init_finish(const int32_t* __restr
         rz[slot] = a;
         sumr2[slot] = b;
         iter[slot] = 0;
-        done[slot] = product ? 0 : ((b > tol[slot] && 0 < maxiter[slot]) ? 0 : 1);   // FG.cpp:2696
+        const uint8_t over = product ? 0 : ((b > tol[slot] && 0 < maxiter[slot]) ? 0 : 1);   // FG.cpp:2696
+        done[slot] = over;
+        h.iter[slot] = 0;
+        h.done[slot] = over;
     }
 }
 
@@ -2183,18 +2190,19 @@ hipError_t launch_update(hipStream_t s, int kpad, int64_t Nnm, int64_t Npad, con
 
 hipError_t launch_beta(hipStream_t s, int kpad, const double* partial, int64_t nparts, double* rz,
                        double* sumr2, const int32_t* maxiter, const double* tol, int32_t* iter,
-                       uint8_t* done, const uint8_t* live, const uint8_t* kind, float* beta) {
+                       uint8_t* done, const uint8_t* live, const uint8_t* kind, float* beta, SlotHost h) {
     hipLaunchKernelGGL(k_beta, dim3((unsigned)kpad), dim3(256), 0, s, kpad, partial, nparts, rz, sumr2,
-                       maxiter, tol, iter, done, live, kind, beta);
+                       maxiter, tol, iter, done, live, kind, beta, h);
     return hipGetLastError();
 }
 
 hipError_t launch_pupdate(hipStream_t s, int kpad, int64_t Nnm, int64_t Npad, const float* beta,
-                          const uint8_t* done, const uint8_t* live, const uint8_t* kind, const float* Z, float* P) {
+                          const uint8_t* done, const uint8_t* live, const uint8_t* kind, const float* Z, float* P,
+                          SlotHost h, int32_t step) {
     (void)Nnm;
     if (kpad != EW) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_pupdate, dim3(nblk(Npad * (EW / 4), 256)), dim3(256), 0, s, Npad, beta, done,
-                       live, kind, Z, P);
+                       live, kind, Z, P, h.seq, step);
     return hipGetLastError();
 }
 
@@ -2211,9 +2219,9 @@ hipError_t launch_cols_init(hipStream_t s, const float* B, int k, const int32_t*
 
 hipError_t launch_cols_init_finish(hipStream_t s, int k, const int32_t* slots, int kpad, const double* partial,
                                    int64_t nparts, double* rz, double* sumr2, const int32_t* maxiter,
-                                   const double* tol, int32_t* iter, uint8_t* done, int product) {
+                                   const double* tol, int32_t* iter, uint8_t* done, int product, SlotHost h) {
     hipLaunchKernelGGL(k_cols_init_finish, dim3((unsigned)k), dim3(256), 0, s, slots, kpad, partial, nparts, rz,
-                       sumr2, maxiter, tol, iter, done, product);
+                       sumr2, maxiter, tol, iter, done, product, h);
     return hipGetLastError();
 }
 

@@ -116,11 +116,9 @@ void free_engine(Engine& e) {
     dfree(e.rz); dfree(e.sumr2); dfree(e.pap); dfree(e.alpha); dfree(e.beta);
     dfree(e.iter); dfree(e.done); dfree(e.slot_state);
     dfree(e.partial); dfree(e.stage); dfree(e.stageB); dfree(e.ypart);
-    if (e.h_done) (void)hipHostFree(e.h_done);
-    if (e.h_iter) (void)hipHostFree(e.h_iter);
+    if (e.host.iter) (void)hipHostFree(e.host.iter);
     if (e.h_state) (void)hipHostFree(e.h_state);
-    e.h_done = nullptr;
-    e.h_iter = nullptr;
+    e.host = SlotHost{};
     e.h_state = nullptr;
     e.d_list = e.h_list = e.slot_sys = e.h_slot_sys = e.maxiter = e.h_maxiter = e.d_take = e.h_take = nullptr;
     e.tol = e.h_tol = nullptr;
@@ -213,8 +211,12 @@ int engine_reserve(saige_ctx* c, Engine& e, int kpad, int nsys) {
     np = std::max<int64_t>(np, vec_max_parts(Np, kpad) * kpad);
     e.nparts = np;
     SAIGE_HIP_TRY(dalloc(&e.partial, np * 2));
-    SAIGE_HIP_TRY(hipHostMalloc((void**)&e.h_done, kpad, hipHostMallocDefault));
-    SAIGE_HIP_TRY(hipHostMalloc((void**)&e.h_iter, sizeof(int32_t) * kpad, hipHostMallocDefault));
+    const size_t hostb = sizeof(int32_t) * (size_t)(kpad + 1) + (size_t)kpad;      // iter, seq, done
+    SAIGE_HIP_TRY(hipHostMalloc((void**)&e.host.iter, hostb, hipHostMallocDefault));
+    std::memset(e.host.iter, 0, hostb);
+    e.host.seq = e.host.iter + kpad;
+    e.host.done = reinterpret_cast<uint8_t*>(e.host.seq + 1);
+    e.steps = 0;
     e.kpad = kpad;
     e.width = kpad;
     e.nsys = nsys;
@@ -367,7 +369,7 @@ int engine_add_batch(saige_ctx* c, Engine& e, int k, const int32_t* slots, const
     SAIGE_HIP_TRY(launch_cols_init(st, B, k, e.d_list, e.d_list + e.kpad, e.kpad, N, Np, e.minv, e.mask, e.X,
                                    e.R, e.Z, e.P, e.partial, &np, product));
     SAIGE_HIP_TRY(launch_cols_init_finish(st, k, e.d_list, e.kpad, e.partial, np, e.rz, e.sumr2, e.maxiter, e.tol,
-                                          e.iter, e.done, product));
+                                          e.iter, e.done, product, e.host));
     SAIGE_HIP_TRY(hipStreamSynchronize(st));
     return SAIGE_OK;
 }
@@ -430,6 +432,20 @@ const GemvPlan* gemv_plan(saige_ctx* c, int* rc) {
     return &c->triv;
 }
 
+// Waits until the last launched iteration's slot state is in e.host; the
+// iteration's update of P may still run, and the next launches follow it on the
+// stream.  An idle or failed stream ends the wait whatever the host sees.
+hipError_t wait_step(saige_ctx* c, Engine& e) {
+    for (int spin = 0; __atomic_load_n(e.host.seq, __ATOMIC_ACQUIRE) != e.steps; spin++) {
+        __builtin_ia32_pause();
+        if ((spin & 1023) == 1023) {
+            const hipError_t q = hipStreamQuery(c->stream);
+            if (q != hipErrorNotReady) return q;
+        }
+    }
+    return hipEventSynchronize(c->ev1);
+}
+
 int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t* iters_out) {
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
@@ -446,8 +462,6 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
     a.mode = 1;
     a.kind = e.kind;
     a.xout = e.X;
-    SAIGE_HIP_TRY(hipMemcpyAsync(e.h_done, e.done, e.kpad, hipMemcpyDeviceToHost, st));
-    SAIGE_HIP_TRY(hipStreamSynchronize(st));
     // 32-column halves of the block that hold an occupied slot; the GEMM skips
     // the others (a done slot that is not yet taken is recomputed unchanged)
     int halves = 0, nlive = 0;
@@ -477,7 +491,7 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
     if (narrow) halves = nc.width == 48 ? 3 : 1;   // for the shape and the statistics below
     for (int it = 0; it < n_iter; it++) {
         bool any = false;
-        for (int k = 0; k < e.kpad; k++) any |= (e.h_live[k] && !e.h_done[k]);
+        for (int k = 0; k < e.kpad; k++) any |= (e.h_live[k] && !e.host.done[k]);
         if (!any) break;
         int64_t np = 0;
         SAIGE_HIP_TRY(hipEventRecord(c->ev0, st));
@@ -494,10 +508,10 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
         SAIGE_HIP_TRY(launch_update(st, e.kpad, N, Np, e.alpha, e.done, e.live, e.kind, e.minv, e.slot_sys, e.X, e.R,
                                     e.Z, e.P, e.AP, e.partial, &np2));
         SAIGE_HIP_TRY(launch_beta(st, e.kpad, e.partial, np2, e.rz, e.sumr2, e.maxiter, e.tol, e.iter, e.done,
-                                  e.live, e.kind, e.beta));
-        SAIGE_HIP_TRY(launch_pupdate(st, e.kpad, N, Np, e.beta, e.done, e.live, e.kind, e.Z, e.P));
-        SAIGE_HIP_TRY(hipMemcpyAsync(e.h_done, e.done, e.kpad, hipMemcpyDeviceToHost, st));
-        SAIGE_HIP_TRY(hipStreamSynchronize(st));
+                                  e.live, e.kind, e.beta, e.host));
+        e.steps = (int32_t)((uint32_t)e.steps + 1u);
+        SAIGE_HIP_TRY(launch_pupdate(st, e.kpad, N, Np, e.beta, e.done, e.live, e.kind, e.Z, e.P, e.host, e.steps));
+        SAIGE_HIP_TRY(wait_step(c, e));
         float ms = 0.f;
         SAIGE_HIP_TRY(hipEventElapsedTime(&ms, c->ev0, c->ev1));
         const int kind = quarter       ? SAIGE_LAUNCH_GEMM_QUARTER
@@ -506,12 +520,9 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
         e.gemm_seconds[kind] += ms * 1e-3;
         e.gemm_launches[kind]++;
     }
-    SAIGE_HIP_TRY(hipMemcpyAsync(e.h_iter, e.iter, 4 * e.kpad, hipMemcpyDeviceToHost, st));
-    SAIGE_HIP_TRY(hipMemcpyAsync(e.h_done, e.done, e.kpad, hipMemcpyDeviceToHost, st));
-    SAIGE_HIP_TRY(hipStreamSynchronize(st));
     for (int k = 0; k < e.kpad; k++) {
-        if (done_out) done_out[k] = e.h_live[k] ? e.h_done[k] : 1;
-        if (iters_out) iters_out[k] = e.h_live[k] ? e.h_iter[k] : 0;
+        if (done_out) done_out[k] = e.h_live[k] ? e.host.done[k] : 1;
+        if (iters_out) iters_out[k] = e.h_live[k] ? e.host.iter[k] : 0;
     }
     return SAIGE_OK;
 }

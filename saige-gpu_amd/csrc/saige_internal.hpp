@@ -151,6 +151,17 @@ struct Solve1 {
     void release();
 };
 
+// Slot state in pinned host memory, written by the kernels that change it: the
+// host learns what has stopped without a copy, and beside the last kernel of the
+// iteration (four copies and three waits per call of one iteration took 45 to 80
+// us of a null fit's 1500).  seq: the number of the last iteration whose done and
+// iter are there.
+struct SlotHost {
+    uint8_t* done = nullptr;
+    int32_t* iter = nullptr;
+    int32_t* seq = nullptr;
+};
+
 struct Engine {
     int width = 0;        // live slot capacity (<= EW)
     int nsys = 0;
@@ -192,9 +203,8 @@ struct Engine {
     int32_t* h_take = nullptr;
     int32_t* h_maxiter = nullptr;
     double* h_tol = nullptr;
-    // pinned host mirrors
-    uint8_t* h_done = nullptr;
-    int32_t* h_iter = nullptr;
+    SlotHost host;                // the slots' state as the host sees it (pinned)
+    int32_t steps = 0;            // iterations launched
     int32_t* h_slot_sys = nullptr;
     uint8_t* h_live = nullptr;
     // device time of the GRM product launches by kind: [1] GEMM over one
@@ -505,16 +515,16 @@ hipError_t launch_update(hipStream_t s, int kpad, int64_t Nnm, int64_t Npad, con
                          const float* AP, double* partial, int64_t* nparts);
 hipError_t launch_beta(hipStream_t s, int kpad, const double* partial, int64_t nparts, double* rz,
                        double* sumr2, const int32_t* maxiter, const double* tol, int32_t* iter,
-                       uint8_t* done, const uint8_t* live, const uint8_t* kind, float* beta);
+                       uint8_t* done, const uint8_t* live, const uint8_t* kind, float* beta, SlotHost h);
 hipError_t launch_pupdate(hipStream_t s, int kpad, int64_t Nnm, int64_t Npad, const float* beta,
                           const uint8_t* done, const uint8_t* live, const uint8_t* kind, const float* Z,
-                          float* P);
+                          float* P, SlotHost h, int32_t step);
 hipError_t launch_cols_init(hipStream_t s, const float* B, int k, const int32_t* slots, const int32_t* sys,
                             int kpad, int64_t Nnm, int64_t Npad, const float* minv, const uint8_t* mask, float* X,
                             float* R, float* Z, float* P, double* partial, int64_t* nparts, int product);
 hipError_t launch_cols_init_finish(hipStream_t s, int k, const int32_t* slots, int kpad, const double* partial,
                                    int64_t nparts, double* rz, double* sumr2, const int32_t* maxiter,
-                                   const double* tol, int32_t* iter, uint8_t* done, int product);
+                                   const double* tol, int32_t* iter, uint8_t* done, int product, SlotHost h);
 // slot results to columns cols[j] (nullptr: j) of a column-major buffer
 hipError_t launch_cols_gather(hipStream_t s, const float* src, int k, const int32_t* slots, const int32_t* cols,
                               int kpad, int64_t Nnm, int64_t ld, float* dst);
