@@ -17,6 +17,7 @@
 #include "saige_internal.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -662,20 +663,40 @@ __device__ __forceinline__ f32x16 mfma_x3(u32x4 ah, u32x4 am, u32x4 al, u32x4 bh
 }
 
 
-__global__ __launch_bounds__(256) void k_split_p(const float* __restrict__ in, int64_t G,
-                                                 u32x4* __restrict__ pb) {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= G * EW) return;
-    const int64_t g = t / EW;
-    const int n = (int)(t % EW);
+// PERM: group g = 4c + j holds rows 32c + 4j + [0, 4) and 32c + 16 + 4j + [0, 4)
+// instead, the row order of the lower-triangle product's use 2
+template <bool PERM>
+__device__ __forceinline__ void split_p_group(const float* __restrict__ in, int64_t G, int64_t g, int n,
+                                              u32x4* __restrict__ pb) {
+    const int64_t r0 = PERM ? 32 * (g >> 2) + 4 * (g & 3) : 8 * g, r1 = r0 + (PERM ? 16 : 4);
     float x[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) x[e] = in[(8 * g + e) * EW + n];
+    for (int e = 0; e < 8; e++) x[e] = in[(e < 4 ? r0 + e : r1 + e - 4) * EW + n];
     u32x4 h, m, l;
     split3_8(make_float4(x[0], x[1], x[2], x[3]), make_float4(x[4], x[5], x[6], x[7]), h, m, l);
     pb[g * EW + n] = h;
     pb[(G + g) * EW + n] = m;
     pb[(2 * G + g) * EW + n] = l;
+}
+
+__global__ __launch_bounds__(256) void k_split_p(const float* __restrict__ in, int64_t G,
+                                                 u32x4* __restrict__ pb) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= G * EW) return;
+    split_p_group<false>(in, G, t / EW, (int)(t % EW), pb);
+}
+
+// both orders: pb, then pb2
+__global__ __launch_bounds__(256) void k_split_p2(const float* __restrict__ in, int64_t G, u32x4* __restrict__ pb,
+                                                  u32x4* __restrict__ pb2) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= 2 * G * EW) return;
+    const int64_t g = t / EW;
+    const int n = (int)(t % EW);
+    if (g < G)
+        split_p_group<false>(in, G, g, n, pb);
+    else
+        split_p_group<true>(in, G, g - G, n, pb2);
 }
 
 template <int RT, int PD, int W>
@@ -1292,6 +1313,147 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
         for (int t = 0; t < NQ; t++)
 #pragma unroll
             for (int a = 0; a < 4; a++) yp[(int64_t)(wv * 32 + 16 * r + 4 * g + a) * YS + 16 * t + ln] = acc1[r][t][a];
+}
+
+// k_gemm_flat<NWV, NQ, SP>: k_gemm_t16's partials, bit by bit, from all of S.  At
+// few samples the triangle's items are fewer than the CUs, each a serial walk of
+// up to 96 chunks by twelve waves (N = 4000: 56 items).  Here a wave owns a strip
+// of 32 rows and its workgroup four strips of one row set, and use 2 needs no
+// transpose: S_IJ^T is the block of S right of the diagonal in strip J's own
+// rows.  An item is the four strips' piece of
+// * a use-1 item of the row set (slot >= 0), the same chunks in the same order,
+//   or
+// * use 2 of some row sets R' > R (slot < 0): per chunk I of them P_I^T S_JI^T
+//   from zero, K in the order k_gemm_t16 has it (P's pieces in that order from
+//   pb2, S's columns 4g + [0, 4) and 16 + 4g + [0, 4)), summed over the chunks of
+//   one row set in wave order and stored as its partial.
+// The use-2 items are independent, so they can be as short as fills the chip;
+// the time is that of the longest use-1 item or of the bytes, twice the
+// triangle's.  P's pieces are staged per chunk for the four strips, in two LDS
+// buffers; making a chunk's operands during the one before gained nothing.  us
+// per 64- / 16-column launch, k_gemm_t16 and this: N = 1000 73 / 35 and 20 / 14,
+// 4000 277 / 130 and 70 / 50, 10,000 286 / 133 and 127 / 106.
+template <int NWV, int NQ, int SP>
+__global__ __launch_bounds__(256) void k_gemm_flat(const float* __restrict__ S, int64_t ld,
+                                                   const u32x4* __restrict__ pb, const u32x4* __restrict__ pb2,
+                                                   const int4* __restrict__ items, float* __restrict__ y1p,
+                                                   float* __restrict__ y2p, ColMap cm) {
+    constexpr int PD = NQ == 4 ? 3 : 4, RING = PD + 1;    // chunks requested ahead (64 columns: the registers)
+    constexpr int NSTG = 192 * NQ, STG = (NSTG + 255) / 256, YS = 16 * NQ;
+    __shared__ u32x4 sB[2][12 * YS];                 // a chunk's P pieces, [(g*3 + piece)*16*NQ + n]
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = lane >> 4, ln = lane & 15;
+    const int4 item = items[blockIdx.x];
+    const int64_t strip = 4 * (int64_t)item.x + wv, ca = item.y, cb = item.z, slot = item.w;
+    const int64_t nch = ld / 32, G = ld / 8, NR = (nch + NWV - 1) / NWV, R = strip / NWV;
+    auto run = [&](auto u2tag) {
+        constexpr bool U2 = decltype(u2tag)::value;
+        const u32x4* bsrc[STG];
+        int bdi[STG];
+#pragma unroll
+        for (int s = 0; s < STG; s++) {
+            const int k = tid + s * 256 < NSTG ? tid + s * 256 : tid % NSTG;
+            const int gp = k / YS, kk = k % YS;
+            bsrc[s] = (U2 ? pb2 : pb) + ((int64_t)(gp % 3) * G + gp / 3) * EW + (NQ < 4 ? map_col(cm, kk) : kk);
+            bdi[s] = gp * YS + kk;
+        }
+        const float* srow = S + (32 * strip + ln) * ld + (U2 ? 4 : 8) * g;
+        u32x4 ring[RING][4], bring[RING][STG];
+        auto issue = [&](int u, int64_t ch) {
+            ch = ch < cb ? ch : cb - 1;              // past the end: the last chunk again, unused
+#pragma unroll
+            for (int s = 0; s < STG; s++) bring[u][s] = bsrc[s][4 * ch * EW];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                ring[u][k] = *reinterpret_cast<const u32x4*>(srow + (int64_t)(k >> 1) * 16 * ld + ch * 32 +
+                                                             (k & 1) * (U2 ? 16 : 4));
+        };
+        // use 1: [row tile][column tile] over the item; use 2: [j group][column
+        // tile] over a row set
+        f32x4 acc[2][NQ];
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int t = 0; t < NQ; t++) acc[r][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        int w = 0;                                   // use 2: the chunk's wave in its row set
+        float* dst = y2p + (tri_y2_first<NWV>(strip, NR) + (ca / NWV - R - 1)) * (32 * YS) + ln * YS + 4 * g;
+        auto step = [&](int u, int64_t c) {
+            u32x4* sb = sB[(c - ca) & 1];
+#pragma unroll
+            for (int s = 0; s < STG; s++) sb[bdi[s]] = bring[u][s];
+            lds_barrier();
+            issue((u + PD) % RING, c + PD);
+            __builtin_amdgcn_sched_barrier(0);       // what is ahead is asked for first
+            const u32x4* bb = sb + g * 3 * YS + ln;
+            u32x4 h[2], m[2], l[2];
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const float4 a = __builtin_bit_cast(float4, ring[u][2 * r]),
+                             b = __builtin_bit_cast(float4, ring[u][2 * r + 1]);
+                if constexpr (SP == 3)
+                    split3_8(a, b, h[r], m[r], l[r]);
+                else
+                    split2_8(a, b, h[r], m[r]);
+            }
+#pragma unroll
+            for (int t = 0; t < NQ; t++) {
+                const u32x4 ph = bb[16 * t], pm = bb[YS + 16 * t], pl = bb[2 * YS + 16 * t];
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    if (U2) {
+                        f32x4 c2 = {0.0f, 0.0f, 0.0f, 0.0f};
+                        if constexpr (SP == 3)
+                            c2 = mfma16_x3(ph, pm, pl, h[r], m[r], l[r], c2);
+                        else
+                            c2 = mfma16_b2(ph, pm, pl, h[r], m[r], c2);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[r][t][e] = w == 0 ? c2[e] : acc[r][t][e] + c2[e];
+                    } else if constexpr (SP == 3) {
+                        acc[r][t] = mfma16_x3(h[r], m[r], l[r], ph, pm, pl, acc[r][t]);
+                    } else {
+                        acc[r][t] = mfma16_a2(h[r], m[r], ph, pm, pl, acc[r][t]);
+                    }
+                }
+            }
+            if (U2) {
+                w++;
+                if (w == NWV || c + 1 == nch) {
+                    // row tile r's column 16r + ln, rhs 16t + 4g + [0, 4); a last
+                    // row set with fewer strips adds its missing waves' zeros
+                    const float z = w < NWV ? 0.0f : -0.0f;
+#pragma unroll
+                    for (int r = 0; r < 2; r++)
+#pragma unroll
+                        for (int t = 0; t < NQ; t++)
+                            *reinterpret_cast<float4*>(dst + 16 * r * YS + 16 * t) =
+                                make_float4(acc[r][t][0] + z, acc[r][t][1] + z, acc[r][t][2] + z, acc[r][t][3] + z);
+                    dst += 32 * YS;
+                    w = 0;
+                }
+            }
+        };
+#pragma unroll
+        for (int d = 0; d < PD; d++) issue(d, ca + d);
+        int64_t c = ca;
+        for (; c + RING <= cb; c += RING) {
+#pragma unroll
+            for (int u = 0; u < RING; u++) step(u, c + u);
+        }
+#pragma unroll
+        for (int u = 0; u < RING - 1; u++)
+            if (c + u < cb) step(u, c + u);
+        if (U2) return;
+        float* yp = y1p + (slot * 32 * NWV + 32 * (strip - R * NWV)) * YS;
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int t = 0; t < NQ; t++)
+#pragma unroll
+                for (int a = 0; a < 4; a++) yp[(int64_t)(16 * r + 4 * g + a) * YS + 16 * t + ln] = acc[r][t][a];
+    };
+    if (slot < 0)
+        run(std::true_type());
+    else
+        run(std::false_type());
 }
 
 // k_tri_reduce: Y[row][q] = the row set's use-1 partials (rtab[R] = {first
@@ -1939,6 +2101,7 @@ hipError_t gemv_plan_build(GemvPlan& t, int64_t Npad, int ch) {
 
 void tri_plan_free(TriPlan& t) {
     if (t.items) (void)hipFree(t.items);
+    if (t.flat) (void)hipFree(t.flat);
     if (t.rtab) (void)hipFree(t.rtab);
     if (t.y1p) (void)hipFree(t.y1p);
     if (t.y2p) (void)hipFree(t.y2p);
@@ -1986,8 +2149,39 @@ static std::vector<int4> tri_dispatch_order(const std::vector<int4>& items, int 
     return out;
 }
 
+// Rows up to which a launch of this width runs as k_gemm_flat, where its bytes
+// (all of S in FP32) begin to take longer than k_gemm_t16's walk of the triangle:
+// us of k_gemm_t16 and k_gemm_flat at 10,240, 14,080 and 20,224 rows: 64 columns
+// 286, 296, 325 and 127, 216, 420; 48: 241, 250, 273 and 115, 192, 393; 32: 184,
+// 190, 205 and 114, 184, 375; 16: 133, 139, 161 and 106, 170, 345.
+// SAIGE_TRI_FLAT_MAX=rows sets one limit for every width (the bits are the same).
+static int64_t tri_flat_rows(int width) {
+    if (const char* e = std::getenv("SAIGE_TRI_FLAT_MAX")) return std::atoll(e);
+    return width <= 16 ? 11264 : width <= 32 ? 14080 : 16384;
+}
+
+// k_gemm_flat's items: per group of four strips the use-1 items of its row set,
+// and its use-2 row sets in runs that make about three items per CU, at most
+// eight row sets each; longest first
+static std::vector<int4> tri_flat_items(const std::vector<int4>& items, int64_t nch, int nwv) {
+    const int64_t nr = (nch + nwv - 1) / nwv, gr = nwv / 4;
+    std::vector<int4> out;
+    int64_t sets = 0;
+    for (const int4& it : items)
+        for (int64_t q = gr * it.x; q < std::min(gr * (it.x + 1), nch / 4); q++)
+            out.push_back(make_int4((int)q, it.y, it.z, it.w));
+    for (int64_t q = 0; q < nch / 4; q++) sets += nr - 1 - q / gr;
+    const int64_t run = std::min<int64_t>(8, std::max<int64_t>(1, sets / 768));
+    for (int64_t q = 0; q < nch / 4; q++)
+        for (int64_t r = q / gr + 1; r < nr; r += run)
+            out.push_back(make_int4((int)q, (int)(r * nwv), (int)std::min((r + run) * nwv, nch), -1));
+    std::stable_sort(out.begin(), out.end(), [](const int4& a, const int4& b) { return a.z - a.y > b.z - b.y; });
+    return out;
+}
+
 hipError_t tri_plan_build(TriPlan& t, int64_t Npad, int nwv, int ch) {
-    if (t.items && t.Npad == Npad && t.nwv == nwv && t.ch == ch) return hipSuccess;
+    if (t.items && t.Npad == Npad && t.nwv == nwv && t.ch == ch && (t.nflat > 0) == (Npad <= tri_flat_rows(EW)))
+        return hipSuccess;
     tri_plan_free(t);
     if ((nwv != 8 && nwv != 12) || ch < 1 || Npad <= 0 || Npad % 256 != 0) return hipErrorInvalidValue;
     const int64_t nch = Npad / 32, nr = (nch + nwv - 1) / nwv;
@@ -2003,6 +2197,8 @@ hipError_t tri_plan_build(TriPlan& t, int64_t Npad, int nwv, int ch) {
         items.push_back(make_int4((int)R, (int)off, (int)std::min(off + nwv, nch), (int)slot++));
         rtab[(size_t)R] = make_int2((int)first, (int)(slot - first));
     }
+    std::vector<int4> flat;
+    if (Npad <= tri_flat_rows(EW)) flat = tri_flat_items(items, nch, nwv);
     items = tri_dispatch_order(items, nwv, ch);
     const int64_t y2 = nwv == 8 ? tri_y2_first<8>(nch, nr) : tri_y2_first<12>(nch, nr);
     t.Npad = Npad;
@@ -2012,17 +2208,35 @@ hipError_t tri_plan_build(TriPlan& t, int64_t Npad, int nwv, int ch) {
     t.nr = nr;
     t.y1_slots = slot;
     t.y2_slots = y2;
+    t.nflat = (int64_t)flat.size();
     hipError_t e = hipMalloc(&t.items, sizeof(int4) * items.size());
     if (e == hipSuccess) e = hipMalloc(&t.rtab, sizeof(int2) * rtab.size());
     if (e == hipSuccess) e = hipMalloc(&t.y1p, sizeof(float) * (size_t)(slot * 32 * nwv * EW));
     if (e == hipSuccess) e = hipMalloc(&t.y2p, sizeof(float) * (size_t)(std::max<int64_t>(y2, 1) * 32 * EW));
     if (e == hipSuccess) e = hipMemcpy(t.items, items.data(), sizeof(int4) * items.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(t.rtab, rtab.data(), sizeof(int2) * rtab.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess && t.nflat) e = hipMalloc(&t.flat, sizeof(int4) * flat.size());
+    if (e == hipSuccess && t.nflat) e = hipMemcpy(t.flat, flat.data(), sizeof(int4) * flat.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) tri_plan_free(t);
     return e;
 }
 
 namespace {
+template <int NWV, int NQ>
+void launch_tri_reduce(hipStream_t s, int64_t Npad, const TriPlan& t, ColMap cm, float* ypart) {
+    constexpr int QW = 4 * NQ, NT = tri_reduce_threads(QW);     // Npad is a multiple of NT / QW
+    hipLaunchKernelGGL((k_tri_reduce<NWV, QW>), dim3((unsigned)(Npad / (NT / QW))), dim3(NT), 0, s, t.y1p, t.y2p,
+                       t.rtab, Npad, cm, ypart);
+}
+
+template <int NWV, int NQ, int SP>
+void launch_flat(hipStream_t s, GrmMat m, int64_t Npad, const u32x4* pb, const u32x4* pb2, const TriPlan& t,
+                 ColMap cm, float* ypart) {
+    hipLaunchKernelGGL((k_gemm_flat<NWV, NQ, SP>), dim3((unsigned)t.nflat), dim3(256), 0, s, m.S, Npad, pb, pb2,
+                       t.flat, t.y1p, t.y2p, cm);
+    launch_tri_reduce<NWV, NQ>(s, Npad, t, cm, ypart);
+}
+
 template <int NWV, int PD, int NQ, int SP>
 void launch_t16(hipStream_t s, dim3 grid, GrmMat m, int64_t Npad, const u32x4* pb, const float* in,
                 const TriPlan& t, ColMap cm, float* ypart) {
@@ -2032,9 +2246,7 @@ void launch_t16(hipStream_t s, dim3 grid, GrmMat m, int64_t Npad, const u32x4* p
     else
         hipLaunchKernelGGL((k_gemm_t16<NWV, PD, NQ, SP, false>), grid, dim3(64 * NWV), 0, s, m.S, m.s24, Npad, pb, in,
                            t.items, t.y1p, t.y2p, cm);
-    constexpr int QW = 4 * NQ, NT = tri_reduce_threads(QW);     // Npad is a multiple of NT / QW
-    hipLaunchKernelGGL((k_tri_reduce<NWV, QW>), dim3((unsigned)(Npad / (NT / QW))), dim3(NT), 0, s, t.y1p, t.y2p,
-                       t.rtab, Npad, cm, ypart);
+    launch_tri_reduce<NWV, NQ>(s, Npad, t, cm, ypart);
 }
 
 // the lower-triangle product over the launch's 64 columns, or the 16, 32 or 48
@@ -2044,7 +2256,6 @@ hipError_t launch_tri(hipStream_t s, GrmMat m, int64_t Npad, const float* in, fl
                       int halves, const NarrowCols* narrow, const TriPlan& t) {
     const int64_t G = Npad / 8;
     u32x4* pb = reinterpret_cast<u32x4*>(ypart + (int64_t)GSPLIT_MAX * Npad * EW);
-    hipLaunchKernelGGL(k_split_p, dim3((unsigned)(G * EW / 256)), dim3(256), 0, s, in, G, pb);
     const dim3 grid((unsigned)t.nitems);
     const bool deep = pd == 3;
     const NarrowCols half = NarrowCols::tile(32, halves == 2 ? 32 : 0);
@@ -2052,13 +2263,24 @@ hipError_t launch_tri(hipStream_t s, GrmMat m, int64_t Npad, const float* in, fl
     ColMap cm{};
     if (narrow)
         for (int k = 0; k < narrow->width; k++) cm.w[k / 4] |= (uint32_t)narrow->col[k] << (8 * (k % 4));
-    if (narrow && narrow->width == 16) {
+    const int width = narrow ? narrow->width : EW;
+    if (t.nflat && Npad <= tri_flat_rows(width)) {
+        u32x4* pb2 = reinterpret_cast<u32x4*>(ypart + 2 * Npad * EW);       // slices that this product leaves free
+        hipLaunchKernelGGL(k_split_p2, dim3((unsigned)(2 * G * EW / 256)), dim3(256), 0, s, in, G, pb, pb2);
+        if (width == 16) launch_flat<NWV, 1, SP>(s, m, Npad, pb, pb2, t, cm, ypart);
+        else if (width == 32) launch_flat<NWV, 2, SP>(s, m, Npad, pb, pb2, t, cm, ypart);
+        else if (width == 48) launch_flat<NWV, 3, SP>(s, m, Npad, pb, pb2, t, cm, ypart);
+        else launch_flat<NWV, 4, SP>(s, m, Npad, pb, pb2, t, cm, ypart);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(k_split_p, dim3((unsigned)(G * EW / 256)), dim3(256), 0, s, in, G, pb);
+    if (width == 16) {
         if (deep) launch_t16<NWV, 2, 1, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
         else launch_t16<NWV, 1, 1, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
-    } else if (narrow && narrow->width == 48) {
+    } else if (width == 48) {
         if (deep) launch_t16<NWV, 2, 3, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
         else launch_t16<NWV, 1, 3, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
-    } else if (narrow) {
+    } else if (width == 32) {
         if (deep) launch_t16<NWV, 2, 2, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
         else launch_t16<NWV, 1, 2, SP>(s, grid, m, Npad, pb, in, t, cm, ypart);
     } else {

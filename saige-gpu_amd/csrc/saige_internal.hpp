@@ -90,6 +90,8 @@ struct TriPlan {
     int ch = 0;                  // most chunks per item left of the diagonal
     int64_t nitems = 0, nr = 0, y1_slots = 0, y2_slots = 0;
     int4* items = nullptr;       // device [nitems], longest first
+    int64_t nflat = 0;           // > 0: few rows, launches may run as k_gemm_flat over these items:
+    int4* flat = nullptr;        // {group of four strips, first and end chunk, use-1 slot or -1}
     int2* rtab = nullptr;        // device [nr]
     float* y1p = nullptr;        // [y1_slots][32*nwv][W], W = the launch's width (<= EW)
     float* y2p = nullptr;        // [y2_slots][32][W]
