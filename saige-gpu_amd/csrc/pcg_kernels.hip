@@ -933,10 +933,12 @@ __global__ __launch_bounds__(768) void k_gemm_x3w(const float* __restrict__ S, i
 // * use 2: Y_J^T[tile t][16*jg + .] = P_I^T T_jg per j-group jg, stored to
 //   the wave's use-2 tile [column j][rhs] in LDS.
 // The NWV use-2 tiles of a chunk are summed in LDS in wave order and stored
-// as the partial of (chunk, row set) in y2p.  With eight waves the LDS holds
-// two such tiles, and chunk c's sum is formed in chunk c+1's iteration,
-// beside its MFMA work, so one barrier per chunk suffices; twelve waves'
-// tiles fit once, and the sum follows a second barrier in the chunk's own
+// as the partial of (chunk, row set) in y2p.  With eight waves, or up to 32
+// columns, the LDS holds two such tiles, and chunk c's sum is formed in chunk
+// c+1's iteration, beside its MFMA work, so one barrier per chunk suffices (32
+// columns at N = 50,000 and 100,000: 1047 and 4820 us with two barriers, 985 and
+// 4500 with one; 16: 893 and 3410, 870 and 3360); wider tiles of twelve waves
+// fit once, and the sum follows a second barrier in the chunk's own
 // iteration.  Use 1 accumulates in registers over the item and is stored as
 // the item's partial in y1p.  k_tri_reduce sums, for each row, its row set's
 // use-1 partials in slot order and then its chunk's use-2 partials in
@@ -945,8 +947,9 @@ __global__ __launch_bounds__(768) void k_gemm_x3w(const float* __restrict__ S, i
 // live columns (a 16-column launch does a quarter of a full one's MFMA work)
 // and a column's bits still do not depend on its co-tenants.  A narrow launch
 // takes any 16, 32 or 48 block columns (a map of launch column -> block column),
-// so that many live columns anywhere in the block run in one.  The arithmetic of an output column depends only on its own
-// column of P, in whatever position of the MFMA operands it sits.
+// so that many live columns anywhere in the block run in one.  The arithmetic of
+// an output column depends only on its own column of P, in whatever position of
+// the MFMA operands it sits.
 // Eight waves have registers for a software-pipelined loop: chunk c's pieces
 // are split during chunk c-1, beside that chunk's MFMAs.  Twelve waves split
 // each chunk at its own turn, PD chunks of raw data ahead.
@@ -957,10 +960,16 @@ __global__ __launch_bounds__(768) void k_gemm_x3w(const float* __restrict__ S, i
 // a zero product leaves an accumulator unchanged, so on such an S both forms
 // give the same bits.
 
-// a use-2 tile in LDS: [column j][64 rhs], float4 slot s of row j stored at
-// slot s ^ (j % 16), so the column-per-lane writes and row-wise reads both
-// spread over all banks
-__device__ __forceinline__ int tri_sr_index(int j, int q) { return j * 64 + 4 * ((q >> 2) ^ (j & 15)) + (q & 3); }
+// a use-2 tile in LDS: [column j][launch columns], 16, 32 or 64 floats a row; the
+// float4 slots of row j permuted so that the column-per-lane writes (eight lanes
+// at a time, neighbouring rows) and row-wise reads both spread over all banks
+template <int NQ>
+constexpr int tri_sr_row = NQ <= 2 ? 16 * NQ : 64;
+template <int NQ>
+__device__ __forceinline__ int tri_sr_index(int j, int q) {
+    const int x = NQ == 1 ? (j >> 1) & 3 : NQ == 2 ? j & 7 : j & 15;
+    return j * tri_sr_row<NQ> + 4 * ((q >> 2) ^ x) + (q & 3);
+}
 
 // index of the first use-2 partial of chunk c: chunk c' has NR - 1 - c'/NWV
 template <int NWV>
@@ -1047,9 +1056,10 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
     constexpr int NSTG = 192 * NQ;                   // P pieces a chunk needs: 4 groups x 3 pieces x 16*NQ columns
     constexpr int STG = (NSTG + NTH - 1) / NTH;      // P pieces staged per thread and chunk
     constexpr int YS = 16 * NQ;                      // row stride of the partials: the launch's columns
-    __shared__ u32x4 sB0[12 * 64], sB1[12 * 64];     // a chunk's P pieces, [(g*3 + piece)*64 + n]
-    constexpr int SRB = NWV == 8 ? 2 : 1;            // use-2 tile buffers
-    __shared__ float sR[SRB][NWV * 32 * 64];         // use-2 results, [wave][column j][launch column]
+    __shared__ u32x4 sB0[12 * YS], sB1[12 * YS];     // a chunk's P pieces, [(g*3 + piece)*16*NQ + n]
+    constexpr int SRB = NWV == 8 || NQ <= 2 ? 2 : 1; // use-2 tile buffers
+    constexpr int SRT = 32 * tri_sr_row<NQ>;         // floats of a use-2 tile
+    __shared__ float sR[SRB][NWV * SRT];             // use-2 results, [wave][column j][launch column]
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = lane >> 4, ln = lane & 15;
     const int4 item = items[blockIdx.x];
     const int64_t R = item.x, ca = item.y, cb = item.z, slot = item.w;
@@ -1062,7 +1072,6 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
     const u32x4* strip = C24 ? reinterpret_cast<const u32x4*>(S24 + s24_block((valid ? rw : ld - 32) / 32, 0) * S24_BLOCK) +
                                    lane
                              : nullptr;
-    constexpr int c0 = 0;                            // the launch's first column in LDS and partials
     // the block column of launch column k (of 16 * NQ)
     auto gcol = [&](int k) { return NQ < 4 ? map_col(cm, k) : k; };
     // staging: element k of a chunk's NSTG pieces is launch column k % (16*NQ)
@@ -1075,7 +1084,7 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
         const int k = tid + s * NTH < NSTG ? tid + s * NTH : tid % NSTG;
         const int gp = k / (16 * NQ), kk = k % (16 * NQ);
         bsrc[s] = pb + ((int64_t)(gp % 3) * G + gp / 3) * EW + gcol(kk);
-        bdi[s] = gp * 64 + c0 + kk;
+        bdi[s] = gp * YS + kk;
     }
     // E_jg as B operand: lane (ln, g) holds K = columns 8g + [0, 8) of column
     // ln, E_jg[k][n] = 1 when k == 16*jg + n
@@ -1149,13 +1158,13 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
             if (wv < NR2) {
                 const int o = (wv * 64 + lane) * V;
                 const int j = o / (16 * NQ), ql = o % (16 * NQ);
-                const float* src = sr + tri_sr_index(j, ql);
+                const float* src = sr + tri_sr_index<NQ>(j, ql);
                 float* dst = y2p + (tri_y2_first<NWV>(cc, NR) + (R - cc / NWV - 1)) * (32 * YS) + j * YS + ql;
                 if constexpr (V == 4) {
                     float4 sum = *reinterpret_cast<const float4*>(src);
 #pragma unroll
                     for (int w = 1; w < NWV; w++) {
-                        const float4 v = *reinterpret_cast<const float4*>(src + w * 32 * 64);
+                        const float4 v = *reinterpret_cast<const float4*>(src + w * SRT);
                         sum.x += v.x;
                         sum.y += v.y;
                         sum.z += v.z;
@@ -1166,7 +1175,7 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
                     float2 sum = *reinterpret_cast<const float2*>(src);
 #pragma unroll
                     for (int w = 1; w < NWV; w++) {
-                        const float2 v = *reinterpret_cast<const float2*>(src + w * 32 * 64);
+                        const float2 v = *reinterpret_cast<const float2*>(src + w * SRT);
                         sum.x += v.x;
                         sum.y += v.y;
                     }
@@ -1174,7 +1183,7 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
                 } else {
                     float sum = src[0];
 #pragma unroll
-                    for (int w = 1; w < NWV; w++) sum += src[w * 32 * 64];
+                    for (int w = 1; w < NWV; w++) sum += src[w * SRT];
                     *dst = sum;
                 }
             }
@@ -1184,16 +1193,16 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
         // the wave's use-2 tile to LDS
         auto chunk_mfma = [&](int par, int64_t c, const u32x4 (&ah)[2], const u32x4 (&am)[2],
                               const u32x4 (&al)[2]) {
-            const u32x4* sb = (par ? sB1 : sB0) + g * 3 * 64 + c0 + ln;
+            const u32x4* sb = (par ? sB1 : sB0) + g * 3 * YS + ln;
 #pragma unroll
             for (int r = 0; r < 2; r++) {
 #pragma unroll
                 for (int t = 0; t < NQ; t++) {
                     const u32x4* bb = sb + 16 * t;
                     if (SP == 3)
-                        acc1[r][t] = mfma16_x3(ah[r], am[r], al[r], bb[0], bb[64], bb[128], acc1[r][t]);
+                        acc1[r][t] = mfma16_x3(ah[r], am[r], al[r], bb[0], bb[YS], bb[2 * YS], acc1[r][t]);
                     else
-                        acc1[r][t] = mfma16_a2(ah[r], am[r], bb[0], bb[64], bb[128], acc1[r][t]);
+                        acc1[r][t] = mfma16_a2(ah[r], am[r], bb[0], bb[YS], bb[2 * YS], acc1[r][t]);
                 }
             }
             if (U2) {
@@ -1203,7 +1212,7 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
                 if (SP == 3) t16_transpose(al, esel, tl);
                 // with two buffers, chunk c's tile goes to buffer c & 1, last
                 // read for chunk c-2 before this chunk's barrier
-                float* dst = sR[SRB == 2 ? (c & 1) : 0] + wv * 32 * 64;
+                float* dst = sR[SRB == 2 ? (c & 1) : 0] + wv * SRT;
 #pragma unroll
                 for (int t = 0; t < NQ; t++) {
 #pragma unroll
@@ -1214,7 +1223,7 @@ __global__ __launch_bounds__(64 * NWV) void k_gemm_t16(const float* __restrict__
                         else
                             c2 = mfma16_b2(pah[t], pam[t], pal[t], th[jg], tm[jg], c2);
                         // c2[a]: rhs 16t + 4g + a, column 16*jg + ln
-                        *reinterpret_cast<float4*>(dst + tri_sr_index(16 * jg + ln, 16 * t + 4 * g)) =
+                        *reinterpret_cast<float4*>(dst + tri_sr_index<NQ>(16 * jg + ln, 16 * t + 4 * g)) =
                             make_float4(c2[0], c2[1], c2[2], c2[3]);
                     }
                 }
