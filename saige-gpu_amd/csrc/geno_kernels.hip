@@ -358,18 +358,21 @@ __device__ __forceinline__ float lut_pick(const float4 L, int g) {
 // the markers strictly in order (z*z rounded, then added).  The order makes
 // it a chain of Mqc dependent additions per sample, so what bounds it is the
 // number of instructions a wave issues between two of them.  A workgroup owns
-// 256 samples, one per thread (64 bytes of each marker's row), and walks
-// tiles of DG_MK markers:
-// * the tile's codes go to LDS per sample, a byte for every two markers: their
-//   two codes, times 8;
-// * the tile's squares go to LDS as a 16-entry table (z^2 of the first marker,
-//   z^2 of the second) for every two markers, so that byte is a table offset
-//   and one 8-byte read gives two addends: per two markers a bit-field
-//   extract, the read and two additions.
-// Both are double-buffered and the next tile's loads are in flight while a
-// tile is summed.  Markers past the end have zero tables.  At N = 100,000,
-// M = 150,000: 1.99 ms (15.3 ms with a byte load and two selects per marker
-// and sample); at 1000 x 10,000: 115 us (863 us).
+// 256 samples (64 bytes of each marker's row) and walks tiles of DG_MK markers.
+// Four waves make a tile:
+// * its codes go to LDS per sample, a byte for every two markers: their two
+//   codes, times 8;
+// * its squares go to LDS as a 16-entry table (z^2 of the first marker, z^2 of
+//   the second) for every two markers, so that byte is a table offset and one
+//   8-byte read gives two addends;
+// and four add up the one before it, a sample per thread: per two markers a
+// bit-field extract, the read and two additions, the reads eight pairs ahead so
+// that there is one wait for sixteen additions.  Both are double-buffered and the
+// next tile's loads are in flight while a tile is made.  Markers past the end
+// have zero tables.  1000 x 10,000: 61 us (115 with the same four waves making
+// and adding, 863 with a byte load and two selects per marker and sample);
+// 24,009 x 20,003: 126 us; 100,000 x 150,000: 1.66 ms (1.99, 15.3), where 391
+// workgroups load 256 CUs unevenly.
 constexpr int DG_MK = 128;                       // markers per tile
 constexpr int DG_PITCH = DG_MK / 8 + 4;          // dwords per sample
 constexpr int DG_PLANE = 16 * DG_PITCH + 4;      // samples s, s + 16, ... stand together
@@ -377,13 +380,14 @@ constexpr int DG_PLANE = 16 * DG_PITCH + 4;      // samples s, s + 16, ... stand
 // 16-byte reads (consecutive samples) both spread over all banks
 __device__ __forceinline__ int dg_sample(int s) { return (s & 15) * DG_PLANE + (s >> 4) * DG_PITCH; }
 
-__global__ __launch_bounds__(256) void k_diag_std(const uint8_t* __restrict__ packed,
+__global__ __launch_bounds__(512) void k_diag_std(const uint8_t* __restrict__ packed,
                                                   const float4* __restrict__ lut, int64_t Mqc,
                                                   int64_t Nnm, int64_t ldp,
                                                   float* __restrict__ diag) {
     __shared__ __attribute__((aligned(16))) float2 tab[2][DG_MK / 2 * 16];
     __shared__ __attribute__((aligned(16))) uint32_t cod[2][16 * DG_PLANE];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x & 255;
+    const bool adds = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) == 0;
     const int64_t ntile = (Mqc + DG_MK - 1) / DG_MK;
     // loads: dword column c4 (samples 16*c4 + [0, 16)) of markers 8*mo + [0, 8)
     const int c4 = tid & 15, mo = tid >> 4;
@@ -436,39 +440,65 @@ __global__ __launch_bounds__(256) void k_diag_std(const uint8_t* __restrict__ pa
         }
         left -= DG_MK;
     };
+    if (!adds) {
+        // tile t + 1 is made while tile t is summed; its buffer's last reader
+        // was tile t - 1, before the barrier
+        fetch();
+        put(std::integral_constant<int, 0>());
+        if (ntile > 1) fetch();
+        lds_barrier();
+        auto step = [&](auto nxt, int64_t t) {
+            if (t + 1 < ntile) {
+                put(nxt);
+                if (t + 2 < ntile) fetch();
+            }
+            lds_barrier();
+        };
+        for (int64_t t = 0; t < ntile; t += 2) {
+            step(std::integral_constant<int, 1>(), t);
+            if (t + 1 < ntile) step(std::integral_constant<int, 0>(), t + 1);
+        }
+        return;
+    }
     float d = 0.0f;
     auto sum = [&](auto buf) {
+        constexpr int NG = DG_MK / 16;               // groups of eight pairs
         const uint32_t* cp = cod[buf] + dg_sample(tid);
         const char* tp = reinterpret_cast<const char*>(tab[buf]);
+        uint4 q[2];
+        float2 s[2][8];
+        auto codes = [&](int h) { q[h & 1] = *reinterpret_cast<const uint4*>(cp + 4 * h); };
+        auto read = [&](int g) {
+            const uint4 c = q[(g >> 1) & 1];
+            const uint32_t v[2] = {g & 1 ? c.z : c.x, g & 1 ? c.w : c.y};
 #pragma unroll
-        for (int g = 0; g < DG_MK / 32; g++) {
-            const uint4 q = *reinterpret_cast<const uint4*>(cp + 4 * g);
-            const uint32_t v[4] = {q.x, q.y, q.z, q.w};
-            float2 s[16];
+            for (int u = 0; u < 8; u++)
+                s[g & 1][u] =
+                    *reinterpret_cast<const float2*>(tp + 128 * (8 * g + u) + ((v[u >> 2] >> (8 * (u & 3))) & 255u));
+        };
+        codes(0);
+        codes(1);
+        read(0);
 #pragma unroll
-            for (int u = 0; u < 16; u++)
-                s[u] = *reinterpret_cast<const float2*>(tp + 128 * (16 * g + u) + ((v[u >> 2] >> (8 * (u & 3))) & 255u));
+        for (int g = 0; g < NG; g++) {
+            // the next group's addends are asked for before this one's are added:
+            // one wait a group
+            if (g + 1 < NG) read(g + 1);
+            if ((g & 1) && g / 2 + 2 < NG / 2) codes(g / 2 + 2);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < 16; u++) d = __fadd_rn(__fadd_rn(d, s[u].x), s[u].y);
+            for (int u = 0; u < 8; u++) d = __fadd_rn(__fadd_rn(d, s[g & 1][u].x), s[g & 1][u].y);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // sum tile t from buffer buf while tile t + 1 goes to the other one,
-    // whose last reader was tile t - 1, before the barrier
-    auto step = [&](auto buf, int64_t t) {
-        if (t + 1 < ntile) {
-            put(std::integral_constant<int, 1 - decltype(buf)::value>());
-            if (t + 2 < ntile) fetch();
-        }
-        sum(buf);
-        lds_barrier();
-    };
-    fetch();
-    put(std::integral_constant<int, 0>());
-    if (ntile > 1) fetch();
     lds_barrier();
     for (int64_t t = 0; t < ntile; t += 2) {
-        step(std::integral_constant<int, 0>(), t);
-        if (t + 1 < ntile) step(std::integral_constant<int, 1>(), t + 1);
+        sum(std::integral_constant<int, 0>());
+        lds_barrier();
+        if (t + 1 < ntile) {
+            sum(std::integral_constant<int, 1>());
+            lds_barrier();
+        }
     }
     const int64_t i = (int64_t)blockIdx.x * 256 + tid;
     if (i < Nnm) diag[i] = d;
@@ -633,7 +663,7 @@ hipError_t launch_lut(hipStream_t s, const int32_t* markers, int64_t nmark, cons
 hipError_t launch_diag_std(hipStream_t s, const uint8_t* packed, const float4* lut, int64_t Mqc,
                            int64_t Nnm, int64_t ldp, float* diag) {
     if (Mqc <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_diag_std, dim3((unsigned)((Nnm + 255) / 256)), dim3(256), 0, s, packed, lut,
+    hipLaunchKernelGGL(k_diag_std, dim3((unsigned)((Nnm + 255) / 256)), dim3(512), 0, s, packed, lut,
                        Mqc, Nnm, ldp, diag);
     return hipGetLastError();
 }
