@@ -336,22 +336,29 @@ __global__ __launch_bounds__(512) void k_syrk_pk256(const uint8_t* __restrict__ 
 //   BF16 pipe instead of the FP32 one (1/16 of its rate).  The second term
 //   depends on the column alone: its sum over the markers is formed in FP64
 //   beforehand and taken off at the store (center).
-// Per chunk of BK markers each thread decodes two operand rows' worth of its
-// byte row through two tables (one for SYRK_HI), then every wave adds the
-// products of its block in a fixed order.  LDS: two buffers of the operands
+// Per chunk of BK markers each decoding thread makes two operand rows' worth of
+// its byte row through two tables (one for SYRK_HI), and every multiplying wave
+// adds the products of its block in a fixed order.  LDS: two buffers of the operands
 // (four for the multi-piece forms), so the next chunk's decode runs beside
 // this chunk's MFMAs.  SYRK_SPLIT: threads of the lower half decode the row
 // panel (hi, lo), of the upper half the column panel; SYRK_FP32: the lower
 // half the row operand and the column's lo, the upper half its hi and mid.
 //
-// T: the 256 tile (8 waves of 64 x 128) does the most MFMA work per decoded
-// value and is bound by the matrix pipe and its power (split GRM at N = 40,000:
-// 1380 TFLOP/s of BF16 products); a small GRM has too few of its tiles for 256
-// CUs, each walking all markers, and takes 128 (4 waves of 64 x 64) or 64 (4
-// waves of 32 x 32) tiles, see syrk_pk_tile.  The per-element order is the
-// same for every T: bitwise equal S.
+// T: the 256 tile (8 waves of 64 x 128, each decoding too) does the most MFMA
+// work per decoded value and is bound by the matrix pipe and its power (split GRM
+// at N = 40,000: 1380 TFLOP/s of BF16 products, the clock at 1.6 GHz); a small
+// GRM has too few of its tiles for 256 CUs, each walking all markers, and takes
+// 128 (4 waves of 64 x 64) or 64 (4 waves of 32 x 32) tiles, see syrk_pk_tile.
+// There a wave has a SIMD to itself and issues one instruction in about seven
+// cycles, so the 230 instructions of a chunk's decode took longer than its
+// products: four waves multiply and two groups of four decode, each every other
+// chunk.  us over 8192 markers with every wave doing both and so: one round of 64
+// tiles 130 and 82, of 128 tiles 277 and 195; 2080 of 128 tiles (N = 8000) 1708
+// and 1688.  The per-element order is the same for every T: bitwise equal S.
+constexpr int syrk_pk_threads(int T) { return T == 256 ? 512 : 768; }
+
 template <int T, int F>
-__global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t* __restrict__ tp, int64_t nchunk,
+__global__ __launch_bounds__(syrk_pk_threads(T)) void k_syrk_pk(const uint8_t* __restrict__ tp, int64_t nchunk,
                                                                   int64_t k0, int64_t k1, SyrkTables tb,
                                                                   const int2* __restrict__ tiles, int64_t nblk,
                                                                   float* S, const float* S0, int64_t ldS,
@@ -364,11 +371,12 @@ __global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t*
     constexpr int WC = 2;                            // waves across the tile's columns
     constexpr int MI = T == 64 ? 1 : 2, NI = T == 256 ? 4 : MI;
     constexpr int NPROD = F == SYRK_HI ? 1 : 3;
+    constexpr bool ROLES = T != 256;                 // waves 0 to 3 multiply, two groups of four decode
     __shared__ __attribute__((aligned(16))) __hip_bfloat16 s0[NOP * T * P];
     __shared__ __attribute__((aligned(16))) __hip_bfloat16 s1[NOP * T * P];
     const int2 t = tiles[xcd_remap(blockIdx.x, nblk)];
     const int64_t bi = t.x, bj = t.y;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = ROLES ? threadIdx.x & 255 : threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int wr = wv / WC, wc = wv % WC;
     // half (0, 1), octet and byte row of this thread
     const int h = tid / HALF, o = tid % OCT, b = (tid % HALF) / OCT;
@@ -397,6 +405,7 @@ __global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t*
 
     uint64_t raw0, raw1, l0[8], l1[8];
     auto fetch = [&](int64_t kc) {
+        kc = kc < k1 ? kc : k1 - 1;                  // past the end: the last chunk again, unused
         const int64_t off = BK == 64 ? kc * 256 : (kc >> 1) * 256 + (kc & 1) * 4;
         raw0 = g0[off];
         if (F == SYRK_FP32) raw1 = g1[off];
@@ -407,8 +416,10 @@ __global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t*
             for (int e = 0; e < 8; e++) l1[e] = t1[kc * BK + e];
         }
     };
-    // decode the chunk held in the registers into buffer d, fetching chunk kn
-    auto decode_next = [&](__hip_bfloat16* d, int64_t kn) {
+    // decode the chunk held in the registers, row by row to f(row, its operands),
+    // fetching chunk kn
+    constexpr int NW = F == SYRK_HI ? 1 : 2;         // operands a thread decodes
+    auto decode = [&](int64_t kn, auto f) {
         const uint64_t c0 = raw0, c1 = F == SYRK_FP32 ? raw1 : raw0;
         uint32_t lo0[8], hi0[8], lo1[8], hi1[8];
         split_bytes(l0, lo0, hi0);
@@ -416,9 +427,16 @@ __global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t*
         fetch(kn);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            *reinterpret_cast<u32x4*>(d + dst + j * P) = decode_row_perm(lo0, hi0, c0, j);
-            if (F != SYRK_HI) *reinterpret_cast<u32x4*>(d + dst + OPS + j * P) = decode_row_perm(lo1, hi1, c1, j);
+            const u32x4 v0 = decode_row_perm(lo0, hi0, c0, j);
+            f(j, v0, F != SYRK_HI ? decode_row_perm(lo1, hi1, c1, j) : v0);
         }
+    };
+    auto put_row = [&](__hip_bfloat16* d, int j, u32x4 v0, u32x4 v1) {
+        *reinterpret_cast<u32x4*>(d + dst + j * P) = v0;
+        if (F != SYRK_HI) *reinterpret_cast<u32x4*>(d + dst + OPS + j * P) = v1;
+    };
+    auto decode_to = [&](__hip_bfloat16* d, int64_t kn) {
+        decode(kn, [&](int j, u32x4 v0, u32x4 v1) { put_row(d, j, v0, v1); });
     };
     auto multiply = [&](const __hip_bfloat16* d) {
 #pragma unroll
@@ -466,7 +484,7 @@ __global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t*
     // then its share of the decode's VALU instructions
     auto step = [&](const __hip_bfloat16* cur, __hip_bfloat16* nxt, int64_t kc) {
         constexpr int NM = MI * NI * (BK / 16) * NPROD;
-        decode_next(nxt, kc + 2 < k1 ? kc + 2 : k1 - 1);
+        decode_to(nxt, kc + 2);
         multiply(cur);
 #pragma unroll
         for (int i = 0; i < NM; i++) {
@@ -475,10 +493,60 @@ __global__ __launch_bounds__(T == 256 ? 512 : 256) void k_syrk_pk(const uint8_t*
         }
         lds_barrier();
     };
-    fetch(k0);
-    decode_next(s0, k0 + 1 < k1 ? k0 + 1 : k0);
-    lds_barrier();
     int64_t kc = k0;
+    if constexpr (ROLES) {
+        // one barrier per chunk: chunk kc is multiplied while kc + 1 is put into the
+        // other buffer by the group that decoded it a chunk ago, and the other
+        // group decodes kc + 2
+        u32x4 dec[NW][4];
+        auto hold = [&](int j, u32x4 v0, u32x4 v1) {
+            dec[0][j] = v0;
+            if (F != SYRK_HI) dec[NW - 1][j] = v1;
+        };
+        auto put = [&](__hip_bfloat16* d) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) put_row(d, j, dec[0][j], dec[NW - 1][j]);
+        };
+        const int role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+        if (role == 1) {
+            fetch(k0);
+            decode_to(s0, k0 + 2);
+            lds_barrier();
+            for (; kc + 2 <= k1; kc += 2) {
+                decode(kc + 4, hold);
+                lds_barrier();
+                put(s0);
+                lds_barrier();
+            }
+            return;
+        }
+        if (role == 2) {
+            fetch(k0 + 1);
+            decode(k0 + 3, hold);
+            lds_barrier();
+            for (; kc + 2 <= k1; kc += 2) {
+                put(s1);
+                lds_barrier();
+                decode(kc + 5, hold);
+                lds_barrier();
+            }
+            return;
+        }
+        lds_barrier();
+        for (; kc + 2 <= k1; kc += 2) {
+            multiply(s0);
+            lds_barrier();
+            multiply(s1);
+            lds_barrier();
+        }
+        if (kc < k1) multiply(s0);
+        store_block<MI, NI, F == SYRK_SPLIT>(S, S0, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane,
+                                             acc, accumulate, F == SYRK_FP32 ? tb.center : nullptr);
+        return;
+    }
+    fetch(k0);
+    decode_to(s0, k0 + 1);
+    lds_barrier();
     for (; kc + 2 <= k1; kc += 2) {
         step(s0, s1, kc);
         step(s1, s0, kc + 1);
@@ -738,7 +806,7 @@ static void launch_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, 
                       int accumulate) {
     constexpr int BK = T == 64 ? 64 : 32;
     const int64_t nt = op.Npad / T, nblk = nt * (nt + 1) / 2;
-    hipLaunchKernelGGL((k_syrk_pk<T, F>), dim3((unsigned)nblk), dim3(T == 256 ? 512 : 256), 0, s, op.tp, op.nchunk,
+    hipLaunchKernelGGL((k_syrk_pk<T, F>), dim3((unsigned)nblk), dim3(syrk_pk_threads(T)), 0, s, op.tp, op.nchunk,
                        (int64_t)0, op.nchunk * (64 / BK), op.tb, tiles, nblk, S, S0, op.Npad, accumulate);
 }
 
@@ -782,23 +850,22 @@ hipError_t launch_grm_block(hipStream_t s, const float* S, int64_t ld, int64_t n
 }
 
 // Tile edge of the 2-bit-input SYRK at Npad rows (every size gives the same
-// bits): the one of least time by a model of rounds on 256 CUs, in us for the
-// split form over 8192 markers.  A 256 tile fills a CU and takes 525 us
-// whatever their number up to 256; two 128 tiles share a CU (390 us; 290 us
-// alone); 64 tiles run at 0.36 us each, at least 130 us.  Measured us at
-// N = 1000, 2000, 3000, 4000, 8000, 20,000: 64 tiles 144, 292, 454, 726, 2477,
-// 13,996; 128 tiles 293, 301, 394, 644, 1708, 9335; 256 tiles 534, 538, 548,
-// 556, 1745, 8053; the other forms cross at the same places.
+// bits): the one of least time by a model of rounds of one tile per CU, in us
+// over 8192 markers.  Measured us with 64, 128 and 256 tiles, split form: N = 1000
+// 82, 171, 522; 1500 163, 185, 523; 2500 335, 195, 524; 3000 418, 367, 525; 4000
+// 746, 574, 558; 5000 1031, 735, 574; 8000 2554, 1688, 1749; 12,000 5726, 3367,
+// 3026; SYRK_FP32 within 5% of it; SYRK_HI: 1000 47, 87, 167; 2500 152, 94, 173;
+// 3000 196, 182, 177; 4000 352, 276, 180; 8000 1117, 804, 616.
 // SAIGE_SYRK_TILE=64, 128 or 256 sets it (the tests compare them).
-int syrk_pk_tile(int64_t Npad) {
+int syrk_pk_tile(int64_t Npad, int form) {
     if (const char* env = std::getenv("SAIGE_SYRK_TILE")) {
         const int t = std::atoi(env);
         if (t == 64 || t == BT || t == BT2) return t;
     }
-    auto tiles = [&](int64_t T) { return (double)(Npad / T) * (double)(Npad / T + 1) / 2.0; };
-    const double t256 = 525.0 * std::ceil(tiles(256) / 256.0);
-    const double t128 = tiles(128) <= 256.0 ? 290.0 : 390.0 * std::ceil(tiles(128) / 512.0);
-    const double t64 = std::max(130.0, 60.0 + 0.36 * tiles(64));
+    auto rounds = [&](int64_t T) { return std::ceil((double)(Npad / T) * (double)(Npad / T + 1) / 512.0); };
+    const bool hi = form == SYRK_HI;
+    const double t64 = (hi ? 47.0 : 82.0) * rounds(64), t128 = (hi ? 92.0 : 190.0) * rounds(BT);
+    const double r256 = rounds(BT2), t256 = hi ? (r256 > 1 ? 200.0 : 178.0) * r256 : (r256 > 1 ? 580.0 : 545.0) * r256;
     if (t256 <= t128 && t256 <= t64) return BT2;
     return t128 <= t64 ? BT : 64;
 }

@@ -1129,7 +1129,7 @@ hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1,
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad;
     const int form = precision == SAIGE_GRM_FP32 ? SYRK_FP32 : (precision == SAIGE_GRM_BF16_SPLIT ? SYRK_SPLIT : SYRK_HI);
-    const int tile = syrk_pk_tile(Np);
+    const int tile = syrk_pk_tile(Np, form);
     // super-blocks of 1024 rows in the dispatch order
     const std::vector<int2> order = syrk_tile_order(Np / tile, 1024 / tile);
     SyrkOperands op;

@@ -415,7 +415,7 @@ std::vector<int2> syrk_tile_order(int64_t nt, int64_t g);
 // symmetric.
 hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, const float* S0,
                           int accumulate, int tile);
-int syrk_pk_tile(int64_t Npad);
+int syrk_pk_tile(int64_t Npad, int form);
 // copy each diagonal tile's lower half onto its upper half (tile edge `tile`)
 hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile);
 // out[nr][nc] (contiguous) = S[i][j] / m for S at its block's first element
