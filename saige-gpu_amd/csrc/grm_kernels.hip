@@ -1,7 +1,9 @@
-// GRM SYRK on CDNA4 matrix cores: S (+)= Zp Zp^T for one marker panel.
+// GRM SYRK on CDNA4 matrix cores: S = Z Z^T from the 2-bit genotypes
+// (k_syrk_pk256, k_syrk_pk), or S (+)= Zp Zp^T for one marker panel
+// (k_syrk_bf16).
 //
-// Zp is the standardised panel, [Npad][ldz] row-major (sample rows, marker
-// columns), so both MFMA operands are K-contiguous rows of the same matrix.
+// Both MFMA operands are marker-contiguous rows of the same matrix of
+// standardised genotypes.
 // Each workgroup computes one tile of the lower triangle (tile row >= tile
 // column) and writes it and its mirror into the full row-major S.
 // Tile order: the host lists the triangle's tiles grouped into 8x8-tile
@@ -11,8 +13,8 @@
 // i.e. 16-24 distinct 128-row panels of Zp, whose current K chunk fits in
 // that XCD's 4 MB L2.
 //
-// Operand staging: global -> registers (prefetch of the next K chunk while
-// the current one is multiplied) -> LDS -> MFMA fragments.
+// Operand staging: global -> registers (the next K chunk while the current one
+// is multiplied; decoded there from 2 bits) -> LDS -> MFMA fragments.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>

@@ -1,15 +1,16 @@
 // PCG kernels on the resident GRM S = Z Z^T (K = S / Mqc).
 //
-// Column blocks are [Npad][kpad] row-major (kpad = 1 for the plain
-// single-RHS path, 64 for the block path).  Rows >= Nnm are zero in every
-// vector and in S, so padded rows never contribute.
+// Column blocks are [Npad][64] row-major, a single column is [Npad].  Rows >=
+// Nnm are zero in every vector and in S, so padded rows never contribute.
 //
 // Products:
-//   k_gemv  (kpad 1): one wave per row, float4 streaming of S; FP32 dot.
-//   k_gemm  (kpad 64): FP32 MFMA 32x32x2; a workgroup owns 128 rows x 64
-//                      columns and walks the full row panel of S, so S is
-//                      read from HBM exactly once per product.
-// Both fuse the Sigma epilogue of getCrossprod (FG.cpp:2397-2425):
+//   one column: k_gemv_tri24 / k_gemv_tri over the lower triangle (24-bit or
+//     FP32), or k_gemv over all of S;
+//   64 columns: k_gemm_t16 over the lower triangle (k_gemm_flat at few rows),
+//     k_gemm_x3 / k_gemm_x3w over all of S, on the BF16 MFMA; k_gemm_part and
+//     k_gemm_half on the FP32 MFMA.
+// Their epilogues (k_gemv*, k_gemm_epi) are the Sigma part of getCrossprod
+// (FG.cpp:2397-2425):
 //   Ap = tau0 * (p * (1/w)) + tau1 * ((S p) / Mqc), masked to the system's
 //   samples, and emit per-workgroup FP64 partials of p^T Ap.
 // Reductions of partials always run in one fixed order, so a column's

@@ -123,7 +123,7 @@ struct GemmConfig {
     int mode = GEMM_FP32;
 };
 
-// The width-1 solver's device state and what it publishes to the host
+// The single-right-hand-side solver's device state and what it publishes to the host
 // (page-locked, coherent): the iteration last decided, the iteration count and
 // whether the solve is over.
 struct P1State {
