@@ -62,10 +62,18 @@ __device__ __forceinline__ float round16(float x) {
 // by its bytes (S0's triangle read, S written): 1000 of 20,000 markers left out
 // at N = 20,000 take 1.54 ms; a copy of S first and requests at their use took
 // 2.7.
+// R16 and s24: each 32 x 32 block of the lower triangle is also stored in three
+// bytes a value (s24_block), turned in the wave's scratch (S24_SCRATCH floats of
+// LDS); beside a whole build's products this costs nothing that shows, a pass of
+// its own over S took 1.07 ms at N = 40,000 and 6.7 ms at 100,000.
+constexpr int S24_PITCH = 36;
+constexpr int S24_SCRATCH = 32 * S24_PITCH;
+
 template <int MI, int NI, bool R16>
 __device__ __forceinline__ void store_block(float* S, const float* S0, int64_t ldS, int64_t row0, int64_t col0,
                                             bool mirror, int lane, const f32x16 (&acc)[MI][NI], int accumulate,
-                                            const float* center = nullptr) {
+                                            const float* center = nullptr, uint8_t* s24 = nullptr,
+                                            float* scratch = nullptr) {
     float s0[2][16];
     auto request = [&](int k) {
         const float* p = S0 + (row0 + k / NI * 32 + 4 * (lane >> 5)) * ldS + col0 + k % NI * 32 + (lane & 31);
@@ -95,6 +103,38 @@ __device__ __forceinline__ void store_block(float* S, const float* S0, int64_t l
             if (mirror) {
                 float4* dst = reinterpret_cast<float4*>(S + col * ldS + row);
                 *dst = make_float4(v[0], v[1], v[2], v[3]);
+            }
+            if constexpr (R16) {
+                if (s24) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        scratch[(8 * g + 4 * (lane >> 5) + e) * S24_PITCH + (lane & 31)] = v[e];
+                }
+            }
+        }
+        if constexpr (R16) {
+            const int64_t I = row0 / 32 + mi, J = col0 / 32 + ni;
+            if (s24 && J < I) {
+                const int ln = lane & 15, o = lane >> 4;
+                u32x4* dst = reinterpret_cast<u32x4*>(s24 + s24_block(I, J) * S24_BLOCK) + lane;
+                u32x4 lo;
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    const u32x4* p = reinterpret_cast<const u32x4*>(scratch + (16 * r + ln) * S24_PITCH + 8 * o);
+                    const u32x4 a = p[0], b = p[1];
+                    // upper halves; then byte 1 of two words each
+                    dst[64 * r] = u32x4{__builtin_amdgcn_perm(a[1], a[0], 0x07060302u),
+                                        __builtin_amdgcn_perm(a[3], a[2], 0x07060302u),
+                                        __builtin_amdgcn_perm(b[1], b[0], 0x07060302u),
+                                        __builtin_amdgcn_perm(b[3], b[2], 0x07060302u)};
+                    lo[2 * r] = __builtin_amdgcn_perm(a[1], a[0], 0x0C0C0501u) |
+                                (__builtin_amdgcn_perm(a[3], a[2], 0x0C0C0501u) << 16);
+                    lo[2 * r + 1] = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0501u) |
+                                    (__builtin_amdgcn_perm(b[3], b[2], 0x0C0C0501u) << 16);
+                }
+                dst[128] = lo;
+                __builtin_amdgcn_wave_barrier();
             }
         }
     }
@@ -364,7 +404,7 @@ __global__ __launch_bounds__(syrk_pk_threads(T)) void k_syrk_pk(const uint8_t* _
                                                                   int64_t k0, int64_t k1, SyrkTables tb,
                                                                   const int2* __restrict__ tiles, int64_t nblk,
                                                                   float* S, const float* S0, int64_t ldS,
-                                                                  int accumulate) {
+                                                                  int accumulate, uint8_t* __restrict__ s24) {
     constexpr int BK = T == 64 ? 64 : 32;            // markers per chunk
     constexpr int P = BK + 8;                        // LDS row pitch (bf16 elements), conflict-free 16-byte reads
     constexpr int NOP = F == SYRK_HI ? 2 : 4;        // operands in LDS
@@ -495,6 +535,14 @@ __global__ __launch_bounds__(syrk_pk_threads(T)) void k_syrk_pk(const uint8_t* _
         }
         lds_barrier();
     };
+    // s1 is the waves' scratch: after the last chunk but one (behind its barrier)
+    // nothing reads or writes it
+    static_assert(sizeof(s1) >= sizeof(float) * S24_SCRATCH * (T == 256 ? 8 : 4), "");
+    auto store = [&]() {
+        store_block<MI, NI, F == SYRK_SPLIT>(S, S0, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane,
+                                             acc, accumulate, F == SYRK_FP32 ? tb.center : nullptr, s24,
+                                             reinterpret_cast<float*>(s1) + wv * S24_SCRATCH);
+    };
     int64_t kc = k0;
     if constexpr (ROLES) {
         // one barrier per chunk: chunk kc is multiplied while kc + 1 is put into the
@@ -542,8 +590,7 @@ __global__ __launch_bounds__(syrk_pk_threads(T)) void k_syrk_pk(const uint8_t* _
             lds_barrier();
         }
         if (kc < k1) multiply(s0);
-        store_block<MI, NI, F == SYRK_SPLIT>(S, S0, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane,
-                                             acc, accumulate, F == SYRK_FP32 ? tb.center : nullptr);
+        store();
         return;
     }
     fetch(k0);
@@ -554,8 +601,7 @@ __global__ __launch_bounds__(syrk_pk_threads(T)) void k_syrk_pk(const uint8_t* _
         step(s1, s0, kc + 1);
     }
     if (kc < k1) multiply(s0);
-    store_block<MI, NI, F == SYRK_SPLIT>(S, S0, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane, acc,
-                                         accumulate, F == SYRK_FP32 ? tb.center : nullptr);
+    store();
 }
 
 // Re-tile the packed genotypes for the SYRK: block (p, c) byte (b, m) = byte
@@ -805,15 +851,16 @@ void SyrkOperands::release() {
 
 template <int T, int F>
 static void launch_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, const float* S0,
-                      int accumulate) {
+                      int accumulate, uint8_t* s24 = nullptr) {
     constexpr int BK = T == 64 ? 64 : 32;
     const int64_t nt = op.Npad / T, nblk = nt * (nt + 1) / 2;
     hipLaunchKernelGGL((k_syrk_pk<T, F>), dim3((unsigned)nblk), dim3(syrk_pk_threads(T)), 0, s, op.tp, op.nchunk,
-                       (int64_t)0, op.nchunk * (64 / BK), op.tb, tiles, nblk, S, S0, op.Npad, accumulate);
+                       (int64_t)0, op.nchunk * (64 / BK), op.tb, tiles, nblk, S, S0, op.Npad, accumulate,
+                       s24);
 }
 
 hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, const float* S0,
-                          int accumulate, int tile) {
+                          int accumulate, int tile, uint8_t* s24) {
     if ((tile != 64 && tile != BT && tile != BT2) || op.Npad % tile != 0 || !op.block) return hipErrorInvalidValue;
     if (op.form == SYRK_HI && tile == BT2) {
         const int64_t nt = op.Npad / BT2, nblk = nt * (nt + 1) / 2;
@@ -823,9 +870,9 @@ hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* til
         if (tile == BT) launch_pk<128, SYRK_HI>(s, op, tiles, S, S0, accumulate);
         else launch_pk<64, SYRK_HI>(s, op, tiles, S, S0, accumulate);
     } else if (op.form == SYRK_SPLIT) {
-        if (tile == BT2) launch_pk<256, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate);
-        else if (tile == BT) launch_pk<128, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate);
-        else launch_pk<64, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate);
+        if (tile == BT2) launch_pk<256, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate, s24);
+        else if (tile == BT) launch_pk<128, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate, s24);
+        else launch_pk<64, SYRK_SPLIT>(s, op, tiles, S, S0, accumulate, s24);
     } else {
         if (tile == BT2) launch_pk<256, SYRK_FP32>(s, op, tiles, S, S0, accumulate);
         else if (tile == BT) launch_pk<128, SYRK_FP32>(s, op, tiles, S, S0, accumulate);

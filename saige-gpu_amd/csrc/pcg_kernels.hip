@@ -38,18 +38,7 @@ __device__ __forceinline__ float wave_sum_f(float v) {
 }
 
 // ------------------------------------------------------- 24-bit triangle
-// A value of at most 16 significant bits (the split GRM's storage) has its
-// low 8 FP32 bits zero: three bytes hold it.  The products that stream the
-// lower triangle are bound by its bytes, so they read it in this form where
-// it is there (15 GB instead of 20 at N = 100,000): 32 x 32 blocks (I, J),
-// J < I, of 3 KB each, block (I, J) at I (I - 1) / 2 + J, so that a strip of 32
-// rows is one contiguous stream.  Within a block lane (ln = l % 16, g = l / 16)
-// owns rows 16 r + ln (r = 0, 1), columns 8 g + [0, 8), the layout of the MFMA
-// operands: [r][lane] 16 bytes, the upper halves of its eight words (the first
-// BF16 piece by truncation, as it stands), then [lane] 16 bytes, the third byte
-// of the eight words of r = 0 and of r = 1.
-constexpr int64_t S24_BLOCK = 3072;
-__host__ __device__ __forceinline__ int64_t s24_block(int64_t I, int64_t J) { return I * (I - 1) / 2 + J; }
+// The layout is at s24_block.
 
 // elements 2k and 2k + 1 (k < 4) of a lane's row from h[k] and their third bytes
 // in l[k / 2]
@@ -58,31 +47,6 @@ __device__ __forceinline__ uint32_t s24_lo(u32x4 h, const uint32_t (&l)[2], int 
 }
 __device__ __forceinline__ uint32_t s24_hi(u32x4 h, const uint32_t (&l)[2], int k) {
     return __builtin_amdgcn_perm(h[k], l[k >> 1], 0x0706000Cu | (uint32_t)((2 * (k & 1) + 1) << 8));
-}
-
-// k_pack24: one wave per block of the FP32 triangle.  Reads 20 GB and writes 15
-// GB at N = 100,000: 6.7 ms, 5.2 TB/s.
-__global__ __launch_bounds__(256) void k_pack24(const float* __restrict__ S, int64_t ld, uint8_t* __restrict__ out) {
-    const int lane = threadIdx.x & 63, ln = lane & 15, g = lane >> 4;
-    const int64_t I = blockIdx.y + 1;
-    const int64_t J = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (J >= I) return;
-    u32x4* dst = reinterpret_cast<u32x4*>(out + s24_block(I, J) * S24_BLOCK);
-    u32x4 lo;
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-        const float* p = S + (32 * I + 16 * r + ln) * ld + 32 * J + 8 * g;
-        const u32x4 a = *reinterpret_cast<const u32x4*>(p), b = *reinterpret_cast<const u32x4*>(p + 4);
-        const u32x4 h = {__builtin_amdgcn_perm(a[1], a[0], 0x07060302u), __builtin_amdgcn_perm(a[3], a[2], 0x07060302u),
-                         __builtin_amdgcn_perm(b[1], b[0], 0x07060302u), __builtin_amdgcn_perm(b[3], b[2], 0x07060302u)};
-        // byte 1 of four words
-        const uint32_t a01 = __builtin_amdgcn_perm(a[1], a[0], 0x0C0C0501u), a23 = __builtin_amdgcn_perm(a[3], a[2], 0x0C0C0501u);
-        const uint32_t b01 = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0501u), b23 = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0501u);
-        lo[2 * r] = a01 | (a23 << 16);
-        lo[2 * r + 1] = b01 | (b23 << 16);
-        dst[64 * r + lane] = h;
-    }
-    dst[128 + lane] = lo;
 }
 
 // --------------------------------------------------------------- GEMV
@@ -2029,13 +1993,6 @@ int64_t gemm_max_parts(int64_t Npad) { return Npad / EROWS; }
 int64_t vec_max_parts(int64_t Npad, int) { return Npad / VROWS; }
 
 int64_t s24_bytes(int64_t Npad) { return s24_block(Npad / 32, 0) * S24_BLOCK; }
-
-hipError_t launch_pack24(hipStream_t s, const float* S, int64_t Npad, uint8_t* out) {
-    const int64_t nb = Npad / 32;
-    if (nb < 2) return hipSuccess;
-    hipLaunchKernelGGL(k_pack24, dim3((unsigned)((nb + 2) / 4), (unsigned)(nb - 1)), dim3(256), 0, s, S, Npad, out);
-    return hipGetLastError();
-}
 
 hipError_t launch_grm_gemv(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, const float* in,
                            float* out, VecArgs a, double* partial, int64_t* nparts, const GemvPlan* tri) {

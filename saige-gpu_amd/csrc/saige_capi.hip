@@ -259,33 +259,29 @@ GrmView grm_view(const saige_ctx* c, int loco) {
     return {{c->d_grm, s16, c->s24_ok ? c->d_s24 : nullptr}, c->d_diag, c->Mqc, c->diag_one};
 }
 
-// Makes the 24-bit triangle of a split GRM when its bytes leave room for
-// everything else a cohort of this size may take: a second GRM (leave one
-// chromosome out) and the products' scratch, a quarter of a GRM at most, and 8
-// GB.  Without it the products read the FP32 triangle.  Asynchronous on the
-// context's stream.
-hipError_t make_s24(saige_ctx* c) {
+// Device memory for a GRM's 24-bit triangle, or null: only for the split form,
+// and when its bytes leave room for everything else a cohort of this size may
+// take: a second GRM (leave one chromosome out) and the products' scratch, a
+// quarter of a GRM at most, and 8 GB.  Without it the products read the FP32
+// triangle.  What it holds is not valid until the caller sets s24_ok.
+uint8_t* reserve_s24(saige_ctx* c, int precision) {
     c->s24_ok = false;
-    if (c->grm_precision != SAIGE_GRM_BF16_SPLIT) {
+    if (precision != SAIGE_GRM_BF16_SPLIT) {
         dfree(c->d_s24);
-        return hipSuccess;
+        return nullptr;
     }
     const int64_t bytes = s24_bytes(c->Npad), grm = 4 * c->Npad * c->Npad;
-    if (bytes == 0) return hipSuccess;
     if (!c->d_s24) {
         size_t free_b = 0, total_b = 0;
-        const hipError_t e = hipMemGetInfo(&free_b, &total_b);
-        if (e != hipSuccess) return e;
-        if ((int64_t)free_b < bytes + grm + grm / 4 + ((int64_t)8 << 30)) return hipSuccess;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess ||
+            (int64_t)free_b < bytes + grm + grm / 4 + ((int64_t)8 << 30))
+            return nullptr;
         if (dalloc(&c->d_s24, bytes) != hipSuccess) {
             (void)hipGetLastError();
             c->d_s24 = nullptr;
-            return hipSuccess;
         }
     }
-    const hipError_t e = launch_pack24(c->stream, c->d_grm, c->Npad, c->d_s24);
-    c->s24_ok = e == hipSuccess;
-    return e;
+    return c->d_s24;
 }
 
 int check_loco(const saige_ctx* c) {
@@ -1122,10 +1118,11 @@ int saige_get_diag_of_kin(saige_ctx* c, float* out) {
 namespace {
 // S = (nothing, S0 plus, S0 minus) the GRM part of markers [j0, j1) from the
 // 2-bit genotypes, in the operand form of `precision` (accumulate: 0, 1, -1; S0
-// may be S).  Waits for the stream; t (may be null): device seconds between its
-// start and end.
+// may be S).  s24 (may be null): the 24-bit triangle of a split S, written too.
+// Waits for the stream; t (may be null): device seconds between its start and
+// end.
 hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1, float* S, const float* S0,
-                            int accumulate, double* t) {
+                            int accumulate, double* t, uint8_t* s24) {
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad;
     const int form = precision == SAIGE_GRM_FP32 ? SYRK_FP32 : (precision == SAIGE_GRM_BF16_SPLIT ? SYRK_SPLIT : SYRK_HI);
@@ -1139,7 +1136,7 @@ hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1,
         e = hipMemcpyAsync(d_tiles, order.data(), sizeof(int2) * order.size(), hipMemcpyHostToDevice, st);
     if (e == hipSuccess && t) e = hipEventRecord(c->ev0, st);
     if (e == hipSuccess) e = op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j0, j1);
-    if (e == hipSuccess) e = launch_syrk_pk(st, op, d_tiles, S, S0, accumulate, tile);
+    if (e == hipSuccess) e = launch_syrk_pk(st, op, d_tiles, S, S0, accumulate, tile, s24);
     if (e == hipSuccess && t) e = hipEventRecord(c->ev1, st);
     const hipError_t w = hipStreamSynchronize(st);
     if (e == hipSuccess) e = w;
@@ -1179,10 +1176,10 @@ int saige_build_grm(saige_ctx* c, int precision) {
     c->loco_inplace = false;
     if (precision != SAIGE_GRM_BF16_PANEL) {
         // 2-bit operands straight into the MFMA SYRK: no Z panel
-        hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, nullptr, 0, &c->grm_seconds);
+        uint8_t* s24 = reserve_s24(c, precision);
+        const hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, nullptr, 0, &c->grm_seconds, s24);
         c->grm_precision = precision;
-        if (e == hipSuccess) e = make_s24(c);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        c->s24_ok = e == hipSuccess && s24;
         if (e != hipSuccess) {
             set_error("GRM build failed: %s", hipGetErrorString(e));
             return e == hipErrorOutOfMemory ? SAIGE_E_NOMEM : SAIGE_E_DEVICE;
@@ -1190,8 +1187,7 @@ int saige_build_grm(saige_ctx* c, int precision) {
         c->grm_ready = true;
         return SAIGE_OK;
     }
-    c->s24_ok = false;
-    dfree(c->d_s24);
+    reserve_s24(c, precision);       // none for panels
     const int64_t kc = syrk_kchunk_bf16();
     size_t free_b = 0, total_b = 0;
     SAIGE_HIP_TRY(hipMemGetInfo(&free_b, &total_b));
@@ -1522,10 +1518,11 @@ int saige_pcg_block(saige_ctx* c, const float* w, const float* tau, const float*
 namespace {
 // S = S0 (+/-) Z_r Z_r^T over GRM markers [start, end], with the kernel and
 // operand precision the resident S was built with (accumulate: 1 add, -1
-// subtract; S0 may be S).
-hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, const float* S0, int accumulate) {
+// subtract; S0 may be S); s24 as in syrk_from_packed.
+hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, const float* S0, int accumulate,
+                      uint8_t* s24 = nullptr) {
     if (c->grm_precision != SAIGE_GRM_BF16_PANEL)
-        return syrk_from_packed(c, c->grm_precision, start, end + 1, S, S0, accumulate, nullptr);
+        return syrk_from_packed(c, c->grm_precision, start, end + 1, S, S0, accumulate, nullptr, s24);
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
     if (S != S0) {                   // the panels add to S one after another
@@ -1570,10 +1567,12 @@ static int restore_full_grm(saige_ctx* c) {
                 set_error("live LOCO slots use the in-place LOCO GRM; take them before using the full GRM");
                 return SAIGE_E_STATE;
             }
-    hipError_t e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, c->d_grm, 1);
-    // the sums may differ from the first build's in the last bit
-    if (e == hipSuccess) e = make_s24(c);
+    // the sums may differ from the first build's in the last bit, so the 24-bit
+    // triangle is made anew
+    uint8_t* s24 = reserve_s24(c, c->grm_precision);
+    hipError_t e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, c->d_grm, 1, s24);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    c->s24_ok = e == hipSuccess && s24;
     if (e != hipSuccess) {
         set_error("restoring the GRM after an in-place LOCO range failed: %s", hipGetErrorString(e));
         return SAIGE_E_DEVICE;

@@ -293,7 +293,7 @@ struct saige_ctx {
     float* d_diag = nullptr;                     // [Npad] sum z^2
     // GRM S = Z Z^T, [Npad][Npad] FP32
     float* d_grm = nullptr;
-    // the split GRM's lower triangle in three bytes a value (launch_pack24), when
+    // the split GRM's lower triangle in three bytes a value (s24_block), when
     // there is room for it; s24_ok: it holds d_grm's present values
     uint8_t* d_s24 = nullptr;
     bool s24_ok = false;
@@ -409,12 +409,25 @@ hipError_t launch_std_panel_bf16(hipStream_t s, const uint8_t* packed, const flo
 hipError_t launch_syrk_bf16(hipStream_t s, const __hip_bfloat16* Zp, int64_t Npad, int64_t ldz,
                             int64_t kdim, const int2* tiles, float* S, int accumulate);
 std::vector<int2> syrk_tile_order(int64_t nt, int64_t g);
+// A value of at most 16 significant bits (the split GRM's storage) has its
+// low 8 FP32 bits zero: three bytes hold it.  The products that stream the
+// lower triangle are bound by its bytes, so they read it in this form where
+// it is there (15 GB instead of 20 at N = 100,000): 32 x 32 blocks (I, J),
+// J < I, of 3 KB each, block (I, J) at I (I - 1) / 2 + J, so that a strip of 32
+// rows is one contiguous stream.  Within a block lane (ln = l % 16, g = l / 16)
+// owns rows 16 r + ln (r = 0, 1), columns 8 g + [0, 8), the layout of the MFMA
+// operands: [r][lane] 16 bytes, the upper halves of its eight words (the first
+// BF16 piece by truncation, as it stands), then [lane] 16 bytes, the third byte
+// of the eight words of r = 0 and of r = 1.
+constexpr int64_t S24_BLOCK = 3072;
+__host__ __device__ __forceinline__ int64_t s24_block(int64_t I, int64_t J) { return I * (I - 1) / 2 + J; }
+
 // the 2-bit-input SYRK of op on T x T tiles (64, 128 or 256; tiles from
 // syrk_tile_order(Npad / tile, ...)); accumulate: 0 overwrite, 1 S = S0 + the
 // product, -1 S = S0 - the product (S0 may be S).  S comes out exactly
-// symmetric.
+// symmetric.  s24 (split form; or null): S's lower triangle in three bytes too.
 hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, const float* S0,
-                          int accumulate, int tile);
+                          int accumulate, int tile, uint8_t* s24);
 int syrk_pk_tile(int64_t Npad, int form);
 // copy each diagonal tile's lower half onto its upper half (tile edge `tile`)
 hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile);
@@ -450,10 +463,9 @@ struct GrmMat {
     // storage): the lower-triangle block product then splits S into two BF16
     // pieces instead of three, with the same bits
     bool s16 = false;
-    const uint8_t* s24 = nullptr;    // such an S's lower triangle in three bytes a value (launch_pack24), or null
+    const uint8_t* s24 = nullptr;    // such an S's lower triangle in three bytes a value (s24_block), or null
 };
 int64_t s24_bytes(int64_t Npad);
-hipError_t launch_pack24(hipStream_t s, const float* S, int64_t Npad, uint8_t* out);
 
 // arguments of a single-column product's epilogue
 struct VecArgs {

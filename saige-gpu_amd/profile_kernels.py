@@ -9,7 +9,7 @@ and HBM counters (FETCH_SIZE, WRITE_SIZE) of each can be read per dispatch:
 
 Kernels exercised: decode/QC (k_decode_stats), repack, diag, the GRM SYRK
 (2-bit input k_syrk_pk256 for --grm bf16; k_syrk_pk<256, SYRK_SPLIT>, hi.hi +
-hi.lo + lo.hi from two tables, k_mirror_diag and k_pack24 for bf16_split; --grm takes a
+hi.lo + lo.hi from two tables, and k_mirror_diag for bf16_split; --grm takes a
 comma-separated list, built in turn, the last one resident), the
 autotuner's block-GEMM shapes, the tuned 64-column block GEMM (k_split_p +
 k_gemm_t16 + k_tri_reduce + k_gemm_epi in the default --gemm-mode

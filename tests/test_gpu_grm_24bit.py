@@ -12,10 +12,11 @@ from fixtures import random_bed
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N", [200, 257, 513, 2305, 7200])
-def test_three_byte_triangle(session, monkeypatch, N):
+@pytest.mark.parametrize("N,tile", [(200, "64"), (257, "128"), (513, "64"), (513, "256"), (2305, "128"), (7200, "256")])
+def test_three_byte_triangle(session, monkeypatch, N, tile):
     M = 320
-    print(f"case: three-byte triangle N={N}", flush=True)
+    monkeypatch.setenv("SAIGE_SYRK_TILE", tile)
+    print(f"case: three-byte triangle N={N} tile={tile}", flush=True)
     body, _, _ = random_bed(N, M, 0.01, seed=N, maf_lo=0.05, maf_hi=0.5)
     session.setminMAFforGRM(0.01)
     session.setmaxMissingRateforGRM(0.15)
