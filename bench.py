@@ -39,15 +39,18 @@ FP32_MFMA_PEAK = 157.3
 # (mode, N, rt, pd, nsplit).  Sources: PROFILE_FILES
 PROFILED_GEMM_TRAFFIC = {("fp32", 100_000, 1, 3, 8): (42.10 + 0.205 + 0.108 + 0.026) * 1e9,
                          ("bf16x3", 100_000, 1, 3, 8): (0.064 + 41.579 + 0.152) * 1e9,
-                         # lower triangle on 16x16 tiles, on the split GRM (two pieces of
-                         # S): all four kernels of a launch (pd 3 spills)
-                         ("bf16x3_tri", 100_000, 1, 1, 8): (25.27 + 4.08) * 1e9,
-                         ("bf16x3_tri", 100_000, 2, 1, 8): (26.63 + 5.54) * 1e9,
-                         ("bf16x3_tri", 100_000, 1, 3, 8): (46.77 + 6.12) * 1e9,
-                         ("bf16x3_tri", 100_000, 2, 3, 8): (29.99 + 9.17) * 1e9}
+                         # lower triangle on 16x16 tiles, on the split GRM's three-byte
+                         # copy: all four kernels of a launch
+                         ("bf16x3_tri", 100_000, 1, 1, 8): (16.15 + 3.79 + 0.05 + 4.01 + 0.09) * 1e9}
 PROFILE_FILES = {"fp32": "profiles/kernels_N100k_M150k_bf16.md", "bf16x3": "profiles/gemm_bf16x3_N100k_M150k.md",
-                 "bf16x3_tri": "profiles/kernels_N100k_M150k_split_grm.md"}
+                 "bf16x3_tri": "profiles/kernels_cases.md"}
 BF16_MFMA_PEAK = 2500.0
+
+
+def tri_bytes(grm_precision):
+    """Bytes of S's lower triangle over N^2: two values of four bytes per pair,
+    or, on the split GRM where its copy fits the device (N = 100k), of three."""
+    return 1.5 if grm_precision == "bf16_split" else 2.0
 
 
 def log(*a):
@@ -632,9 +635,10 @@ def main():
         plain_s = time.perf_counter() - tp
         g3, n3 = sess.engine_stats("gemv")
         gemv_avg = (g3 - g2) / max(1, n3 - n2)
-        # GB/s of S the product needs: its lower triangle (2 N^2 bytes) in the
-        # default mode, all of it (4 N^2) in the "full" one
-        gemv_bytes = (2.0 if sess.gemv_mode() == "tri" else 4.0) * N * N
+        # GB/s of S the product needs: its lower triangle (2 N^2 bytes; three
+        # bytes a value, 1.5 N^2, on the split GRM) in the default mode, all of
+        # it (4 N^2) in the "full" one
+        gemv_bytes = (4.0 if sess.gemv_mode() != "tri" else tri_bytes(sess.grm_precision())) * N * N
         plain = {"seconds": plain_s, "fits_per_hour": 3600.0 / plain_s, "pcg_iters": pr["pcg_iters"],
                  "grm_products": pr["pcg_iters"] + pr["n_products"],
                  "n_solves": pr["n_solves"], "gemv_ms": gemv_avg * 1e3, "gemv_mode": sess.gemv_mode(),
@@ -775,8 +779,9 @@ def main():
         roofline["kernel"] = ("k_split_p + k_gemm_t16 + k_tri_reduce + k_gemm_epi (block-PCG GRM x 64 RHS from "
                               "the lower triangle on 16x16x32 MFMA tiles, P as three BF16 pieces, S as " +
                               ("two (the split GRM's 16-bit values)" if npc == 5 else "three") + ")")
-        roofline["bytes"] = f"2*N^2 = {2.0 * N * N:.3e} B of S's lower triangle per launch"
-        roofline["hbm_GBs_of_triangle"] = 2.0 * N * N / gemm_avg / 1e9
+        tb = tri_bytes(sess.grm_precision())
+        roofline["bytes"] = f"{tb:g}*N^2 = {tb * N * N:.3e} B of S's lower triangle per launch"
+        roofline["hbm_GBs_of_triangle"] = tb * N * N / gemm_avg / 1e9
         roofline["bf16_piece_products"] = {"tflops": npc * gemm_flop / gemm_avg / 1e12, "peak": BF16_MFMA_PEAK,
                                            "frac": npc * gemm_flop / gemm_avg / 1e12 / BF16_MFMA_PEAK,
                                            "note": f"{npc} BF16 piece products per FP32 product (the emulation's "
