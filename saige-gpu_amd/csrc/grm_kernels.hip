@@ -64,8 +64,9 @@ __device__ __forceinline__ float round16(float x) {
 // 2.7.
 // R16 and s24: each 32 x 32 block of the lower triangle is also stored in three
 // bytes a value (s24_block), turned in the wave's scratch (S24_SCRATCH floats of
-// LDS); beside a whole build's products this costs nothing that shows, a pass of
-// its own over S took 1.07 ms at N = 40,000 and 6.7 ms at 100,000.
+// LDS): about 1 ms of a 214 ms build at N = 40,000, a fifth more bytes in the
+// stores between two tiles; a pass of its own over S takes as long there and 6.7
+// ms at 100,000.
 constexpr int S24_PITCH = 36;
 constexpr int S24_SCRATCH = 32 * S24_PITCH;
 
