@@ -191,11 +191,14 @@ __device__ __forceinline__ float row16_sum(float x) {
 
 // k_gemv_tri24: k_gemv_tri on the 24-bit triangle, the same items and partials.
 // A wave's strip is a stream of 3 KB blocks, eight per 256-column chunk.  Lane
-// (ln, g) holds rows ln and 16 + ln and eight columns of a block: use 1 adds into
-// two accumulators per lane, use 2 into eight per block, which are summed over
-// the 16 lanes of a column group (DPP) and left in LDS per strip.  Diagonal
-// items read the FP32 square.  Bound by S's bytes: 2.64 ms at N = 100,000 (5.7
-// TB/s), 3.43 on the FP32 triangle; 0.69 ms at 50,000.
+// (ln, g) holds rows ln and 16 + ln and eight columns of a block: use 1 gives two
+// sums of eight products per lane and block, use 2 eight of two, which are summed
+// over the 16 lanes of a column group (DPP) and left in LDS per strip.  Use 1's
+// block sums are added in pairs over a chunk's eight blocks and the chunks'
+// one after another, so that its error stays that of k_gemv_tri's sums of four:
+// one chain over the item's up to 768 products was 3 to 6 times further off.
+// Diagonal items read the FP32 square.  Bound by S's bytes: 2.64 ms at N =
+// 100,000 (5.7 TB/s), 3.43 on the FP32 triangle; 0.69 ms at 50,000.
 __global__ __launch_bounds__(512) void k_gemv_tri24(const float* __restrict__ S, const uint8_t* __restrict__ S24,
                                                     int64_t ld, const float* __restrict__ x,
                                                     const int4* __restrict__ items, float* __restrict__ y1p,
@@ -224,6 +227,7 @@ __global__ __launch_bounds__(512) void k_gemv_tri24(const float* __restrict__ S,
     const u32x4* strip = reinterpret_cast<const u32x4*>(S24 + s24_block(r0 / 32, 0) * S24_BLOCK) + lane;
     float acc0 = 0.0f, acc1 = 0.0f;
     for (int64_t c = ca; c < cb; c++) {
+        float y0[8], y1[8];                     // the blocks' sums of this chunk
         const u32x4* bp = strip + 8 * c * (S24_BLOCK / 16);
         u32x4 h0[8], h1[8], lo[8];
 #pragma unroll
@@ -243,10 +247,8 @@ __global__ __launch_bounds__(512) void k_gemv_tri24(const float* __restrict__ S,
             for (int k = 0; k < 4; k++) {
                 const float a0 = __uint_as_float(s24_lo(h0[b], l0, k)), a1 = __uint_as_float(s24_hi(h0[b], l0, k));
                 const float b0 = __uint_as_float(s24_lo(h1[b], l1, k)), b1 = __uint_as_float(s24_hi(h1[b], l1, k));
-                acc0 = __fmaf_rn(a0, xv[2 * k], acc0);
-                acc1 = __fmaf_rn(b0, xv[2 * k], acc1);
-                acc0 = __fmaf_rn(a1, xv[2 * k + 1], acc0);
-                acc1 = __fmaf_rn(b1, xv[2 * k + 1], acc1);
+                y0[b] = __fmaf_rn(a1, xv[2 * k + 1], k == 0 ? a0 * xv[0] : __fmaf_rn(a0, xv[2 * k], y0[b]));
+                y1[b] = __fmaf_rn(b1, xv[2 * k + 1], k == 0 ? b0 * xv[0] : __fmaf_rn(b0, xv[2 * k], y1[b]));
                 z[2 * k] = __fmaf_rn(b0, xr1, a0 * xr0);
                 z[2 * k + 1] = __fmaf_rn(b1, xr1, a1 * xr0);
             }
@@ -258,6 +260,8 @@ __global__ __launch_bounds__(512) void k_gemv_tri24(const float* __restrict__ S,
                 d[1] = make_float4(z[4], z[5], z[6], z[7]);
             }
         }
+        acc0 += ((y0[0] + y0[1]) + (y0[2] + y0[3])) + ((y0[4] + y0[5]) + (y0[6] + y0[7]));
+        acc1 += ((y1[0] + y1[1]) + (y1[2] + y1[3])) + ((y1[4] + y1[5]) + (y1[6] + y1[7]));
         // buffer c & 1 was last read for chunk c-2, before chunk c-1's barrier
         lds_barrier();
         if (wv == (int)(c & 7)) {
