@@ -160,6 +160,12 @@ int saige_get_grm_block(saige_ctx* ctx, int64_t r0, int64_t c0, int64_t nr, int6
 double saige_last_grm_seconds(const saige_ctx* ctx);
 /* The SAIGE_GRM_* precision the resident GRM was built with, -1 if none. */
 int saige_grm_precision(const saige_ctx* ctx);
+/* Bytes per value of the copy of the resident GRM's lower triangle that the
+ * lower-triangle products read: 3 when the split GRM has its three-byte copy,
+ * else 4 (the FP32 GRM itself), 0 if no GRM is built.  Results are the same
+ * bit by bit.  The copy is made when device memory allows (1.5 N^2 bytes);
+ * SAIGE_GRM_24BIT=0 in the environment of saige_build_grm does without it. */
+int saige_grm_triangle_bytes(const saige_ctx* ctx);
 
 /* getCrossprodMatAndKin / parallelCrossProd (FG.cpp:1953-1981, 1669-1708):
  * y = K b.  Replaces gpuSymMatMult::sym_sgemv (GPU.hpp:30, GPU.cu:211-252). */

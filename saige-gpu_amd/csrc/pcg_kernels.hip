@@ -189,7 +189,8 @@ __device__ __forceinline__ float row16_sum(float x) {
     return x;
 }
 
-// k_gemv_tri24: k_gemv_tri on the 24-bit triangle, the same items and partials.
+// k_gemv_tri24<C24>: k_gemv_tri for the split GRM, on its 24-bit triangle, the same
+// items and partials.
 // A wave's strip is a stream of 3 KB blocks, eight per 256-column chunk.  Lane
 // (ln, g) holds rows ln and 16 + ln and eight columns of a block: use 1 gives two
 // sums of eight products per lane and block, use 2 eight of two, which are summed
@@ -199,6 +200,11 @@ __device__ __forceinline__ float row16_sum(float x) {
 // one chain over the item's up to 768 products was 3 to 6 times further off.
 // Diagonal items read the FP32 square.  Bound by S's bytes: 2.64 ms at N =
 // 100,000 (5.7 TB/s), 3.43 on the FP32 triangle; 0.69 ms at 50,000.
+// Without the 24-bit triangle (C24 false) a lane reads the same values from S, so
+// that a product's bits do not depend on the memory that was free when the GRM was
+// built (N = 20,000, 50,000, 100,000: 0.22, 0.95, 3.65 ms; k_gemv_tri, whose order
+// is another, 0.20, 0.93, 3.56; with the 24-bit triangle 0.15, 0.71, 2.72).
+template <bool C24>
 __global__ __launch_bounds__(512) void k_gemv_tri24(const float* __restrict__ S, const uint8_t* __restrict__ S24,
                                                     int64_t ld, const float* __restrict__ x,
                                                     const int4* __restrict__ items, float* __restrict__ y1p,
@@ -224,34 +230,55 @@ __global__ __launch_bounds__(512) void k_gemv_tri24(const float* __restrict__ S,
         return;
     }
     const float xr0 = x[r0 + ln], xr1 = x[r0 + 16 + ln];
-    const u32x4* strip = reinterpret_cast<const u32x4*>(S24 + s24_block(r0 / 32, 0) * S24_BLOCK) + lane;
+    const u32x4* strip =
+        C24 ? reinterpret_cast<const u32x4*>(S24 + s24_block(r0 / 32, 0) * S24_BLOCK) + lane : nullptr;
+    const float* row = S + (r0 + ln) * ld + 8 * g;
+    // a block's eight values of a row: the 24-bit form's words, or S's
+    auto values = [&](const u32x4& p, const u32x4& q, uint32_t l0, uint32_t l1, float (&v)[8]) {
+        const uint32_t l[2] = {l0, l1};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            v[2 * k] = __uint_as_float(C24 ? s24_lo(p, l, k) : k < 2 ? p[2 * k] : q[2 * k - 4]);
+            v[2 * k + 1] = __uint_as_float(C24 ? s24_hi(p, l, k) : k < 2 ? p[2 * k + 1] : q[2 * k - 3]);
+        }
+    };
     float acc0 = 0.0f, acc1 = 0.0f;
     for (int64_t c = ca; c < cb; c++) {
         float y0[8], y1[8];                     // the blocks' sums of this chunk
-        const u32x4* bp = strip + 8 * c * (S24_BLOCK / 16);
-        u32x4 h0[8], h1[8], lo[8];
+        // rows ln and 16 + ln: the upper halves and the third bytes, or S's words
+        u32x4 h0[8], h1[8], lo[8], q0[8], q1[8];
 #pragma unroll
         for (int b = 0; b < 8; b++) {
-            h0[b] = bp[b * 192];
-            h1[b] = bp[b * 192 + 64];
-            lo[b] = bp[b * 192 + 128];
+            if constexpr (C24) {
+                const u32x4* bp = strip + (8 * c + b) * (S24_BLOCK / 16);
+                h0[b] = bp[0];
+                h1[b] = bp[64];
+                lo[b] = bp[128];
+            } else {
+                const float* p = row + TV_COLS * c + 32 * b;
+                h0[b] = *reinterpret_cast<const u32x4*>(p);
+                q0[b] = *reinterpret_cast<const u32x4*>(p + 4);
+                h1[b] = *reinterpret_cast<const u32x4*>(p + 16 * ld);
+                q1[b] = *reinterpret_cast<const u32x4*>(p + 16 * ld + 4);
+            }
         }
 #pragma unroll
         for (int b = 0; b < 8; b++) {
             const float* xc = x + TV_COLS * c + 32 * b + 8 * g;
             const float4 xa = *reinterpret_cast<const float4*>(xc), xb = *reinterpret_cast<const float4*>(xc + 4);
             const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-            const uint32_t l0[2] = {lo[b][0], lo[b][1]}, l1[2] = {lo[b][2], lo[b][3]};
-            float z[8];
+            float u[8], v[8], z[8];
+            values(h0[b], q0[b], lo[b][0], lo[b][1], u);
+            values(h1[b], q1[b], lo[b][2], lo[b][3], v);
+            y0[b] = u[0] * xv[0];
+            y1[b] = v[0] * xv[0];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const float a0 = __uint_as_float(s24_lo(h0[b], l0, k)), a1 = __uint_as_float(s24_hi(h0[b], l0, k));
-                const float b0 = __uint_as_float(s24_lo(h1[b], l1, k)), b1 = __uint_as_float(s24_hi(h1[b], l1, k));
-                y0[b] = __fmaf_rn(a1, xv[2 * k + 1], k == 0 ? a0 * xv[0] : __fmaf_rn(a0, xv[2 * k], y0[b]));
-                y1[b] = __fmaf_rn(b1, xv[2 * k + 1], k == 0 ? b0 * xv[0] : __fmaf_rn(b0, xv[2 * k], y1[b]));
-                z[2 * k] = __fmaf_rn(b0, xr1, a0 * xr0);
-                z[2 * k + 1] = __fmaf_rn(b1, xr1, a1 * xr0);
+            for (int k = 1; k < 8; k++) {
+                y0[b] = __fmaf_rn(u[k], xv[k], y0[b]);
+                y1[b] = __fmaf_rn(v[k], xv[k], y1[b]);
             }
+#pragma unroll
+            for (int k = 0; k < 8; k++) z[k] = __fmaf_rn(v[k], xr1, u[k] * xr0);
 #pragma unroll
             for (int k = 0; k < 8; k++) z[k] = row16_sum(z[k]);
             if (ln == 15) {
@@ -2002,10 +2029,14 @@ hipError_t launch_grm_gemv(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, c
                            float* out, VecArgs a, double* partial, int64_t* nparts, const GemvPlan* tri) {
     if (tri) {
         if (tri->Npad != Npad || !tri->items || Npad % TV_ROWS != 0) return hipErrorInvalidValue;
-        if (m.s24)
-            hipLaunchKernelGGL(k_gemv_tri24, dim3((unsigned)tri->nitems), dim3(512), 0, s, m.S, m.s24, Npad, in,
-                               tri->items, tri->y1p, tri->y2p, a.over, a.iter);
-        else
+        if (m.by24) {
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)tri->nitems), dim3(512), 0, s, m.S, m.s24, Npad, in,
+                                   tri->items, tri->y1p, tri->y2p, a.over, a.iter);
+            };
+            if (m.s24) go(k_gemv_tri24<true>);
+            else go(k_gemv_tri24<false>);
+        } else
             hipLaunchKernelGGL(k_gemv_tri, dim3((unsigned)tri->nitems), dim3(512), 0, s, m.S, Npad, in, tri->items,
                                tri->y1p, tri->y2p, a.over, a.iter);
         const int64_t nb = Npad / TV_ROWS;

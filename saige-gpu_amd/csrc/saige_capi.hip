@@ -254,19 +254,21 @@ struct GrmView {
 
 GrmView grm_view(const saige_ctx* c, int loco) {
     const char* pieces = std::getenv("SAIGE_GEMM_S_PIECES");
-    const bool s16 = c->grm_precision == SAIGE_GRM_BF16_SPLIT && !(pieces && std::atoi(pieces) == 3);
-    if (loco) return {{c->loco_inplace ? c->d_grm : c->d_grm_loco, s16, nullptr}, c->d_diag_loco, c->loco_m, 0};
-    return {{c->d_grm, s16, c->s24_ok ? c->d_s24 : nullptr}, c->d_diag, c->Mqc, c->diag_one};
+    const bool split = c->grm_precision == SAIGE_GRM_BF16_SPLIT, s16 = split && !(pieces && std::atoi(pieces) == 3);
+    if (loco) return {{c->loco_inplace ? c->d_grm : c->d_grm_loco, s16, nullptr, false}, c->d_diag_loco, c->loco_m, 0};
+    return {{c->d_grm, s16, c->s24_ok ? c->d_s24 : nullptr, split}, c->d_diag, c->Mqc, c->diag_one};
 }
 
 // Device memory for a GRM's 24-bit triangle, or null: only for the split form,
 // and when its bytes leave room for everything else a cohort of this size may
 // take: a second GRM (leave one chromosome out) and the products' scratch, a
 // quarter of a GRM at most, and 8 GB.  Without it the products read the FP32
-// triangle.  What it holds is not valid until the caller sets s24_ok.
+// triangle, with the same bits; SAIGE_GRM_24BIT=0 does without it.  What it holds
+// is not valid until the caller sets s24_ok.
 uint8_t* reserve_s24(saige_ctx* c, int precision) {
     c->s24_ok = false;
-    if (precision != SAIGE_GRM_BF16_SPLIT) {
+    const char* env = std::getenv("SAIGE_GRM_24BIT");
+    if (precision != SAIGE_GRM_BF16_SPLIT || (env && std::atoi(env) == 0)) {
         dfree(c->d_s24);
         return nullptr;
     }
@@ -1245,6 +1247,8 @@ int saige_build_grm(saige_ctx* c, int precision) {
 double saige_last_grm_seconds(const saige_ctx* c) { return c ? c->grm_seconds : 0.0; }
 
 int saige_grm_precision(const saige_ctx* c) { return c && c->grm_ready ? c->grm_precision : -1; }
+
+int saige_grm_triangle_bytes(const saige_ctx* c) { return c && c->grm_ready ? (c->s24_ok ? 3 : 4) : 0; }
 
 int saige_get_grm_block(saige_ctx* c, int64_t r0, int64_t c0, int64_t nr, int64_t nc, float* out) {
     CHECK_CTX(c);

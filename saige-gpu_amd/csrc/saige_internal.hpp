@@ -464,6 +464,9 @@ struct GrmMat {
     // pieces instead of three, with the same bits
     bool s16 = false;
     const uint8_t* s24 = nullptr;    // such an S's lower triangle in three bytes a value (s24_block), or null
+    // the split GRM: single-column products add in k_gemv_tri24's order, with
+    // s24 or without
+    bool by24 = false;
 };
 int64_t s24_bytes(int64_t Npad);
 

@@ -99,6 +99,7 @@ SIGNATURES = {
     "saige_get_grm_block": (_int, [_c_p, _i64, _i64, _i64, _i64, _c_p]),
     "saige_last_grm_seconds": (_f64, [_c_p]),
     "saige_grm_precision": (_int, [_c_p]),
+    "saige_grm_triangle_bytes": (_int, [_c_p]),
     "saige_probes_device_rows": (_int, [_c_p, _c_p, _i64, ctypes.c_uint64, _i64, _int, _c_p, _i64]),
     "saige_alloc_host": (_int, [_c_p, _i64, ctypes.POINTER(_c_p)]),
     "saige_free_host": (_int, [_c_p, _c_p]),

@@ -191,6 +191,10 @@ class Session:
         p = int(self._L.saige_grm_precision(self.ctx))
         return next((k for k, v in self._GRM_PRECISIONS.items() if v == p), None)
 
+    def grm_triangle_bytes(self):
+        """Bytes per value of the triangle the products read (0: no GRM)."""
+        return int(self._L.saige_grm_triangle_bytes(self.ctx))
+
     def grm_block(self, r0, c0, nr, nc):
         out = np.zeros((nr, nc), np.float32)
         check(self._L.saige_get_grm_block(self.ctx, int(r0), int(c0), int(nr), int(nc), ptr(out)))
