@@ -53,8 +53,9 @@ __device__ __forceinline__ float round16(float x) {
 // Store a wave's block of 32*MI rows from row0 and 32*NI columns from col0,
 // mirrored for off-diagonal tiles; accumulate: +1 S = S0 + block, -1 S = S0 -
 // block (LOCO: one chromosome's markers left out), 0 store.  S0 may be S.
-// center: the column's value taken off each sum first (nullptr: none).  R16:
-// the stored values (after the add or subtract) rounded by round16.
+// center: the column's value taken off each sum first, in rows below `rows` (the
+// padded ones stay zero); nullptr: none.  R16: the stored values (after the add or
+// subtract) rounded by round16.
 // Accumulator layout of a 32x32 MFMA block: lane l, register r holds row
 // 8*(r/4) + 4*(l/32) + (r%4), column l%32.  A block's S0 values are requested
 // before the block ahead of it is stored (no entry that is read is stored by
@@ -73,8 +74,8 @@ constexpr int S24_SCRATCH = 32 * S24_PITCH;
 template <int MI, int NI, bool R16>
 __device__ __forceinline__ void store_block(float* S, const float* S0, int64_t ldS, int64_t row0, int64_t col0,
                                             bool mirror, int lane, const f32x16 (&acc)[MI][NI], int accumulate,
-                                            const float* center = nullptr, uint8_t* s24 = nullptr,
-                                            float* scratch = nullptr) {
+                                            const float* center = nullptr, int64_t rows = 0,
+                                            uint8_t* s24 = nullptr, float* scratch = nullptr) {
     float s0[2][16];
     auto request = [&](int k) {
         const float* p = S0 + (row0 + k / NI * 32 + 4 * (lane >> 5)) * ldS + col0 + k % NI * 32 + (lane & 31);
@@ -94,7 +95,7 @@ __device__ __forceinline__ void store_block(float* S, const float* S0, int64_t l
             float v[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                v[e] = center ? acc[mi][ni][4 * g + e] - cc : acc[mi][ni][4 * g + e];
+                v[e] = center && row + e < rows ? acc[mi][ni][4 * g + e] - cc : acc[mi][ni][4 * g + e];
                 if (accumulate > 0) v[e] = s0[k & 1][4 * g + e] + v[e];
                 else if (accumulate < 0) v[e] = s0[k & 1][4 * g + e] - v[e];
                 if (R16) v[e] = round16(v[e]);
@@ -541,7 +542,7 @@ __global__ __launch_bounds__(syrk_pk_threads(T)) void k_syrk_pk(const uint8_t* _
     static_assert(sizeof(s1) >= sizeof(float) * S24_SCRATCH * (T == 256 ? 8 : 4), "");
     auto store = [&]() {
         store_block<MI, NI, F == SYRK_SPLIT>(S, S0, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane,
-                                             acc, accumulate, F == SYRK_FP32 ? tb.center : nullptr, s24,
+                                             acc, accumulate, F == SYRK_FP32 ? tb.center : nullptr, tb.rows, s24,
                                              reinterpret_cast<float*>(s1) + wv * S24_SCRATCH);
     };
     int64_t kc = k0;
@@ -826,6 +827,7 @@ hipError_t SyrkOperands::build(hipStream_t s, int form_, const uint8_t* packed, 
     if (nsl) {
         tb.corr = reinterpret_cast<double*>(p);
         tb.center = reinterpret_cast<float*>(p + b_cor);
+        tb.rows = Nnm;
         part = reinterpret_cast<double*>(p + b_cor + b_cen);
     }
     hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)((npanel + 3) / 4), (unsigned)nchunk), dim3(256), 0, s, packed,

@@ -243,6 +243,7 @@ struct SyrkTables {
     uint64_t* t[4] = {nullptr, nullptr, nullptr, nullptr};
     double* corr = nullptr;        // [markers][3]
     float* center = nullptr;       // [Npad]
+    int64_t rows = 0;              // the samples: rows that have a center taken off
 };
 
 // The operands of a 2-bit-input SYRK over markers [j0, j1): the genotypes
