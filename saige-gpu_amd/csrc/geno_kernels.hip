@@ -8,6 +8,7 @@
 // contraction into FMA changes a rounding step.
 #include "saige_internal.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -636,18 +637,30 @@ hipError_t launch_repack(hipStream_t s, const uint8_t* bed, int64_t bpm, const i
                          int64_t ldp, uint8_t* out) {
     if (nmark == 0) return hipSuccess;
     const int64_t lds = 16 * ((bpm + 3) / 4);
-    if (!subidx) {
-        hipLaunchKernelGGL(k_repack_id, dim3((unsigned)((nmark + 3) / 4)), dim3(256), 0, s, bed, bpm, markers, nmark,
-                           stats, Nnm, ldp, out);
-    } else if (lds <= REPACK_LDS_BYTES) {
+    if (subidx && lds > REPACK_LDS_BYTES) {
+        hipLaunchKernelGGL(k_repack_far, dim3(grid_for(nmark, 16384)), dim3(256), 0, s, bed, bpm, markers, nmark,
+                           stats, subidx, Nnm, ldp, out);
+        return hipGetLastError();
+    }
+    if (subidx) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_repack_sub),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)REPACK_LDS_BYTES);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_repack_sub, dim3((unsigned)((nmark + 3) / 4)), dim3(512), (size_t)lds, s, bed, bpm,
-                           markers, nmark, stats, subidx, Nnm, ldp, out);
-    } else {
-        hipLaunchKernelGGL(k_repack_far, dim3(grid_for(nmark, 16384)), dim3(256), 0, s, bed, bpm, markers, nmark,
-                           stats, subidx, Nnm, ldp, out);
+    }
+    // four markers per workgroup; a launch has fewer than 2^32 threads, so the
+    // markers go in passes
+    constexpr int64_t PASS = (int64_t)1 << 24;
+    for (int64_t m0 = 0; m0 < nmark; m0 += PASS) {
+        const int64_t n = std::min(PASS, nmark - m0);
+        const dim3 grid((unsigned)((n + 3) / 4));
+        if (!subidx)
+            hipLaunchKernelGGL(k_repack_id, grid, dim3(256), 0, s, bed, bpm, markers + m0, n, stats, Nnm, ldp,
+                               out + m0 * ldp);
+        else
+            hipLaunchKernelGGL(k_repack_sub, grid, dim3(512), (size_t)lds, s, bed, bpm, markers + m0, n, stats, subidx,
+                               Nnm, ldp, out + m0 * ldp);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
     }
     return hipGetLastError();
 }
