@@ -800,35 +800,55 @@ static int64_t center_slices(int64_t n, int64_t Npad) {
     return std::max<int64_t>(1, std::min<int64_t>({(n + 31) / 32, (2048 + blocks - 1) / blocks, (int64_t)512}));
 }
 
+namespace {
+// the parts of SyrkOperands' block: tiled genotypes, tables, then (SYRK_FP32)
+// corr, center, slices
+struct OperandParts {
+    int64_t c0, nchunk, n, npanel, ntab, nsl, tp, tab, cor, cen, total;
+    OperandParts(int form, int64_t Npad, int64_t j0, int64_t j1) {
+        c0 = j0 / 64;
+        nchunk = (j1 + 63) / 64 - c0;
+        npanel = Npad / BT;
+        n = nchunk * 64;
+        ntab = form == SYRK_HI ? 1 : (form == SYRK_SPLIT ? 2 : 4);
+        nsl = form == SYRK_FP32 ? center_slices(n, Npad) : 0;
+        tp = npanel * nchunk * 2048;
+        tab = 8 * n;
+        cor = nsl ? round_up(24 * n, 256) : 0;
+        cen = nsl ? round_up(4 * Npad, 256) : 0;
+        total = tp + ntab * tab + cor + cen + 8 * nsl * Npad;
+    }
+};
+}  // namespace
+
+int64_t SyrkOperands::bytes(int form, int64_t Npad, int64_t j0, int64_t j1) {
+    return OperandParts(form, Npad, j0, j1).total;
+}
+
 hipError_t SyrkOperands::build(hipStream_t s, int form_, const uint8_t* packed, const float4* lut, int64_t Mqc,
                                int64_t Nnm, int64_t Npad_, int64_t ldp, int64_t j0, int64_t j1) {
     release();
     if (j0 < 0 || j1 > Mqc || j0 >= j1 || Npad_ % 256 != 0 || 4 * ldp < Npad_) return hipErrorInvalidValue;
     form = form_;
     Npad = Npad_;
-    const int64_t c0 = j0 / 64;
-    nchunk = (j1 + 63) / 64 - c0;
-    const int64_t npanel = Npad / BT, n = nchunk * 64;
-    const int ntab = form == SYRK_HI ? 1 : (form == SYRK_SPLIT ? 2 : 4);
-    const int64_t nsl = form == SYRK_FP32 ? center_slices(n, Npad) : 0;
-    // one block: tiled genotypes, tables, then (SYRK_FP32) corr, center, slices
-    const int64_t b_tp = npanel * nchunk * 2048, b_tab = 8 * n;
-    const int64_t b_cor = nsl ? round_up(24 * n, 256) : 0, b_cen = nsl ? round_up(4 * Npad, 256) : 0;
-    hipError_t e = hipMalloc(&block, (size_t)(b_tp + ntab * b_tab + b_cor + b_cen + 8 * nsl * Npad));
+    const OperandParts q(form, Npad, j0, j1);
+    const int64_t c0 = q.c0, npanel = q.npanel, n = q.n, nsl = q.nsl;
+    nchunk = q.nchunk;
+    hipError_t e = hipMalloc(&block, (size_t)q.total);
     if (e != hipSuccess) {
         block = nullptr;
         return e;
     }
     uint8_t* p = static_cast<uint8_t*>(block);
     tp = p;
-    p += b_tp;
-    for (int q = 0; q < ntab; q++, p += b_tab) tb.t[q] = reinterpret_cast<uint64_t*>(p);
+    p += q.tp;
+    for (int k = 0; k < q.ntab; k++, p += q.tab) tb.t[k] = reinterpret_cast<uint64_t*>(p);
     double* part = nullptr;
     if (nsl) {
         tb.corr = reinterpret_cast<double*>(p);
-        tb.center = reinterpret_cast<float*>(p + b_cor);
+        tb.center = reinterpret_cast<float*>(p + q.cor);
         tb.rows = Nnm;
-        part = reinterpret_cast<double*>(p + b_cor + b_cen);
+        part = reinterpret_cast<double*>(p + q.cor + q.cen);
     }
     hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)((npanel + 3) / 4), (unsigned)nchunk), dim3(256), 0, s, packed,
                        Mqc, Nnm, ldp, npanel, c0, nchunk, tp);

@@ -1118,11 +1118,20 @@ int saige_get_diag_of_kin(saige_ctx* c, float* out) {
 }
 
 namespace {
+// SAIGE_GRM_PANEL_MARKERS caps the markers of one panel, or of one pass of the
+// FP32 form (tests use it to force several, i.e. the accumulating SYRK)
+int64_t panel_cap(int64_t markers) {
+    const char* env = std::getenv("SAIGE_GRM_PANEL_MARKERS");
+    return env ? std::min(markers, std::max<int64_t>(64, std::atoll(env) / 64 * 64)) : markers;
+}
+
 // S = (nothing, S0 plus, S0 minus) the GRM part of markers [j0, j1) from the
 // 2-bit genotypes, in the operand form of `precision` (accumulate: 0, 1, -1; S0
 // may be S).  s24 (may be null): the 24-bit triangle of a split S, written too.
-// Waits for the stream; t (may be null): device seconds between its start and
-// end.
+// The FP32 form goes in passes of fewer markers that add up in S where memory has
+// no room for all markers' operands (Npad / 4 bytes a marker), half of what is
+// free each; the others, whose stored values a pass would round, do not.  Waits
+// for the stream; t (may be null): device seconds between its start and end.
 hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1, float* S, const float* S0,
                             int accumulate, double* t, uint8_t* s24) {
     hipStream_t st = c->stream;
@@ -1137,8 +1146,27 @@ hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1,
     if (e == hipSuccess)
         e = hipMemcpyAsync(d_tiles, order.data(), sizeof(int2) * order.size(), hipMemcpyHostToDevice, st);
     if (e == hipSuccess && t) e = hipEventRecord(c->ev0, st);
-    if (e == hipSuccess) e = op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j0, j1);
-    if (e == hipSuccess) e = launch_syrk_pk(st, op, d_tiles, S, S0, accumulate, tile, s24);
+    int64_t pass = form == SYRK_FP32 ? panel_cap(j1 - j0) : j1 - j0;
+    for (int64_t j = j0; j < j1 && e == hipSuccess; j += pass) {
+        pass = std::min(pass, j1 - j);
+        e = op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j, j + pass);
+        if (e == hipErrorOutOfMemory && form == SYRK_FP32 && pass > 64) {
+            (void)hipGetLastError();
+            size_t free_b = 0, total_b = 0;
+            if ((e = hipMemGetInfo(&free_b, &total_b)) != hipSuccess) break;
+            while (pass > 64 && SyrkOperands::bytes(form, Np, j, j + pass) > (int64_t)(free_b / 2))
+                pass = std::max<int64_t>(64, pass / 2 / 64 * 64);
+            e = op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j, j + pass);
+        }
+        if (e == hipSuccess)
+            e = j == j0 ? launch_syrk_pk(st, op, d_tiles, S, S0, accumulate, tile, s24)
+                        : launch_syrk_pk(st, op, d_tiles, S, S, accumulate < 0 ? -1 : 1, tile, s24);
+        if (j + pass < j1) {                 // the next pass's operands take this one's place
+            const hipError_t w = hipStreamSynchronize(st);
+            if (e == hipSuccess) e = w;
+            op.release();
+        }
+    }
     if (e == hipSuccess && t) e = hipEventRecord(c->ev1, st);
     const hipError_t w = hipStreamSynchronize(st);
     if (e == hipSuccess) e = w;
@@ -1199,12 +1227,7 @@ int saige_build_grm(saige_ctx* c, int precision) {
     pw = std::max<int64_t>(kc, pw / 64 * 64);
     const int64_t full = round_up(c->Mqc, 64);
     pw = std::min(pw, full);
-    // SAIGE_GRM_PANEL_MARKERS caps the panel width (tests use it to force
-    // several panels, i.e. the accumulate path of the SYRK)
-    if (const char* env = std::getenv("SAIGE_GRM_PANEL_MARKERS")) {
-        const int64_t cap = std::max<int64_t>(64, std::atoll(env) / 64 * 64);
-        pw = std::min(pw, cap);
-    }
+    pw = panel_cap(pw);
     void* d_panel = nullptr;
     SAIGE_HIP_TRY(hipMalloc(&d_panel, (size_t)(Np * pw * 2)));
     const std::vector<int2> order = syrk_tile_order(Np / syrk_tile(), 8);
@@ -1545,8 +1568,7 @@ hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, const 
     if (e == hipSuccess) e = hipMemGetInfo(&free_b, &total_b);
     int64_t pw = std::min<int64_t>((int64_t)32 << 30, (int64_t)(free_b / 2)) / (Np * 2);
     pw = std::min(std::max<int64_t>(kc, pw / 64 * 64), round_up(cnt, 64));
-    if (const char* env = std::getenv("SAIGE_GRM_PANEL_MARKERS"))
-        pw = std::min(pw, std::max<int64_t>(64, std::atoll(env) / 64 * 64));
+    pw = panel_cap(pw);
     if (e == hipSuccess) e = hipMalloc(&d_panel, (size_t)(Np * pw * 2));
     for (int64_t j0 = start; j0 <= end && e == hipSuccess; j0 += pw) {
         const int64_t np = std::min(pw, end + 1 - j0);

@@ -259,6 +259,7 @@ struct SyrkOperands {
     SyrkTables tb;
     hipError_t build(hipStream_t s, int form, const uint8_t* packed, const float4* lut, int64_t Mqc, int64_t Nnm,
                      int64_t Npad, int64_t ldp, int64_t j0, int64_t j1);
+    static int64_t bytes(int form, int64_t Npad, int64_t j0, int64_t j1);   // the block's size
     void release();
 };
 

@@ -1,0 +1,98 @@
+"""Calls that have to succeed with little device memory left: the rest of the
+device is held by untouched allocations while they run."""
+import contextlib
+import ctypes
+
+import numpy as np
+import pytest
+
+from fixtures import random_bed
+
+pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def only_free(session, left):
+    """Holds device memory so that about `left` bytes stay free."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+    hip.hipFree.argtypes = [ctypes.c_void_p]
+    held, piece = [], 1 << 38
+    try:
+        while piece >= 1 << 22:
+            over = session.device_memory()[0] - left
+            if over < 1 << 22:
+                break
+            p = ctypes.c_void_p()
+            if over >= piece and hip.hipMalloc(ctypes.byref(p), piece) == 0:
+                held.append(p)
+            else:
+                piece //= 2
+        hip.hipGetLastError()
+        yield
+    finally:
+        for p in held:
+            hip.hipFree(p)
+
+
+def load(session, N, M, seed=3):
+    body, _, _ = random_bed(N, M, 0.01, seed=seed, maf_lo=0.05, maf_hi=0.5)
+    session.setminMAFforGRM(0.01)
+    session.setmaxMissingRateforGRM(0.15)
+    session.setgeno_bytes(body, N, M)
+
+
+def test_fp32_grm_passes_add_up(session, monkeypatch):
+    """The FP32 GRM in passes of 128 markers is the FP32 sum of the passes' GRMs
+    (powers of two of markers, so that K names S exactly)."""
+    N = 700
+    print("case: FP32 GRM in passes", flush=True)
+    body, _, _ = random_bed(N, 256, 0.0, seed=2, maf_lo=0.1, maf_hi=0.5)
+    body = body.reshape(256, -1)
+    session.setminMAFforGRM(0.01)
+    session.setmaxMissingRateforGRM(0.15)
+    part = []
+    for j in (0, 128):
+        session.setgeno_bytes(body[j:j + 128].ravel(), N, 128)
+        assert session.getMsub_MAFge_minMAFtoConstructGRM() == 128
+        session.build_grm("fp32")
+        part.append(session.grm_block(0, 0, N, N) * np.float32(128))
+    session.setgeno_bytes(body.ravel(), N, 256)
+    monkeypatch.setenv("SAIGE_GRM_PANEL_MARKERS", "128")
+    session.build_grm("fp32")
+    S = session.grm_block(0, 0, N, N) * np.float32(256)
+    assert np.array_equal(S, part[0] + part[1])
+    # a range of two passes, taken off
+    session.setStartEndIndex(30, 230, 0)
+    monkeypatch.delenv("SAIGE_GRM_PANEL_MARKERS")
+    e = np.zeros(N, np.float32)
+    e[5] = 1.0
+    y = session.getCrossprodMatAndKin_LOCO(e)
+    session.setStartEndIndex(30, 230, 0)
+    z = session.getCrossprodMatAndKin_LOCO(e)
+    # FP32 sums of at most 256 products of |z| < 7 in two groupings
+    assert np.max(np.abs(y - z)) <= 256 * 49 * 256 / 55 * 2.0 ** -24
+
+
+def test_fp32_grm_without_room_for_all_markers(session):
+    """Memory for a part of the markers' operands only: the build goes in passes."""
+    N, M = 1000, 1 << 19
+    print("case: FP32 GRM with little memory", flush=True)
+    rng = np.random.default_rng(4)
+    body = rng.integers(0, 256, (4096, (N + 3) // 4), dtype=np.uint8)
+    session.setminMAFforGRM(0.0)
+    session.setmaxMissingRateforGRM(1.0)
+    try:
+        session.setgeno_bytes(np.tile(body, (M // 4096, 1)).ravel(), N, M)
+        session.build_grm("fp32")
+        K = session.grm_block(0, 0, N, N)
+        # all operands: 1024 / 4 bytes of genotypes and 56 of tables a marker
+        with only_free(session, 96 << 20):
+            assert session.device_memory()[0] < M * (256 + 56)
+            session.build_grm("fp32")
+        L = session.grm_block(0, 0, N, N)
+        # FP32 sums over M markers in two groupings, random signs off the diagonal
+        assert np.max(np.abs(K - L)) <= 4 * np.sqrt(M) * 2.0 ** -24 * np.max(np.abs(K))
+        assert np.any(K != L)
+    finally:
+        load(session, 200, 64)
