@@ -161,11 +161,17 @@ void clear_geno(saige_ctx* c) {
     c->N = c->M = c->Nnm = c->Npad = c->Mqc = c->Mvr = c->ldp = 0;
 }
 
+// the kept blocks that an ingest takes after its decode
+void free_kept_cohort(saige_ctx* c) {
+    for (KeptBlock* b : {&c->kb_packed, &c->kb_packed_vr, &c->kb_lut, &c->kb_lut_vr, &c->kb_vec, &c->kb_block})
+        b->release();
+}
+
 void free_geno(saige_ctx* c) {
     clear_geno(c);
-    for (KeptBlock* b : {&c->kb_stats, &c->kb_packed, &c->kb_packed_vr, &c->kb_lut, &c->kb_lut_vr, &c->kb_vec,
-                         &c->kb_lists, &c->kb_block})
-        b->release();
+    free_kept_cohort(c);
+    c->kb_stats.release();
+    c->kb_lists.release();
 }
 
 int64_t count_lines(const char* path, int* err) {
@@ -700,9 +706,18 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
     // sample list and the marker list, each at a multiple of 256 bytes
     const int64_t o_rset = round_up(all_in ? 0 : 16 * ldm, 256), o_sub = o_rset + round_up(M, 256),
                   o_list = o_sub + round_up(4 * n_sub, 256);
+    // blocks kept from the last cohort must not stand in the way of this one's:
+    // where memory runs out, those not yet taken over go first
+    auto reserve = [&](auto take) {
+        if (!take()) return true;
+        free_kept_cohort(c);
+        return !take();
+    };
     int rc = SAIGE_OK;
     do {
-        if (c->kb_lists.reserve(o_list + 4 * M) || c->kb_stats.reserve((int64_t)sizeof(MarkerStat) * M)) {
+        if (!reserve([&] {
+                return c->kb_lists.reserve(o_list + 4 * M) || c->kb_stats.reserve((int64_t)sizeof(MarkerStat) * M);
+            })) {
             set_error("device allocation failed (setgeno)");
             rc = SAIGE_E_NOMEM;
             break;
@@ -745,10 +760,13 @@ int setgeno_device_impl(saige_ctx* c, const uint8_t* d_bed, int64_t N, int64_t M
         }
         c->Mqc = (int64_t)c->qc_index.size();
         c->Mvr = (int64_t)c->vr_index.size();
-        if (c->kb_packed.reserve((c->Mqc + PACKED_PAD_ROWS) * c->ldp) || c->kb_packed_vr.reserve(c->Mvr * c->ldp) ||
-            c->kb_lut.reserve((int64_t)sizeof(float4) * (c->Mqc + PACKED_PAD_ROWS)) ||
-            c->kb_lut_vr.reserve((int64_t)sizeof(float4) * c->Mvr) ||
-            c->kb_vec.reserve((int64_t)sizeof(float) * 5 * c->Npad)) {
+        if (!reserve([&] {
+                return c->kb_packed.reserve((c->Mqc + PACKED_PAD_ROWS) * c->ldp) ||
+                       c->kb_packed_vr.reserve(c->Mvr * c->ldp) ||
+                       c->kb_lut.reserve((int64_t)sizeof(float4) * (c->Mqc + PACKED_PAD_ROWS)) ||
+                       c->kb_lut_vr.reserve((int64_t)sizeof(float4) * c->Mvr) ||
+                       c->kb_vec.reserve((int64_t)sizeof(float) * 5 * c->Npad);
+            })) {
             set_error("device allocation failed (packed genotypes)");
             rc = SAIGE_E_NOMEM;
             break;
@@ -1284,10 +1302,13 @@ int saige_get_grm_block(saige_ctx* c, int64_t r0, int64_t c0, int64_t nr, int64_
     if (nr == 0 || nc == 0) return SAIGE_OK;
     // rows divided on the device into a contiguous block (at most 64 MB, or one
     // row) and copied from there: a pitched copy goes to the host row by row
-    const int64_t rows = std::min(nr, std::max<int64_t>(1, ((int64_t)16 << 20) / nc));
-    if (c->kb_block.reserve((int64_t)sizeof(float) * rows * nc)) {
-        set_error("device allocation failed (GRM block)");
-        return SAIGE_E_NOMEM;
+    int64_t rows = std::min(nr, std::max<int64_t>(1, ((int64_t)16 << 20) / nc));
+    while (c->kb_block.reserve((int64_t)sizeof(float) * rows * nc)) {
+        if (rows == 1) {
+            set_error("device allocation failed (GRM block)");
+            return SAIGE_E_NOMEM;
+        }
+        rows = (rows + 1) / 2;               // where memory is short: fewer rows at a time
     }
     float* d = static_cast<float*>(c->kb_block.p);
     for (int64_t i = 0; i < nr; i += rows) {

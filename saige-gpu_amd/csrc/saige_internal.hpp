@@ -217,17 +217,21 @@ struct Engine {
 
 // A device block that outlives the cohort it was made for (a context reads
 // one after another): reserve() keeps the block when it is large enough and
-// not more than twice (plus 64 MB) too large, else replaces it.
+// not more than 64 MB too large, else replaces it.
 struct KeptBlock {
     void* p = nullptr;
     int64_t cap = 0;
     hipError_t reserve(int64_t bytes) {
         if (bytes < 16) bytes = 16;
-        if (p && cap >= bytes && cap <= 2 * bytes + ((int64_t)64 << 20)) return hipSuccess;
+        if (p && cap >= bytes && cap <= bytes + ((int64_t)64 << 20)) return hipSuccess;
         release();
         const hipError_t e = hipMalloc(&p, (size_t)bytes);
-        if (e == hipSuccess) cap = bytes;
-        else p = nullptr;
+        if (e == hipSuccess) {
+            cap = bytes;
+        } else {
+            p = nullptr;
+            (void)hipGetLastError();         // or the next launch's check would report it
+        }
         return e;
     }
     void release() {

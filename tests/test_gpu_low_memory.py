@@ -11,16 +11,26 @@ from fixtures import random_bed
 pytestmark = pytest.mark.gpu
 
 
+def hip_runtime():
+    return ctypes.CDLL("libamdhip64.so")
+
+
+def free_memory():
+    f, t = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip_runtime().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+    return f.value
+
+
 @contextlib.contextmanager
-def only_free(session, left):
+def only_free(left):
     """Holds device memory so that about `left` bytes stay free."""
-    hip = ctypes.CDLL("libamdhip64.so")
+    hip = hip_runtime()
     hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
     hip.hipFree.argtypes = [ctypes.c_void_p]
     held, piece = [], 1 << 38
     try:
         while piece >= 1 << 22:
-            over = session.device_memory()[0] - left
+            over = free_memory() - left
             if over < 1 << 22:
                 break
             p = ctypes.c_void_p()
@@ -87,12 +97,55 @@ def test_fp32_grm_without_room_for_all_markers(session):
         session.build_grm("fp32")
         K = session.grm_block(0, 0, N, N)
         # all operands: 1024 / 4 bytes of genotypes and 56 of tables a marker
-        with only_free(session, 96 << 20):
-            assert session.device_memory()[0] < M * (256 + 56)
+        with only_free(96 << 20):
+            assert free_memory() < M * (256 + 56)
             session.build_grm("fp32")
         L = session.grm_block(0, 0, N, N)
         # FP32 sums over M markers in two groupings, random signs off the diagonal
         assert np.max(np.abs(K - L)) <= 4 * np.sqrt(M) * 2.0 ** -24 * np.max(np.abs(K))
         assert np.any(K != L)
+    finally:
+        load(session, 200, 64)
+
+
+def many_markers(N, M):
+    """A .bed body of M markers that repeats 1000 random ones."""
+    body = np.random.default_rng(N).integers(0, 256, (1000, (N + 3) // 4), dtype=np.uint8)
+    return np.tile(body, (M // 1000, 1)).ravel()
+
+
+def test_kept_blocks_are_bounded(session):
+    """A cohort of half the last one's size does not keep the last one's memory:
+    at most 64 MB too much in each of an ingest's eight blocks."""
+    print("case: kept blocks' bound", flush=True)
+    N, large, small = 4000, 1250000, 650000
+    session.setminMAFforGRM(0.0)
+    session.setmaxMissingRateforGRM(1.0)
+    try:
+        load(session, 200, 64)
+        session.setminMAFforGRM(0.0)
+        session.setmaxMissingRateforGRM(1.0)
+        before = free_memory()
+        session.setgeno_bytes(many_markers(N, small), N, small)
+        fresh = before - free_memory()
+        session.setgeno_bytes(many_markers(N, large), N, large)
+        session.setgeno_bytes(many_markers(N, small), N, small)
+        assert before - free_memory() <= fresh + 8 * (64 << 20)
+    finally:
+        load(session, 200, 64)
+
+
+def test_ingest_gives_up_kept_blocks(session):
+    """A cohort that fits only without the last one's blocks."""
+    print("case: ingest beside kept blocks", flush=True)
+    session.setminMAFforGRM(0.0)
+    session.setmaxMissingRateforGRM(1.0)
+    try:
+        session.setgeno_bytes(many_markers(4000, 1250000), 4000, 1250000)      # 1.3 GB of genotypes
+        M = 7000000
+        with only_free(200 << 20):
+            # 0.26 GB of lists and stats first, then 1.0 GB of genotypes and tables
+            session.setgeno_bytes(many_markers(8, M), 8, M)
+        assert session.getMsub_MAFge_minMAFtoConstructGRM() == M
     finally:
         load(session, 200, 64)
