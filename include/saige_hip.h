@@ -163,8 +163,11 @@ int saige_grm_precision(const saige_ctx* ctx);
 /* Bytes per value of the copy of the resident GRM's lower triangle that the
  * lower-triangle products read: 3 when the split GRM has its three-byte copy,
  * else 4 (the FP32 GRM itself), 0 if no GRM is built.  Results are the same
- * bit by bit.  The copy is made when device memory allows (1.5 N^2 bytes);
- * SAIGE_GRM_24BIT=0 in the environment of saige_build_grm does without it. */
+ * bit by bit.  The copy (1.5 N^2 bytes) is made by saige_build_grm when that
+ * leaves a second GRM, a quarter of one and 8 GB free.  It is given back when an
+ * allocation of this context would fail otherwise, and for the second GRM of a
+ * leave-out range; other users of the device cannot reach it: build the GRM with
+ * SAIGE_GRM_24BIT=0 in the environment to do without. */
 int saige_grm_triangle_bytes(const saige_ctx* ctx);
 
 /* getCrossprodMatAndKin / parallelCrossProd (FG.cpp:1953-1981, 1669-1708):
@@ -390,7 +393,9 @@ int saige_get_gemm_mode(const saige_ctx* ctx, int* mode);
 int saige_set_gemv_mode(saige_ctx* ctx, int mode);
 int saige_get_gemv_mode(const saige_ctx* ctx, int* mode);
 
-/* Free and total device memory (hipMemGetInfo), for admission control. */
+/* Free and total device memory (hipMemGetInfo), for admission control; the
+ * GRM's three-byte copy, which the context gives back on demand, counts as
+ * free. */
 int saige_device_memory(saige_ctx* ctx, int64_t* free_bytes, int64_t* total_bytes);
 /* Device bytes one engine system (w, tau, sample mask) occupies. */
 int64_t saige_engine_system_bytes(const saige_ctx* ctx);

@@ -70,13 +70,56 @@ template <typename T>
 hipError_t dalloc(T** p, int64_t count) {
     *p = nullptr;
     if (count <= 0) count = 1;
-    return hipMalloc((void**)p, sizeof(T) * (size_t)count);
+    const hipError_t e = hipMalloc((void**)p, sizeof(T) * (size_t)count);
+    if (e != hipSuccess) (void)hipGetLastError();       // or the next launch's check would report it
+    return e;
 }
 
 template <typename T>
 void dfree(T*& p) {
     if (p) (void)hipFree((void*)p);
     p = nullptr;
+}
+
+// While one lives the 24-bit triangle stays where it is.
+class S24Use {
+public:
+    explicit S24Use(saige_ctx* c) : c_(c) { count(1); }
+    S24Use(const S24Use&) = delete;
+    S24Use& operator=(const S24Use&) = delete;
+    ~S24Use() { count(-1); }
+
+private:
+    void count(int d) {
+        std::lock_guard<std::mutex> lk(c_->s24_mu);
+        c_->s24_uses += d;
+    }
+    saige_ctx* c_;
+};
+
+// Frees the 24-bit triangle; false when there is none or it is in use.
+bool give_back_s24(saige_ctx* c) {
+    std::lock_guard<std::mutex> lk(c->s24_mu);
+    if (!c->d_s24 || c->s24_uses) return false;
+    dfree(c->d_s24);
+    c->s24_ok = false;
+    return true;
+}
+
+// take() allocates device memory (a SAIGE_* code or a hipError_t) and can be run
+// again after a failure: where memory runs out, the 24-bit triangle, which the
+// products can do without, is given back for it.  No S24Use may live around it.
+bool no_memory(int rc) { return rc == SAIGE_E_NOMEM; }
+bool no_memory(hipError_t e) { return e == hipErrorOutOfMemory; }
+template <typename F>
+auto with_room(saige_ctx* c, F take) {
+    auto r = take();
+    if (!no_memory(r)) return r;
+    (void)hipGetLastError();
+    if (!give_back_s24(c)) return r;
+    r = take();
+    if (no_memory(r)) (void)hipGetLastError();
+    return r;
 }
 
 // the per-slot state block: lists [2][kpad] and slot systems, maxiter [kpad]
@@ -139,8 +182,8 @@ void clear_geno(saige_ctx* c) {
     c->d_packed = c->d_packed_vr = nullptr;
     c->d_lut = c->d_lut_vr = nullptr;
     c->d_diag = c->d_vec = nullptr;
-    dfree(c->d_grm); dfree(c->d_s24); dfree(c->d_grm_loco);
-    c->s24_ok = false;
+    dfree(c->d_grm); dfree(c->d_grm_loco);
+    give_back_s24(c);
     dfree(c->d_diag_loco);
     dfree(c->d_mv_in); dfree(c->d_mv_blk); dfree(c->d_mv_out); dfree(c->d_mv_ypart);
     dfree(c->d_dots_partial); dfree(c->d_dots_out);
@@ -188,8 +231,7 @@ int64_t count_lines(const char* path, int* err) {
 }
 
 // Allocate and fill the slot engine: kpad columns, nsys systems.
-int engine_reserve(saige_ctx* c, Engine& e, int kpad, int nsys) {
-    if (e.kpad == kpad && e.nsys >= nsys && e.X) return SAIGE_OK;
+int engine_alloc(saige_ctx* c, Engine& e, int kpad, int nsys) {
     free_engine(e);
     const int64_t Np = c->Npad;
     SAIGE_HIP_TRY(dalloc(&e.X, Np * kpad));
@@ -246,50 +288,57 @@ int engine_reserve(saige_ctx* c, Engine& e, int kpad, int nsys) {
     return SAIGE_OK;
 }
 
+int engine_reserve(saige_ctx* c, Engine& e, int kpad, int nsys) {
+    if (e.kpad == kpad && e.nsys >= nsys && e.X) return SAIGE_OK;
+    return with_room(c, [&] { return engine_alloc(c, e, kpad, nsys); });
+}
+
 // The GRM a product uses: the full one (S/Mqc, diag) or the LOCO one
 // (S_loco/M_loco, diag_loco; getDiagOfSigma_LOCO ignores the diag-as-one
 // option, FG.cpp:2368-2392).  The split GRM and its LOCO ranges have values of
 // at most 16 significant bits; SAIGE_GEMM_S_PIECES=3 has the block GEMM take
 // them as any others (the same bits, more work).
 struct GrmView {
+    S24Use use;
     GrmMat S;
     const float* diag;
     int64_t m;
     int diag_one;
 };
 
-GrmView grm_view(const saige_ctx* c, int loco) {
+// Taken after the call's allocations (with_room).
+GrmView grm_view(saige_ctx* c, int loco) {
     const char* pieces = std::getenv("SAIGE_GEMM_S_PIECES");
     const bool split = c->grm_precision == SAIGE_GRM_BF16_SPLIT, s16 = split && !(pieces && std::atoi(pieces) == 3);
-    if (loco) return {{c->loco_inplace ? c->d_grm : c->d_grm_loco, s16, nullptr, false}, c->d_diag_loco, c->loco_m, 0};
-    return {{c->d_grm, s16, c->s24_ok ? c->d_s24 : nullptr, split}, c->d_diag, c->Mqc, c->diag_one};
+    if (loco)
+        return {S24Use(c), {c->loco_inplace ? c->d_grm : c->d_grm_loco, s16, nullptr, false}, c->d_diag_loco,
+                c->loco_m, 0};
+    return {S24Use(c), {c->d_grm, s16, c->s24_ok ? c->d_s24 : nullptr, split}, c->d_diag, c->Mqc, c->diag_one};
 }
 
-// Device memory for a GRM's 24-bit triangle, or null: only for the split form,
+// Takes device memory for a GRM's 24-bit triangle: only for the split form,
 // and when its bytes leave room for everything else a cohort of this size may
 // take: a second GRM (leave one chromosome out) and the products' scratch, a
 // quarter of a GRM at most, and 8 GB.  Without it the products read the FP32
-// triangle, with the same bits; SAIGE_GRM_24BIT=0 does without it.  What it holds
-// is not valid until the caller sets s24_ok.
-uint8_t* reserve_s24(saige_ctx* c, int precision) {
-    c->s24_ok = false;
+// triangle, with the same bits; SAIGE_GRM_24BIT=0 does without it, and it is given
+// back when the context needs the memory (with_room).  What it holds is not valid
+// until s24_ok says so (syrk_from_packed).
+void reserve_s24(saige_ctx* c, int precision) {
     const char* env = std::getenv("SAIGE_GRM_24BIT");
     if (precision != SAIGE_GRM_BF16_SPLIT || (env && std::atoi(env) == 0)) {
-        dfree(c->d_s24);
-        return nullptr;
+        give_back_s24(c);
+        return;
     }
+    std::lock_guard<std::mutex> lk(c->s24_mu);
+    c->s24_ok = false;
     const int64_t bytes = s24_bytes(c->Npad), grm = 4 * c->Npad * c->Npad;
     if (!c->d_s24) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess ||
             (int64_t)free_b < bytes + grm + grm / 4 + ((int64_t)8 << 30))
-            return nullptr;
-        if (dalloc(&c->d_s24, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            c->d_s24 = nullptr;
-        }
+            return;
+        if (dalloc(&c->d_s24, bytes) != hipSuccess) c->d_s24 = nullptr;
     }
-    return c->d_s24;
 }
 
 int check_loco(const saige_ctx* c) {
@@ -403,7 +452,8 @@ constexpr int TRI_CHUNKS = 96;
 // waves, rt 2: 8), when that mode is on
 int ensure_tri(saige_ctx* c) {
     if (c->gemm_cfg.mode != GEMM_BF16X3_TRI) return SAIGE_OK;
-    const hipError_t e = tri_plan_build(c->tri, c->Npad, c->gemm_cfg.rt == 2 ? 8 : 12, TRI_CHUNKS);
+    const hipError_t e =
+        with_room(c, [&] { return tri_plan_build(c->tri, c->Npad, c->gemm_cfg.rt == 2 ? 8 : 12, TRI_CHUNKS); });
     if (e != hipSuccess) {
         saige::set_error("lower-triangle product scratch for Npad=%lld: %s", (long long)c->Npad,
                          hipGetErrorString(e));
@@ -428,7 +478,7 @@ int triv_chunks(int64_t Npad) {
 const GemvPlan* gemv_plan(saige_ctx* c, int* rc) {
     *rc = SAIGE_OK;
     if (c->gemv_mode != SAIGE_GEMV_TRI) return nullptr;
-    const hipError_t e = gemv_plan_build(c->triv, c->Npad, triv_chunks(c->Npad));
+    const hipError_t e = with_room(c, [&] { return gemv_plan_build(c->triv, c->Npad, triv_chunks(c->Npad)); });
     if (e != hipSuccess) {
         saige::set_error("lower-triangle GEMV scratch for Npad=%lld: %s", (long long)c->Npad, hipGetErrorString(e));
         *rc = e == hipErrorOutOfMemory ? SAIGE_E_NOMEM : SAIGE_E_DEVICE;
@@ -560,14 +610,16 @@ int engine_take_batch(saige_ctx* c, Engine& e, int k, const int32_t* slots, floa
 
 int ensure_dots_scratch(saige_ctx* c) {
     if (c->d_dots_partial) return SAIGE_OK;
-    if (dalloc(&c->d_dots_partial, col_dots_partial_doubles(c->Npad, EW)) ||
-        dalloc(&c->d_dots_out, (int64_t)EW * col_dots_max())) {
-        dfree(c->d_dots_partial);
-        dfree(c->d_dots_out);
-        set_error("device allocation failed (dot scratch)");
-        return SAIGE_E_NOMEM;
-    }
-    return SAIGE_OK;
+    return with_room(c, [&] {
+        if (dalloc(&c->d_dots_partial, col_dots_partial_doubles(c->Npad, EW)) ||
+            dalloc(&c->d_dots_out, (int64_t)EW * col_dots_max())) {
+            dfree(c->d_dots_partial);
+            dfree(c->d_dots_out);
+            set_error("device allocation failed (dot scratch)");
+            return SAIGE_E_NOMEM;
+        }
+        return SAIGE_OK;
+    });
 }
 
 // FP64 dots of k columns (engine slots or a column-major device buffer) with
@@ -990,7 +1042,7 @@ int saige_setgeno_host(saige_ctx* c, const uint8_t* body, int64_t N, int64_t M, 
     }
     uint8_t* d_bed = nullptr;
     const int64_t bytes = M * ((N + 3) / 4);
-    SAIGE_HIP_TRY(dalloc(&d_bed, bytes));
+    SAIGE_HIP_TRY(with_room(c, [&] { return dalloc(&d_bed, bytes); }));
     hipError_t e = hipMemcpy(d_bed, body, (size_t)bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         dfree(d_bed);
@@ -1145,13 +1197,14 @@ int64_t panel_cap(int64_t markers) {
 
 // S = (nothing, S0 plus, S0 minus) the GRM part of markers [j0, j1) from the
 // 2-bit genotypes, in the operand form of `precision` (accumulate: 0, 1, -1; S0
-// may be S).  s24 (may be null): the 24-bit triangle of a split S, written too.
+// may be S).  s24: S is to be the context's whole split GRM, and its 24-bit
+// triangle, where there is memory for it (reserve_s24), is written too.
 // The FP32 form goes in passes of fewer markers that add up in S where memory has
 // no room for all markers' operands (Npad / 4 bytes a marker), half of what is
 // free each; the others, whose stored values a pass would round, do not.  Waits
 // for the stream; t (may be null): device seconds between its start and end.
 hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1, float* S, const float* S0,
-                            int accumulate, double* t, uint8_t* s24) {
+                            int accumulate, double* t, bool s24) {
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad;
     const int form = precision == SAIGE_GRM_FP32 ? SYRK_FP32 : (precision == SAIGE_GRM_BF16_SPLIT ? SYRK_SPLIT : SYRK_HI);
@@ -1160,35 +1213,33 @@ hipError_t syrk_from_packed(saige_ctx* c, int precision, int64_t j0, int64_t j1,
     const std::vector<int2> order = syrk_tile_order(Np / tile, 1024 / tile);
     SyrkOperands op;
     int2* d_tiles = nullptr;
-    hipError_t e = dalloc(&d_tiles, (int64_t)order.size());
+    hipError_t e = with_room(c, [&] { return dalloc(&d_tiles, (int64_t)order.size()); });
     if (e == hipSuccess)
         e = hipMemcpyAsync(d_tiles, order.data(), sizeof(int2) * order.size(), hipMemcpyHostToDevice, st);
     if (e == hipSuccess && t) e = hipEventRecord(c->ev0, st);
     int64_t pass = form == SYRK_FP32 ? panel_cap(j1 - j0) : j1 - j0;
     for (int64_t j = j0; j < j1 && e == hipSuccess; j += pass) {
         pass = std::min(pass, j1 - j);
-        e = op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j, j + pass);
+        auto build = [&] { return op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j, j + pass); };
+        e = with_room(c, build);
         if (e == hipErrorOutOfMemory && form == SYRK_FP32 && pass > 64) {
-            (void)hipGetLastError();
             size_t free_b = 0, total_b = 0;
             if ((e = hipMemGetInfo(&free_b, &total_b)) != hipSuccess) break;
             while (pass > 64 && SyrkOperands::bytes(form, Np, j, j + pass) > (int64_t)(free_b / 2))
                 pass = std::max<int64_t>(64, pass / 2 / 64 * 64);
-            e = op.build(st, form, c->d_packed, c->d_lut, c->Mqc, c->Nnm, Np, c->ldp, j, j + pass);
+            e = with_room(c, build);
         }
+        const S24Use use(c);
+        uint8_t* d_s24 = s24 ? c->d_s24 : nullptr;
         if (e == hipSuccess)
-            e = j == j0 ? launch_syrk_pk(st, op, d_tiles, S, S0, accumulate, tile, s24)
-                        : launch_syrk_pk(st, op, d_tiles, S, S, accumulate < 0 ? -1 : 1, tile, s24);
-        if (j + pass < j1) {                 // the next pass's operands take this one's place
-            const hipError_t w = hipStreamSynchronize(st);
-            if (e == hipSuccess) e = w;
-            op.release();
-        }
+            e = j == j0 ? launch_syrk_pk(st, op, d_tiles, S, S0, accumulate, tile, d_s24)
+                        : launch_syrk_pk(st, op, d_tiles, S, S, accumulate < 0 ? -1 : 1, tile, d_s24);
+        if (e == hipSuccess && t) e = hipEventRecord(c->ev1, st);
+        const hipError_t w = hipStreamSynchronize(st);
+        if (e == hipSuccess) e = w;
+        op.release();                        // the next pass's operands take this one's place
+        if (s24) c->s24_ok = e == hipSuccess && d_s24;
     }
-    if (e == hipSuccess && t) e = hipEventRecord(c->ev1, st);
-    const hipError_t w = hipStreamSynchronize(st);
-    if (e == hipSuccess) e = w;
-    op.release();
     dfree(d_tiles);
     float ms = 0.f;
     if (e == hipSuccess && t) e = hipEventElapsedTime(&ms, c->ev0, c->ev1);
@@ -1224,10 +1275,10 @@ int saige_build_grm(saige_ctx* c, int precision) {
     c->loco_inplace = false;
     if (precision != SAIGE_GRM_BF16_PANEL) {
         // 2-bit operands straight into the MFMA SYRK: no Z panel
-        uint8_t* s24 = reserve_s24(c, precision);
-        const hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, nullptr, 0, &c->grm_seconds, s24);
+        reserve_s24(c, precision);
+        const hipError_t e = syrk_from_packed(c, precision, 0, c->Mqc, c->d_grm, nullptr, 0, &c->grm_seconds,
+                                              precision == SAIGE_GRM_BF16_SPLIT);
         c->grm_precision = precision;
-        c->s24_ok = e == hipSuccess && s24;
         if (e != hipSuccess) {
             set_error("GRM build failed: %s", hipGetErrorString(e));
             return e == hipErrorOutOfMemory ? SAIGE_E_NOMEM : SAIGE_E_DEVICE;
@@ -1303,7 +1354,7 @@ int saige_get_grm_block(saige_ctx* c, int64_t r0, int64_t c0, int64_t nr, int64_
     // rows divided on the device into a contiguous block (at most 64 MB, or one
     // row) and copied from there: a pitched copy goes to the host row by row
     int64_t rows = std::min(nr, std::max<int64_t>(1, ((int64_t)16 << 20) / nc));
-    while (c->kb_block.reserve((int64_t)sizeof(float) * rows * nc)) {
+    while (with_room(c, [&] { return c->kb_block.reserve((int64_t)sizeof(float) * rows * nc); })) {
         if (rows == 1) {
             set_error("device allocation failed (GRM block)");
             return SAIGE_E_NOMEM;
@@ -1322,10 +1373,26 @@ int saige_get_grm_block(saige_ctx* c, int64_t r0, int64_t c0, int64_t nr, int64_
 
 namespace {
 int reserve_solve1(saige_ctx* c) {
-    const hipError_t e = c->s1.reserve(c->Npad);
+    const hipError_t e = with_room(c, [&] { return c->s1.reserve(c->Npad); });
     if (e == hipSuccess) return SAIGE_OK;
     set_error("device allocation failed (single-column vectors): %s", hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? SAIGE_E_NOMEM : SAIGE_E_DEVICE;
+}
+
+// the block products' own scratch (not the engine's, so that live engine slots
+// are untouched)
+int ensure_mv_scratch(saige_ctx* c) {
+    if (c->d_mv_in) return SAIGE_OK;
+    const int64_t Np = c->Npad, N = c->Nnm;
+    return with_room(c, [&] {
+        if (dalloc(&c->d_mv_in, N * EW) || dalloc(&c->d_mv_blk, Np * EW) || dalloc(&c->d_mv_out, Np * EW) ||
+            dalloc(&c->d_mv_ypart, gemm_ypart_floats(Np))) {
+            dfree(c->d_mv_in); dfree(c->d_mv_blk); dfree(c->d_mv_out); dfree(c->d_mv_ypart);
+            set_error("device allocation failed (block product scratch)");
+            return SAIGE_E_NOMEM;
+        }
+        return SAIGE_OK;
+    });
 }
 
 // zeroes rows [Nnm, Npad) of a vector (padded rows read as zero in products)
@@ -1341,13 +1408,13 @@ static int grm_matvec(saige_ctx* c, int loco, const float* B, int64_t k, float* 
     }
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
-    const GrmView g = grm_view(c, loco);
     if (k == 1) {
         if (int rc = reserve_solve1(c)) return rc;
         Solve1& v = c->s1;
         int prc = 0;
         const GemvPlan* tv = gemv_plan(c, &prc);
         if (prc) return prc;
+        const GrmView g = grm_view(c, loco);
         VecArgs va;
         va.mqc = (float)g.m;
         SAIGE_HIP_TRY(hipMemcpyAsync(v.p, B, 4 * N, hipMemcpyHostToDevice, st));
@@ -1357,19 +1424,12 @@ static int grm_matvec(saige_ctx* c, int loco, const float* B, int64_t k, float* 
         SAIGE_HIP_TRY(hipStreamSynchronize(st));
         return SAIGE_OK;
     }
+    if (int rc = ensure_tri(c)) return rc;
+    if (int rc = ensure_mv_scratch(c)) return rc;
+    const GrmView g = grm_view(c, loco);
     SigmaArgs a{};
     a.mqc = (float)g.m;
     a.mode = 0;
-    if (int rc = ensure_tri(c)) return rc;
-    // own scratch (not the engine's), so live engine slots are untouched
-    if (!c->d_mv_in) {
-        if (dalloc(&c->d_mv_in, N * EW) || dalloc(&c->d_mv_blk, Np * EW) || dalloc(&c->d_mv_out, Np * EW) ||
-            dalloc(&c->d_mv_ypart, gemm_ypart_floats(Np))) {
-            dfree(c->d_mv_in); dfree(c->d_mv_blk); dfree(c->d_mv_out); dfree(c->d_mv_ypart); dfree(c->d_mv_ypart);
-            set_error("device allocation failed (grm_matvec)");
-            return SAIGE_E_NOMEM;
-        }
-    }
     float *d_in = c->d_mv_in, *d_blk = c->d_mv_blk, *d_out = c->d_mv_out;
     hipError_t e = hipSuccess;
     for (int64_t k0 = 0; k0 < k && e == hipSuccess; k0 += EW) {
@@ -1421,7 +1481,7 @@ static int get_diag_of_sigma(saige_ctx* c, int loco, const float* w, const float
     float* d_minv = c->d_vec + 2 * Np;
     float* d_d = c->d_vec + 3 * Np;
     uint8_t* d_mask = nullptr;
-    SAIGE_HIP_TRY(dalloc(&d_mask, Np));
+    SAIGE_HIP_TRY(with_room(c, [&] { return dalloc(&d_mask, Np); }));
     SAIGE_HIP_TRY(hipMemcpyAsync(d_w, w, 4 * N, hipMemcpyHostToDevice, st));
     const GrmView g = grm_view(c, loco);
     SAIGE_HIP_TRY(launch_sigma_setup(st, d_w, nullptr, g.diag, N, Np, tau[0], tau[1], (float)g.m, g.diag_one,
@@ -1447,10 +1507,10 @@ static int get_crossprod(saige_ctx* c, int loco, const float* b, const float* w,
     Solve1& v = c->s1;
     hipStream_t st = c->stream;
     const int64_t Np = c->Npad, N = c->Nnm;
-    const GrmView g = grm_view(c, loco);
     int prc = 0;
     const GemvPlan* tv = gemv_plan(c, &prc);
     if (prc) return prc;
+    const GrmView g = grm_view(c, loco);
     SAIGE_HIP_TRY(hipMemcpyAsync(v.w, w, 4 * N, hipMemcpyHostToDevice, st));
     SAIGE_HIP_TRY(hipMemcpyAsync(v.p, b, 4 * N, hipMemcpyHostToDevice, st));
     SAIGE_HIP_TRY(zero_tail(c, v.p));
@@ -1485,10 +1545,10 @@ static int pcg1(saige_ctx* c, int loco, const float* w, const float* tau, const 
     Solve1& v = c->s1;
     hipStream_t st = c->stream;
     const int64_t N = c->Nnm;
-    const GrmView g = grm_view(c, loco);
     int prc = 0;
     const GemvPlan* tv = gemv_plan(c, &prc);
     if (prc) return prc;
+    const GrmView g = grm_view(c, loco);
     int it = 0;
     SAIGE_HIP_TRY(solve1(st, v, w, b, x, g.S, g.diag, N, tau[0], tau[1], (float)g.m, g.diag_one, maxiter, (double)tol,
                          tv, &it));
@@ -1568,7 +1628,7 @@ namespace {
 // operand precision the resident S was built with (accumulate: 1 add, -1
 // subtract; S0 may be S); s24 as in syrk_from_packed.
 hipError_t range_syrk(saige_ctx* c, int64_t start, int64_t end, float* S, const float* S0, int accumulate,
-                      uint8_t* s24 = nullptr) {
+                      bool s24 = false) {
     if (c->grm_precision != SAIGE_GRM_BF16_PANEL)
         return syrk_from_packed(c, c->grm_precision, start, end + 1, S, S0, accumulate, nullptr, s24);
     hipStream_t st = c->stream;
@@ -1616,10 +1676,10 @@ static int restore_full_grm(saige_ctx* c) {
             }
     // the sums may differ from the first build's in the last bit, so the 24-bit
     // triangle is made anew
-    uint8_t* s24 = reserve_s24(c, c->grm_precision);
-    hipError_t e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, c->d_grm, 1, s24);
+    reserve_s24(c, c->grm_precision);
+    hipError_t e = range_syrk(c, c->loco_start, c->loco_end, c->d_grm, c->d_grm, 1,
+                              c->grm_precision == SAIGE_GRM_BF16_SPLIT);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    c->s24_ok = e == hipSuccess && s24;
     if (e != hipSuccess) {
         set_error("restoring the GRM after an in-place LOCO range failed: %s", hipGetErrorString(e));
         return SAIGE_E_DEVICE;
@@ -1656,20 +1716,26 @@ int saige_set_start_end_index(saige_ctx* c, int64_t start, int64_t end, int chro
     // full-GRM use (SAIGE_LOCO_INPLACE=1 forces this).
     const char* env = std::getenv("SAIGE_LOCO_INPLACE");
     const bool force_inplace = env && std::atoi(env) != 0;
-    if (!c->d_diag_loco && dalloc(&c->d_diag_loco, Np)) {
+    if (!c->d_diag_loco && with_room(c, [&] { return dalloc(&c->d_diag_loco, Np); })) {
         set_error("device allocation failed (LOCO diagonal)");
         return SAIGE_E_NOMEM;
     }
     bool two_buffers = !force_inplace && c->d_grm_loco != nullptr;
     if (!force_inplace && !two_buffers) {
-        size_t free_b = 0, total_b = 0;
-        SAIGE_HIP_TRY(hipMemGetInfo(&free_b, &total_b));
-        if ((int64_t)free_b >= 4 * Np * Np + ((int64_t)4 << 30) && dalloc(&c->d_grm_loco, Np * Np) == hipSuccess)
-            two_buffers = true;
+        // with the 24-bit triangle's memory where it does not fit beside it
+        const hipError_t e = with_room(c, [&] {
+            size_t free_b = 0, total_b = 0;
+            const hipError_t m = hipMemGetInfo(&free_b, &total_b);
+            if (m != hipSuccess) return m;
+            return (int64_t)free_b < 4 * Np * Np + ((int64_t)4 << 30) ? hipErrorOutOfMemory
+                                                                       : dalloc(&c->d_grm_loco, Np * Np);
+        });
+        if (!no_memory(e)) SAIGE_HIP_TRY(e);
+        two_buffers = e == hipSuccess;
     }
     c->loco_ready = false;
     float* d_rdiag = nullptr;
-    if (dalloc(&d_rdiag, Np)) {
+    if (with_room(c, [&] { return dalloc(&d_rdiag, Np); })) {
         set_error("device allocation failed (LOCO)");
         return SAIGE_E_NOMEM;
     }
@@ -1980,18 +2046,6 @@ int engine_idle(const saige_ctx* c, const char* what) {
             }
     return SAIGE_OK;
 }
-
-int ensure_mv_scratch(saige_ctx* c) {
-    if (c->d_mv_in) return SAIGE_OK;
-    const int64_t Np = c->Npad, N = c->Nnm;
-    if (dalloc(&c->d_mv_in, N * EW) || dalloc(&c->d_mv_blk, Np * EW) || dalloc(&c->d_mv_out, Np * EW) ||
-        dalloc(&c->d_mv_ypart, gemm_ypart_floats(Np))) {
-        dfree(c->d_mv_in); dfree(c->d_mv_blk); dfree(c->d_mv_out); dfree(c->d_mv_ypart);
-        set_error("device allocation failed (block product scratch)");
-        return SAIGE_E_NOMEM;
-    }
-    return SAIGE_OK;
-}
 }  // namespace
 
 int saige_autotune(saige_ctx* c, int reps, double* ms_table) {
@@ -2009,15 +2063,15 @@ int saige_autotune(saige_ctx* c, int reps, double* ms_table) {
     a.mqc = (float)c->Mqc;
     a.mode = 0;
     // time one shape: one warm-up launch, then reps launches between events
-    const GrmMat S = grm_view(c, 0).S;
     const NarrowCols q0 = NarrowCols::tile(16, 0);
     auto time_shape = [&](GemmConfig g, int halves, double* out_ms, bool q = false) -> hipError_t {
         const NarrowCols* quarter = q ? &q0 : nullptr;
-        hipError_t e = launch_grm_gemm(st, S, Np, N, c->d_mv_blk, c->d_mv_out, a, nullptr, nullptr, c->d_mv_ypart,
+        const GrmView v = grm_view(c, 0);
+        hipError_t e = launch_grm_gemm(st, v.S, Np, N, c->d_mv_blk, c->d_mv_out, a, nullptr, nullptr, c->d_mv_ypart,
                                        g, halves, &c->tri, quarter);
         if (e == hipSuccess) e = hipEventRecord(c->ev0, st);
         for (int r = 0; r < reps && e == hipSuccess; r++)
-            e = launch_grm_gemm(st, S, Np, N, c->d_mv_blk, c->d_mv_out, a, nullptr, nullptr, c->d_mv_ypart, g,
+            e = launch_grm_gemm(st, v.S, Np, N, c->d_mv_blk, c->d_mv_out, a, nullptr, nullptr, c->d_mv_ypart, g,
                                 halves, &c->tri, quarter);
         if (e == hipSuccess) e = hipEventRecord(c->ev1, st);
         if (e == hipSuccess) e = hipEventSynchronize(c->ev1);
@@ -2259,6 +2313,10 @@ int saige_device_memory(saige_ctx* c, int64_t* free_bytes, int64_t* total_bytes)
     CHECK_CTX(c);
     size_t f = 0, t = 0;
     SAIGE_HIP_TRY(hipMemGetInfo(&f, &t));
+    {
+        std::lock_guard<std::mutex> lk(c->s24_mu);
+        if (c->d_s24) f += (size_t)s24_bytes(c->Npad);      // given back on demand
+    }
     if (free_bytes) *free_bytes = (int64_t)f;
     if (total_bytes) *total_bytes = (int64_t)t;
     return SAIGE_OK;
@@ -2289,7 +2347,7 @@ int saige_alloc_device(saige_ctx* c, int64_t bytes, void** out) {
         set_error("invalid allocation request");
         return SAIGE_E_ARG;
     }
-    SAIGE_HIP_TRY(hipMalloc(out, (size_t)bytes));
+    SAIGE_HIP_TRY(with_room(c, [&] { return hipMalloc(out, (size_t)bytes); }));
     // zeroed, so that what a caller reads before writing it does not depend on
     // what the block held before
     hipError_t e = hipMemsetAsync(*out, 0, (size_t)bytes, c->stream);

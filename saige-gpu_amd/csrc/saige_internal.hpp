@@ -303,6 +303,8 @@ struct saige_ctx {
     // there is room for it; s24_ok: it holds d_grm's present values
     uint8_t* d_s24 = nullptr;
     bool s24_ok = false;
+    std::mutex s24_mu;                           // guards the two and:
+    int s24_uses = 0;                            // work under way that reads or writes it (S24Use)
     // LOCO (setStartEndIndex, FG.cpp:3067): S minus one range of GRM markers
     float* d_grm_loco = nullptr;                 // [Npad][Npad]
     float* d_diag_loco = nullptr;                // [Npad]

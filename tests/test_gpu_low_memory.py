@@ -149,3 +149,54 @@ def test_ingest_gives_up_kept_blocks(session):
         assert session.getMsub_MAFge_minMAFtoConstructGRM() == M
     finally:
         load(session, 200, 64)
+
+
+COPY = 632 * 631 // 2 * 3072                         # bytes: 32 x 32 blocks left of the diagonal
+
+
+@pytest.fixture
+def split_grm(session):
+    """A split GRM of 20,224 samples: 1.6 GB, its three-byte triangle 0.6."""
+    session.setminMAFforGRM(0.0)
+    session.setmaxMissingRateforGRM(1.0)
+    session.setgeno_bytes(many_markers(20224, 1000), 20224, 1000)
+    session.set_gemm_mode("bf16x3_tri")
+    session.build_grm("bf16_split")
+    assert session.grm_triangle_bytes() == 3
+    yield np.random.default_rng(1).standard_normal((20224, 20)).astype(np.float32)
+    session.set_gemm_mode("fp32")
+    load(session, 200, 64)
+
+
+def test_three_byte_copy_is_given_back(session, split_grm):
+    """Allocations of the context take the copy's memory when there is no other,
+    and the products' bits stay."""
+    print("case: the three-byte triangle's memory", flush=True)
+    B = split_grm
+    assert session.device_memory()[0] - free_memory() == COPY
+    y = session.getCrossprodMatAndKin(B[:, 0])
+    with only_free(64 << 20):
+        Y = session.grm_matvec(B)                    # 0.15 GB of scratch on its first call
+        assert session.grm_triangle_bytes() == 4
+        assert np.array_equal(session.getCrossprodMatAndKin(B[:, 0]), y)
+    session.build_grm("bf16_split")
+    assert session.grm_triangle_bytes() == 3
+    assert np.array_equal(session.grm_matvec(B), Y)
+    with only_free(64 << 20):
+        p = session.alloc_device(400 << 20)
+        session.free_device(p)
+        assert session.grm_triangle_bytes() == 4
+        with pytest.raises(Exception):               # nothing left to give
+            session.alloc_device(2 << 30)
+        assert np.array_equal(session.getCrossprodMatAndKin(B[:, 0]), y)
+
+
+def test_second_grm_takes_the_copys_memory(session, split_grm):
+    """A leave-out range gets its own GRM (1.6 GB, with 4 GB to spare) where it
+    fits without the copy."""
+    print("case: a leave-out GRM beside the three-byte triangle", flush=True)
+    with only_free((4 << 30) + 1300000000):
+        before = free_memory()
+        session.setStartEndIndex(10, 40, 0)
+        assert session.grm_triangle_bytes() == 4
+        assert before + COPY - free_memory() > 1500 << 20
