@@ -334,7 +334,10 @@ int saige_engine_use_loco(saige_ctx* ctx, int on);
  * ms_table (may be NULL) receives 24 per-launch times in ms: the 16 full
  * shapes in the order of saige_autotune_candidates, then the one-half
  * shapes (rt, pd) = (1,1), (2,1), (1,3), (2,3), then the 16-column shapes of
- * the lower-triangle mode in the same order (-1 in other modes).  Call it
+ * the lower-triangle mode in the same order (-1 in other modes).  Shapes that
+ * differ only in what has no effect are timed once and read the same: rt and pd
+ * of one-half launches in the FP32 mode, pd in the lower-triangle mode at few
+ * rows (up to 16,384, 14,080 and 11,264 for 64, 32 and 16 columns).  Call it
  * once before solving; results are reproducible for a fixed shape.
  * SAIGE_E_STATE if the engine has live slots. */
 int saige_autotune(saige_ctx* ctx, int reps, double* ms_table);
@@ -347,7 +350,8 @@ int saige_set_gemm_config(saige_ctx* ctx, int rt, int pd, int nsplit);
  * a shape is tuned or set, the library takes the prefetch depth it has
  * measured better for the launch's width in place of pd (the same bits). */
 int saige_get_gemm_config(const saige_ctx* ctx, int* rt, int* pd, int* nsplit, double* tuned_ms);
-/* Shape of one-half launches (nsplit as the full shape). */
+/* Shape of one-half launches (nsplit as the full shape; rt and pd have no
+ * effect in the FP32 mode). */
 int saige_get_gemm_config_half(const saige_ctx* ctx, int* rt, int* pd, double* tuned_ms);
 /* Shape of 16-column launches (lower-triangle mode; rt as the full shape). */
 int saige_get_gemm_config_quarter(const saige_ctx* ctx, int* rt, int* pd, double* tuned_ms);

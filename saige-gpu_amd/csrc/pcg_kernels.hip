@@ -2162,6 +2162,8 @@ static int64_t tri_flat_rows(int width) {
     return width <= 16 ? 11264 : width <= 32 ? 14080 : 16384;
 }
 
+bool tri_is_flat(const TriPlan& t, int width) { return t.nflat && t.Npad <= tri_flat_rows(width); }
+
 // k_gemm_flat's items: per group of four strips the use-1 items of its row set,
 // and its use-2 row sets in runs that make about three items per CU, at most
 // eight row sets each; longest first
@@ -2266,7 +2268,7 @@ hipError_t launch_tri(hipStream_t s, GrmMat m, int64_t Npad, const float* in, fl
     if (narrow)
         for (int k = 0; k < narrow->width; k++) cm.w[k / 4] |= (uint32_t)narrow->col[k] << (8 * (k % 4));
     const int width = narrow ? narrow->width : EW;
-    if (t.nflat && Npad <= tri_flat_rows(width)) {
+    if (tri_is_flat(t, width)) {
         u32x4* pb2 = reinterpret_cast<u32x4*>(ypart + 2 * Npad * EW);       // slices that this product leaves free
         hipLaunchKernelGGL(k_split_p2, dim3((unsigned)(2 * G * EW / 256)), dim3(256), 0, s, in, G, pb, pb2);
         if (width == 16) launch_flat<NWV, 1, SP>(s, m, Npad, pb, pb2, t, cm, ypart);

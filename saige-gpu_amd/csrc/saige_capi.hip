@@ -2097,8 +2097,12 @@ int saige_autotune(saige_ctx* c, int reps, double* ms_table) {
         if (tri && g.nsplit != 8) continue;
         c->gemm_cfg = g;
         if (int rc = ensure_tri(c)) return rc;
-        double per = 0.0;
-        SAIGE_HIP_TRY(time_shape(g, 3, &per));
+        // shapes that differ in a parameter without effect run one kernel, which
+        // is timed once: here the depth at few rows of the lower-triangle mode
+        double per = -1.0;
+        for (int j = 0; j < i && tri && tri_is_flat(c->tri, EW); j++)
+            if (kGemmCandidates[j].rt == g.rt && tfull[j] >= 0.0) per = tfull[j];
+        if (per < 0.0) SAIGE_HIP_TRY(time_shape(g, 3, &per));
         tfull[i] = per;
         if (ms_table) ms_table[i] = per;
         if (best_ms < 0.0 || per < best_ms) {
@@ -2135,14 +2139,15 @@ int saige_autotune(saige_ctx* c, int reps, double* ms_table) {
             for (int i = 0; i < kNumHalfCandidates; i++) {
                 if (kHalfCandidates[i].rt != rt) continue;
                 const GemmConfig g{rt, 8, kHalfCandidates[i].pd, mode};
-                double per = 0.0;
-                SAIGE_HIP_TRY(time_shape(g, 1, &per));
+                double per = mh;
+                if (mh < 0.0 || !tri_is_flat(c->tri, 32)) SAIGE_HIP_TRY(time_shape(g, 1, &per));
                 if (ms_table) ms_table[kNumGemmCandidates + i] = per;
                 if (mh < 0.0 || per < mh) {
                     bh = g;
                     mh = per;
                 }
-                SAIGE_HIP_TRY(time_shape(g, 1, &per, true));
+                per = mq;
+                if (mq < 0.0 || !tri_is_flat(c->tri, 16)) SAIGE_HIP_TRY(time_shape(g, 1, &per, true));
                 if (ms_table) ms_table[kNumGemmCandidates + kNumHalfCandidates + i] = per;
                 if (mq < 0.0 || per < mq) {
                     bq = g;
@@ -2165,8 +2170,9 @@ int saige_autotune(saige_ctx* c, int reps, double* ms_table) {
     for (int i = 0; i < kNumHalfCandidates && !tri; i++) {
         GemmConfig g{kHalfCandidates[i].rt, best.nsplit, kHalfCandidates[i].pd, mode};
         if (ms_table) ms_table[kNumGemmCandidates + i] = -1.0;
-        double per = 0.0;
-        SAIGE_HIP_TRY(time_shape(g, 1, &per));
+        // the FP32 mode has one half kernel whatever rt and pd
+        double per = best_h_ms;
+        if (per < 0.0 || mode != GEMM_FP32) SAIGE_HIP_TRY(time_shape(g, 1, &per));
         if (ms_table) ms_table[kNumGemmCandidates + i] = per;
         if (best_h_ms < 0.0 || per < best_h_ms) {
             best_h = g;

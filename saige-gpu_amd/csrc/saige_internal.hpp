@@ -99,6 +99,9 @@ struct TriPlan {
 // builds (or keeps, when Npad/nwv/ch match) the plan; frees on failure
 hipError_t tri_plan_build(TriPlan& t, int64_t Npad, int nwv, int ch);
 void tri_plan_free(TriPlan& t);
+// a launch of this many columns runs as k_gemm_flat, which has no prefetch depth
+// to choose
+bool tri_is_flat(const TriPlan& t, int width);
 
 // The lower-triangle GEMV's work list and partials: row sets of 256 rows,
 // chunks of 256 columns; items as in TriPlan (at most ch chunks left of the
