@@ -491,7 +491,7 @@ __global__ __launch_bounds__(256) void k_gemm_part(const float* __restrict__ S, 
 // 172, 356, 712, 3030 us; staging both halves took 195, 415, 830, 3460).  Few
 // rows leave them on too few CUs or unevenly on all (N = 10,240: 320 workgroups
 // on 256 CUs), and one-wave workgroups, which spread evenly, pay their own
-// staging: see HALF_ONE_WAVE.
+// staging: see half_one_wave.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_gemm_half(const float* __restrict__ S, int64_t ld,
                                                        const float* __restrict__ in, float* __restrict__ ypart,
@@ -2295,10 +2295,18 @@ hipError_t launch_tri(hipStream_t s, GrmMat m, int64_t Npad, const float* in, fl
 }
 }  // namespace
 
-// Rows up to which a one-half FP32 product runs one-wave workgroups: us per
-// product with one and with four waves at 1024, 2560, 5120, 10,240, 14,080 and
-// 20,224 rows: 7.5, 17.4, 34.2, 111, 217, 487 and 8.5, 17.6, 34.0, 126, 172, 356.
-constexpr int64_t HALF_ONE_WAVE = 12288;
+// When a one-half FP32 product runs one-wave workgroups, by the number of
+// four-wave ones (rows / 128 times the column slices) over 256 CUs: fewer than
+// half the CUs would have one, or some CUs two and most one.  us per product
+// (epilogue included) with one and with four waves at 64, 80, 96, 110 of them
+// (one slice): 189, 266, 319, 362 and 205, 277, 326, 375; 128 (1, 2, 4 slices)
+// 417, 112, 38.8 and 421, 111, 39.3; 256 (2, 4, 8) 246, 72.8, 32.5 and 238, 68.6,
+// 32.0; 316 (2), 320 (4, 8) 417, 124, 44.0 and 475, 137, 47.0; 384 (4, 8) 180, 53.9
+// and 172, 51.7; 512 (4, 8) 253, 81.1 and 214, 69.5.
+static bool half_one_wave(int64_t Npad, int nsplit) {
+    const int64_t w = Npad / 128 * nsplit;
+    return w < 128 || (w > 256 && w < 384);
+}
 
 hipError_t launch_grm_gemm(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, const float* in,
                            float* out, SigmaArgs a, double* partial, int64_t* nparts, float* ypart, GemmConfig g,
@@ -2359,7 +2367,7 @@ hipError_t launch_grm_gemm(hipStream_t s, GrmMat m, int64_t Npad, int64_t Nnm, c
         else
             hipLaunchKernelGGL((k_gemm_x3<2, 1, 2>), grid, dim3(256), 0, s, S, Npad, pb, ypart, halves);
     } else if (halves != 3) {
-        if (Npad <= HALF_ONE_WAVE)
+        if (half_one_wave(Npad, nsplit))
             hipLaunchKernelGGL((k_gemm_half<1>), dim3((unsigned)(Npad / 32), nsplit), dim3(64), 0, s, S, Npad, in,
                                ypart, halves - 1);
         else
