@@ -43,8 +43,11 @@ extern "C" {
 #define SAIGE_GRM_FP32 0        /* 2-bit genotypes; z_i z_j = (g_i - c) beta z_j + a term of
                                    j alone: g - c whole, beta z in three BF16 pieces (24
                                    bits), three products on the BF16 MFMA with FP32
-                                   accumulation, the terms of j alone in FP64; an FP32
-                                   sum over the markers' exact products               */
+                                   accumulation, the terms of j alone summed in FP64 and
+                                   rounded once to FP32.  A heterozygote's z is the mean
+                                   of the two homozygotes' FP32 values, so a product is
+                                   within about 2^-23 of the marker's largest one; S is
+                                   the FP32 sum of the products                        */
 #define SAIGE_GRM_BF16 1        /* 2-bit genotypes standardised to BF16 inside the SYRK,
                                    BF16 MFMA with FP32 accumulation                    */
 #define SAIGE_GRM_BF16_PANEL 2  /* same arithmetic from materialised BF16 Z panels     */
@@ -93,7 +96,9 @@ int saige_set_vr_random_markers(saige_ctx* ctx, const int32_t* idx_host, int64_t
  *                        samples (subSampleInGeno)
  *   indicator          : N flags (indicatorGenoSamplesWithPheno); NULL derives
  *                        them from sub_sample_in_geno
- *   is_diag_of_kin_set_as_one : isDiagofKinSetAsOne */
+ *   is_diag_of_kin_set_as_one : isDiagofKinSetAsOne
+ * The device blocks it fills stay with the context and are used again by the
+ * next cohort when large enough and at most 64 MB too large. */
 int saige_setgeno(saige_ctx* ctx, const char* bed_file, const char* bim_file,
                   const char* fam_file, const int32_t* sub_sample_in_geno, int64_t n_sub,
                   const uint8_t* indicator, int is_diag_of_kin_set_as_one);
@@ -262,7 +267,10 @@ int saige_engine_add_products(saige_ctx* ctx, int k, const int32_t* slots, const
 int saige_engine_take_batch(saige_ctx* ctx, int k, const int32_t* slots, float* X_host);
 /* Run `n_iter` iterations on every live slot.  done[slot] = 1 when the slot
  * has stopped; iters[slot] = its iteration count (either may be NULL; each
- * holds 64 entries). */
+ * holds 64 entries).  Returns when both are known; the last iteration's update
+ * of the search directions, which no call shows, may still run then.  Every
+ * later call on the context comes after it, and an error in it is reported by
+ * one of those. */
 int saige_engine_step(saige_ctx* ctx, int n_iter, uint8_t* done_host, int32_t* iters_host);
 /* Copy the solution of a slot to host and free the slot. */
 int saige_engine_take(saige_ctx* ctx, int slot, float* x_host);
@@ -405,7 +413,9 @@ int saige_device_memory(saige_ctx* ctx, int64_t* free_bytes, int64_t* total_byte
 int64_t saige_engine_system_bytes(const saige_ctx* ctx);
 /* Seconds of device time spent in the engines' GRM product launches of one
  * kind, and their count (HIP events around each launch). */
-#define SAIGE_LAUNCH_GEMV 0       /* products of saige_pcg1's solver             */
+#define SAIGE_LAUNCH_GEMV 0       /* products of saige_pcg1's solver (up to 7168 rows,
+                                     where they are not launches of their own: its
+                                     whole iterations)                            */
 #define SAIGE_LAUNCH_GEMM_HALF 1  /* block GEMM over 32 columns: one half, or (lower
                                      triangle) at most 32 occupied slots anywhere */
 #define SAIGE_LAUNCH_GEMM_FULL 2  /* block GEMM over all 64 columns, or (lower
