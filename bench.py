@@ -47,10 +47,16 @@ PROFILE_FILES = {"fp32": "profiles/kernels_N100k_M150k_bf16.md", "bf16x3": "prof
 BF16_MFMA_PEAK = 2500.0
 
 
-def tri_bytes(grm_precision):
-    """Bytes of S's lower triangle over N^2: two values of four bytes per pair,
-    or, on the split GRM where its copy fits the device (N = 100k), of three."""
-    return 1.5 if grm_precision == "bf16_split" else 2.0
+def tri_bytes(sess):
+    """Bytes of S's lower triangle over N^2: N^2 / 2 values of four bytes, or of
+    three where the split GRM has its copy."""
+    return sess.grm_triangle_bytes() / 2.0
+
+
+def full_width(sess):
+    """Device seconds and count of the 64-column GEMM launches."""
+    (s, n), (s48, n48) = sess.engine_stats("gemm_full"), sess.engine_stats("gemm_48")
+    return s - s48, n - n48
 
 
 def log(*a):
@@ -421,7 +427,7 @@ def c4_leg(args):
     tune = sess.autotune(reps=3)
     log(f"C4 autotune: rt{tune['rt']}/pd{tune['pd']}/s{tune['nsplit']} {tune['ms']:.2f} ms")
     opt = D.Options(nrun=30)
-    g0, n0 = sess.engine_stats("gemm_full")
+    g0, n0 = full_width(sess)
     t0 = time.perf_counter()
     handles, sch = D.fit_batched(sess, [{"trait": "binary", "y": y, "X": X}], opt)
     if handles[0].error is not None:
@@ -430,8 +436,8 @@ def c4_leg(args):
     t1 = time.perf_counter()
     vr = D.variance_ratio(sess, fit, y, X, "binary", categories, opt, vr_pool=True, num_markers=100)
     t2 = time.perf_counter()
-    g1, n1 = sess.engine_stats("gemm_full")
-    gemm_avg = (g1 - g0) / max(1, n1 - n0)
+    g1, n1 = full_width(sess)
+    gemm_avg = (g1 - g0) / (n1 - n0) if n1 > n0 else tune["ms"] * 1e-3    # none that wide: the tuned one
     out = {"config": "C4", "N": N, "M": M, "Mqc": Mqc, "grm": args.grm, "grm_seconds": grm_s,
            "grm_tflops": grm_tflops if args.grm != "bf16_split" else None,
            "grm_GB": 4.0 * (N + 255) // 256 * 256 * ((N + 255) // 256 * 256) / 1e9,
@@ -439,7 +445,7 @@ def c4_leg(args):
            "variance_ratios": [row[0] for row in vr["table"]], "vr_markers": [len(r) for r in vr["ratios"]],
            "gemm_avg_ms": gemm_avg * 1e3, "gemm_tflops": 2.0 * N * N * 64 / gemm_avg / 1e12,
            # bytes of S a product must read: its lower triangle in that mode
-           "gemm_hbm_GBs": (2.0 if args.gemm_mode == "bf16x3_tri" else 4.0) * N * N / gemm_avg / 1e9,
+           "gemm_hbm_GBs": (tri_bytes(sess) if args.gemm_mode == "bf16x3_tri" else 4.0) * N * N / gemm_avg / 1e9,
            "gemm_mode": args.gemm_mode, "gemm_autotune": tune}
     log(f"C4: fit {t1 - t0:.1f}s theta {fit['theta']}, VR {t2 - t1:.1f}s ratios {out['variance_ratios']}")
     print(json.dumps(out))
@@ -550,16 +556,20 @@ def main():
     # (saige_fit_null_batch), the path an R or C++ caller reaches
     for _ in range(args.warmup):
         native_step()
-    g0, n0_ = sess.engine_stats("gemm_full")
+    w0, l0 = sess.engine_stats("gemm_48")
+    g0, n0_ = full_width(sess)
     h0, m0 = sess.engine_stats("gemm_half")
     q0_, k0 = sess.engine_stats("gemm_quarter")
     t0 = time.perf_counter()
     for _ in range(args.steps):
         nat = native_step()
     t1 = time.perf_counter()
-    g1, n1 = sess.engine_stats("gemm_full")
+    w1, l1 = sess.engine_stats("gemm_48")
+    g1, n1 = full_width(sess)
     h1, m1 = sess.engine_stats("gemm_half")
     q1_, k1 = sess.engine_stats("gemm_quarter")
+    wide_launches = l1 - l0
+    wide_avg = (w1 - w0) / max(1, wide_launches)
     half_launches = m1 - m0
     half_avg = (h1 - h0) / max(1, half_launches)
     quarter_launches = k1 - k0
@@ -568,14 +578,15 @@ def main():
     fits = len(jobs) * args.steps
     fits_per_hour = fits / (t1 - t0) * 3600.0
     gemm_launches = n1 - n0_
-    gemm_avg = (g1 - g0) / max(1, gemm_launches)
+    # no launch that wide: the tuned one's time
+    gemm_avg = (g1 - g0) / gemm_launches if gemm_launches else tune["ms"] * 1e-3
     gemm_flop = 2.0 * N * N * 64
     gemm_tflops = gemm_flop / gemm_avg / 1e12
     nat_s = step_s
     log(f"C++ drivers (saige_fit_null_batch): {step_s:.3f}s/step, {fits_per_hour:.1f} fits/h, {gemm_launches} "
-        f"64-column GEMMs avg {gemm_avg * 1e3:.2f} ms ({gemm_tflops:.1f} TFLOP/s), {half_launches} 32-column GEMMs "
-        f"avg {half_avg * 1e3:.2f} ms, {quarter_launches} 16-column GEMMs avg {quarter_avg * 1e3:.2f} ms "
-        f"({(g1 - g0 + h1 - h0 + q1_ - q0_) / args.steps:.3f}s of GEMM per step), theta "
+        f"64-column GEMMs avg {gemm_avg * 1e3:.2f} ms ({gemm_tflops:.1f} TFLOP/s), {wide_launches} 48-column GEMMs "
+        f"avg {wide_avg * 1e3:.2f} ms, {half_launches} 32-column GEMMs avg {half_avg * 1e3:.2f} ms, {quarter_launches} 16-column GEMMs avg {quarter_avg * 1e3:.2f} ms "
+        f"({(g1 - g0 + w1 - w0 + h1 - h0 + q1_ - q0_) / args.steps:.3f}s of GEMM per step), theta "
         f"{[list(np.round(r['theta'], 4)) for r in nat]}")
 
     # the same rounds through the Python drivers and scheduler (the
@@ -635,10 +646,10 @@ def main():
         plain_s = time.perf_counter() - tp
         g3, n3 = sess.engine_stats("gemv")
         gemv_avg = (g3 - g2) / max(1, n3 - n2)
-        # GB/s of S the product needs: its lower triangle (2 N^2 bytes; three
-        # bytes a value, 1.5 N^2, on the split GRM) in the default mode, all of
-        # it (4 N^2) in the "full" one
-        gemv_bytes = (4.0 if sess.gemv_mode() != "tri" else tri_bytes(sess.grm_precision())) * N * N
+        # GB/s of S the product needs: its lower triangle (2 N^2 bytes; 1.5 N^2
+        # where the split GRM has its three-byte copy) in the default mode, all
+        # of it (4 N^2) in the "full" one
+        gemv_bytes = (4.0 if sess.gemv_mode() != "tri" else tri_bytes(sess)) * N * N
         plain = {"seconds": plain_s, "fits_per_hour": 3600.0 / plain_s, "pcg_iters": pr["pcg_iters"],
                  "grm_products": pr["pcg_iters"] + pr["n_products"],
                  "n_solves": pr["n_solves"], "gemv_ms": gemv_avg * 1e3, "gemv_mode": sess.gemv_mode(),
@@ -750,6 +761,8 @@ def main():
 
     sess.free_device(dev)
     traffic = PROFILED_GEMM_TRAFFIC.get((args.gemm_mode, N, tune["rt"], tune["pd"], tune["nsplit"]))
+    if args.gemm_mode == "bf16x3_tri" and sess.grm_triangle_bytes() != 3:
+        traffic = None                                   # profiled on the three-byte copy
     common = {"traffic": traffic,
               "traffic_source": PROFILE_FILES[args.gemm_mode] + " (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE)",
               "avg_launch_ms": gemm_avg * 1e3, "launches": gemm_launches}
@@ -767,6 +780,7 @@ def main():
     roofline = {"bound": "mfma", "achieved": gemm_tflops, "peak": FP32_MFMA_PEAK, "unit": "TFLOP/s",
                 "frac": gemm_tflops / FP32_MFMA_PEAK,
                 "algorithmic": f"2*N^2*64 = {gemm_flop:.3e} FP32 flop per launch (64 right-hand sides)",
+                "width_48": narrow(wide_avg, wide_launches, 48),
                 "half_width": narrow(half_avg, half_launches, 32),
                 "quarter_width": narrow(quarter_avg, quarter_launches, 16), **common}
     if args.gemm_mode == "fp32":
@@ -779,7 +793,7 @@ def main():
         roofline["kernel"] = ("k_split_p + k_gemm_t16 + k_tri_reduce + k_gemm_epi (block-PCG GRM x 64 RHS from "
                               "the lower triangle on 16x16x32 MFMA tiles, P as three BF16 pieces, S as " +
                               ("two (the split GRM's 16-bit values)" if npc == 5 else "three") + ")")
-        tb = tri_bytes(sess.grm_precision())
+        tb = tri_bytes(sess)
         roofline["bytes"] = f"{tb:g}*N^2 = {tb * N * N:.3e} B of S's lower triangle per launch"
         roofline["hbm_GBs_of_triangle"] = tb * N * N / gemm_avg / 1e9
         roofline["bf16_piece_products"] = {"tflops": npc * gemm_flop / gemm_avg / 1e12, "peak": BF16_MFMA_PEAK,

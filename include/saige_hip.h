@@ -422,6 +422,7 @@ int64_t saige_engine_system_bytes(const saige_ctx* ctx);
                                      triangle) 48 of them                        */
 #define SAIGE_LAUNCH_GEMM_QUARTER 3 /* lower-triangle block GEMM over 16 columns
                                      (at most 16 occupied slots, anywhere)       */
+#define SAIGE_LAUNCH_GEMM_48 4    /* those of SAIGE_LAUNCH_GEMM_FULL over 48 columns */
 int saige_engine_stats(const saige_ctx* ctx, int kind, double* gemm_seconds, int64_t* gemm_launches);
 
 /* ------------------------------------------------------- synthetic data */

@@ -573,6 +573,10 @@ int engine_step(saige_ctx* c, Engine& e, int n_iter, uint8_t* done_out, int32_t*
                                        : SAIGE_LAUNCH_GEMM_HALF;
         e.gemm_seconds[kind] += ms * 1e-3;
         e.gemm_launches[kind]++;
+        if (narrow && nc.width == 48) {
+            e.gemm_seconds[SAIGE_LAUNCH_GEMM_48] += ms * 1e-3;
+            e.gemm_launches[SAIGE_LAUNCH_GEMM_48]++;
+        }
     }
     for (int k = 0; k < e.kpad; k++) {
         if (done_out) done_out[k] = e.h_live[k] ? e.host.done[k] : 1;
@@ -2305,7 +2309,7 @@ int saige_engine_stats(const saige_ctx* c, int kind, double* secs, int64_t* laun
         set_error("null context");
         return SAIGE_E_ARG;
     }
-    if (kind < 0 || kind > 3) {
+    if (kind < 0 || kind > SAIGE_LAUNCH_GEMM_48) {
         set_error("unknown launch kind %d", kind);
         return SAIGE_E_ARG;
     }

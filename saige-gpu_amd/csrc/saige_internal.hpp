@@ -213,9 +213,10 @@ struct Engine {
     int32_t* h_slot_sys = nullptr;
     uint8_t* h_live = nullptr;
     // device time of the GRM product launches by kind: [1] GEMM over one
-    // 32-column half, [2] GEMM over both halves, [3] over 16 columns
-    double gemm_seconds[4] = {0.0, 0.0, 0.0, 0.0};   // by SAIGE_LAUNCH_* kind
-    int64_t gemm_launches[4] = {0, 0, 0, 0};
+    // 32-column half, [2] GEMM over both halves, [3] over 16 columns, [4] those
+    // of [2] over 48
+    double gemm_seconds[5] = {0.0, 0.0, 0.0, 0.0, 0.0};   // by SAIGE_LAUNCH_* kind
+    int64_t gemm_launches[5] = {0, 0, 0, 0, 0};
 };
 
 // A device block that outlives the cohort it was made for (a context reads

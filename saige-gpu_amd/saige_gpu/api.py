@@ -523,14 +523,14 @@ class Session:
 
     def engine_stats(self, kind=None):
         """Device seconds and launch count of the GRM product launches: for one
-        kind ("gemv", "gemm_half", "gemm_full", "gemm_quarter") or summed over
-        all."""
+        kind ("gemv", "gemm_half", "gemm_full", "gemm_quarter", or "gemm_48",
+        those of "gemm_full" over 48 columns) or summed over all."""
         kinds = self.LAUNCH_KINDS if kind is None else (kind,)
         tot_s, tot_n = 0.0, 0
         for k in kinds:
             s = ctypes.c_double(0.0)
             n = ctypes.c_int64(0)
-            check(self._L.saige_engine_stats(self.ctx, self.LAUNCH_KINDS.index(k), ctypes.byref(s),
+            check(self._L.saige_engine_stats(self.ctx, (self.LAUNCH_KINDS + ("gemm_48",)).index(k), ctypes.byref(s),
                                              ctypes.byref(n)))
             tot_s += float(s.value)
             tot_n += int(n.value)
