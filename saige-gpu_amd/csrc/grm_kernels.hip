@@ -53,9 +53,8 @@ __device__ __forceinline__ float round16(float x) {
 // Store a wave's block of 32*MI rows from row0 and 32*NI columns from col0,
 // mirrored for off-diagonal tiles; accumulate: +1 S = S0 + block, -1 S = S0 -
 // block (LOCO: one chromosome's markers left out), 0 store.  S0 may be S.
-// center: the column's value taken off each sum first, in rows below `rows` (the
-// padded ones stay zero); nullptr: none.  R16: the stored values (after the add or
-// subtract) rounded by round16.
+// center: the column's value taken off each sum first (nullptr: none).  R16:
+// the stored values (after the add or subtract) rounded by round16.
 // Accumulator layout of a 32x32 MFMA block: lane l, register r holds row
 // 8*(r/4) + 4*(l/32) + (r%4), column l%32.  A block's S0 values are requested
 // before the block ahead of it is stored (no entry that is read is stored by
@@ -74,8 +73,8 @@ constexpr int S24_SCRATCH = 32 * S24_PITCH;
 template <int MI, int NI, bool R16>
 __device__ __forceinline__ void store_block(float* S, const float* S0, int64_t ldS, int64_t row0, int64_t col0,
                                             bool mirror, int lane, const f32x16 (&acc)[MI][NI], int accumulate,
-                                            const float* center = nullptr, int64_t rows = 0,
-                                            uint8_t* s24 = nullptr, float* scratch = nullptr) {
+                                            const float* center = nullptr, uint8_t* s24 = nullptr,
+                                            float* scratch = nullptr) {
     float s0[2][16];
     auto request = [&](int k) {
         const float* p = S0 + (row0 + k / NI * 32 + 4 * (lane >> 5)) * ldS + col0 + k % NI * 32 + (lane & 31);
@@ -95,7 +94,7 @@ __device__ __forceinline__ void store_block(float* S, const float* S0, int64_t l
             float v[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                v[e] = center && row + e < rows ? acc[mi][ni][4 * g + e] - cc : acc[mi][ni][4 * g + e];
+                v[e] = center ? acc[mi][ni][4 * g + e] - cc : acc[mi][ni][4 * g + e];
                 if (accumulate > 0) v[e] = s0[k & 1][4 * g + e] + v[e];
                 else if (accumulate < 0) v[e] = s0[k & 1][4 * g + e] - v[e];
                 if (R16) v[e] = round16(v[e]);
@@ -542,7 +541,7 @@ __global__ __launch_bounds__(syrk_pk_threads(T)) void k_syrk_pk(const uint8_t* _
     static_assert(sizeof(s1) >= sizeof(float) * S24_SCRATCH * (T == 256 ? 8 : 4), "");
     auto store = [&]() {
         store_block<MI, NI, F == SYRK_SPLIT>(S, S0, ldS, bi * T + wr * 32 * MI, bj * T + wc * 32 * NI, bi != bj, lane,
-                                             acc, accumulate, F == SYRK_FP32 ? tb.center : nullptr, tb.rows, s24,
+                                             acc, accumulate, F == SYRK_FP32 ? tb.center : nullptr, s24,
                                              reinterpret_cast<float*>(s1) + wv * S24_SCRATCH);
     };
     int64_t kc = k0;
@@ -770,12 +769,16 @@ __global__ __launch_bounds__(256) void k_center_sum(const double* __restrict__ p
 // GRM's cross terms add hi.lo and lo.hi to the two mirror entries of a
 // diagonal tile in opposite orders; this keeps S exactly symmetric, with the
 // lower triangle's values, as off-diagonal tiles are mirrored.  Block (t, r):
-// row r of tile t; its threads write column r of the upper part.
-__global__ __launch_bounds__(256) void k_mirror_diag(float* __restrict__ S, int64_t ld, int T) {
+// row r of tile t; its threads write column r of the upper part.  Rows and
+// columns from `rows` on (ld: none) are set to zero: the FP32 form's store takes
+// the columns' centers off the padded rows' zeros too (leaving them out there
+// took the SYRK of 5003 samples 8 us of 1350, here it takes 1.3).
+__global__ __launch_bounds__(256) void k_mirror_diag(float* __restrict__ S, int64_t ld, int T, int64_t rows) {
     const int64_t t = blockIdx.x, r = blockIdx.y;
-    const int64_t base = t * T;
+    const int64_t base = t * T, i = base + r;
     for (int64_t c = threadIdx.x; c < r; c += blockDim.x)
-        S[(base + c) * ld + base + r] = S[(base + r) * ld + base + c];
+        S[(base + c) * ld + i] = i < rows ? S[i * ld + base + c] : 0.0f;
+    for (int64_t c = (i < rows ? rows : 0) + threadIdx.x; c < ld; c += blockDim.x) S[i * ld + c] = 0.0f;
 }
 
 // out[nr][nc] = S[r0 + i][c0 + j] / m, rounded once (div_rn): the read-back of a
@@ -834,6 +837,7 @@ hipError_t SyrkOperands::build(hipStream_t s, int form_, const uint8_t* packed, 
     const OperandParts q(form, Npad, j0, j1);
     const int64_t c0 = q.c0, npanel = q.npanel, n = q.n, nsl = q.nsl;
     nchunk = q.nchunk;
+    rows = Nnm;
     hipError_t e = hipMalloc(&block, (size_t)q.total);
     if (e != hipSuccess) {
         block = nullptr;
@@ -847,7 +851,6 @@ hipError_t SyrkOperands::build(hipStream_t s, int form_, const uint8_t* packed, 
     if (nsl) {
         tb.corr = reinterpret_cast<double*>(p);
         tb.center = reinterpret_cast<float*>(p + q.cor);
-        tb.rows = Nnm;
         part = reinterpret_cast<double*>(p + q.cor + q.cen);
     }
     hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)((npanel + 3) / 4), (unsigned)nchunk), dim3(256), 0, s, packed,
@@ -904,13 +907,15 @@ hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* til
     hipError_t e = hipGetLastError();
     // the multi-piece forms reach a diagonal tile's two mirror entries by
     // different sums: keep S exactly symmetric
-    if (e == hipSuccess && op.form != SYRK_HI) e = launch_mirror_diag(s, S, op.Npad, tile);
+    if (e == hipSuccess && op.form != SYRK_HI)
+        e = launch_mirror_diag(s, S, op.Npad, tile, op.form == SYRK_FP32 ? op.rows : op.Npad);
     return e;
 }
 
-hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile) {
+hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile, int64_t rows) {
     if (tile <= 0 || Npad % tile != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_mirror_diag, dim3((unsigned)(Npad / tile), (unsigned)tile), dim3(256), 0, s, S, Npad, tile);
+    hipLaunchKernelGGL(k_mirror_diag, dim3((unsigned)(Npad / tile), (unsigned)tile), dim3(256), 0, s, S, Npad, tile,
+                       rows);
     return hipGetLastError();
 }
 

@@ -251,7 +251,6 @@ struct SyrkTables {
     uint64_t* t[4] = {nullptr, nullptr, nullptr, nullptr};
     double* corr = nullptr;        // [markers][3]
     float* center = nullptr;       // [Npad]
-    int64_t rows = 0;              // the samples: rows that have a center taken off
 };
 
 // The operands of a 2-bit-input SYRK over markers [j0, j1): the genotypes
@@ -262,7 +261,7 @@ enum SyrkForm { SYRK_HI = 0, SYRK_SPLIT = 1, SYRK_FP32 = 2 };
 struct SyrkOperands {
     void* block = nullptr;
     int form = SYRK_HI;
-    int64_t Npad = 0, nchunk = 0;
+    int64_t Npad = 0, nchunk = 0, rows = 0;          // rows: the samples
     uint8_t* tp = nullptr;
     SyrkTables tb;
     hipError_t build(hipStream_t s, int form, const uint8_t* packed, const float4* lut, int64_t Mqc, int64_t Nnm,
@@ -441,8 +440,9 @@ __host__ __device__ __forceinline__ int64_t s24_block(int64_t I, int64_t J) { re
 hipError_t launch_syrk_pk(hipStream_t s, const SyrkOperands& op, const int2* tiles, float* S, const float* S0,
                           int accumulate, int tile, uint8_t* s24);
 int syrk_pk_tile(int64_t Npad, int form);
-// copy each diagonal tile's lower half onto its upper half (tile edge `tile`)
-hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile);
+// copy each diagonal tile's lower half onto its upper half (tile edge `tile`);
+// rows and columns from `rows` on set to zero
+hipError_t launch_mirror_diag(hipStream_t s, float* S, int64_t Npad, int tile, int64_t rows);
 // out[nr][nc] (contiguous) = S[i][j] / m for S at its block's first element
 hipError_t launch_grm_block(hipStream_t s, const float* S, int64_t ld, int64_t nr, int64_t nc, float m, float* out);
 hipError_t launch_sub(hipStream_t s, const float* a, const float* b, int64_t n, float* out);
