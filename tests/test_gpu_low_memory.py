@@ -2,6 +2,7 @@
 device is held by untouched allocations while they run."""
 import contextlib
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -16,9 +17,16 @@ def hip_runtime():
 
 
 def free_memory():
+    """Free device memory once it has stopped changing: the driver returns freed
+    blocks some time after the call."""
     f, t = ctypes.c_size_t(), ctypes.c_size_t()
-    assert hip_runtime().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
-    return f.value
+    last, same = -1, 0
+    while same < 8:
+        assert hip_runtime().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        same = same + 1 if f.value == last else 0
+        last = f.value
+        time.sleep(0.02)
+    return last
 
 
 @contextlib.contextmanager
@@ -27,17 +35,24 @@ def only_free(left):
     hip = hip_runtime()
     hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
     hip.hipFree.argtypes = [ctypes.c_void_p]
-    held, piece = [], 1 << 38
+
+    def take(n):
+        p = ctypes.c_void_p()
+        return p if hip.hipMalloc(ctypes.byref(p), n) == 0 else None
+
+    # what hipMemGetInfo calls free is less than what can be allocated: hold
+    # `left`, take all there is, let `left` go
+    free_memory()
+    room, held, piece = take(left), [], 1 << 38
     try:
+        assert room
         while piece >= 1 << 22:
-            over = free_memory() - left
-            if over < 1 << 22:
-                break
-            p = ctypes.c_void_p()
-            if over >= piece and hip.hipMalloc(ctypes.byref(p), piece) == 0:
+            p = take(piece)
+            if p:
                 held.append(p)
             else:
                 piece //= 2
+        hip.hipFree(room)
         hip.hipGetLastError()
         yield
     finally:
