@@ -372,7 +372,7 @@ __device__ __forceinline__ float lut_pick(const float4 L, int g) {
 // next tile's loads are in flight while a tile is made.  Markers past the end
 // have zero tables.  1000 x 10,000: 61 us (115 with the same four waves making
 // and adding, 863 with a byte load and two selects per marker and sample);
-// 24,009 x 20,003: 126 us; 100,000 x 150,000: 1.66 ms (1.99, 15.3), where 391
+// 24,008 x 20,003: 126 us; 100,000 x 150,000: 1.66 ms (1.99, 15.3), where 391
 // workgroups load 256 CUs unevenly.
 constexpr int DG_MK = 128;                       // markers per tile
 constexpr int DG_PITCH = DG_MK / 8 + 4;          // dwords per sample

@@ -388,8 +388,8 @@ __global__ __launch_bounds__(512) void k_syrk_pk256(const uint8_t* __restrict__ 
 // half the row operand and the column's lo, the upper half its hi and mid.
 //
 // T: the 256 tile (8 waves of 64 x 128, each decoding too) does the most MFMA
-// work per decoded value and is bound by the matrix pipe and its power (split GRM
-// at N = 40,000: 1380 TFLOP/s of BF16 products, the clock at 1.6 GHz); a small
+// work per decoded value (split GRM at N = 40,000, M = 60,000: 1350 TFLOP/s of BF16
+// products, the matrix pipe busy 63% of the cycles at 2.08 GHz); a small
 // GRM has too few of its tiles for 256 CUs, each walking all markers, and takes
 // 128 (4 waves of 64 x 64) or 64 (4 waves of 32 x 32) tiles, see syrk_pk_tile.
 // There a wave has a SIMD to itself and issues one instruction in about seven
