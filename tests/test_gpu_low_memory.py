@@ -188,7 +188,8 @@ def test_three_byte_copy_is_given_back(session, split_grm):
     and the products' bits stay."""
     print("case: the three-byte triangle's memory", flush=True)
     B = split_grm
-    assert session.device_memory()[0] - free_memory() == COPY
+    free = free_memory()
+    assert session.device_memory()[0] - free == COPY
     y = session.getCrossprodMatAndKin(B[:, 0])
     with only_free(64 << 20):
         Y = session.grm_matvec(B)                    # 0.15 GB of scratch on its first call
